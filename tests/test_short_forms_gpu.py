@@ -1,0 +1,51 @@
+"""The whole-solve kernels of the small systems take short forms of the division, the square root, the logarithm and the
+exponential where an iteration's operands are in their ranges, and the general forms otherwise: results at and across the
+edges of those ranges against the scalar C oracle, bit for bit."""
+import pytest
+import torch
+
+import torchode_amd as to
+from helpers import assert_identical, c_oracle_solve, gpu_solve
+
+pytestmark = pytest.mark.gpu
+
+# (tolerances and exponents: inside the ranges; at their edges; absolute tolerance zero or below 2^-40; relative tolerance
+# above 1/16; exponents of the error ratio above 1/2)
+CONTROLLERS = {
+    "inside": dict(kind="pid", atol=1e-6, rtol=1e-4, pcoeff=0.2, icoeff=0.5, dcoeff=0.05),
+    "edge": dict(kind="pid", atol=2.0**-40, rtol=2.0**-4, pcoeff=1.0, icoeff=1.5, dcoeff=0.0),
+    "tiny-atol": dict(kind="integral", atol=1e-13, rtol=1e-4),
+    "large-rtol": dict(kind="integral", atol=1e-4, rtol=0.07),
+    "steep": dict(kind="pid", atol=1e-5, rtol=1e-3, pcoeff=1.2, icoeff=1.6, dcoeff=0.1),
+}
+
+
+@pytest.mark.parametrize("dtype", [torch.float32, torch.float64], ids=["f32", "f64"])
+@pytest.mark.parametrize("controller", CONTROLLERS)
+@pytest.mark.parametrize("name,method", [("vdp", "tsit5"), ("lorenz", "dopri5"), ("linear_decay", "tsit5"), ("linear_decay", "dopri5")])
+def test_ranges_of_the_controller(name, method, controller, dtype):
+    w = to.workloads.make(name, batch=130, dtype=dtype)
+    spec = CONTROLLERS[controller]
+    ref = c_oracle_solve(w.f, w.y0, w.t_eval, method, spec)
+    for fast in ("one", True):
+        assert_identical(gpu_solve(w.f, w.y0, w.t_eval, method, spec, fast=fast), ref)
+
+
+@pytest.mark.parametrize("dtype", [torch.float32, torch.float64], ids=["f32", "f64"])
+@pytest.mark.parametrize("features", [1, 2, 3, 4, 8])
+def test_scaled_errors_of_every_size(features, dtype):
+    """Linear decay from states of 2^-140 ... 2^100 in one wavefront, some exactly zero: scaled errors that are zero, far
+    below and above the range of the short forms, next to ordinary ones; evaluation points from the first step on."""
+    B = 97
+    g = torch.Generator().manual_seed(5)
+    exponent = torch.linspace(-140, 100, B, dtype=torch.float64)[torch.randperm(B, generator=g)]
+    y0 = (torch.randn((B, features), generator=g, dtype=torch.float64) * 2.0 ** exponent[:, None]).to(dtype)
+    y0[::7, 0] = 0.0
+    y0[5] = 0.0
+    f = to.LinearDecay((torch.rand((B, features), generator=g, dtype=torch.float64) * 3 + 0.1).to(dtype))
+    t_eval = (torch.rand((B, 1), generator=g, dtype=torch.float64) * torch.tensor([[0.0, 1e-30, 1e-9, 0.01, 0.3, 0.31, 0.9, 1.0]], dtype=torch.float64)).to(dtype)
+    spec = dict(kind="pid", atol=1e-6, rtol=1e-4, pcoeff=0.2, icoeff=0.5, dcoeff=0.05)
+    for method in ("dopri5", "tsit5"):
+        ref = c_oracle_solve(f, y0, t_eval, method, spec)
+        for fast in ("one", True):
+            assert_identical(gpu_solve(f, y0, t_eval, method, spec, fast=fast), ref)

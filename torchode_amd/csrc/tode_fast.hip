@@ -26,12 +26,16 @@ template <typename T> struct FastOut {
     int64_t *n_steps, *n_accepted, *n_initialized, *status;
 };
 
+// Wavefronts per SIMD that the registers are held to: 64 registers, eight wavefronts, where a kernel needs a few more than
+// that left to itself (Lorenz float32: 69 registers, seven wavefronts; its spills at 64 lie outside the loop).
+constexpr int fast_wavefronts(size_t size, int features, int nhist, bool record) { return size == 4 && features <= 3 && nhist <= 1 && !record ? 8 : 1; }
+
 // NHIST: how many history factors the controller multiplies in (0 integral, 1 PI, 2 PID).
 // RECORD: the loop state before every iteration of the wavefront goes to p.rec_* (tode_solve_record), as the general
 // kernel writes it: entry i is the state before iteration i; a sample that has finished repeats its last state with
 // `running` 0, up to the record's capacity.  A record that is too short raises TODE_FLAG_NEEDS_GENERAL.
 template <typename T, int METHOD, int CTRL, int NHIST, typename Term, bool STAGE_YS, bool RECORD = false>
-__global__ void __launch_bounds__(64) solve_fast_kernel(const SolveParams<T> p, const FastOut<T> o) {
+__global__ void __launch_bounds__(64, fast_wavefronts(sizeof(T), Term::F, NHIST, RECORD)) solve_fast_kernel(const SolveParams<T> p, const FastOut<T> o) {
     using Tab = typename std::conditional<METHOD == 1, Tsit5Tab, Dopri5Tab>::type;
     constexpr int F = Term::F;
     constexpr int P = Term::P;
@@ -77,15 +81,23 @@ __global__ void __launch_bounds__(64) solve_fast_kernel(const SolveParams<T> p, 
     const T dir = fwd ? (T)1 : (T)-1;
     const T tlo = tmin(ts, te), thi = tmax(te, ts);
 
+    // From here on times are multiplied by the sample's direction (+-1: exact), so that "a has reached b" is dir * a >= dir * b
+    // in either direction; behind the last evaluation point lies one that no step reaches (not as another row in LDS: at 20
+    // points a workgroup's rows fill exactly the 1/32 of LDS that eight wavefronts per SIMD leave it).
+    const T never = (T)__builtin_huge_val();
     bool bail = false;
+    const T te_first = te_s[lane];
     {
-        T prev_te = te_s[lane];
+        T prev_te = dir * te_first;
+        te_s[lane] = prev_te;
         for (int e = 1; e < E; ++e) {
-            T cur = te_s[e * 64 + lane];
-            if (!(fwd ? cur >= prev_te : cur <= prev_te)) bail = true;
+            const T cur = dir * te_s[e * 64 + lane];
+            te_s[e * 64 + lane] = cur;
+            if (!(cur >= prev_te)) bail = true;
             prev_te = cur;
         }
     }
+    auto point = [&](int e) -> T { return e < E ? te_s[e * 64 + lane] : never; };
 
     T t = ts, dt;
     if (p.dt0) {
@@ -95,23 +107,22 @@ __global__ void __launch_bounds__(64) solve_fast_kernel(const SolveParams<T> p, 
         dt = initial_step<T, CTRL, Term>(cp, rhs, ts, y, dir, abs_(te - ts), k[0]);
     }
     dt = tclamp(dt, tlo - t, thi - t);
-    // logarithms of the previous two accepted error ratios (both start at 1, log 1 = 0)
     StepFactor<T, NHIST> step_factor;  // with the logarithms of the previous two accepted error ratios (both start at 1)
     int cursor = 0;
-    T *ys_g = p.ys + bs * (long long)EF;
-    if (te_s[lane] == ts) {
+    // (a wavefront's block of ys is far below 4 GiB: launch_fast)
+    T *ys_block = p.ys + b0 * (long long)EF;
+    const unsigned ys_row = (unsigned)(live ? lane : 0) * (unsigned)E;
+    if (te_first == ts) {
 #pragma unroll
         for (int f = 0; f < F; ++f) {
             if (STAGE_YS)
                 ys_s[f * 65 + lane] = y[f];
             else if (live)
-                ys_g[f] = y[f];
+                ys_block[ys_row * F + f] = y[f];
         }
         cursor = 1;
     }
-    // direction-normalised times: multiplying by +-1 is exact, so dir*a >= dir*b decides
-    // "a has reached b in the direction of time" without a branch
-    T dte_next = dir * te_s[(cursor < E ? cursor : E - 1) * 64 + lane];
+    T dte_next = point(cursor);
     const T dte_end = dir * te;
 
     int n_steps = 0, n_acc = 0;
@@ -124,13 +135,12 @@ __global__ void __launch_bounds__(64) solve_fast_kernel(const SolveParams<T> p, 
         for (int f = 0; f < F; ++f) odd_start = odd_start || !finite_(y[f]) || !finite_(k[0][f]);
         bail = bail || (live && odd_start);
     }
-    bool active = live && !bail;
+    // lanes whose sample is still stepping, and lanes whose sample needs the general kernel
+    lanes_t active = lanes_where(live && !bail), bail_lanes = lanes_where(bail);
     const T e1 = (T)cp.e1, e2 = (T)cp.e2, e3 = (T)cp.e3;
     const int step_limit = p.max_steps < TODE_HARD_STEP_LIMIT ? p.max_steps : TODE_HARD_STEP_LIMIT;
 
-    // (RECORD) iterations of this wavefront so far = the record's next entry; the last two accepted error ratios as
-    // values (the step factor keeps their logarithms)
-    long long iteration = 0;
+    // (RECORD) the last two accepted error ratios as values (the step factor keeps their logarithms)
     T ratio_prev = 1, ratio_prev_prev = 1;
     bool record_full = false;
     auto keep = [&](long long at, bool running) {
@@ -146,12 +156,14 @@ __global__ void __launch_bounds__(64) solve_fast_kernel(const SolveParams<T> p, 
     // iterations with the clamped step t_end - t: with evaluation points that is seen only in the status of that step,
     // which is a success unless its error ratio is not finite.  The sample sits through one more iteration here, as
     // an inactive lane whose error ratio is looked at.
-    bool idle = false;
-    while (__any(active || idle)) {
-        if (RECORD) keep(iteration++, active);
+    lanes_t idle = 0;
+    int iteration = 0;  // of this wavefront, so far
+    for (lanes_t counted = active; counted; counted = active | idle) {
+        if (RECORD) keep(iteration, holds(active));
+        ++iteration;
         // ---- stages (runge_kutta.py:255-263) ----
         const T t0 = t;
-        T y1[F], err[F];
+        T y1[F];
 #pragma unroll
         for (int i = 1; i < 7; ++i) {
             T tn = fma_((T)Tab::c[i], dt, t0);
@@ -160,7 +172,8 @@ __global__ void __launch_bounds__(64) solve_fast_kernel(const SolveParams<T> p, 
             for (int f = 0; f < F; ++f) {
                 T s = 0;
 #pragma unroll
-                for (int j = 0; j < i; ++j) s = fma_((T)Tab::a[i][j], k[j][f], s);
+                for (int j = 0; j < i; ++j)
+                    if (Tab::a[i][j] != 0.0) s = fma_((T)Tab::a[i][j], k[j][f], s);  // (a zero weight: weighted_k's FINITE)
                 yi[f] = fma_(dt, s, y[f]);
             }
             rhs(tn, yi, k[i]);
@@ -169,87 +182,80 @@ __global__ void __launch_bounds__(64) solve_fast_kernel(const SolveParams<T> p, 
                 for (int f = 0; f < F; ++f) y1[f] = yi[f];
             }
         }
-        weighted_k<T, F, Tab, -1, true>(dt, k, err);
 
-        // ---- step size control (step_size_controllers.py:370-429, 715-774) ----
-        bool unordered;
-        const T ratio = error_ratio_common<T, F>(cp, y, y1, err, unordered);
-        const bool accept = ratio < (T)1;
-        // a NaN or infinite ratio is a non-success status: leave it to the general kernel (the ratio is at least 1e-38)
-        bool sane = !unordered && ratio < (T)__builtin_huge_val();
-        bail = bail || (idle && !sane);
-        idle = false;
-        T factor = step_factor(cp.safety, sane ? ratio : (T)1, e1, e2, e3, active);
-        sane = sane && factor == factor;  // (a product of an underflowed and an overflowed power)
+        // ---- error estimate and step size control (step_size_controllers.py:370-429, 715-774) ----
+        lanes_t insane;  // (a NaN or infinite ratio is a non-success status: left to the general kernel)
+        T factor;
+        const T ratio = control_common<T, F, NHIST, Tab>(cp, dt, k, y, y1, counted, step_factor, e1, e2, e3, factor, insane);
+        const lanes_t accept = lanes_where(ratio < (T)1), move = accept & active;
+        bail_lanes |= idle & insane;
+        idle = 0;
         factor = clamp_ordered(factor, cp.fmin, cp.fmax);
         const T dt_next = dt * factor;
 
-        const bool move = accept && active;
-        const T t_new = move ? (t0 + dt) : t0;
-        const T dt_new = dir * t_new;
-        const bool running_new = dt_new < dte_end;
-        n_steps += active ? 1 : 0;
-        n_acc += move ? 1 : 0;
+        t = holds(move) ? (t0 + dt) : t0;
+        const T dt_new = dir * t;
+        const lanes_t running = lanes_where(dt_new < dte_end);
+        n_acc += holds(move) ? 1 : 0;
 
         // ---- dense output (adjoints.py:215-234) ----
-        bool hit = active && cursor < E && dt_new >= dte_next;
-        if (__any(hit)) {
+        if (holds(active) && dt_new >= dte_next) {
             T q[5][F];
-            quartic<T, F, METHOD>(dt, y, y1, k, q);
-            do {
-                T out[F];
-                quartic_eval<T, F>(q, t0, dt, dir * dte_next, out);
-                if (hit) {
+            quartic<T, F, METHOD, true>(dt, y, y1, k, q);
+            const StepPosition<T> position(t0, dt);
+            auto write_points = [&](auto plain) {
+                do {
+                    T out[F];
+                    quartic_at_unit<T, F>(q, position.template at<decltype(plain)::value>(dir, dte_next), out);
+                    T *row = ys_block + (ys_row + (unsigned)cursor) * F;
 #pragma unroll
                     for (int f = 0; f < F; ++f) {
                         if (STAGE_YS)
                             ys_s[(cursor * F + f) * 65 + lane] = out[f];
                         else
-                            ys_g[cursor * F + f] = out[f];
+                            row[f] = out[f];
                     }
-                }
-                cursor += hit ? 1 : 0;
-                const T nxt = dir * te_s[(cursor < E ? cursor : E - 1) * 64 + lane];
-                dte_next = hit ? nxt : dte_next;
-                hit = hit && cursor < E && dt_new >= dte_next;
-            } while (__any(hit));
+                    ++cursor;
+                    dte_next = point(cursor);
+                } while (dt_new >= dte_next);
+            };
+            if (position.plain == lanes_where(true))
+                write_points(std::true_type());
+            else
+                write_points(std::false_type());
         }
 
         // ---- state update (adjoints.py:150-155, 247-255) ----
 #pragma unroll
         for (int f = 0; f < F; ++f) {
-            y[f] = move ? y1[f] : y[f];
-            k[0][f] = move ? k[6][f] : k[0][f];
+            y[f] = holds(move) ? y1[f] : y[f];
+            k[0][f] = holds(move) ? k[6][f] : k[0][f];
         }
-        t = t_new;
-        {
-            const T dtn = running_new ? dt_next : dt;
-            const T dtc = clamp_ordered(dtn, tlo - t, thi - t);
-            dt = active ? dtc : dt;
-        }
-        if (NHIST >= 1) step_factor.shift(active && running_new && accept);
+        // (a finished sample no longer runs: its step stays what this clamp made it)
+        dt = clamp_ordered(holds(running) ? dt_next : dt, tlo - t, thi - t);
+        if (NHIST >= 1) step_factor.shift(holds(running & accept));
         if (RECORD && CTRL == 1) {
-            const bool shift = active && running_new && accept;
+            const bool shift = holds(running & accept);
             ratio_prev_prev = shift ? ratio_prev : ratio_prev_prev;
             ratio_prev = shift ? ratio : ratio_prev;
         }
-        {
-            // non-finite error ratio or max_steps reached: not the common case
-            const bool failed = active && (!sane || n_steps >= step_limit);
-            const bool finished = active && !failed && !running_new;
-            if (__any(finished)) {
-                // a sample whose state or derivative at the end is not finite shows up in later iterations of the
-                // reference loop with another status; one that landed past t_end is looked at in the next iteration
-                bool odd = false;
+        // non-finite error ratio or max_steps reached: not the common case
+        const lanes_t failed = active & (iteration >= step_limit ? ~(lanes_t)0 : insane);
+        const lanes_t ended = active & (failed | ~running);
+        if (ended) {
+            n_steps = holds(ended) ? iteration : n_steps;
+            // a sample whose state or derivative at the end is not finite shows up in later iterations of the
+            // reference loop with another status; one that landed past t_end is looked at in the next iteration
+            bool odd = false;
 #pragma unroll
-                for (int f = 0; f < F; ++f) odd = odd || !settles_(y[f], k[0][f]);
-                bail = bail || (finished && odd);
-                idle = finished && !odd && !(t == te);
-            }
-            bail = bail || failed;
-            active = active && !failed && running_new;
+            for (int f = 0; f < F; ++f) odd = odd || !settles_(y[f], k[0][f]);
+            const lanes_t finished = ended & ~failed, odd_lanes = lanes_where(odd);
+            bail_lanes |= failed | (finished & odd_lanes);
+            idle = finished & ~odd_lanes & ~lanes_where(t == te);
+            active &= ~ended;
         }
     }
+    bail = holds(bail_lanes);
 
     if (live) {
         o.n_steps[b] = n_steps;

@@ -117,32 +117,117 @@ __device__ __forceinline__ float pow2i(float, int q) { return __int_as_float((q 
 __device__ __forceinline__ double pow2i(double, int q) { return __longlong_as_double((long long)(q + 0x3ff) << 52); }
 template <typename T> __device__ __forceinline__ T ldexp2k(T d, int e) { return d * pow2i(T(0), e >> 1) * pow2i(T(0), e - (e >> 1)); }
 
+// ---------------------------------------------------------------------------
+// The correctly rounded quotient, reciprocal, square root and power of two without the scaling and
+// the special cases of the general forms, for operands that are known to need neither: a Newton step
+// on the hardware's estimate and one correction through the exact (fused) remainder.  A loop
+// iteration of the small systems holds three to four divisions, a square root and two powers, and
+// runs at the rate at which a SIMD issues vector instructions: 11 -> 6 instructions per float32
+// division, 11 -> 3 for the logarithm's reciprocal, 17 -> 5 per square root, 7 -> 1 per power of two.
+// Same values, by proof or exhaustively:
+//  * float32 reciprocal, square root: equal to 1 / x and sqrt(x) for every mantissa (1 <= x < 4, checked on
+//    the hardware; both scale exactly with even powers of two while nothing underflows);
+//  * float32 quotient: r is the correctly rounded reciprocal, n * r is less than two units off, and the
+//    corrected quotient errs by less than 2^-22 units before its rounding.  The mantissa pairs whose
+//    quotient lies that close to a rounding boundary are those with 2^k n = (2j + 1) d + s, |s| <= 8:
+//    all of them (to |s| = 32) were enumerated, none is rounded to the wrong side;
+//  * float64: the iterations that the general forms run on operands they do not have to scale.
+// Measured with the lane conditions below, on whole solves: Van der Pol float32 B = 65536 (tode_pair.hip) 0.147 -> 0.121 ms,
+// float64 B = 20011 0.175 -> 0.145 ms; Lorenz float32 B = 40009 0.063 -> 0.052 ms, B = 1 048 576 (tode_fast.hip, eight
+// wavefronts per SIMD, where additions and products are issued at twice the rate of what was removed) 0.51 -> 0.50 ms.
+// Ranges: quotient d in [2^-40, 2^124], n = 0 or n / d in [2^-60, 2^60] (remainders exact, no intermediate
+// result subnormal); root in [2^-100, 2^100]; reciprocal in [1, 4).
+// ---------------------------------------------------------------------------
+__device__ __forceinline__ float reciprocal_plain(float x) {
+    const float r = __builtin_amdgcn_rcpf(x);
+    return fma_(fma_(-x, r, 1.0f), r, r);
+}
+__device__ __forceinline__ double reciprocal_estimate(double x) {
+    double r = __builtin_amdgcn_rcp(x);
+    r = fma_(fma_(-x, r, 1.0), r, r);
+    return fma_(fma_(-x, r, 1.0), r, r);
+}
+__device__ __forceinline__ double reciprocal_plain(double x) {
+    const double r = reciprocal_estimate(x);
+    return fma_(fma_(-x, r, 1.0), r, r);
+}
+__device__ __forceinline__ float reciprocal_estimate(float x) { return reciprocal_plain(x); }
+// n / d from n, d and reciprocal_estimate(d)
+template <typename T> __device__ __forceinline__ T quotient_with(T n, T d, T r) {
+    const T q = n * r;
+    return fma_(fma_(-d, q, n), r, q);
+}
+template <typename T> __device__ __forceinline__ T quotient_plain(T n, T d) { return quotient_with(n, d, reciprocal_estimate(d)); }
+__device__ __forceinline__ float sqrt_plain(float a) {
+    const float y = __builtin_amdgcn_rsqf(a), g = a * y, h = 0.5f * y;
+    return fma_(fma_(-g, g, a), h, g);
+}
+__device__ __forceinline__ double sqrt_plain(double a) {
+    const double y = __builtin_amdgcn_rsq(a);
+    double g = a * y, h = y * 0.5;
+    const double r = fma_(-h, g, 0.5);
+    g = fma_(g, r, g);
+    h = fma_(h, r, h);
+    g = fma_(fma_(-g, g, a), h, g);
+    return fma_(fma_(-g, g, a), h, g);
+}
+__device__ __forceinline__ float ldexp_plain(float x, int q) { return __builtin_amdgcn_ldexpf(x, q); }
+__device__ __forceinline__ double ldexp_plain(double x, int q) { return __builtin_amdgcn_ldexp(x, q); }
+
+// Conditions of a wavefront's lanes as one scalar: the logic of a loop that the whole wavefront runs together -- who still
+// steps, who moved, who ended -- is then a handful of scalar instructions, where conditions kept per lane across branches
+// cost the compiler's merges of lane masks (60 of them per iteration of the stepper loop, 25 this way).
+typedef unsigned long long lanes_t;
+__device__ __forceinline__ lanes_t lanes_where(bool c) { return __builtin_amdgcn_ballot_w64(c); }
+__device__ __forceinline__ bool holds(lanes_t lanes) { return __builtin_amdgcn_inverse_ballot_w64(lanes); }
+
+// The double-word sums below in which the low part is known: with the larger operand first the exact error of a sum takes
+// two more operations instead of five, and a difference of two values within a factor two of each other has none.
+template <typename T> __device__ __forceinline__ DW<T> dw_add2_ordered(T larger, DW<T> y) {  // |larger| >= |y.x|
+    const T s = larger + y.x;
+    return dw(s, (y.x - (s - larger)) + y.y);
+}
+
+// (m - 1) / (m + 1) as a double-word, 0.74 < m < 1.51.  PLAIN: m - 1 is exact, the error of m + 1 is m - ((m + 1) - 1), and
+// the division's reciprocal, of an operand in [1.74, 2.51], takes its short form.
+template <bool PLAIN, typename T> __device__ __forceinline__ DW<T> log_argument(T m) {
+    if (!PLAIN) return dw_div(dw_add2((T)-1, m), dw_add2((T)1, m));
+    const T n = m - (T)1, d = m + (T)1, dl = m - (d - (T)1);
+    const T t = reciprocal_plain(d);
+    const T s = n * t, u = fmapn(t, n, s), v = fmanp(dl, t, fmanp(d, t, (T)1));
+    return dw(s, fma_(s, v, u));
+}
+
+// PLAIN: d is a normal number.
 // log of a positive finite d as a double-word
-__device__ __forceinline__ DW<float> logk(float d) {
-    const bool o = d < 1.17549435e-38f;
+template <bool PLAIN = false> __device__ __forceinline__ DW<float> logk(float d) {
+    const bool o = !PLAIN && d < 1.17549435e-38f;
     d = o ? d * 18446744073709551616.0f : d;  // 2^64
     const float d43 = d * (1.0f / 0.75f);
     int e = ((__float_as_int(d43) >> 23) & 0xff) - 0x7f;
     const float m = __int_as_float(__float_as_int(d) - (e << 23));  // d * 2^-e
     e = o ? e - 64 : e;
-    DW<float> x = dw_div(dw_add2(-1.0f, m), dw_add2(1.0f, m));
-    DW<float> x2 = dw_squ(x);
+    const DW<float> x = log_argument<PLAIN>(m);
+    const DW<float> x2 = dw_squ(x);
     float t = 0.240320354700088500976562f;
     t = fma_(t, x2.x, 0.285112679004669189453125f);
     t = fma_(t, x2.x, 0.400007992982864379882812f);
     const DW<float> c = dw(0.66666662693023681640625f, 3.69183861259614332084311e-09f);
     DW<float> s = dw_mul(dw(0.69314718246459960938f, -1.904654323148236017e-09f), (float)e);
     s = dw_add(s, dw_scale(x, 2.0f));
-    s = dw_add(s, dw_mul(dw_mul(x2, x), dw_add2(dw_mul(x2, t), c)));
+    const DW<float> xt = dw_mul(x2, t);  // (at most 0.017)
+    const DW<float> p = PLAIN ? dw_add2_ordered(c.x, dw(xt.x, xt.y + c.y)) : dw_add2(xt, c);
+    s = dw_add(s, dw_mul(dw_mul(x2, x), p));
     return s;
 }
 
-// exp of a double-word
-__device__ __forceinline__ float expk(DW<float> d) {
+// exp of a double-word.  PLAIN: |d| is at most 60, so that neither end of the range is near.
+template <bool PLAIN = false> __device__ __forceinline__ float expk(DW<float> d) {
     float u = (d.x + d.y) * 1.442695040888963407359924681001892137426645954152985934135449406931f;
     const float fq = __builtin_rintf(u);
     const int q = (int)fq;
-    DW<float> s = dw_add2(d, fq * -0.693145751953125f);
+    // (15 bits times a small integer: an exact product.  PLAIN: and one that lies within a factor two of d, or is zero)
+    DW<float> s = PLAIN ? dw(fma_(fq, -0.693145751953125f, d.x), d.y) : dw_add2(d, fq * -0.693145751953125f);
     s = dw_add2(s, fq * -1.428606765330187045e-06f);
     s = dw_normalize(s);
     u = 0.00136324646882712841033936f;
@@ -153,19 +238,20 @@ __device__ __forceinline__ float expk(DW<float> d) {
     DW<float> t = dw_add(s, dw_mul(dw_squ(s), u));
     t = dw_add(1.0f, t);
     u = t.x + t.y;
+    if (PLAIN) return ldexp_plain(u, q);
     u = ldexp2k(u, q);
     return d.x < -104.0f ? 0.0f : u;
 }
 
 // ---- double ----
-__device__ __forceinline__ DW<double> logk(double d) {
-    const bool o = d < 2.2250738585072014e-308;
+template <bool PLAIN = false> __device__ __forceinline__ DW<double> logk(double d) {
+    const bool o = !PLAIN && d < 2.2250738585072014e-308;
     d = o ? d * 18446744073709551616.0 : d;
     const double d43 = d * (1.0 / 0.75);
     int e = (int)((__double2hiint(d43) >> 20) & 0x7ff) - 0x3ff;
     const double m = __hiloint2double(__double2hiint(d) - (e << 20), __double2loint(d));
     e = o ? e - 64 : e;
-    DW<double> x = dw_div(dw_add2(-1.0, m), dw_add2(1.0, m));
+    DW<double> x = log_argument<PLAIN>(m);
     DW<double> x2 = dw_squ(x);
     const double z = x2.x, z2 = z * z, z4 = z2 * z2, z8 = z4 * z4;
     const double p01 = fma_(z, 0.285714285714249172087875, 0.400000000000000077715612);
@@ -184,11 +270,11 @@ __device__ __forceinline__ DW<double> logk(double d) {
     return s;
 }
 
-__device__ __forceinline__ double expk(DW<double> d) {
+template <bool PLAIN = false> __device__ __forceinline__ double expk(DW<double> d) {
     double u = (d.x + d.y) * 1.442695040888963407359924681001892137426645954152985934135449406931;
     const double dq = __builtin_rint(u);
     const int q = (int)dq;
-    DW<double> s = dw_add2(d, dq * -.69314718055966295651160180568695068359375);
+    DW<double> s = PLAIN ? dw(fma_(dq, -.69314718055966295651160180568695068359375, d.x), d.y) : dw_add2(d, dq * -.69314718055966295651160180568695068359375);
     s = dw_add2(s, dq * -.28235290563031577122588448175013436025525412068e-12);
     s = dw_normalize(s);
     const double z = s.x, z2 = z * z, z4 = z2 * z2, z8 = z4 * z4;
@@ -202,6 +288,7 @@ __device__ __forceinline__ double expk(DW<double> d) {
     DW<double> t = dw_add(1.0, s);
     t = dw_add(t, dw_mul(dw_squ(s), u));
     u = t.x + t.y;
+    if (PLAIN) return ldexp_plain(u, q);
     u = ldexp2k(u, q);
     return d.x < -1000.0 ? 0.0 : u;
 }
@@ -219,11 +306,19 @@ template <typename T> __device__ __forceinline__ T powk(DW<T> lg, T y) {
 template <typename T, int NHIST> struct StepFactor {
     DW<T> lg, lg_prev, lg_pprev;
     __device__ __forceinline__ StepFactor() : lg(dw((T)0, (T)0)), lg_prev(dw((T)0, (T)0)), lg_pprev(dw((T)0, (T)0)) {}
-    __device__ __forceinline__ T operator()(T safety, T ratio, T e1, T e2, T e3, bool) {
+    __device__ __forceinline__ T operator()(T safety, T ratio, T e1, T e2, T e3) {
         lg = logk(ratio);
         T factor = safety * powk<T>(lg, e1);
         if (NHIST >= 1) factor = factor * powk<T>(lg_prev, e2);
         if (NHIST >= 2) factor = factor * powk<T>(lg_pprev, e3);
+        return factor;
+    }
+    // the same for a ratio in [2^-50, 2^50] and exponents of at most 1/2 in magnitude
+    __device__ __forceinline__ T plain(T safety, T ratio, T e1, T e2, T e3) {
+        lg = logk<true>(ratio);
+        T factor = safety * expk<true>(dw_mul(lg, e1));
+        if (NHIST >= 1) factor = factor * expk<true>(dw_mul(lg_prev, e2));
+        if (NHIST >= 2) factor = factor * expk<true>(dw_mul(lg_pprev, e3));
         return factor;
     }
     // the ratio just used becomes the previous one where `shift` (an accepted step of a running sample)
@@ -348,6 +443,7 @@ template <typename T> struct CtrlParams {
     double e1, e2, e3;         // pow exponents: ratio, prev, prev_prev
     int has_dt_min, has_dt_max;
     int skip2, skip3;          // exponent is +-0: the factor is exactly 1
+    int plain;                 // tolerances and exponents in the ranges that control_common's short forms need
     // an exponent that ATen does not compute through pow (kernels that share one logarithm
     // between the powers do not take such a controller)
     bool shortcut_exponent() const {
@@ -379,7 +475,9 @@ template <typename T, int F> __device__ __forceinline__ T rms(const T (&v)[F]) {
 // arguments so that the float64 -> T conversion happens at compile time.
 // With MAGNITUDE_ONLY the first product is taken as it is instead of being added to zero: the
 // two differ in the sign of a zero sum at most, which a caller that only uses |out| never sees.
-template <typename T, int F, typename Tab, int ROW, bool MAGNITUDE_ONLY = false>
+// FINITE: terms with a zero weight are left out.  0 * k is a zero unless k is not finite, and a step with such a k is
+// given up by the callers that ask for this (its other slopes carry it into the error estimate).
+template <typename T, int F, typename Tab, int ROW, bool MAGNITUDE_ONLY = false, bool FINITE = false>
 __device__ __forceinline__ void weighted_k(T dt, const T (&k)[7][F], T (&out)[F]) {
 #pragma unroll
     for (int f = 0; f < F; ++f) out[f] = 0;
@@ -387,6 +485,7 @@ __device__ __forceinline__ void weighted_k(T dt, const T (&k)[7][F], T (&out)[F]
     for (int s = 0; s < 7; ++s) {
         constexpr int R = ROW < 0 ? 0 : ROW;
         const T ws = ROW < 0 ? (T)Tab::b_err[s] : (T)Tab::w[R][s];
+        if (FINITE && ws == (T)0) continue;
         T p = dt * ws;
 #pragma unroll
         for (int f = 0; f < F; ++f) {
@@ -436,35 +535,92 @@ template <int F> struct DivSqrtCorrected {
     }
     static __device__ __forceinline__ float exact(float x) { return x / DivSqrtConstant<F>::c; }
 };
+// float64, F == 2: 1/c rounds with an error of 0.26 half units, so that x * (1/c) is within one unit of x / c for every x
+// and Markstein's theorem makes the corrected value the correctly rounded quotient; 11 -> 3 instructions.  F == 3: 0.79
+// half units, the product may be one and a half units off; a second correction starts within one.  (Arguments below
+// 2^-900 take the division.)
+template <> struct DivSqrtFeatures<double, 2> {
+    static constexpr bool corrected = true;
+    static __device__ __forceinline__ double fast(double x) {
+        constexpr double c = 0x1.6a09e667f3bcdp+0, rc = 0x1.6a09e667f3bccp-1;
+        return quotient_with(x, c, rc);
+    }
+    static __device__ __forceinline__ double exact(double x) { return x / 0x1.6a09e667f3bcdp+0; }
+};
+template <> struct DivSqrtFeatures<double, 3> {
+    static constexpr bool corrected = true;
+    static __device__ __forceinline__ double fast(double x) {
+        constexpr double c = 0x1.bb67ae8584caap+0, rc = 0x1.279a74590331dp-1;
+        const double q = quotient_with(x, c, rc);
+        return fma_(fma_(-q, c, x), rc, q);
+    }
+    static __device__ __forceinline__ double exact(double x) { return x / 0x1.bb67ae8584caap+0; }
+};
 template <> struct DivSqrtFeatures<float, 2> : DivSqrtCorrected<2> {};
 template <> struct DivSqrtFeatures<float, 3> : DivSqrtCorrected<3> {};
 
-// Error ratio for the kernels that cover the common case only (and hand every batch with a
-// non-finite value to the general kernel): the same operations as error_ratio() with the
-// hardware's maximum in place of the NaN-propagating one.  The two differ for a NaN operand alone;
-// `unordered` is raised for one (a NaN in y0, y1, err or the sum), and the caller must then leave
-// the common case rather than use the returned value.  An infinite operand takes the same path
-// through both.
-template <typename T, int F>
-__device__ __forceinline__ T error_ratio_common(const CtrlParams<T> &cp, const T (&y0)[F], const T (&y1)[F], const T (&err)[F],
-                                                bool &unordered) {
+// max(|a|, |b|), max and min of two values that are not NaN, one instruction each (the compiler puts a canonicalising
+// maximum in front of every operand of fmax that it cannot prove quiet).
+__device__ __forceinline__ float max_abs(float a, float b) {
+    float r;
+    asm("v_max_f32 %0, |%1|, |%2|" : "=v"(r) : "v"(a), "v"(b));
+    return r;
+}
+__device__ __forceinline__ double max_abs(double a, double b) {
+    double r;
+    asm("v_max_f64 %0, |%1|, |%2|" : "=v"(r) : "v"(a), "v"(b));
+    return r;
+}
+__device__ __forceinline__ float max_ordered(float a, float b) {
+    float r;
+    asm("v_max_f32 %0, %1, %2" : "=v"(r) : "v"(a), "v"(b));
+    return r;
+}
+__device__ __forceinline__ double max_ordered(double a, double b) {
+    double r;
+    asm("v_max_f64 %0, %1, %2" : "=v"(r) : "v"(a), "v"(b));
+    return r;
+}
+__device__ __forceinline__ float min_ordered(float a, float b) {
+    float r;
+    asm("v_min_f32 %0, %1, %2" : "=v"(r) : "v"(a), "v"(b));
+    return r;
+}
+__device__ __forceinline__ double min_ordered(double a, double b) {
+    double r;
+    asm("v_min_f64 %0, %1, %2" : "=v"(r) : "v"(a), "v"(b));
+    return r;
+}
+
+// The upper 32 bits of a value, and of the bounds below (for float32: all of it).
+__device__ __forceinline__ unsigned high_bits(float x) { return __float_as_uint(x); }
+__device__ __forceinline__ unsigned high_bits(double x) { return (unsigned)__double2hiint(x); }
+template <typename T> __device__ __forceinline__ constexpr unsigned power_of_two_bits(int e) {
+    return sizeof(T) == 4 ? (unsigned)(e + 127) << 23 : (unsigned)(e + 1023) << 20;
+}
+
+// Error ratio and step factor (before its clip) for the kernels that cover the common case only: the operations of
+// error_ratio() and StepFactor.  With the short forms above wherever every lane that counts (`counted`: its sample is
+// still stepping, or sits through an idle step) has its operands in their ranges, which nearly every iteration of an
+// ordinary solve does; otherwise, for the whole wavefront, with the general ones.  The test: every scaled error zero or
+// at least 2^-60 (for float64, 2^-400: nothing below 2^-1022 hides in a zero upper half that could reach the sum of
+// squares), their sum of squares in [2^-100, 2^100] -- which a NaN anywhere in the step fails: it reaches the error
+// estimate through the last stage.  `insane`: the lanes whose ratio is not finite or whose factor is not a number; the
+// caller must leave the common case there and not use the values.
+template <typename T, int F, int NHIST, typename Tab>
+__device__ __forceinline__ T control_common(const CtrlParams<T> &cp, T dt, const T (&k)[7][F], const T (&y0)[F], const T (&y1)[F], lanes_t counted,
+                                            StepFactor<T, NHIST> &step_factor, T e1, T e2, T e3, T &factor, lanes_t &insane) {
     using Div = DivSqrtFeatures<T, F>;
-    T q[F], x[F];
-    bool nan = false, small = false;
+    T err[F], q[F], x[F], eb[F], acc = 0;
+    weighted_k<T, F, Tab, -1, true, true>(dt, k, err);
+    unsigned smallest = 0xffffffffu;
 #pragma unroll
     for (int f = 0; f < F; ++f) {
-        nan = nan || __builtin_isunordered(y0[f], y1[f]);
-        const T m = hwmax(abs_(y0[f]), abs_(y1[f]));
-        const T eb = fma_(cp.rtol, m, cp.atol);
-        q[f] = abs_(err[f]) / eb;
+        eb[f] = fma_(cp.rtol, max_abs(y0[f], y1[f]), cp.atol);
+        q[f] = quotient_plain(abs_(err[f]), eb[f]);
         x[f] = Div::fast(q[f]);
-        if (Div::corrected) small = small || (q[f] < (T)0x1p-100f && q[f] > (T)0);
+        smallest = min(smallest, high_bits(q[f]) - 1u);  // (zero wraps round to the largest)
     }
-    if (Div::corrected && __builtin_expect(__any(small), 0)) {  // (one branch for all features, after their divisions)
-#pragma unroll
-        for (int f = 0; f < F; ++f) x[f] = Div::exact(q[f]);
-    }
-    T acc = 0;
 #pragma unroll
     for (int f = 0; f < F; ++f) {
         if (F <= 3)
@@ -474,13 +630,43 @@ __device__ __forceinline__ T error_ratio_common(const CtrlParams<T> &cp, const T
             acc = acc + sq;
         }
     }
-    const T r = sqrt_(acc);
-    unordered = nan || r != r;
-    return hwmax(r, (T)1e-38);
+    constexpr unsigned lowest = power_of_two_bits<T>(sizeof(T) == 4 ? -60 : -400) - 1u;
+    constexpr unsigned from = power_of_two_bits<T>(-100), width = power_of_two_bits<T>(100) - from;
+    const lanes_t outside = lanes_where(smallest < lowest) | lanes_where(high_bits(acc) - from >= width);
+    T ratio = sqrt_plain(acc);
+    factor = step_factor.plain(cp.safety, ratio, e1, e2, e3);
+    insane = 0;
+    if (__builtin_expect((counted & outside) != 0 || !cp.plain, 0)) {
+        bool nan = false;
+        asm volatile("" : "+v"(dt));  // (the error estimate formed again: keeping it for this rare branch would cost F registers)
+        weighted_k<T, F, Tab, -1, true, true>(dt, k, err);
+#pragma unroll
+        for (int f = 0; f < F; ++f) {
+            nan = nan || __builtin_isunordered(y0[f], y1[f]);
+            x[f] = (abs_(err[f]) / fma_(cp.rtol, hwmax(abs_(y0[f]), abs_(y1[f])), cp.atol));
+            x[f] = Div::exact(x[f]);
+        }
+        acc = 0;
+#pragma unroll
+        for (int f = 0; f < F; ++f) {
+            if (F <= 3)
+                acc = fma_(x[f], x[f], acc);
+            else {
+                const T sq = x[f] * x[f];
+                acc = acc + sq;
+            }
+        }
+        const T r = sqrt_(acc);
+        ratio = hwmax(r, (T)1e-38);
+        const bool sane = !nan && r == r && ratio < (T)__builtin_huge_val();  // (the ratio is at least 1e-38)
+        factor = step_factor(cp.safety, sane ? ratio : (T)1, e1, e2, e3);
+        insane = ~lanes_where(sane && factor == factor);  // (a product of an underflowed and an overflowed power)
+    }
+    return ratio;
 }
 
 // clamp(x, lo, hi) for operands that are known not to be NaN.
-template <typename T> __device__ __forceinline__ T clamp_ordered(T x, T lo, T hi) { return hwmin(hwmax(x, lo), hi); }
+template <typename T> __device__ __forceinline__ T clamp_ordered(T x, T lo, T hi) { return min_ordered(max_ordered(x, lo), hi); }
 
 // dt factor (step_size_controllers.py:289-294, 598-620).
 template <typename T, int CTRL> __device__ __forceinline__ T dt_factor(const CtrlParams<T> &cp, T ratio, T prev, T prev_prev) {
@@ -528,7 +714,7 @@ __device__ __forceinline__ int limit_step(const CtrlParams<T> &cp, TT dt_min, TT
 
 // Quartic coefficients of the dense output, lowest power first.
 // Tsit5: tsit5.py:123-139.  Dopri5: dopri5.py:53-60 -> interpolation.py:138-170.
-template <typename T, int F, int METHOD>
+template <typename T, int F, int METHOD, bool FINITE = false>
 __device__ __forceinline__ void quartic(T dt, const T (&y0)[F], const T (&y1)[F], const T (&k)[7][F], T (&q)[5][F]) {
     if (METHOD == 1) {
 #pragma unroll
@@ -541,7 +727,7 @@ __device__ __forceinline__ void quartic(T dt, const T (&y0)[F], const T (&y1)[F]
         weighted_k<T, F, Tsit5Tab, 2>(dt, k, q[4]);
     } else {
         T ymid[F];
-        weighted_k<T, F, Dopri5Tab, 0>(dt, k, ymid);
+        weighted_k<T, F, Dopri5Tab, 0, false, FINITE>(dt, k, ymid);
 #pragma unroll
         for (int f = 0; f < F; ++f) {
             T f0 = dt * k[0][f], f1 = dt * k[6][f];
@@ -583,6 +769,37 @@ template <typename T, int F, typename TT = T> __device__ __forceinline__ void qu
         y = fma_(y, x, q[1][f]);
         y = fma_(y, x, q[0][f]);
         out[f] = y;
+    }
+}
+
+// Where evaluation points lie within a step, x = (t - t0) / ((t0 + dt) - t0) (interpolation.py:25-40), for many points of
+// one step: the step's reciprocal is formed once and a point costs a product and a correction (quotient_with) where
+// `plain` says that the operands are in the range of that form.  A point in [t0, t0 + dt] is t0 itself or at least
+// 2^-25 |t0| away, so |t0| >= 2^-30 |den| puts the quotient above 2^-55; the step before that (t0 = 0 or near it) divides.
+template <typename T> struct StepPosition {
+    T t0, den, r;
+    lanes_t plain;
+    __device__ __forceinline__ StepPosition(T t0_, T dt) : t0(t0_) {
+        const T t1 = t0 + dt, d = t1 - t0;
+        den = abs_(d) > (T)0 ? d : (T)1;
+        r = reciprocal_estimate(den);
+        plain = lanes_where(abs_(den) >= (T)0x1p-40) & lanes_where(abs_(den) <= (T)0x1p+40) & lanes_where(abs_(t0) >= abs_(den) * (T)0x1p-30);
+    }
+    // t = dir * dte with dir = +-1 (an exact product)
+    template <bool PLAIN> __device__ __forceinline__ T at(T dir, T dte) const {
+        const T n = fma_(dir, dte, -t0);
+        return PLAIN ? quotient_with(n, den, r) : n / den;
+    }
+};
+// Horner on x, lowest power first in q.
+template <typename T, int F> __device__ __forceinline__ void quartic_at_unit(const T (&q)[5][F], T x, T (&out)[F]) {
+#pragma unroll
+    for (int f = 0; f < F; ++f) {
+        T y = q[4][f];
+        y = fma_(y, x, q[3][f]);
+        y = fma_(y, x, q[2][f]);
+        y = fma_(y, x, q[1][f]);
+        out[f] = fma_(y, x, q[0][f]);
     }
 }
 

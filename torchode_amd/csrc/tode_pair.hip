@@ -9,7 +9,7 @@
 // dense output -- so each group of 64 samples gets two wavefronts:
 //   * the STEPPER runs the adaptive loop (stages, error ratio, step size control,
 //     state update) and, after every attempted step, leaves the step's
-//     (t0, dt, y0, y1, k_0..k_6, new time, active flag) in LDS;
+//     (t0, dt, y0, y1, k_0..k_6, new time) in LDS;
 //   * the EVALUATOR picks that record up one barrier later, builds the quartic
 //     interpolant and writes the evaluation points the step passed, while the
 //     stepper is already computing the next step.
@@ -35,7 +35,7 @@ __global__ void __launch_bounds__(128) solve_pair_kernel(const SolveParams<T> p,
     using Tab = typename std::conditional<METHOD == 1, Tsit5Tab, Dopri5Tab>::type;
     constexpr int F = Term::F;
     constexpr int P = Term::P;
-    constexpr int NF = 4 + 9 * F;  // record: t0, dt, dir*t_new, active, y[F], y1[F], k[7][F]
+    constexpr int NF = 3 + 9 * F;  // record: t0, dt, dir*t_new (-inf once the sample has finished), y[F], y1[F], k[7][F]
     extern __shared__ __align__(16) unsigned char smem_raw[];
     const int lane = threadIdx.x & 63;
     const int wave = threadIdx.x >> 6;
@@ -56,7 +56,7 @@ __global__ void __launch_bounds__(128) solve_pair_kernel(const SolveParams<T> p,
 
     T *rec = reinterpret_cast<T *>(smem_raw);                // [2][NF][64]
     int *ctl = reinterpret_cast<int *>(rec + 2 * NF * 64);   // [2] "stepper is done" per phase
-    T *te_s = reinterpret_cast<T *>(ctl + 4);                // [E][64] when STAGE_TE
+    T *te_s = reinterpret_cast<T *>(ctl + 4);                // [E + 1][64] when STAGE_TE
 
     const T ts = p.t_start[bs * p.ts_stride], te = p.t_end[bs * p.te_stride];
     const bool fwd = te > ts;
@@ -87,8 +87,8 @@ __global__ void __launch_bounds__(128) solve_pair_kernel(const SolveParams<T> p,
         bool odd_start = !finite_(dt) || !finite_(ts) || !finite_(te);
 #pragma unroll
         for (int f = 0; f < F; ++f) odd_start = odd_start || !finite_(y[f]) || !finite_(k[0][f]);
-        bool bail = live && odd_start;
-        bool active = live && !odd_start;
+        // lanes whose sample is still stepping, and lanes whose sample needs the general kernel
+        lanes_t active = lanes_where(live && !odd_start), bail_lanes = lanes_where(live && odd_start);
         const int step_limit = p.max_steps < TODE_HARD_STEP_LIMIT ? p.max_steps : TODE_HARD_STEP_LIMIT;
         const T e1 = (T)cp.e1, e2 = (T)cp.e2, e3 = (T)cp.e3;
 
@@ -108,15 +108,15 @@ __global__ void __launch_bounds__(128) solve_pair_kernel(const SolveParams<T> p,
         // later iterations with the clamped step t_end - t: with evaluation points that is seen only in the status of
         // that step, a success unless its error ratio is not finite.  The sample sits through one more iteration here,
         // as an inactive lane whose error ratio is looked at.
-        bool idle = false;
+        lanes_t idle = 0;
         int phase = 0;
         for (;; ++phase) {
-            const bool any = __any(active || idle);
-            if (any) {
-                if (RECORD) keep(phase, active);
+            const lanes_t counted = active | idle;
+            if (counted) {
+                if (RECORD) keep(phase, holds(active));
                 // ---- stages (runge_kutta.py:255-263) ----
                 const T t0 = t;
-                T y1[F], err[F];
+                T y1[F];
 #pragma unroll
                 for (int i = 1; i < 7; ++i) {
                     T tn = fma_((T)Tab::c[i], dt, t0);
@@ -125,7 +125,8 @@ __global__ void __launch_bounds__(128) solve_pair_kernel(const SolveParams<T> p,
                     for (int f = 0; f < F; ++f) {
                         T s = 0;
 #pragma unroll
-                        for (int j = 0; j < i; ++j) s = fma_((T)Tab::a[i][j], k[j][f], s);
+                        for (int j = 0; j < i; ++j)
+                            if (Tab::a[i][j] != 0.0) s = fma_((T)Tab::a[i][j], k[j][f], s);  // (a zero weight: weighted_k's FINITE)
                         yi[f] = fma_(dt, s, y[f]);
                     }
                     rhs(tn, yi, k[i]);
@@ -135,83 +136,71 @@ __global__ void __launch_bounds__(128) solve_pair_kernel(const SolveParams<T> p,
                     }
                 }
                 // hand the attempted step to the evaluator (everything it needs is known now)
-                const bool pre_active = active;
                 T *r = rec + (phase & 1) * NF * 64 + lane;
                 r[0 * 64] = t0;
                 r[1 * 64] = dt;
 #pragma unroll
                 for (int f = 0; f < F; ++f) {
-                    r[(4 + f) * 64] = y[f];
-                    if (METHOD != 1) r[(4 + F + f) * 64] = y1[f];  // (Tsit5's interpolant does not look at the step's result)
+                    r[(3 + f) * 64] = y[f];
+                    if (METHOD != 1) r[(3 + F + f) * 64] = y1[f];  // (Tsit5's interpolant does not look at the step's result)
                 }
 #pragma unroll
                 for (int s = 0; s < 7; ++s)
 #pragma unroll
-                    for (int f = 0; f < F; ++f) r[(4 + 2 * F + s * F + f) * 64] = k[s][f];
+                    for (int f = 0; f < F; ++f) r[(3 + 2 * F + s * F + f) * 64] = k[s][f];
 
-                weighted_k<T, F, Tab, -1, true>(dt, k, err);
-
-                // ---- step size control (step_size_controllers.py:370-429, 715-774) ----
-                bool unordered;
-                const T ratio = error_ratio_common<T, F>(cp, y, y1, err, unordered);
-                const bool accept = ratio < (T)1;
-                bool sane = !unordered && ratio < (T)__builtin_huge_val();  // (the ratio is at least 1e-38)
-                bail = bail || (idle && !sane);
-                idle = false;
-                T factor = step_factor(cp.safety, sane ? ratio : (T)1, e1, e2, e3, active);
-                sane = sane && factor == factor;  // (a product of an underflowed and an overflowed power)
+                // ---- error estimate and step size control (step_size_controllers.py:370-429, 715-774) ----
+                lanes_t insane;  // (a NaN or infinite ratio is a non-success status: left to the general kernel)
+                T factor;
+                const T ratio = control_common<T, F, NHIST, Tab>(cp, dt, k, y, y1, counted, step_factor, e1, e2, e3, factor, insane);
+                const lanes_t accept = lanes_where(ratio < (T)1), move = accept & active;
+                bail_lanes |= idle & insane;
+                idle = 0;
                 factor = clamp_ordered(factor, cp.fmin, cp.fmax);
                 const T dt_next = dt * factor;
 
-                const bool move = accept && active;
-                const T t_new = move ? (t0 + dt) : t0;
-                const T dt_new = dir * t_new;
-                const bool running_new = dt_new < dte_end;
-                n_steps += active ? 1 : 0;
-                n_acc += move ? 1 : 0;
-                r[2 * 64] = dt_new;
-                r[3 * 64] = pre_active ? (T)1 : (T)0;
+                t = holds(move) ? (t0 + dt) : t0;
+                const T dt_new = dir * t;
+                const lanes_t running = lanes_where(dt_new < dte_end);
+                n_acc += holds(move) ? 1 : 0;
+                r[2 * 64] = holds(active) ? dt_new : (T)-__builtin_huge_val();  // (a finished sample passes no point)
 
                 // ---- state update (adjoints.py:150-155, 247-255) ----
 #pragma unroll
                 for (int f = 0; f < F; ++f) {
-                    y[f] = move ? y1[f] : y[f];
-                    k[0][f] = move ? k[6][f] : k[0][f];
+                    y[f] = holds(move) ? y1[f] : y[f];
+                    k[0][f] = holds(move) ? k[6][f] : k[0][f];
                 }
-                t = t_new;
-                {
-                    const T dtn = running_new ? dt_next : dt;
-                    const T dtc = clamp_ordered(dtn, tlo - t, thi - t);
-                    dt = active ? dtc : dt;
-                }
-                if (NHIST >= 1) step_factor.shift(active && running_new && accept);
+                // (a finished sample no longer runs: its step stays what this clamp made it)
+                dt = clamp_ordered(holds(running) ? dt_next : dt, tlo - t, thi - t);
+                if (NHIST >= 1) step_factor.shift(holds(running & accept));
                 if (RECORD && CTRL == 1) {
-                    const bool shift = active && running_new && accept;
+                    const bool shift = holds(running & accept);
                     ratio_prev_prev = shift ? ratio_prev : ratio_prev_prev;
                     ratio_prev = shift ? ratio : ratio_prev;
                 }
-                {
-                    const bool failed = active && (!sane || n_steps >= step_limit);
-                    const bool finished = active && !failed && !running_new;
-                    if (__any(finished)) {
-                        // a sample whose state or derivative at the end is not finite shows up in later iterations of
-                        // the reference loop with another status, and so does, without evaluation points, one that
-                        // landed past t_end (in the interpolant of the batch's last step); with evaluation points
-                        // such a sample is looked at in the next iteration
-                        bool odd = end_only && !(t == te);
+                const lanes_t failed = active & (phase + 1 >= step_limit ? ~(lanes_t)0 : insane);
+                const lanes_t ended = active & (failed | ~running);
+                if (ended) {
+                    n_steps = holds(ended) ? phase + 1 : n_steps;
+                    // a sample whose state or derivative at the end is not finite shows up in later iterations of
+                    // the reference loop with another status, and so does, without evaluation points, one that
+                    // landed past t_end (in the interpolant of the batch's last step); with evaluation points
+                    // such a sample is looked at in the next iteration
+                    bool odd = end_only && !(t == te);
 #pragma unroll
-                        for (int f = 0; f < F; ++f) odd = odd || !settles_(y[f], k[0][f]);
-                        bail = bail || (finished && odd);
-                        idle = finished && !odd && !(t == te);
-                    }
-                    bail = bail || failed;
-                    active = active && !failed && running_new;
+                    for (int f = 0; f < F; ++f) odd = odd || !settles_(y[f], k[0][f]);
+                    const lanes_t finished = ended & ~failed, odd_lanes = lanes_where(odd);
+                    bail_lanes |= failed | (finished & odd_lanes);
+                    idle = finished & ~odd_lanes & ~lanes_where(t == te);
+                    active &= ~ended;
                 }
             }
-            if (lane == 0) ctl[phase & 1] = any ? 0 : 1;
+            if (lane == 0) ctl[phase & 1] = counted ? 0 : 1;
             __syncthreads();
-            if (!any) break;
+            if (!counted) break;
         }
+        bool bail = holds(bail_lanes);
 
         if (RECORD) {  // the state every sample is left in, for every later iteration of the batch
             for (long long at = phase; at < p.rec_capacity; ++at) keep(at, false);
@@ -257,62 +246,76 @@ __global__ void __launch_bounds__(128) solve_pair_kernel(const SolveParams<T> p,
             }
         }
         // (LDS accesses of one wavefront complete in order; te_s is private to this wave)
-        auto te_at = [&](int e) -> T { return end_only ? te : (STAGE_TE ? te_s[e * 64 + lane] : tev_g[e]); };
+        // From here on times are multiplied by the sample's direction (exact), and behind the last point lies one that no
+        // step reaches: whether a step has passed the next point is one comparison.
+        const T never = (T)__builtin_huge_val();
         bool bail = false;
-        {
-            T prev_te = te_at(0);
+        const T te_first = end_only ? te : (STAGE_TE ? te_s[lane] : tev_g[0]);
+        if (!end_only) {
+            T prev_te = dir * te_first;
+            if (STAGE_TE) te_s[lane] = prev_te;
             for (int e = 1; e < E; ++e) {
-                T cur = te_at(e);
-                if (!(fwd ? cur >= prev_te : cur <= prev_te)) bail = true;
+                const T cur = dir * (STAGE_TE ? te_s[e * 64 + lane] : tev_g[e]);
+                if (STAGE_TE) te_s[e * 64 + lane] = cur;
+                if (!(cur >= prev_te)) bail = true;
                 prev_te = cur;
             }
+            if (STAGE_TE) te_s[E * 64 + lane] = never;
         }
-        T *ys_g = p.ys + bs * (long long)E * F;
+        auto point = [&](int e) -> T {
+            if (end_only) return e == 0 ? dir * te : never;
+            if (STAGE_TE) return te_s[e * 64 + lane];
+            return e < E ? dir * tev_g[e] : never;
+        };
+        // (a workgroup's block of ys is far below 4 GiB: launch_pair)
+        T *ys_block = p.ys + b0 * (long long)E * F;
+        const unsigned ys_row = (unsigned)(live ? lane : 0) * (unsigned)E;
         int cursor = 0;
-        if (te_at(0) == ts) {
+        if (te_first == ts) {
             if (live) {
 #pragma unroll
-                for (int f = 0; f < F; ++f) ys_g[f] = p.y0[bs * F + f];
+                for (int f = 0; f < F; ++f) ys_block[ys_row * F + f] = p.y0[bs * F + f];
             }
             cursor = 1;
         }
-        T dte_next = dir * te_at(cursor < E ? cursor : E - 1);
+        T dte_next = live ? point(cursor) : never;
 
         for (int phase = 0;; ++phase) {
-            if (phase > 0) {
-                const T *r = rec + ((phase - 1) & 1) * NF * 64 + lane;
-                const T dt_new = r[2 * 64];
-                const bool was_active = live && !bail && r[3 * 64] != (T)0;
-                bool hit = was_active && cursor < E && dt_new >= dte_next;
-                if (__any(hit)) {
-                    const T t0 = r[0 * 64], dt = r[1 * 64];
-                    T y[F], y1[F], k[7][F], q[5][F];
+            __syncthreads();
+            const T *r = rec + (phase & 1) * NF * 64 + lane;
+            const int done = ctl[phase & 1];
+            const T dt_new = r[2 * 64];
+            if (done) break;
+            if (dt_new >= dte_next) {
+                const T t0 = r[0 * 64], dt = r[1 * 64];
+                T y[F], y1[F], k[7][F], q[5][F];
 #pragma unroll
-                    for (int f = 0; f < F; ++f) {
-                        y[f] = r[(4 + f) * 64];
-                        y1[f] = METHOD != 1 ? r[(4 + F + f) * 64] : (T)0;
-                    }
+                for (int f = 0; f < F; ++f) {
+                    y[f] = r[(3 + f) * 64];
+                    y1[f] = METHOD != 1 ? r[(3 + F + f) * 64] : (T)0;
+                }
 #pragma unroll
-                    for (int s = 0; s < 7; ++s)
+                for (int s = 0; s < 7; ++s)
 #pragma unroll
-                        for (int f = 0; f < F; ++f) k[s][f] = r[(4 + 2 * F + s * F + f) * 64];
-                    quartic<T, F, METHOD>(dt, y, y1, k, q);
+                    for (int f = 0; f < F; ++f) k[s][f] = r[(3 + 2 * F + s * F + f) * 64];
+                quartic<T, F, METHOD, true>(dt, y, y1, k, q);
+                const StepPosition<T> position(t0, dt);
+                auto write_points = [&](auto plain) {
                     do {
                         T out[F];
-                        quartic_eval<T, F>(q, t0, dt, dir * dte_next, out);
-                        if (hit) {
+                        quartic_at_unit<T, F>(q, position.template at<decltype(plain)::value>(dir, dte_next), out);
+                        T *row = ys_block + (ys_row + (unsigned)cursor) * F;
 #pragma unroll
-                            for (int f = 0; f < F; ++f) ys_g[cursor * F + f] = out[f];
-                        }
-                        cursor += hit ? 1 : 0;
-                        const T nxt = dir * te_at(cursor < E ? cursor : E - 1);
-                        dte_next = hit ? nxt : dte_next;
-                        hit = hit && cursor < E && dt_new >= dte_next;
-                    } while (__any(hit));
-                }
+                        for (int f = 0; f < F; ++f) row[f] = out[f];
+                        ++cursor;
+                        dte_next = point(cursor);
+                    } while (dt_new >= dte_next);
+                };
+                if (position.plain == lanes_where(true))
+                    write_points(std::true_type());
+                else
+                    write_points(std::false_type());
             }
-            __syncthreads();
-            if (ctl[phase & 1]) break;
         }
 
         if (live) o.n_initialized[b] = cursor;
@@ -327,14 +330,17 @@ __global__ void __launch_bounds__(128) solve_pair_kernel(const SolveParams<T> p,
 template <typename T, int METHOD, int CTRL, typename Term>
 static int launch_pair(const tode_solve_args &a, const tode_controller &c, const PairOut<T> &o, hipStream_t stream, bool *used) {
     *used = false;
-    constexpr int NF = 4 + 9 * Term::F;
+    constexpr int NF = 3 + 9 * Term::F;
     const long long blocks = (a.batch + 63) / 64;
     // worthwhile only while the single-wave kernel would leave SIMDs with <= 2 wavefronts
     if (blocks == 0 || blocks > 2 * 1024) return TODE_OK;
     const size_t rec_bytes = (size_t)2 * NF * 64 * sizeof(T) + 16;
-    const size_t te_bytes = (size_t)a.n_eval * 64 * sizeof(T);
-    const size_t budget = (size_t)(160 * 1024) / 4 - 512;  // four workgroups (eight wavefronts) per CU
-    if (rec_bytes > budget) return TODE_OK;
+    const size_t te_bytes = a.n_eval > 0 ? ((size_t)a.n_eval + 1) * 64 * sizeof(T) : 0;
+    if ((size_t)a.n_eval * Term::F >= ((size_t)1 << 24)) return TODE_OK;  // (32-bit offsets into a workgroup's block of ys)
+    // LDS: up to four workgroups (eight wavefronts) have to share a compute unit, fewer in a batch that does not have them
+    const long long per_cu = (blocks + 255) / 256;
+    const size_t budget = (size_t)(160 * 1024) / (size_t)(per_cu < 4 ? per_cu : 4) - 512;
+    if (rec_bytes > 36 * 1024) return TODE_OK;  // (four features in float64: the records alone would fill a quarter of it)
     const bool stage_te = rec_bytes + te_bytes <= budget;
     const size_t lds = rec_bytes + (stage_te ? te_bytes : 0);
     constexpr bool RECORD = TODE_INSTANTIATE_RECORD != 0;

@@ -239,6 +239,9 @@ template <typename T> static CtrlParams<T> make_ctrl(const tode_controller &c, d
     }
     cp.skip2 = ((double)(T)cp.e2 == 0.0);
     cp.skip3 = ((double)(T)cp.e3 == 0.0);
+    // (control_common: error bounds in [2^-40, 2^124] for any finite state, powers of ratios that stay within 2^+-64)
+    auto small = [](double e) { return e >= -0.5 && e <= 0.5; };
+    cp.plain = cp.atol >= (T)0x1p-40 && cp.atol <= (T)0x1p+40 && cp.rtol >= (T)0 && cp.rtol <= (T)0.0625 && small(cp.e1) && small(cp.e2) && small(cp.e3);
     return cp;
 }
 
