@@ -510,7 +510,8 @@ int tode_step_stats(const tode_step_state *state, int64_t *out_n_steps, int64_t 
  * in the reference.  A hook for tests and profiles, which have to address each kernel on inputs of their choice.
  * 0 (default): two wavefronts per 64 samples (a stepper and a dense-output evaluator) while the batch would
  * otherwise leave SIMDs with at most two wavefronts, one wavefront per 64 samples above that; 1: always one
- * wavefront; 2: two wavefronts or TODE_E_UNSUPPORTED.  Both kernels produce identical bits.
+ * wavefront; 2: two wavefronts or TODE_E_UNSUPPORTED; 3: two wavefronts with a sample's features on lanes of their own (the
+ * choice for the smallest batches) or TODE_E_UNSUPPORTED.  All produce identical bits.
  */
 int tode_set_fast_kernel_variant(int variant);
 

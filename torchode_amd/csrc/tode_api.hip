@@ -224,7 +224,8 @@ const char *tode_source_hash(void) { return TODE_SOURCE_HASH; }
 const char *tode_last_error(void) { return tode::g_error; }
 
 int tode_set_fast_kernel_variant(int variant) {
-    if (variant < 0 || variant > 2) return tode::fail(TODE_E_INVALID, "variant must be 0 (automatic), 1 (one wavefront per 64 samples) or 2 (two wavefronts)");
+    if (variant < 0 || variant > 3)
+        return tode::fail(TODE_E_INVALID, "variant must be 0 (automatic), 1 (one wavefront per 64 samples), 2 (two wavefronts) or 3 (two wavefronts, one feature per lane)");
     tode::g_fast_variant = variant;
     return TODE_OK;
 }
@@ -303,6 +304,12 @@ int tode_solve_builtin_fast(const tode_solve_args *a, const tode_controller *c, 
     if (a->record) {  // the solve and the record of its loop state in one kernel: the stepper of the two-wavefront kernel
                       // writes it for small batches, the single-wavefront kernel otherwise
         if (end_only) return fail(TODE_E_UNSUPPORTED, "a record from the fast entry point needs evaluation points");
+        if (g_fast_variant == 0 || g_fast_variant == 3) {
+            bool used = false;
+            int rc = a->dtype == TODE_F32 ? solve_pair_f32_lanes_record(*a, *c, ns, na, ni, st, s, &used) : solve_pair_f64_lanes_record(*a, *c, ns, na, ni, st, s, &used);
+            if (rc || used) return rc;
+            if (g_fast_variant == 3) return fail(TODE_E_UNSUPPORTED, "the two-wavefront kernel with a sample's features on several lanes does not cover this problem size");
+        }
         if (g_fast_variant == 0 || g_fast_variant == 2) {
             bool used = false;
             int rc = a->dtype == TODE_F32 ? solve_pair_f32_record(*a, *c, ns, na, ni, st, s, &used) : solve_pair_f64_record(*a, *c, ns, na, ni, st, s, &used);
@@ -310,6 +317,13 @@ int tode_solve_builtin_fast(const tode_solve_args *a, const tode_controller *c, 
             if (g_fast_variant == 2) return fail(TODE_E_UNSUPPORTED, "the two-wavefront kernel does not cover this problem size");
         }
         return a->dtype == TODE_F32 ? solve_fast_f32_record(*a, *c, ns, na, ni, st, s) : solve_fast_f64_record(*a, *c, ns, na, ni, st, s);
+    }
+    if (g_fast_variant == 0 || g_fast_variant == 3) {
+        // smaller batches yet: those two with a sample's features on lanes of their own
+        bool used = false;
+        int rc = a->dtype == TODE_F32 ? solve_pair_f32_lanes(*a, *c, ns, na, ni, st, s, &used) : solve_pair_f64_lanes(*a, *c, ns, na, ni, st, s, &used);
+        if (rc || used) return rc;
+        if (g_fast_variant == 3) return fail(TODE_E_UNSUPPORTED, "the two-wavefront kernel with a sample's features on several lanes does not cover this problem size");
     }
     if (g_fast_variant == 0 || g_fast_variant == 2) {
         // small batches: two wavefronts per group of 64 samples (stepper + dense-output evaluator)

@@ -186,7 +186,7 @@ __global__ void __launch_bounds__(64, fast_wavefronts(sizeof(T), Term::F, NHIST,
         // ---- error estimate and step size control (step_size_controllers.py:370-429, 715-774) ----
         lanes_t insane;  // (a NaN or infinite ratio is a non-success status: left to the general kernel)
         T factor;
-        const T ratio = control_common<T, F, NHIST, Tab>(cp, dt, k, y, y1, counted, step_factor, e1, e2, e3, factor, insane);
+        const T ratio = control_common<T, F, F, 1, NHIST, Tab>(cp, dt, k, y, y1, counted, step_factor, e1, e2, e3, factor, insane);
         const lanes_t accept = lanes_where(ratio < (T)1), move = accept & active;
         bail_lanes |= idle & insane;
         idle = 0;

@@ -300,40 +300,6 @@ template <typename T> __device__ __forceinline__ T powk(DW<T> lg, T y) {
     return (r != r) ? (T)__builtin_huge_val() : r;
 }
 
-// The step factor's powers (step_size_controllers.py:289-294, 598-620) for the kernels that keep
-// the history of accepted error ratios as logarithms: safety * ratio^e1 [* prev^e2 [* prev_prev^e3]],
-// multiplied in this order.  `ratio` is positive and finite.  NHIST = number of history factors.
-template <typename T, int NHIST> struct StepFactor {
-    DW<T> lg, lg_prev, lg_pprev;
-    __device__ __forceinline__ StepFactor() : lg(dw((T)0, (T)0)), lg_prev(dw((T)0, (T)0)), lg_pprev(dw((T)0, (T)0)) {}
-    __device__ __forceinline__ T operator()(T safety, T ratio, T e1, T e2, T e3) {
-        lg = logk(ratio);
-        T factor = safety * powk<T>(lg, e1);
-        if (NHIST >= 1) factor = factor * powk<T>(lg_prev, e2);
-        if (NHIST >= 2) factor = factor * powk<T>(lg_pprev, e3);
-        return factor;
-    }
-    // the same for a ratio in [2^-50, 2^50] and exponents of at most 1/2 in magnitude
-    __device__ __forceinline__ T plain(T safety, T ratio, T e1, T e2, T e3) {
-        lg = logk<true>(ratio);
-        T factor = safety * expk<true>(dw_mul(lg, e1));
-        if (NHIST >= 1) factor = factor * expk<true>(dw_mul(lg_prev, e2));
-        if (NHIST >= 2) factor = factor * expk<true>(dw_mul(lg_pprev, e3));
-        return factor;
-    }
-    // the ratio just used becomes the previous one where `shift` (an accepted step of a running sample)
-    __device__ __forceinline__ void shift(bool s) {
-        if (NHIST >= 2) {
-            lg_pprev.x = s ? lg_prev.x : lg_pprev.x;
-            lg_pprev.y = s ? lg_prev.y : lg_pprev.y;
-        }
-        if (NHIST >= 1) {
-            lg_prev.x = s ? lg.x : lg_prev.x;
-            lg_prev.y = s ? lg.y : lg_prev.y;
-        }
-    }
-};
-
 // x ** y for x >= 0 or NaN, all special cases included.
 template <typename T> __device__ __forceinline__ T pow_(T x, T y) {
     if (y == (T)0 || x == (T)1) return (T)1;
@@ -597,72 +563,6 @@ __device__ __forceinline__ unsigned high_bits(float x) { return __float_as_uint(
 __device__ __forceinline__ unsigned high_bits(double x) { return (unsigned)__double2hiint(x); }
 template <typename T> __device__ __forceinline__ constexpr unsigned power_of_two_bits(int e) {
     return sizeof(T) == 4 ? (unsigned)(e + 127) << 23 : (unsigned)(e + 1023) << 20;
-}
-
-// Error ratio and step factor (before its clip) for the kernels that cover the common case only: the operations of
-// error_ratio() and StepFactor.  With the short forms above wherever every lane that counts (`counted`: its sample is
-// still stepping, or sits through an idle step) has its operands in their ranges, which nearly every iteration of an
-// ordinary solve does; otherwise, for the whole wavefront, with the general ones.  The test: every scaled error zero or
-// at least 2^-60 (for float64, 2^-400: nothing below 2^-1022 hides in a zero upper half that could reach the sum of
-// squares), their sum of squares in [2^-100, 2^100] -- which a NaN anywhere in the step fails: it reaches the error
-// estimate through the last stage.  `insane`: the lanes whose ratio is not finite or whose factor is not a number; the
-// caller must leave the common case there and not use the values.
-template <typename T, int F, int NHIST, typename Tab>
-__device__ __forceinline__ T control_common(const CtrlParams<T> &cp, T dt, const T (&k)[7][F], const T (&y0)[F], const T (&y1)[F], lanes_t counted,
-                                            StepFactor<T, NHIST> &step_factor, T e1, T e2, T e3, T &factor, lanes_t &insane) {
-    using Div = DivSqrtFeatures<T, F>;
-    T err[F], q[F], x[F], eb[F], acc = 0;
-    weighted_k<T, F, Tab, -1, true, true>(dt, k, err);
-    unsigned smallest = 0xffffffffu;
-#pragma unroll
-    for (int f = 0; f < F; ++f) {
-        eb[f] = fma_(cp.rtol, max_abs(y0[f], y1[f]), cp.atol);
-        q[f] = quotient_plain(abs_(err[f]), eb[f]);
-        x[f] = Div::fast(q[f]);
-        smallest = min(smallest, high_bits(q[f]) - 1u);  // (zero wraps round to the largest)
-    }
-#pragma unroll
-    for (int f = 0; f < F; ++f) {
-        if (F <= 3)
-            acc = fma_(x[f], x[f], acc);
-        else {
-            const T sq = x[f] * x[f];
-            acc = acc + sq;
-        }
-    }
-    constexpr unsigned lowest = power_of_two_bits<T>(sizeof(T) == 4 ? -60 : -400) - 1u;
-    constexpr unsigned from = power_of_two_bits<T>(-100), width = power_of_two_bits<T>(100) - from;
-    const lanes_t outside = lanes_where(smallest < lowest) | lanes_where(high_bits(acc) - from >= width);
-    T ratio = sqrt_plain(acc);
-    factor = step_factor.plain(cp.safety, ratio, e1, e2, e3);
-    insane = 0;
-    if (__builtin_expect((counted & outside) != 0 || !cp.plain, 0)) {
-        bool nan = false;
-        asm volatile("" : "+v"(dt));  // (the error estimate formed again: keeping it for this rare branch would cost F registers)
-        weighted_k<T, F, Tab, -1, true, true>(dt, k, err);
-#pragma unroll
-        for (int f = 0; f < F; ++f) {
-            nan = nan || __builtin_isunordered(y0[f], y1[f]);
-            x[f] = (abs_(err[f]) / fma_(cp.rtol, hwmax(abs_(y0[f]), abs_(y1[f])), cp.atol));
-            x[f] = Div::exact(x[f]);
-        }
-        acc = 0;
-#pragma unroll
-        for (int f = 0; f < F; ++f) {
-            if (F <= 3)
-                acc = fma_(x[f], x[f], acc);
-            else {
-                const T sq = x[f] * x[f];
-                acc = acc + sq;
-            }
-        }
-        const T r = sqrt_(acc);
-        ratio = hwmax(r, (T)1e-38);
-        const bool sane = !nan && r == r && ratio < (T)__builtin_huge_val();  // (the ratio is at least 1e-38)
-        factor = step_factor(cp.safety, sane ? ratio : (T)1, e1, e2, e3);
-        insane = ~lanes_where(sane && factor == factor);  // (a product of an underflowed and an overflowed power)
-    }
-    return ratio;
 }
 
 // clamp(x, lo, hi) for operands that are known not to be NaN.

@@ -17,12 +17,21 @@
 // hand-over.  Stepper and evaluator roles alternate between neighbouring
 // workgroups so that every SIMD hosts one of each.
 //
+// In the smallest batches a sample's features get a lane each (the ...Lanes systems of tode_solve.h), 64 / L samples per
+// wavefront: the same kernel with one feature per lane.
+//
 // Same arithmetic, bit for bit, and same contract as tode_fast.hip
 // (TODE_FLAG_NEEDS_GENERAL when the batch leaves the common case).
 //
 // RECORD: the stepper also writes the loop state before every iteration to p.rec_* (tode_solve_record), as
 // tode_fast.hip's recording variant does, for the reverse sweep of a differentiable solve.
 #include "tode_solve.h"
+
+#if TODE_INSTANTIATE_LANES
+#define TODE_PAIR_TERM(name) name##Lanes
+#else
+#define TODE_PAIR_TERM(name) name##Term
+#endif
 
 namespace tode {
 
@@ -33,17 +42,24 @@ template <typename T> struct PairOut {
 template <typename T, int METHOD, int CTRL, int NHIST, typename Term, bool STAGE_TE, bool RECORD = false>
 __global__ void __launch_bounds__(128) solve_pair_kernel(const SolveParams<T> p, const PairOut<T> o) {
     using Tab = typename std::conditional<METHOD == 1, Tsit5Tab, Dopri5Tab>::type;
-    constexpr int F = Term::F;
+    // F features per sample, K of them per lane, L lanes per sample, S samples per wavefront
+    constexpr int F = Term::F, K = Term::K, L = Term::L, S = 64 / L;
     constexpr int P = Term::P;
-    constexpr int NF = 3 + 9 * F;  // record: t0, dt, dir*t_new (-inf once the sample has finished), y[F], y1[F], k[7][F]
+    constexpr int NF = 3 + 9 * K;  // record: t0, dt, dir*t_new (-inf once the sample has finished), y[K], y1[K], k[7][K]
     extern __shared__ __align__(16) unsigned char smem_raw[];
     const int lane = threadIdx.x & 63;
     const int wave = threadIdx.x >> 6;
     const bool stepper = ((wave + (blockIdx.x >> 1)) & 1) == 0;
-    const long long b0 = (long long)blockIdx.x * 64;
-    const long long b = b0 + lane;
-    const int rows = (int)min((long long)64, p.batch - b0);
-    const bool live = lane < rows;
+    const long long b0 = (long long)blockIdx.x * S;
+    const int group = lane / L;  // the lane's sample among the wavefront's
+    const long long b = b0 + group;
+    const int rows = (int)min((long long)S, p.batch - b0);
+    const bool live = group < rows;
+    // the features of the lane (a lane beyond the last feature repeats it and stores nothing), and the lane that stores what
+    // the sample has one of
+    auto feature = [&](int i) { return L == 1 ? i : min(lane_feature<L>(), F - 1); };
+    const bool owns = L == 1 || lane_feature<L>() < F;
+    const bool first_lane = L == 1 || lane_feature<L>() == 0;
     const long long bs = live ? b : b0;
     const CtrlParams<T> &cp = p.cp;
     // Without evaluation points the reference reports the end point alone (adjoints.py:296-311): the
@@ -55,8 +71,8 @@ __global__ void __launch_bounds__(128) solve_pair_kernel(const SolveParams<T> p,
     const int E = end_only ? 1 : p.n_eval;
 
     T *rec = reinterpret_cast<T *>(smem_raw);                // [2][NF][64]
-    int *ctl = reinterpret_cast<int *>(rec + 2 * NF * 64);   // [2] "stepper is done" per phase
-    T *te_s = reinterpret_cast<T *>(ctl + 4);                // [E + 1][64] when STAGE_TE
+    int *ctl = reinterpret_cast<int *>(rec + 2 * NF * 64);   // [2] "stepper is done", by phase
+    T *te_s = reinterpret_cast<T *>(ctl + 4);                // [E + 1][S] when STAGE_TE
 
     const T ts = p.t_start[bs * p.ts_stride], te = p.t_end[bs * p.te_stride];
     const bool fwd = te > ts;
@@ -66,9 +82,9 @@ __global__ void __launch_bounds__(128) solve_pair_kernel(const SolveParams<T> p,
         // =============================== stepper ===============================
         Term rhs;
         rhs.load(p.params + bs * P, p.scalars);
-        T y[F], k[7][F];
+        T y[K], k[7][K];
 #pragma unroll
-        for (int f = 0; f < F; ++f) y[f] = p.y0[bs * F + f];
+        for (int f = 0; f < K; ++f) y[f] = p.y0[bs * F + feature(f)];
         const T tlo = tmin(ts, te), thi = tmax(te, ts);
         T t = ts, dt;
         if (p.dt0) {
@@ -78,7 +94,7 @@ __global__ void __launch_bounds__(128) solve_pair_kernel(const SolveParams<T> p,
             dt = initial_step<T, CTRL, Term>(cp, rhs, ts, y, dir, abs_(te - ts), k[0]);
         }
         dt = tclamp(dt, tlo - t, thi - t);
-        StepFactor<T, NHIST> step_factor;  // with the logarithms of the previous two accepted error ratios (both start at 1)
+        StepFactor<T, NHIST, L> step_factor;  // with the logarithms of the previous two accepted error ratios (both start at 1)
         const T dte_end = dir * te;
         int n_steps = 0, n_acc = 0;
         // The loop below uses the hardware's minimum and maximum, which is the reference's arithmetic as long as no
@@ -86,7 +102,7 @@ __global__ void __launch_bounds__(128) solve_pair_kernel(const SolveParams<T> p,
         // and so does one that produces a non-finite error ratio, step factor or step later.
         bool odd_start = !finite_(dt) || !finite_(ts) || !finite_(te);
 #pragma unroll
-        for (int f = 0; f < F; ++f) odd_start = odd_start || !finite_(y[f]) || !finite_(k[0][f]);
+        for (int f = 0; f < K; ++f) odd_start = odd_start || !finite_(y[f]) || !finite_(k[0][f]);
         // lanes whose sample is still stepping, and lanes whose sample needs the general kernel
         lanes_t active = lanes_where(live && !odd_start), bail_lanes = lanes_where(live && odd_start);
         const int step_limit = p.max_steps < TODE_HARD_STEP_LIMIT ? p.max_steps : TODE_HARD_STEP_LIMIT;
@@ -101,7 +117,17 @@ __global__ void __launch_bounds__(128) solve_pair_kernel(const SolveParams<T> p,
                 return;
             }
             if (!live) return;
-            record_entry<T, T, F>(p, at, b, t, dt, y, k[0], ratio_prev, ratio_prev_prev, running, n_acc);
+            if constexpr (L == 1) {
+                record_entry<T, T, F>(p, at, b, t, dt, y, k[0], ratio_prev, ratio_prev_prev, running, n_acc);
+            } else {
+                const long long i = at * p.batch + b;
+                if (owns) p.rec_y[i * F + feature(0)] = y[0], p.rec_k0[i * F + feature(0)] = k[0][0];
+                if (first_lane) {
+                    p.rec_t[i] = t, p.rec_dt[i] = dt;
+                    p.rec_prev[i] = ratio_prev, p.rec_pprev[i] = ratio_prev_prev;
+                    p.rec_running[i] = running ? 1 : 0, p.rec_n_accepted[i] = n_acc;
+                }
+            }
         };
 
         // A sample that has landed past t_end (t + (t_end - t) rounded upwards) keeps stepping in the reference's
@@ -110,19 +136,20 @@ __global__ void __launch_bounds__(128) solve_pair_kernel(const SolveParams<T> p,
         // as an inactive lane whose error ratio is looked at.
         lanes_t idle = 0;
         int phase = 0;
+        if (lane == 0) ctl[0] = ctl[1] = 0;
         for (;; ++phase) {
             const lanes_t counted = active | idle;
             if (counted) {
                 if (RECORD) keep(phase, holds(active));
                 // ---- stages (runge_kutta.py:255-263) ----
                 const T t0 = t;
-                T y1[F];
+                T y1[K];
 #pragma unroll
                 for (int i = 1; i < 7; ++i) {
                     T tn = fma_((T)Tab::c[i], dt, t0);
-                    T yi[F];
+                    T yi[K];
 #pragma unroll
-                    for (int f = 0; f < F; ++f) {
+                    for (int f = 0; f < K; ++f) {
                         T s = 0;
 #pragma unroll
                         for (int j = 0; j < i; ++j)
@@ -132,7 +159,7 @@ __global__ void __launch_bounds__(128) solve_pair_kernel(const SolveParams<T> p,
                     rhs(tn, yi, k[i]);
                     if (i == 6) {
 #pragma unroll
-                        for (int f = 0; f < F; ++f) y1[f] = yi[f];
+                        for (int f = 0; f < K; ++f) y1[f] = yi[f];
                     }
                 }
                 // hand the attempted step to the evaluator (everything it needs is known now)
@@ -140,19 +167,19 @@ __global__ void __launch_bounds__(128) solve_pair_kernel(const SolveParams<T> p,
                 r[0 * 64] = t0;
                 r[1 * 64] = dt;
 #pragma unroll
-                for (int f = 0; f < F; ++f) {
+                for (int f = 0; f < K; ++f) {
                     r[(3 + f) * 64] = y[f];
-                    if (METHOD != 1) r[(3 + F + f) * 64] = y1[f];  // (Tsit5's interpolant does not look at the step's result)
+                    if (METHOD != 1) r[(3 + K + f) * 64] = y1[f];  // (Tsit5's interpolant does not look at the step's result)
                 }
 #pragma unroll
                 for (int s = 0; s < 7; ++s)
 #pragma unroll
-                    for (int f = 0; f < F; ++f) r[(3 + 2 * F + s * F + f) * 64] = k[s][f];
+                    for (int f = 0; f < K; ++f) r[(3 + 2 * K + s * K + f) * 64] = k[s][f];
 
                 // ---- error estimate and step size control (step_size_controllers.py:370-429, 715-774) ----
                 lanes_t insane;  // (a NaN or infinite ratio is a non-success status: left to the general kernel)
                 T factor;
-                const T ratio = control_common<T, F, NHIST, Tab>(cp, dt, k, y, y1, counted, step_factor, e1, e2, e3, factor, insane);
+                const T ratio = control_common<T, F, K, L, NHIST, Tab>(cp, dt, k, y, y1, counted, step_factor, e1, e2, e3, factor, insane);
                 const lanes_t accept = lanes_where(ratio < (T)1), move = accept & active;
                 bail_lanes |= idle & insane;
                 idle = 0;
@@ -167,7 +194,7 @@ __global__ void __launch_bounds__(128) solve_pair_kernel(const SolveParams<T> p,
 
                 // ---- state update (adjoints.py:150-155, 247-255) ----
 #pragma unroll
-                for (int f = 0; f < F; ++f) {
+                for (int f = 0; f < K; ++f) {
                     y[f] = holds(move) ? y1[f] : y[f];
                     k[0][f] = holds(move) ? k[6][f] : k[0][f];
                 }
@@ -189,14 +216,14 @@ __global__ void __launch_bounds__(128) solve_pair_kernel(const SolveParams<T> p,
                     // such a sample is looked at in the next iteration
                     bool odd = end_only && !(t == te);
 #pragma unroll
-                    for (int f = 0; f < F; ++f) odd = odd || !settles_(y[f], k[0][f]);
+                    for (int f = 0; f < K; ++f) odd = odd || !settles_(y[f], k[0][f]);
                     const lanes_t finished = ended & ~failed, odd_lanes = lanes_where(odd);
                     bail_lanes |= failed | (finished & odd_lanes);
                     idle = finished & ~odd_lanes & ~lanes_where(t == te);
                     active &= ~ended;
                 }
             }
-            if (lane == 0) ctl[phase & 1] = counted ? 0 : 1;
+            if (!counted && lane == 0) ctl[phase & 1] = 1;  // (the evaluator may still be about to look at the other word)
             __syncthreads();
             if (!counted) break;
         }
@@ -207,14 +234,14 @@ __global__ void __launch_bounds__(128) solve_pair_kernel(const SolveParams<T> p,
             if (phase >= p.rec_capacity) record_full = true;
             bail = bail || record_full;
         }
-        if (live) {
+        if (live && first_lane) {
             o.n_steps[b] = n_steps;
             o.n_accepted[b] = n_acc;
             o.status[b] = 0;
-            if (end_only) {
+        }
+        if (live && owns && end_only) {
 #pragma unroll
-                for (int f = 0; f < F; ++f) p.y_idle[b * F + f] = y[f];
-            }
+            for (int f = 0; f < K; ++f) p.y_idle[b * F + feature(f)] = y[f];
         }
         int my_steps = live ? n_steps : 0, my_bail = (live && bail) ? 1 : 0;
 #pragma unroll
@@ -236,7 +263,7 @@ __global__ void __launch_bounds__(128) solve_pair_kernel(const SolveParams<T> p,
             int row = lane / E, e = lane - row * E;
             const int drow = 64 / E, de = 64 - drow * E;
             for (int g = lane; g < n; g += 64) {
-                te_s[e * 64 + row] = src[g];
+                te_s[e * S + row] = src[g];
                 e += de;
                 row += drow;
                 if (e >= E) {
@@ -250,31 +277,31 @@ __global__ void __launch_bounds__(128) solve_pair_kernel(const SolveParams<T> p,
         // step reaches: whether a step has passed the next point is one comparison.
         const T never = (T)__builtin_huge_val();
         bool bail = false;
-        const T te_first = end_only ? te : (STAGE_TE ? te_s[lane] : tev_g[0]);
+        const T te_first = end_only ? te : (STAGE_TE ? te_s[group] : tev_g[0]);
         if (!end_only) {
             T prev_te = dir * te_first;
-            if (STAGE_TE) te_s[lane] = prev_te;
+            if (STAGE_TE) te_s[group] = prev_te;
             for (int e = 1; e < E; ++e) {
-                const T cur = dir * (STAGE_TE ? te_s[e * 64 + lane] : tev_g[e]);
-                if (STAGE_TE) te_s[e * 64 + lane] = cur;
+                const T cur = dir * (STAGE_TE ? te_s[e * S + group] : tev_g[e]);
+                if (STAGE_TE) te_s[e * S + group] = cur;
                 if (!(cur >= prev_te)) bail = true;
                 prev_te = cur;
             }
-            if (STAGE_TE) te_s[E * 64 + lane] = never;
+            if (STAGE_TE) te_s[E * S + group] = never;
         }
         auto point = [&](int e) -> T {
             if (end_only) return e == 0 ? dir * te : never;
-            if (STAGE_TE) return te_s[e * 64 + lane];
+            if (STAGE_TE) return te_s[e * S + group];
             return e < E ? dir * tev_g[e] : never;
         };
         // (a workgroup's block of ys is far below 4 GiB: launch_pair)
         T *ys_block = p.ys + b0 * (long long)E * F;
-        const unsigned ys_row = (unsigned)(live ? lane : 0) * (unsigned)E;
+        const unsigned ys_row = (unsigned)(live ? group : 0) * (unsigned)E;
         int cursor = 0;
         if (te_first == ts) {
-            if (live) {
+            if (live && owns) {
 #pragma unroll
-                for (int f = 0; f < F; ++f) ys_block[ys_row * F + f] = p.y0[bs * F + f];
+                for (int f = 0; f < K; ++f) ys_block[ys_row * F + feature(f)] = p.y0[bs * F + feature(f)];
             }
             cursor = 1;
         }
@@ -288,25 +315,26 @@ __global__ void __launch_bounds__(128) solve_pair_kernel(const SolveParams<T> p,
             if (done) break;
             if (dt_new >= dte_next) {
                 const T t0 = r[0 * 64], dt = r[1 * 64];
-                T y[F], y1[F], k[7][F], q[5][F];
+                T y[K], y1[K], k[7][K], q[5][K];
 #pragma unroll
-                for (int f = 0; f < F; ++f) {
+                for (int f = 0; f < K; ++f) {
                     y[f] = r[(3 + f) * 64];
-                    y1[f] = METHOD != 1 ? r[(3 + F + f) * 64] : (T)0;
+                    y1[f] = METHOD != 1 ? r[(3 + K + f) * 64] : (T)0;
                 }
 #pragma unroll
                 for (int s = 0; s < 7; ++s)
 #pragma unroll
-                    for (int f = 0; f < F; ++f) k[s][f] = r[(3 + 2 * F + s * F + f) * 64];
-                quartic<T, F, METHOD, true>(dt, y, y1, k, q);
+                    for (int f = 0; f < K; ++f) k[s][f] = r[(3 + 2 * K + s * K + f) * 64];
+                quartic<T, K, METHOD, true>(dt, y, y1, k, q);
                 const StepPosition<T> position(t0, dt);
                 auto write_points = [&](auto plain) {
                     do {
-                        T out[F];
-                        quartic_at_unit<T, F>(q, position.template at<decltype(plain)::value>(dir, dte_next), out);
+                        T out[K];
+                        quartic_at_unit<T, K>(q, position.template at<decltype(plain)::value>(dir, dte_next), out);
                         T *row = ys_block + (ys_row + (unsigned)cursor) * F;
 #pragma unroll
-                        for (int f = 0; f < F; ++f) row[f] = out[f];
+                        for (int f = 0; f < K; ++f)
+                            if (owns) row[feature(f)] = out[f];
                         ++cursor;
                         dte_next = point(cursor);
                     } while (dt_new >= dte_next);
@@ -318,7 +346,7 @@ __global__ void __launch_bounds__(128) solve_pair_kernel(const SolveParams<T> p,
             }
         }
 
-        if (live) o.n_initialized[b] = cursor;
+        if (live && first_lane) o.n_initialized[b] = cursor;
         int my_bail = (live && bail) ? 1 : 0;
 #pragma unroll
         for (int off = 32; off > 0; off >>= 1) my_bail = max(my_bail, __shfl_xor(my_bail, off));
@@ -327,20 +355,30 @@ __global__ void __launch_bounds__(128) solve_pair_kernel(const SolveParams<T> p,
     publish_flags(p);
 }
 
+// The largest batch that takes this form.  One sample per lane: up to 2048 groups of 64 samples, above which the
+// single-wavefront kernel has three wavefronts per SIMD by itself.
+template <typename Term> constexpr long long pair_batch_limit() {
+    if constexpr (Term::L == 1)
+        return 2048 * 64;
+    else
+        return Term::most_samples;
+}
+
 template <typename T, int METHOD, int CTRL, typename Term>
 static int launch_pair(const tode_solve_args &a, const tode_controller &c, const PairOut<T> &o, hipStream_t stream, bool *used) {
     *used = false;
-    constexpr int NF = 3 + 9 * Term::F;
-    const long long blocks = (a.batch + 63) / 64;
-    // worthwhile only while the single-wave kernel would leave SIMDs with <= 2 wavefronts
-    if (blocks == 0 || blocks > 2 * 1024) return TODE_OK;
+    constexpr int L = Term::L, S = 64 / L, NF = 3 + 9 * Term::K;
+    const long long blocks = (a.batch + S - 1) / S;
+    if (blocks == 0 || a.batch > pair_batch_limit<Term>()) return TODE_OK;
     const size_t rec_bytes = (size_t)2 * NF * 64 * sizeof(T) + 16;
-    const size_t te_bytes = a.n_eval > 0 ? ((size_t)a.n_eval + 1) * 64 * sizeof(T) : 0;
+    const size_t te_bytes = a.n_eval > 0 ? ((size_t)a.n_eval + 1) * S * sizeof(T) : 0;
     if ((size_t)a.n_eval * Term::F >= ((size_t)1 << 24)) return TODE_OK;  // (32-bit offsets into a workgroup's block of ys)
-    // LDS: up to four workgroups (eight wavefronts) have to share a compute unit, fewer in a batch that does not have them
+    // LDS: up to four workgroups per compute unit for every 64 samples of theirs, fewer in a batch that does not have them
     const long long per_cu = (blocks + 255) / 256;
-    const size_t budget = (size_t)(160 * 1024) / (size_t)(per_cu < 4 ? per_cu : 4) - 512;
-    if (rec_bytes > 36 * 1024) return TODE_OK;  // (four features in float64: the records alone would fill a quarter of it)
+    const size_t budget = (size_t)(160 * 1024) / (size_t)(per_cu < 4 * L ? per_cu : 4 * L) - 512;
+    if (rec_bytes > 36 * 1024) return TODE_OK;  // (four features in float64, one sample per lane: the records alone would fill a quarter of it)
+    // (the same problem without evaluation points stays with the general kernel)
+    if (L > 1 && a.n_eval == 0 && Term::F * sizeof(T) > 24) return TODE_OK;
     const bool stage_te = rec_bytes + te_bytes <= budget;
     const size_t lds = rec_bytes + (stage_te ? te_bytes : 0);
     constexpr bool RECORD = TODE_INSTANTIATE_RECORD != 0;
@@ -385,17 +423,22 @@ static int pair_term(const tode_solve_args &a, const tode_controller &c, int64_t
     switch (a.term) {
     case TODE_TERM_VAN_DER_POL:
         if (a.n_features != 2 || a.n_params != 1) return TODE_OK;
-        return pair_mc<T, VanDerPolTerm<T>>(a, c, o, s, used);
+        return pair_mc<T, TODE_PAIR_TERM(VanDerPol)<T>>(a, c, o, s, used);
     case TODE_TERM_LORENZ63:
         if (a.n_features != 3 || a.n_params != 1) return TODE_OK;
-        return pair_mc<T, Lorenz63Term<T>>(a, c, o, s, used);
+        return pair_mc<T, TODE_PAIR_TERM(Lorenz63)<T>>(a, c, o, s, used);
     case TODE_TERM_LINEAR_DECAY:
         if (a.n_params != a.n_features) return TODE_OK;
         switch (a.n_features) {
-        case 1: return pair_mc<T, LinearDecayTerm<T, 1>>(a, c, o, s, used);
-        case 2: return pair_mc<T, LinearDecayTerm<T, 2>>(a, c, o, s, used);
-        case 3: return pair_mc<T, LinearDecayTerm<T, 3>>(a, c, o, s, used);
-        case 4: return pair_mc<T, LinearDecayTerm<T, 4>>(a, c, o, s, used);
+#if !TODE_INSTANTIATE_LANES
+        case 1: return pair_mc<T, TODE_PAIR_TERM(LinearDecay)<T, 1>>(a, c, o, s, used);
+#endif
+        case 2: return pair_mc<T, TODE_PAIR_TERM(LinearDecay)<T, 2>>(a, c, o, s, used);
+        case 3: return pair_mc<T, TODE_PAIR_TERM(LinearDecay)<T, 3>>(a, c, o, s, used);
+        case 4:
+            // (with the record, four float64 features stay with the single-wavefront kernel in either form)
+            if (TODE_INSTANTIATE_LANES && TODE_INSTANTIATE_RECORD && sizeof(T) == 8) return TODE_OK;
+            return pair_mc<T, TODE_PAIR_TERM(LinearDecay)<T, 4>>(a, c, o, s, used);
         default: return TODE_OK;
         }
     default:
@@ -403,11 +446,16 @@ static int pair_term(const tode_solve_args &a, const tode_controller &c, int64_t
     }
 }
 
-// (each translation unit instantiates one type, with or without the record: TODE_INSTANTIATE_RECORD)
+// (each translation unit instantiates one type and form, with or without the record: TODE_INSTANTIATE_LANES, ..._RECORD)
 #if TODE_INSTANTIATE_RECORD
-#define TODE_PAIR_ENTRY(name) name##_record
+#define TODE_PAIR_ENTRY(name) TODE_PAIR_FORM(name, _record)
 #else
-#define TODE_PAIR_ENTRY(name) name
+#define TODE_PAIR_ENTRY(name) TODE_PAIR_FORM(name, )
+#endif
+#if TODE_INSTANTIATE_LANES
+#define TODE_PAIR_FORM(name, suffix) name##_lanes##suffix
+#else
+#define TODE_PAIR_FORM(name, suffix) name##suffix
 #endif
 #if TODE_INSTANTIATE_F32
 int TODE_PAIR_ENTRY(solve_pair_f32)(const tode_solve_args &a, const tode_controller &c, int64_t *ns, int64_t *na, int64_t *ni, int64_t *st, hipStream_t s, bool *used) {

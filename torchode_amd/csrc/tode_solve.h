@@ -18,7 +18,7 @@ namespace tode {
 // rounding, matching an eager evaluation of the torch expression in the comment.
 // ---------------------------------------------------------------------------
 template <typename T, int F_> struct LinearDecayTerm {  // (-k) * y
-    static constexpr int F = F_;
+    static constexpr int F = F_, K = F_, L = 1;
     static constexpr int P = F_;
     T nk[F_];
     __device__ __forceinline__ void load(const T *par, const double *) {
@@ -40,7 +40,7 @@ template <typename T, int F_> struct LinearDecayTerm {  // (-k) * y
 };
 
 template <typename T> struct VanDerPolTerm {  // dx = v ; dv = ((mu*(1-(x*x)))*v)-x
-    static constexpr int F = 2;
+    static constexpr int F = 2, K = 2, L = 1;
     static constexpr int P = 1;
     T mu;
     __device__ __forceinline__ void load(const T *par, const double *) { mu = par[0]; }
@@ -62,7 +62,7 @@ template <typename T> struct VanDerPolTerm {  // dx = v ; dv = ((mu*(1-(x*x)))*v
 };
 
 template <typename T> struct Lorenz63Term {  // dx=sigma*(y-x); dy=(x*(rho-z))-y; dz=(x*y)-(beta*z)
-    static constexpr int F = 3;
+    static constexpr int F = 3, K = 3, L = 1;
     static constexpr int P = 1;
     T rho, sigma, beta;
     __device__ __forceinline__ void load(const T *par, const double *sc) {
@@ -87,6 +87,102 @@ template <typename T> struct Lorenz63Term {  // dx=sigma*(y-x); dy=(x*(rho-z))-y
         gy[1] = sigma * g[0] - g[1] + x * g[2];
         gy[2] = -(x * g[1]) - beta * g[2];
         gpar[0] += x * g[1];
+    }
+};
+
+// ---------------------------------------------------------------------------
+// The same systems with a sample spread over L neighbouring lanes, one feature each (K = 1; with three features the fourth
+// lane repeats the third): what a sample does per feature then takes one instruction where it took F, at the price of L
+// times the wavefronts.  A lane gets the other features by quad permutations (DPP).  Same operations on the same operands.
+// A SIMD issues for one wavefront every five cycles and for two or more every two to two and a half: while a batch leaves
+// most SIMDs with one or two wavefronts, more and shorter ones cost nothing.  most_samples: where that ends, measured in
+// tode_pair.hip (kernel, one sample per lane against spread; Tsit5 + PID for Van der Pol, Dopri5 + integral otherwise):
+//   Van der Pol float32  B = 4096 90 -> 68 us, 20 000 93 -> 77, 32 768 98 -> 87, 40 000 100 -> 109
+//   Van der Pol float64  B = 4096 123 -> 97 us, 20 011 146 -> 114, 32 768 157 -> 123, 65 536 184 -> 210
+//   Lorenz float32       B = 4096 41 -> 36 us, 8192 40 -> 40, 11 000 40 -> 45
+//   decay, 2 features    B = 8192 27.5 -> 25.6 us, 16 384 30 -> 31
+//   decay, 4, float32    B = 256 33 -> 21 us, 8192 33 -> 30, 11 000 34 -> 34
+//   decay, 4, float64    B = 256 52 -> 27 us (against tode_fast.hip: one sample per lane does not fit), 16 384 54 -> 49, 20 000 55 -> 55
+// ---------------------------------------------------------------------------
+template <int L> __device__ __forceinline__ int lane_feature() { return threadIdx.x & (L - 1); }
+
+// The value that lane J of this lane's group of L (two or four neighbours) holds.
+template <int L, int J> __device__ __forceinline__ int from_lane(int v) {
+    constexpr int control = L == 2 ? (J | (J << 2) | ((2 + J) << 4) | ((2 + J) << 6)) : (J | (J << 2) | (J << 4) | (J << 6));
+    return __builtin_amdgcn_mov_dpp(v, control, 0xf, 0xf, true);
+}
+template <int L, int J> __device__ __forceinline__ float from_lane(float v) { return __int_as_float(from_lane<L, J>(__float_as_int(v))); }
+template <int L, int J> __device__ __forceinline__ double from_lane(double v) {
+    return __hiloint2double(from_lane<L, J>(__double2hiint(v)), from_lane<L, J>(__double2loint(v)));
+}
+
+// The value of the other lane of a pair of neighbours.
+__device__ __forceinline__ int swap_lanes(int v) { return __builtin_amdgcn_mov_dpp(v, 1 | (0 << 2) | (3 << 4) | (2 << 6), 0xf, 0xf, true); }
+__device__ __forceinline__ float swap_lanes(float v) { return __int_as_float(swap_lanes(__float_as_int(v))); }
+__device__ __forceinline__ double swap_lanes(double v) { return __hiloint2double(swap_lanes(__double2hiint(v)), swap_lanes(__double2loint(v))); }
+
+// All F features of a sample from the K a lane holds.
+template <int F, int L, typename T, int K> __device__ __forceinline__ void gather_features(const T (&own)[K], T (&all)[F]) {
+    if constexpr (L == 1) {
+#pragma unroll
+        for (int f = 0; f < F; ++f) all[f] = own[f];
+    } else {
+        static_assert(K == 1 && F <= 4, "one feature per lane of a quad");
+        if constexpr (F > 0) all[0] = from_lane<L, 0>(own[0]);
+        if constexpr (F > 1) all[1] = from_lane<L, 1>(own[0]);
+        if constexpr (F > 2) all[2] = from_lane<L, 2>(own[0]);
+        if constexpr (F > 3) all[3] = from_lane<L, 3>(own[0]);
+    }
+}
+
+template <typename T, int F_> struct LinearDecayLanes {
+    static constexpr int F = F_, K = 1, L = F_ == 2 ? 2 : 4;
+    static constexpr int P = F_;
+    static constexpr int most_samples = F_ == 2 ? 12288 : (F_ == 4 && sizeof(T) == 8) ? 16384 : 8192;
+    T nk;
+    __device__ __forceinline__ void load(const T *par, const double *) { nk = -par[min(lane_feature<L>(), F - 1)]; }
+    __device__ __forceinline__ void operator()(T, const T (&y)[1], T (&dy)[1]) const { dy[0] = nk * y[0]; }
+};
+
+template <typename T> struct VanDerPolLanes {
+    static constexpr int F = 2, K = 1, L = 2;
+    static constexpr int P = 1;
+    static constexpr int most_samples = 32768;
+    T mu;
+    bool second;
+    __device__ __forceinline__ void load(const T *par, const double *) { mu = par[0], second = lane_feature<L>() == 1; }
+    __device__ __forceinline__ void operator()(T, const T (&y)[1], T (&dy)[1]) const {
+        const T other = swap_lanes(y[0]);  // the second lane holds v and gets x, the first gets v
+        const T xx = other * other;
+        const T om = (T)1 - xx;
+        const T m1 = mu * om;
+        const T m2 = m1 * y[0];
+        const T dv = m2 - other;
+        dy[0] = second ? dv : other;
+    }
+};
+
+template <typename T> struct Lorenz63Lanes {
+    static constexpr int F = 3, K = 1, L = 4;
+    static constexpr int P = 1;
+    static constexpr int most_samples = 8192;
+    T rho, sigma, beta;
+    bool first, second;
+    __device__ __forceinline__ void load(const T *par, const double *sc) {
+        rho = par[0];
+        sigma = (T)sc[0];
+        beta = (T)sc[1];
+        first = lane_feature<L>() == 0, second = lane_feature<L>() == 1;
+    }
+    __device__ __forceinline__ void operator()(T, const T (&y)[1], T (&dy)[1]) const {
+        T all[3];
+        gather_features<3, 4>(y, all);
+        const T x = all[0], yy = all[1], z = all[2];
+        const T a = x * (second ? rho - z : yy);     // x (rho - z) or x y
+        const T b = second ? yy : beta * z;
+        const T d = a - b;
+        const T dx = sigma * (yy - x);
+        dy[0] = first ? dx : d;
     }
 };
 
@@ -127,37 +223,152 @@ __device__ __forceinline__ void record_entry(const SolveParams<T, TT> &p, long l
     p.rec_running[i] = running ? 1 : 0, p.rec_n_accepted[i] = n_accepted;
 }
 
+// The step factor's powers (step_size_controllers.py:289-294, 598-620) for the kernels that keep
+// the history of accepted error ratios as logarithms: safety * ratio^e1 [* prev^e2 [* prev_prev^e3]],
+// multiplied in this order.  `ratio` is positive and finite.  NHIST = number of history factors.
+// L > 1: the L lanes of a sample form one of the powers each.
+template <typename T, int NHIST, int L = 1> struct StepFactor {
+    DW<T> lg, lg_prev, lg_pprev;
+    __device__ __forceinline__ StepFactor() : lg(dw((T)0, (T)0)), lg_prev(dw((T)0, (T)0)), lg_pprev(dw((T)0, (T)0)) {}
+    __device__ __forceinline__ T operator()(T safety, T ratio, T e1, T e2, T e3) {
+        lg = logk(ratio);
+        T factor = safety * powk<T>(lg, e1);
+        if (NHIST >= 1) factor = factor * powk<T>(lg_prev, e2);
+        if (NHIST >= 2) factor = factor * powk<T>(lg_pprev, e3);
+        return factor;
+    }
+    // the same for a ratio in [2^-50, 2^50] and exponents of at most 1/2 in magnitude
+    __device__ __forceinline__ T plain(T safety, T ratio, T e1, T e2, T e3) {
+        lg = logk<true>(ratio);
+        if constexpr (L > 1 && NHIST >= 1) {
+            const int j = lane_feature<L>();
+            DW<T> mine = dw(j == 0 ? lg.x : lg_prev.x, j == 0 ? lg.y : lg_prev.y);
+            T e = j == 0 ? e1 : e2;
+            if constexpr (L > 2 && NHIST >= 2) mine = dw(j == 2 ? lg_pprev.x : mine.x, j == 2 ? lg_pprev.y : mine.y), e = j == 2 ? e3 : e;
+            const T power = expk<true>(dw_mul(mine, e));
+            T factor = safety * from_lane<L, 0>(power);
+            factor = factor * from_lane<L, 1>(power);
+            if constexpr (L > 2 && NHIST >= 2) factor = factor * from_lane<L, 2>(power);
+            if constexpr (L == 2 && NHIST >= 2) factor = factor * expk<true>(dw_mul(lg_pprev, e3));
+            return factor;
+        }
+        T factor = safety * expk<true>(dw_mul(lg, e1));
+        if (NHIST >= 1) factor = factor * expk<true>(dw_mul(lg_prev, e2));
+        if (NHIST >= 2) factor = factor * expk<true>(dw_mul(lg_pprev, e3));
+        return factor;
+    }
+    // the ratio just used becomes the previous one where `shift` (an accepted step of a running sample)
+    __device__ __forceinline__ void shift(bool s) {
+        if (NHIST >= 2) {
+            lg_pprev.x = s ? lg_prev.x : lg_pprev.x;
+            lg_pprev.y = s ? lg_prev.y : lg_pprev.y;
+        }
+        if (NHIST >= 1) {
+            lg_prev.x = s ? lg.x : lg_prev.x;
+            lg_prev.y = s ? lg.y : lg_prev.y;
+        }
+    }
+};
+
+// Error ratio and step factor (before its clip) for the kernels that cover the common case only: the operations of
+// error_ratio() and StepFactor.  With the short forms above wherever every lane that counts (`counted`: its sample is
+// still stepping, or sits through an idle step) has its operands in their ranges, which nearly every iteration of an
+// ordinary solve does; otherwise, for the whole wavefront, with the general ones.  The test: every scaled error zero or
+// at least 2^-60 (for float64, 2^-400: nothing below 2^-1022 hides in a zero upper half that could reach the sum of
+// squares), their sum of squares in [2^-100, 2^100] -- which a NaN anywhere in the step fails: it reaches the error
+// estimate through the last stage.  `insane`: the lanes whose ratio is not finite or whose factor is not a number; the
+// caller must leave the common case there and not use the values.
+template <typename T, int F, int K, int L, int NHIST, typename Tab>
+__device__ __forceinline__ T control_common(const CtrlParams<T> &cp, T dt, const T (&k)[7][K], const T (&y0)[K], const T (&y1)[K], lanes_t counted,
+                                            StepFactor<T, NHIST, L> &step_factor, T e1, T e2, T e3, T &factor, lanes_t &insane) {
+    using Div = DivSqrtFeatures<T, F>;
+    auto sum_of_squares = [](const T (&v)[K]) {
+        T x[F], acc = 0;
+        gather_features<F, L>(v, x);
+#pragma unroll
+        for (int f = 0; f < F; ++f) {
+            if (F <= 3)
+                acc = fma_(x[f], x[f], acc);
+            else {
+                const T sq = x[f] * x[f];
+                acc = acc + sq;
+            }
+        }
+        return acc;
+    };
+    T err[K], q[K], x[K], eb[K];
+    weighted_k<T, K, Tab, -1, true, true>(dt, k, err);
+    unsigned smallest = 0xffffffffu;
+#pragma unroll
+    for (int f = 0; f < K; ++f) {
+        eb[f] = fma_(cp.rtol, max_abs(y0[f], y1[f]), cp.atol);
+        q[f] = quotient_plain(abs_(err[f]), eb[f]);
+        x[f] = Div::fast(q[f]);
+        smallest = min(smallest, high_bits(q[f]) - 1u);  // (zero wraps round to the largest)
+    }
+    T acc = sum_of_squares(x);
+    constexpr unsigned lowest = power_of_two_bits<T>(sizeof(T) == 4 ? -60 : -400) - 1u;
+    constexpr unsigned from = power_of_two_bits<T>(-100), width = power_of_two_bits<T>(100) - from;
+    const lanes_t outside = lanes_where(smallest < lowest) | lanes_where(high_bits(acc) - from >= width);
+    T ratio = sqrt_plain(acc);
+    factor = step_factor.plain(cp.safety, ratio, e1, e2, e3);
+    insane = 0;
+    if (__builtin_expect((counted & outside) != 0 || !cp.plain, 0)) {
+        bool nan = false;
+        asm volatile("" : "+v"(dt));  // (the error estimate formed again: keeping it for this rare branch would cost F registers)
+        weighted_k<T, K, Tab, -1, true, true>(dt, k, err);
+#pragma unroll
+        for (int f = 0; f < K; ++f) {
+            nan = nan || __builtin_isunordered(y0[f], y1[f]);
+            x[f] = (abs_(err[f]) / fma_(cp.rtol, hwmax(abs_(y0[f]), abs_(y1[f])), cp.atol));
+            x[f] = Div::exact(x[f]);
+        }
+        acc = sum_of_squares(x);
+        const T r = sqrt_(acc);
+        ratio = hwmax(r, (T)1e-38);
+        const bool sane = !nan && r == r && ratio < (T)__builtin_huge_val();  // (the ratio is at least 1e-38)
+        factor = step_factor(cp.safety, sane ? ratio : (T)1, e1, e2, e3);
+        insane = ~lanes_where(sane && factor == factor);  // (a product of an underflowed and an overflowed power)
+    }
+    return ratio;
+}
+
 // Start step (step_size_controllers.py:431-490 integral, 776-835 PID; the integral
 // copy maps h0 == 0 to d2 = inf, the PID copy does not).
 template <typename T, int CTRL, typename Term>
-__device__ __forceinline__ T initial_step(const CtrlParams<T> &cp, const Term &rhs, T t0, const T (&y0)[Term::F], T dir, T span,
-                                          T (&f0)[Term::F]) {
-    constexpr int F = Term::F;
+__device__ __forceinline__ T initial_step(const CtrlParams<T> &cp, const Term &rhs, T t0, const T (&y0)[Term::K], T dir, T span,
+                                          T (&f0)[Term::K]) {
+    constexpr int F = Term::F, K = Term::K, L = Term::L;
+    auto norm = [](const T (&v)[K]) {
+        T all[F];
+        gather_features<F, L>(v, all);
+        return rms<T, F>(all);
+    };
     rhs(t0, y0, f0);
-    T inv[F], w[F];
+    T inv[K], w[K];
 #pragma unroll
-    for (int f = 0; f < F; ++f) inv[f] = (T)1 / fma_(cp.rtol, abs_(y0[f]), cp.atol);
+    for (int f = 0; f < K; ++f) inv[f] = (T)1 / fma_(cp.rtol, abs_(y0[f]), cp.atol);
 #pragma unroll
-    for (int f = 0; f < F; ++f) w[f] = y0[f] * inv[f];
-    T d0 = rms<T, F>(w);
+    for (int f = 0; f < K; ++f) w[f] = y0[f] * inv[f];
+    T d0 = norm(w);
 #pragma unroll
-    for (int f = 0; f < F; ++f) w[f] = f0[f] * inv[f];
-    T d1 = rms<T, F>(w);
+    for (int f = 0; f < K; ++f) w[f] = f0[f] * inv[f];
+    T d1 = norm(w);
     const T tiny = (T)1e-6;
     T h0 = (d0 < (T)1e-5 || d1 < (T)1e-5) ? tiny : ((T)0.01 * d0) / d1;
     h0 = tmin(h0, span);
     T dh = dir * h0;
-    T y1[F], f1[F];
+    T y1[K], f1[K];
 #pragma unroll
-    for (int f = 0; f < F; ++f) y1[f] = fma_(dh, f0[f], y0[f]);
+    for (int f = 0; f < K; ++f) y1[f] = fma_(dh, f0[f], y0[f]);
     T t1 = fma_(dir, h0, t0);
     rhs(t1, y1, f1);
 #pragma unroll
-    for (int f = 0; f < F; ++f) {
+    for (int f = 0; f < K; ++f) {
         T df = f1[f] - f0[f];
         w[f] = df * inv[f];
     }
-    T d2 = rms<T, F>(w) / h0;
+    T d2 = norm(w) / h0;
     if (CTRL == 0 && h0 == (T)0) d2 = (T)__builtin_huge_val();
     T m = tmax(d1, d2);
     T h1;
@@ -170,7 +381,6 @@ __device__ __forceinline__ T initial_step(const CtrlParams<T> &cp, const Term &r
     }
     return dir * tmin((T)100 * h0, h1);
 }
-
 
 // Pieces of the start step and of the dense output shared by the per-call operators and the
 // whole-solve kernels for long rows.
