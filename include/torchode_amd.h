@@ -393,6 +393,41 @@ int tode_mlp_pack_weights(const void *raw, int64_t n_raw, int32_t matrix_inputs,
  */
 int tode_mlp_pack_weights_for(const void *raw, int64_t n_raw, int32_t n_features, int32_t matrix_inputs, void *packed, void *stream);
 
+/*
+ * Reverse sweep with the perceptron as right-hand side (float32, n_features = 1 ... 64, n_hidden = 1 ... 256): what
+ * surrounds tode_step_finish_backward for one recorded iteration.  Per iteration: tode_mlp_stages forms the six stages
+ * again from the recorded t, dt, y, k0 (y1 is the last stage input); tode_step_finish_backward leaves the cotangents g_*;
+ * tode_mlp_stages_backward takes them through the stages and, where `sums` is not null, adds the iteration's share to the
+ * weights' gradients (accumulate = 0: the sweep's first call, which sets them).  After the last iteration
+ * tode_mlp_weight_gradients adds up the splits: out = W1 [n_hidden x (n_features + 1)] | b1 | W2 | b2.
+ * tode_mlp_pack_weights_reverse packs the same raw weights as tode_mlp_pack_weights_for for the way back.
+ */
+#define TODE_MLP_REVERSE_PACKED_SIZE (144 * 256)
+#define TODE_MLP_SUMS_SIZE (64 * 256 + 256 + 256 + 64 * 256 + 64)
+#define TODE_MLP_MAX_SPLITS 1024
+typedef struct tode_mlp_reverse {
+    int32_t method;              /* TODE_DOPRI5 or TODE_TSIT5 */
+    int32_t n_features, n_hidden;
+    int32_t splits;              /* shares of the rows for the weights' gradients, at most TODE_MLP_MAX_SPLITS */
+    int64_t batch;
+    const void *packed, *packed_reverse;  /* tode_mlp_pack_weights_for (float32), tode_mlp_pack_weights_reverse */
+    const void *t, *dt;          /* [B] the recorded state before the iteration */
+    const void *y, *k0;          /* [B,F] */
+    void *k;                     /* [6,B,F] k_1 .. k_6 */
+    void *stage_inputs;          /* [6,B,F] */
+    void *stage_times;           /* [6,B] */
+    void *hidden;                /* [6,B,256] */
+    void *hidden_cotangents;     /* [6,B,256], null where no weight wants a gradient */
+    void *g_k;                   /* [7,B,F] in and out */
+    void *g_y, *g_y1;            /* [B,F] in (and out: g_y) */
+    void *g_t, *g_dt;            /* [B] in and out */
+    void *sums;                  /* [splits, TODE_MLP_SUMS_SIZE], null where no weight wants a gradient */
+} tode_mlp_reverse;
+int tode_mlp_pack_weights_reverse(const void *raw, int64_t n_raw, int32_t n_features, void *packed, void *stream);
+int tode_mlp_stages(const tode_mlp_reverse *p, void *stream);
+int tode_mlp_stages_backward(const tode_mlp_reverse *p, int32_t accumulate, void *stream);
+int tode_mlp_weight_gradients(const tode_mlp_reverse *p, void *out, void *stream);
+
 /* ------------------------------------------------------------------------- */
 /* Per-step kernels around a right-hand side that lives outside the library   */
 /* ------------------------------------------------------------------------- */

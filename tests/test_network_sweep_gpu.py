@@ -1,0 +1,53 @@
+"""The reverse sweep's kernels for the perceptron (tode_mlp_stages, tode_mlp_stages_backward, tode_mlp_weight_gradients)
+against the same sweep with torch's evaluations of the network and autograd's vector-Jacobian products, over the same
+record, at the edges of their tiles: one sample, a full tile of 16 and one more, more tiles than workgroups; one
+feature, rows that are no multiple of four, all 64; one hidden unit, 255, 256."""
+import math
+
+import pytest
+import torch
+
+import torchode_amd as to
+
+pytestmark = pytest.mark.gpu
+
+
+def _gradients(B, F, H, E, method, controller, through, network, hook=False):
+    g = torch.Generator("cuda").manual_seed(B + F + H)
+    rand = lambda *shape: torch.rand(shape, generator=g, dtype=torch.float64, device="cuda")
+    bound = lambda n, *shape: ((2 * rand(*shape) - 1) * math.sqrt(6.0 / n)).float().requires_grad_()
+    weights = [bound(F + 1 + H, H, F + 1), bound(F + 1 + H, H), bound(F + H, F, H), bound(F + H, F)]
+    y0 = (2 * rand(B, F) - 1).float().requires_grad_()
+    t1 = (0.5 + 0.5 * rand(B)).float()
+    times = dict(t_eval=(t1[:, None] * torch.linspace(0, 1, E, device="cuda")[None, :])) if E else dict(t_start=torch.zeros_like(t1), t_end=t1)
+    f = to.MLPField(*weights)
+    if hook:
+        f.register_forward_hook(lambda module, inputs, output: 2 * output)
+    solver = to.AutoDiffAdjoint(method(), controller(), backprop_through_step_size_control=through)
+    solver.backward_network_kernels = network
+    sol = solver.solve(to.InitialValueProblem(y0, **times), to.ODETerm(f))
+    cotangent = (2 * rand(*sol.ys.shape) - 1).float()
+    return torch.autograd.grad(sol.ys, [y0, *weights], cotangent)
+
+
+@pytest.mark.parametrize("method, controller", [(to.Dopri5, lambda: to.IntegralController(1e-5, 1e-3)), (to.Tsit5, lambda: to.PIDController(1e-5, 1e-3, 0.2, 0.5, 0.0))],
+                         ids=["dopri5-integral", "tsit5-pid"])  # fmt: skip
+@pytest.mark.parametrize("B, F, H, E", [(1, 1, 1, 4), (16, 64, 256, 7), (17, 63, 255, 0), (33, 6, 3, 5), (4113, 64, 256, 3), (300, 4, 100, 20)])
+def test_network_kernels_against_autograd(B, F, H, E, method, controller):
+    """Same record, same decisions.  With the step sizes held constant the two differ by the roundings of float32 sums of at
+    most 6 * 4113 rows or 256 units: 2^-24 times the square root of their number, with a factor of two in hand for
+    products of several such sums, 2e-5 of the 2-norm.  Through the step size rule those are amplified by the
+    derivatives of powers of error ratios (2e-2, as for the other pairs of sweeps)."""
+    for through, bound in ((False, 2e-5), (True, 2e-2)):
+        got = _gradients(B, F, H, E, method, controller, through, True)
+        want = _gradients(B, F, H, E, method, controller, through, False)
+        for a, b in zip(got, want):
+            assert a.shape == b.shape and bool(a.isfinite().all())
+            assert float((a.double() - b.double()).norm()) <= bound * float(b.double().norm()), (through, tuple(a.shape))
+
+
+def test_a_hook_on_the_network_is_called():
+    """A hook that doubles what the network returns: the sweep evaluates the module then, and both settings agree exactly."""
+    got, want = (_gradients(17, 8, 16, 4, to.Dopri5, lambda: to.IntegralController(1e-5, 1e-3), False, network, hook=True) for network in (True, False))
+    for a, b in zip(got, want):
+        assert torch.equal(a, b)

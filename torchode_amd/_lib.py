@@ -16,6 +16,7 @@ LIB_PATH = os.path.join(_HERE, "libtorchode_amd.so")
 ABI_VERSION = 23
 END_ONLY_MAX_BATCH = 2048 * 64  # TODE_END_ONLY_MAX_BATCH
 MLP_PACKED_SIZE = {"float32": 152 * 256, "bfloat16": 92 * 256}
+MLP_SUMS_SIZE, MLP_REVERSE_PACKED_SIZE = 64 * 256 + 256 + 256 + 64 * 256 + 64, 144 * 256  # TODE_MLP_*_SIZE
 MLP_INPUTS = {"float32": 0, "bfloat16": 1}
 F32, F64 = 0, 1
 DOPRI5, TSIT5, HEUN, EULER = 0, 1, 2, 3
@@ -45,6 +46,10 @@ EXPORTS = (
     "tode_solve_workspace_bytes",
     "tode_mlp_pack_weights",
     "tode_mlp_pack_weights_for",
+    "tode_mlp_pack_weights_reverse",
+    "tode_mlp_stages",
+    "tode_mlp_stages_backward",
+    "tode_mlp_weight_gradients",
     "tode_select_end_point",
     "tode_step_begin",
     "tode_step_stage",
@@ -199,6 +204,16 @@ class StepState(C.Structure):
     ]
 
 
+class MlpReverse(C.Structure):
+    """struct tode_mlp_reverse"""
+
+    _fields_ = [(name, C.c_int32) for name in ("method", "n_features", "n_hidden", "splits")] + [("batch", C.c_int64)] + [
+        (name, C.c_void_p)
+        for name in ("packed", "packed_reverse", "t", "dt", "y", "k0", "k", "stage_inputs", "stage_times", "hidden", "hidden_cotangents",
+                     "g_k", "g_y", "g_y1", "g_t", "g_dt", "sums")
+    ]  # fmt: skip
+
+
 class StepAdjoint(C.Structure):
     """struct tode_step_adjoint"""
 
@@ -333,6 +348,14 @@ def load():
         lib.tode_mlp_pack_weights.argtypes = [C.c_void_p, C.c_int64, C.c_int32, C.c_void_p, C.c_void_p]
         lib.tode_mlp_pack_weights_for.restype = C.c_int
         lib.tode_mlp_pack_weights_for.argtypes = [C.c_void_p, C.c_int64, C.c_int32, C.c_int32, C.c_void_p, C.c_void_p]
+        lib.tode_mlp_pack_weights_reverse.restype = C.c_int
+        lib.tode_mlp_pack_weights_reverse.argtypes = [C.c_void_p, C.c_int64, C.c_int32, C.c_void_p, C.c_void_p]
+        lib.tode_mlp_stages.restype = C.c_int
+        lib.tode_mlp_stages.argtypes = [C.POINTER(MlpReverse), C.c_void_p]
+        lib.tode_mlp_stages_backward.restype = C.c_int
+        lib.tode_mlp_stages_backward.argtypes = [C.POINTER(MlpReverse), C.c_int32, C.c_void_p]
+        lib.tode_mlp_weight_gradients.restype = C.c_int
+        lib.tode_mlp_weight_gradients.argtypes = [C.POINTER(MlpReverse), C.c_void_p, C.c_void_p]
         lib.tode_solve_builtin_fast_static.restype = C.c_int
         lib.tode_solve_builtin_fast_static.argtypes = [C.POINTER(SolveArgs), C.POINTER(Controller)] + [C.c_void_p] * 6
         lib.tode_solve_builtin_fast_sync.restype = C.c_int

@@ -498,6 +498,84 @@ def reverse_sweep_whole(adjoint, replay: Replay, term, problem, dt0, record, gra
     return adj, grad_params
 
 
+class NetworkSweep:
+    """The kernels of a reverse sweep with the library's own perceptron as right-hand side (tode_mlp_stages,
+    tode_mlp_stages_backward): the six stages of an iteration in one launch, their reverse in another, the weights'
+    gradients in a third, where autograd takes some two hundred."""
+
+    @staticmethod
+    def takes(adjoint, term, y0, times) -> bool:
+        """An ``MLPField`` as the library ships it, in the shapes the kernels are built for: a subclass, a replaced
+        ``forward`` or a hook on the module (or on all modules) is the user's code and is called as such."""
+        from .builtin_terms import MLPField
+
+        f = term.f
+        if not getattr(adjoint, "backward_network_kernels", True) or type(f) is not MLPField or term.with_args or "forward" in f.__dict__:
+            return False
+        from torch.nn.modules import module as nn_module
+
+        hooks = (f._forward_hooks, f._forward_pre_hooks, f._backward_hooks, f._backward_pre_hooks, nn_module._global_forward_hooks,
+                 nn_module._global_forward_pre_hooks, nn_module._global_backward_hooks, nn_module._global_backward_pre_hooks)  # fmt: skip
+        weights = (f.W1, f.b1, f.W2, f.b2)
+        F, H = f.W2.shape
+        return (
+            not any(hooks)
+            and f.matrix_inputs == "float32"
+            and y0.dtype == torch.float32
+            and times.dtype == torch.float32
+            and all(x.dtype == torch.float32 and x.device == y0.device for x in weights)
+            and F == y0.shape[1]
+            and 1 <= F <= 64
+            and 1 <= H <= 256
+            and [tuple(x.shape) for x in weights] == [(H, F + 1), (H,), (F, H), (F,)]
+            and y0.shape[0] > 0
+        )
+
+    def __init__(self, lib, method_id, f, B, F, g_k, g_y, g_y1, g_t, g_dt, stream):
+        dev, H = g_k.device, f.W2.shape[1]
+        new = lambda *shape: torch.empty(shape, dtype=torch.float32, device=dev)
+        self.lib, self.stream, self.f, self.started = lib, stream, f, False
+        wanted = any(x.requires_grad for x in (f.W1, f.b1, f.W2, f.b2))
+        with torch.no_grad():
+            raw = f.builtin_shared()
+        packed, packed_reverse = new(_lib.MLP_PACKED_SIZE["float32"]), new(_lib.MLP_REVERSE_PACKED_SIZE)
+        _lib.check(lib.tode_mlp_pack_weights_for(raw.data_ptr(), raw.numel(), F, _lib.MLP_INPUTS["float32"], packed.data_ptr(), stream), "tode_mlp_pack_weights_for")
+        _lib.check(lib.tode_mlp_pack_weights_reverse(raw.data_ptr(), raw.numel(), F, packed_reverse.data_ptr(), stream), "tode_mlp_pack_weights_reverse")
+        # One share of the 6 B rows per compute unit and at least 64 rows each: a share ends with 133 KB of sums.
+        splits = max(1, min(256, (6 * B) // 64))
+        self.k, self.inputs, self.times, self.hidden = new(6, B, F), new(6, B, F), new(6, B), new(6, B, 256)
+        self.cotangents = new(6, B, 256) if wanted else None
+        self.sums = new(splits, _lib.MLP_SUMS_SIZE) if wanted else None
+        self.keep = (raw, packed, packed_reverse, g_k, g_y, g_y1, g_t, g_dt)
+        self.args = _lib.MlpReverse(
+            method_id, F, H, splits, B, packed.data_ptr(), packed_reverse.data_ptr(), None, None, None, None, self.k.data_ptr(), self.inputs.data_ptr(),
+            self.times.data_ptr(), self.hidden.data_ptr(), _lib.ptr(self.cotangents), *(x.data_ptr() for x in (g_k, g_y, g_y1, g_t, g_dt)), _lib.ptr(self.sums),
+        )  # fmt: skip
+        self.ref = _lib.C.byref(self.args)
+
+    def stages(self, state):
+        a = self.args
+        a.t, a.dt, a.y, a.k0 = (state[k].data_ptr() for k in ("t", "dt", "y", "k0"))
+        _lib.check(self.lib.tode_mlp_stages(self.ref, self.stream), "tode_mlp_stages")
+        return [state["k0"], *self.k.unbind(0)], self.inputs[5]
+
+    def stages_backward(self):
+        _lib.check(self.lib.tode_mlp_stages_backward(self.ref, int(self.started), self.stream), "tode_mlp_stages_backward")
+        self.started = True
+
+    def weight_gradients(self, params):
+        """The gradients of ``params`` through the weights: autograd carries those of the held tensors on to the leaves."""
+        f = self.f
+        weights = (f.W1, f.b1, f.W2, f.b2)
+        if self.sums is None or not self.started or not params:
+            return [None] * len(params)
+        out = torch.empty(sum(x.numel() for x in weights), dtype=torch.float32, device=self.sums.device)
+        _lib.check(self.lib.tode_mlp_weight_gradients(self.ref, out.data_ptr(), self.stream), "tode_mlp_weight_gradients")
+        grads = [g.view(x.shape) for g, x in zip(out.split([x.numel() for x in weights]), weights)]
+        pairs = [(x, g) for x, g in zip(weights, grads) if x.requires_grad]
+        return list(torch.autograd.grad([x for x, _ in pairs], params, [g for _, g in pairs], allow_unused=True, retain_graph=True))
+
+
 def reverse_sweep_kernels(adjoint, replay: Replay, term, args, problem, dt0_given, dt0, states, hits, grad_ys, params, params_given):
     """The iterations in reverse through the library's reverse kernels (tode_step_finish_backward,
     tode_step_stage_backward): per iteration the stage values are recomputed by the forward stage kernel and ``f``
@@ -568,6 +646,9 @@ def reverse_sweep_kernels(adjoint, replay: Replay, term, args, problem, dt0_give
     ad.g_y, ad.g_y1, ad.g_t, ad.g_dt, ad.g_prev, ad.g_pprev = (x.data_ptr() for x in (g_y, g_y1, g_t, g_dt, g_hist[0], g_hist[1]))
 
     f, with_args = term.f, term.with_args
+    network = None
+    if NetworkSweep.takes(adjoint, term, y0, t_start):
+        network = NetworkSweep(lib, method.method_id, f, B, F, g_k, g_y, g_y1, g_t, g_dt, stream)
 
     def rhs(tt, yy):
         out = f(tt, yy, args) if with_args else f(tt, yy)
@@ -591,7 +672,9 @@ def reverse_sweep_kernels(adjoint, replay: Replay, term, args, problem, dt0_give
         st.ratio_prev, st.ratio_pprev = now["prev"].data_ptr(), now["pprev"].data_ptr()
         st.k[0] = now["k0"].data_ptr()
         ks, inputs = [now["k0"]], [None]
-        for i in range(1, 7):
+        if network is not None:
+            ks, y1 = network.stages(now)
+        for i in range(1, 7 if network is None else 1):
             yi, ti = new(B, F), new(B, dt=ttype)
             st.ystage[i], st.tnode = yi.data_ptr(), ti.data_ptr()
             _lib.check(lib.tode_step_stage(sref, cref, i, stream), "tode_step_stage")
@@ -610,14 +693,16 @@ def reverse_sweep_kernels(adjoint, replay: Replay, term, args, problem, dt0_give
         ad.moved, ad.running_next = moved.data_ptr(), running_next.data_ptr()
         for i in range(7):
             ad.k[i] = ks[i].data_ptr()
-        ad.y1 = inputs[6][0].data_ptr()
+        ad.y1 = (y1 if network is not None else inputs[6][0]).data_ptr()
         names = ("a_y", "a_k0", "a_t", "a_dt", "a_prev", "a_pprev")
         held = [None if adj is None else adj[j] for j in range(6)]
         for name, value in zip(names, held):
             setattr(ad, name, _lib.ptr(value))
         _lib.check(lib.tode_step_finish_backward(aref, cref, stream), "tode_step_finish_backward")
         # ---- the stages reversed: f's vector-Jacobian products by autograd, the sums by the kernel ----
-        for i in range(6, 0, -1):
+        if network is not None:
+            network.stages_backward()
+        for i in range(6 if network is None else 0, 0, -1):
             yi, ti, ki = inputs[i]
             if ki.requires_grad:
                 grads = torch.autograd.grad(ki, [yi, ti] + params, g_k[i], allow_unused=True, retain_graph=True)
@@ -631,6 +716,9 @@ def reverse_sweep_kernels(adjoint, replay: Replay, term, args, problem, dt0_give
             for j, g in enumerate(grads[2:]):
                 grad_params[j] = _add(grad_params[j], g)
         adj = (g_y.clone(), g_k[0].clone(), g_t.clone(), g_dt.clone(), g_hist[0].clone(), g_hist[1].clone())
+
+    if network is not None:
+        grad_params = network.weight_gradients(params)
 
     # the gradients of the times go to the entries of `params` that stand for them
     for given, collected in ((problem_time(replay, "t_start"), g_t_start), (problem_time(replay, "t_end"), g_t_end),

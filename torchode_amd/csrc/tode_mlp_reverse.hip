@@ -1,0 +1,404 @@
+// Reverse sweep of a solve with the two-layer perceptron as right-hand side (float32, up to 64 state values and 256 hidden
+// units): what lies on either side of tode_step_finish_backward for one recorded iteration, and the gradients of the
+// weights.  The reference leaves all of it to autograd over its loop (adjoints.py:135-260); through autograd it is, per
+// iteration, six evaluations of the network and six vector-Jacobian products of some fifteen launches each.  Here:
+//
+//   mlp_stages_kernel           all six stages of the iteration again (a tile of 16 samples per workgroup, laid out as in
+//                               the whole-solve kernel), keeping stage inputs, derivatives and hidden activations;
+//   mlp_stages_backward_kernel  the six stages in reverse: the network's vector-Jacobian product and the stage sums' reverse,
+//                               the cotangents of all stage derivatives in registers between them;
+//   mlp_weight_gradient_kernel  the two outer products over all 6 B rows of the iteration, split over the rows;
+//   mlp_weight_gradient_sum_kernel  the splits' sums added in order, once per sweep.
+//
+// All products are on v_mfma_f32_16x16x4_f32.  For the vector-Jacobian product the weights are packed a second time,
+// transposed (tode_mlp_pack_weights_reverse), so that the same two facts hold as in the forward kernel: every lane keeps its
+// A operands in registers, and the first product's result, lane (q, c) holding the cotangents of hidden units 4q..4q+3 of
+// sample c, is after (1 - h^2) already the second product's B operand.
+#include "tode_mlp.h"
+
+namespace tode {
+
+constexpr int MLP_REVERSE_REGS = 64 + 64 + 16;  // packed values per thread: W2 transposed, W1 transposed, W1's time column
+// sums per split: W1 without its time column as [64 inputs][256 units] | time column | b1 | W2 [64][256] | b2
+constexpr int MLP_SUM_W1T = MLP_F * MLP_H, MLP_SUM_B1 = MLP_SUM_W1T + MLP_H, MLP_SUM_W2 = MLP_SUM_B1 + MLP_H, MLP_SUM_B2 = MLP_SUM_W2 + MLP_F * MLP_H;
+constexpr int MLP_SUMS = MLP_SUM_B2 + MLP_F;
+
+static __global__ void mlp_pack_reverse_kernel(const float *raw, float *packed, int H, int FR) {
+    const int i = blockIdx.x * blockDim.x + threadIdx.x;
+    if (i >= MLP_REVERSE_REGS * 256) return;
+    const int tid = (i / 4) % 256, lane = tid & 63, w = tid >> 6, q = lane >> 4, c = lane & 15;
+    int j = 4 * (i / 1024) + i % 4;
+    const long long o_w2 = (long long)H * (FR + 1) + H;
+    long long src = -1;
+    if (j < 64) {  // W2[16q + kk][64w + 16 tile + c]
+        const int f = 16 * q + j / 4, unit = 64 * w + 16 * (j % 4) + c;
+        if (f < FR && unit < H) src = o_w2 + (long long)f * H + unit;
+    } else if (j < 128) {  // W1[64w + 16 tile + 4q + r][16 it + c]
+        j -= 64;
+        const int input = 16 * (j / 16) + c, unit = 64 * w + 16 * ((j / 4) % 4) + 4 * q + j % 4;
+        if (input < FR && unit < H) src = (long long)unit * (FR + 1) + input;
+    } else {  // W1[64w + 16 tile + 4q + r][time]
+        j -= 128;
+        const int unit = 64 * w + 16 * (j / 4) + 4 * q + j % 4;
+        if (unit < H) src = (long long)unit * (FR + 1) + FR;
+    }
+    packed[i] = src < 0 ? 0.0f : raw[src];
+}
+
+// The lane's four features f0 .. f0 + 3 of a row of FR values: 16 bytes at a time where rows are whole groups of four.
+__device__ __forceinline__ void mlp_get(const float *row, int f0, int FR, float (&v)[4]) {
+    if ((FR & 3) == 0) {
+        const float4 u = f0 < FR ? *reinterpret_cast<const float4 *>(row + f0) : make_float4(0.0f, 0.0f, 0.0f, 0.0f);
+        v[0] = u.x, v[1] = u.y, v[2] = u.z, v[3] = u.w;
+    } else {
+#pragma unroll
+        for (int r = 0; r < 4; ++r) v[r] = f0 + r < FR ? row[f0 + r] : 0.0f;
+    }
+}
+
+__device__ __forceinline__ void mlp_put(float *row, int f0, int FR, const float (&v)[4]) {
+    if ((FR & 3) == 0) {
+        if (f0 < FR) *reinterpret_cast<float4 *>(row + f0) = make_float4(v[0], v[1], v[2], v[3]);
+    } else {
+#pragma unroll
+        for (int r = 0; r < 4; ++r)
+            if (f0 + r < FR) row[f0 + r] = v[r];
+    }
+}
+
+template <int METHOD> __global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2, 2))) mlp_stages_kernel(const tode_mlp_reverse p) {
+    using Tab = typename std::conditional<METHOD == 1, Tsit5Tab, Dopri5Tab>::type;
+    __shared__ MlpShared sh;
+    const int tid = threadIdx.x, lane = tid & 63, w = tid >> 6, q = lane >> 4, c = lane & 15, FR = p.n_features, f0 = 16 * w + 4 * q;
+    const long long B = p.batch, tiles = (B + MLP_TILE - 1) / MLP_TILE;
+    MlpWeights W;
+    mlp_load(W, (const float *)p.packed, tid);
+    for (int i = tid; i < MLP_TILE * MLP_XS; i += 256) sh.x[i] = 0.0f;  // also the zero columns from 65 on
+    __syncthreads();
+    for (long long tile = blockIdx.x; tile < tiles; tile += gridDim.x) {
+        const bool live = tile * MLP_TILE + c < B;
+        const long long b = live ? tile * MLP_TILE + c : B - 1;
+        const float t = ((const float *)p.t)[b], dt = ((const float *)p.dt)[b];
+        float y[4], k[7][4];
+        mlp_get((const float *)p.y + b * FR, f0, FR, y);
+        mlp_get((const float *)p.k0 + b * FR, f0, FR, k[0]);
+#pragma unroll
+        for (int s = 1; s < 7; ++s) {
+            float yi[4];
+#pragma unroll
+            for (int r = 0; r < 4; ++r) {
+                float sum = 0;
+#pragma unroll
+                for (int j = 0; j < s; ++j) sum = fma_((float)Tab::a[s][j], k[j][r], sum);
+                yi[r] = fma_(dt, sum, y[r]);
+            }
+            const float tn = fma_((float)Tab::c[s], dt, t);
+            const long long row = (s - 1) * B + b;
+            if (live) {
+                mlp_put((float *)p.stage_inputs + row * FR, f0, FR, yi);
+                if (w == 0 && q == 0) ((float *)p.stage_times)[row] = tn;
+            }
+            mlp_rhs<true>(sh, W, tn, yi, k[s], live ? (float *)p.hidden + row * MLP_H : nullptr);
+            if (live) mlp_put((float *)p.k + row * FR, f0, FR, k[s]);
+        }
+    }
+}
+
+struct __align__(16) MlpReverseShared {
+    float g[MLP_TILE * MLP_XS];   // cotangent of the stage derivative: [sample][feature]
+    float part[4][4][64][4];      // [16 inputs][wavefront it comes from][lane][4 inputs]
+    float red[4][MLP_TILE][2];
+};
+
+// One wavefront per SIMD: 144 registers of weights, 28 + 24 of stage derivatives and their cotangents.  A workgroup takes
+// several tiles where the batch has more than the grid, so that the weights are loaded once.
+template <int METHOD> __global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(1, 1))) mlp_stages_backward_kernel(const tode_mlp_reverse p) {
+    using Tab = typename std::conditional<METHOD == 1, Tsit5Tab, Dopri5Tab>::type;
+    __shared__ MlpReverseShared sh;
+    const int tid = threadIdx.x, lane = tid & 63, w = tid >> 6, q = lane >> 4, c = lane & 15, FR = p.n_features, f0 = 16 * w + 4 * q;
+    const long long B = p.batch, tiles = (B + MLP_TILE - 1) / MLP_TILE;
+    float w2t[16][4], w1t[4][16], wt[16];
+    {
+        const float4 *src = reinterpret_cast<const float4 *>(p.packed_reverse) + tid;
+#pragma unroll
+        for (int i = 0; i < MLP_REVERSE_REGS / 4; ++i) {
+            const float4 u = src[i * 256];
+            const float v[4] = {u.x, u.y, u.z, u.w};
+#pragma unroll
+            for (int r = 0; r < 4; ++r) {
+                if (i < 16) w2t[i][r] = v[r];
+                else if (i < 32) w1t[(i - 16) / 4][4 * ((i - 16) % 4) + r] = v[r];
+                else wt[4 * (i - 32) + r] = v[r];
+            }
+        }
+    }
+    for (long long tile = blockIdx.x; tile < tiles; tile += gridDim.x) {
+        const bool live = tile * MLP_TILE + c < B;
+        const long long b = live ? tile * MLP_TILE + c : B - 1;
+        const float dt = ((const float *)p.dt)[b];
+        float k[6][4], gk[7][4], gy[4], gy1[4], g_t = 0, g_dt = 0;
+        mlp_get((const float *)p.k0 + b * FR, f0, FR, k[0]);
+#pragma unroll
+        for (int s = 1; s < 6; ++s) mlp_get((const float *)p.k + ((s - 1) * B + b) * FR, f0, FR, k[s]);
+#pragma unroll
+        for (int s = 0; s < 7; ++s) mlp_get((const float *)p.g_k + (s * B + b) * FR, f0, FR, gk[s]);
+        mlp_get((const float *)p.g_y + b * FR, f0, FR, gy);
+        mlp_get((const float *)p.g_y1 + b * FR, f0, FR, gy1);
+#pragma unroll
+        for (int s = 6; s >= 1; --s) {
+            const long long row = (s - 1) * B + b;
+            *reinterpret_cast<float4 *>(sh.g + c * MLP_XS + f0) = make_float4(gk[s][0], gk[s][1], gk[s][2], gk[s][3]);
+            if (s < 6 && live) mlp_put((float *)p.g_k + (s * B + b) * FR, f0, FR, gk[s]);  // (final: the weights' gradients read it)
+            float4 h[4];
+#pragma unroll
+            for (int u = 0; u < 4; ++u) h[u] = *reinterpret_cast<const float4 *>((const float *)p.hidden + row * MLP_H + 64 * w + 16 * u + 4 * q);
+            lds_barrier();
+            float g[16];
+            {
+                const float4 *at = reinterpret_cast<const float4 *>(sh.g + c * MLP_XS + 16 * q);
+#pragma unroll
+                for (int j = 0; j < 4; ++j) {
+                    const float4 v = at[j];
+                    g[4 * j] = v.x, g[4 * j + 1] = v.y, g[4 * j + 2] = v.z, g[4 * j + 3] = v.w;
+                }
+            }
+            mfma_acc d[4];
+#pragma unroll
+            for (int u = 0; u < 4; ++u) d[u] = {0.0f, 0.0f, 0.0f, 0.0f};
+#pragma unroll
+            for (int kk = 0; kk < 16; ++kk)
+#pragma unroll
+                for (int u = 0; u < 4; ++u) d[u] = __builtin_amdgcn_mfma_f32_16x16x4f32(w2t[kk][u], g[kk], d[u], 0, 0, 0);
+            float gt = 0;
+#pragma unroll
+            for (int u = 0; u < 4; ++u) {
+                const float hv[4] = {h[u].x, h[u].y, h[u].z, h[u].w};
+#pragma unroll
+                for (int r = 0; r < 4; ++r) {
+                    d[u][r] = d[u][r] * fma_(-hv[r], hv[r], 1.0f);
+                    gt = fma_(wt[4 * u + r], d[u][r], gt);
+                }
+                if (live && p.hidden_cotangents)
+                    *reinterpret_cast<float4 *>((float *)p.hidden_cotangents + row * MLP_H + 64 * w + 16 * u + 4 * q) = make_float4(d[u][0], d[u][1], d[u][2], d[u][3]);
+            }
+            g_t += gt;
+            g_dt = fma_((float)Tab::c[s], gt, g_dt);
+            mfma_acc acc[4];
+#pragma unroll
+            for (int it = 0; it < 4; ++it) acc[it] = {0.0f, 0.0f, 0.0f, 0.0f};
+#pragma unroll
+            for (int u = 0; u < 4; ++u)
+#pragma unroll
+                for (int r = 0; r < 4; ++r)
+#pragma unroll
+                    for (int it = 0; it < 4; ++it) acc[it] = __builtin_amdgcn_mfma_f32_16x16x4f32(w1t[it][4 * u + r], d[u][r], acc[it], 0, 0, 0);
+#pragma unroll
+            for (int it = 0; it < 4; ++it) *reinterpret_cast<float4 *>(sh.part[it][w][lane]) = make_float4(acc[it][0], acc[it][1], acc[it][2], acc[it][3]);
+            lds_barrier();
+            float4 v[4];
+#pragma unroll
+            for (int from = 0; from < 4; ++from) v[from] = *reinterpret_cast<const float4 *>(sh.part[w][from][lane]);
+            float gi[4] = {(v[0].x + v[1].x) + (v[2].x + v[3].x), (v[0].y + v[1].y) + (v[2].y + v[3].y), (v[0].z + v[1].z) + (v[2].z + v[3].z),
+                           (v[0].w + v[1].w) + (v[2].w + v[3].w)};
+            // the stage's sum reversed (stage_backward_sample)
+#pragma unroll
+            for (int r = 0; r < 4; ++r) {
+                if (s == 6) gi[r] += gy1[r];
+                gy[r] += gi[r];
+                float sum = 0;
+#pragma unroll
+                for (int j = 0; j < s; ++j) {
+                    sum = fma_((float)Tab::a[s][j], k[j][r], sum);
+                    gk[j][r] += (float)Tab::a[s][j] * dt * gi[r];
+                }
+                g_dt = fma_(gi[r], sum, g_dt);
+            }
+        }
+        // the sample's shares of the cotangents of t and dt: four lane groups of four wavefronts
+#pragma unroll
+        for (int off = 16; off < 64; off <<= 1) g_t += __shfl_xor(g_t, off), g_dt += __shfl_xor(g_dt, off);
+        if (q == 0) sh.red[w][c][0] = g_t, sh.red[w][c][1] = g_dt;
+        lds_barrier();  // (the next tile's sums come behind its own barriers, so one set of words is enough)
+        if (live) {
+            mlp_put((float *)p.g_y + b * FR, f0, FR, gy);
+            mlp_put((float *)p.g_k + b * FR, f0, FR, gk[0]);
+            if (w == 0 && q == 0) {
+                ((float *)p.g_t)[b] += (sh.red[0][c][0] + sh.red[1][c][0]) + (sh.red[2][c][0] + sh.red[3][c][0]);
+                ((float *)p.g_dt)[b] += (sh.red[0][c][1] + sh.red[1][c][1]) + (sh.red[2][c][1] + sh.red[3][c][1]);
+            }
+        }
+    }
+}
+
+// The operands of four rows (k of the matrix instructions) for one wavefront: lane (q, c) holds row 4 step + q.
+struct MlpOuterRows {
+    float h[4], d[4], g[4], x[4], t;
+};
+
+__device__ __forceinline__ MlpOuterRows mlp_outer_rows(const tode_mlp_reverse &p, long long row, long long end, int w, int c) {
+    const bool in = row < end;
+    const long long at = in ? row : end - 1;
+    const int FR = p.n_features;
+    MlpOuterRows v;
+#pragma unroll
+    for (int u = 0; u < 4; ++u) {
+        v.h[u] = ((const float *)p.hidden)[at * MLP_H + 64 * w + 16 * u + c];
+        v.d[u] = ((const float *)p.hidden_cotangents)[at * MLP_H + 64 * w + 16 * u + c];
+        const int f = 16 * u + c;
+        v.g[u] = f < FR ? ((const float *)p.g_k)[(p.batch + at) * FR + f] : 0.0f;
+        v.x[u] = f < FR ? ((const float *)p.stage_inputs)[at * FR + f] : 0.0f;
+        v.d[u] = in ? v.d[u] : 0.0f;
+        v.g[u] = in ? v.g[u] : 0.0f;
+    }
+    v.t = ((const float *)p.stage_times)[at];
+    return v;
+}
+
+// dW2[f][u] = sum over rows g[f] h[u],  dW1[u][i] = sum over rows d[u] x[i],  and the biases' and the time column's sums:
+// every workgroup takes a share of the rows and holds all sums of it in registers (wavefront w: units 64w .. 64w + 63, 128
+// accumulators), 32 matrix instructions per four rows with the next four rows' operands on their way.  The sums of a
+// share go to the workgroup's own slot, added to those of the iterations before (`accumulate`).
+__global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2, 2))) mlp_weight_gradient_kernel(const tode_mlp_reverse p, long long rows_per_split, int accumulate) {
+    const int tid = threadIdx.x, lane = tid & 63, w = tid >> 6, q = lane >> 4, c = lane & 15;
+    const long long rows = 6 * p.batch, first = (long long)blockIdx.x * rows_per_split, end = min(rows, first + rows_per_split);
+    mfma_acc a2[4][4], a1[4][4];
+    float at[4], ab[4], ag[4];
+#pragma unroll
+    for (int i = 0; i < 4; ++i) {
+        at[i] = ab[i] = ag[i] = 0;
+#pragma unroll
+        for (int u = 0; u < 4; ++u) a2[i][u] = {0.0f, 0.0f, 0.0f, 0.0f}, a1[i][u] = {0.0f, 0.0f, 0.0f, 0.0f};
+    }
+    if (first < end) {
+        MlpOuterRows here = mlp_outer_rows(p, first + q, end, w, c);
+        for (long long row = first; row < end; row += 4) {
+            const MlpOuterRows next = mlp_outer_rows(p, row + 4 + q, end, w, c);
+#pragma unroll
+            for (int u = 0; u < 4; ++u) {
+#pragma unroll
+                for (int i = 0; i < 4; ++i) {
+                    a2[i][u] = __builtin_amdgcn_mfma_f32_16x16x4f32(here.g[i], here.h[u], a2[i][u], 0, 0, 0);
+                    a1[i][u] = __builtin_amdgcn_mfma_f32_16x16x4f32(here.x[i], here.d[u], a1[i][u], 0, 0, 0);
+                }
+                at[u] = fma_(here.t, here.d[u], at[u]);
+                ab[u] += here.d[u];
+                ag[u] += here.g[u];
+            }
+            here = next;
+        }
+    }
+    float *out = (float *)p.sums + (long long)blockIdx.x * MLP_SUMS;
+    auto put = [&](int i, float v) { out[i] = accumulate ? out[i] + v : v; };
+#pragma unroll
+    for (int u = 0; u < 4; ++u) {
+        const int unit = 64 * w + 16 * u + c;
+#pragma unroll
+        for (int i = 0; i < 4; ++i)
+#pragma unroll
+            for (int r = 0; r < 4; ++r) {
+                put((16 * i + 4 * q + r) * MLP_H + unit, a1[i][u][r]);
+                put(MLP_SUM_W2 + (16 * i + 4 * q + r) * MLP_H + unit, a2[i][u][r]);
+            }
+#pragma unroll
+        for (int off = 16; off < 64; off <<= 1) at[u] += __shfl_xor(at[u], off), ab[u] += __shfl_xor(ab[u], off), ag[u] += __shfl_xor(ag[u], off);
+        if (q == 0) {
+            put(MLP_SUM_W1T + unit, at[u]);
+            put(MLP_SUM_B1 + unit, ab[u]);
+            if (w == 0) put(MLP_SUM_B2 + 16 * u + c, ag[u]);
+        }
+    }
+}
+
+// One thread per sum, the splits in order; out in the order of the weights: W1 [H x (F + 1)] | b1 | W2 [F x H] | b2.
+static __global__ void __launch_bounds__(256) mlp_weight_gradient_sum_kernel(const float *sums, int splits, int H, int FR, float *out) {
+    const int i = blockIdx.x * 256 + threadIdx.x;
+    if (i >= MLP_SUMS) return;
+    const long long o_b1 = (long long)H * (FR + 1), o_w2 = o_b1 + H, o_b2 = o_w2 + (long long)FR * H;
+    long long to = -1;
+    const int row = i / MLP_H, unit = i % MLP_H;  // (of the first part; the others start at multiples of MLP_H as well)
+    if (i < MLP_SUM_W1T) to = (unit < H && row < FR) ? (long long)unit * (FR + 1) + row : -1;
+    else if (i < MLP_SUM_B1) to = unit < H ? (long long)unit * (FR + 1) + FR : -1;
+    else if (i < MLP_SUM_W2) to = unit < H ? o_b1 + unit : -1;
+    else if (i < MLP_SUM_B2) to = (unit < H && row - MLP_F - 2 < FR) ? o_w2 + (long long)(row - MLP_F - 2) * H + unit : -1;
+    else to = i - MLP_SUM_B2 < FR ? o_b2 + (i - MLP_SUM_B2) : -1;
+    if (to < 0) return;
+    float s[4] = {0, 0, 0, 0};
+    for (int k = 0; k < splits; k += 4)
+#pragma unroll
+        for (int j = 0; j < 4; ++j)
+            if (k + j < splits) s[j] += sums[(long long)(k + j) * MLP_SUMS + i];
+    out[to] = (s[0] + s[1]) + (s[2] + s[3]);
+}
+
+static int check_mlp_reverse(const tode_mlp_reverse *p) {
+    if (!p) return fail(TODE_E_INVALID, "null tode_mlp_reverse");
+    if (p->method != TODE_DOPRI5 && p->method != TODE_TSIT5) return fail(TODE_E_INVALID, "unknown method %d", p->method);
+    if (p->n_features < 1 || p->n_features > MLP_F || p->n_hidden < 1 || p->n_hidden > MLP_H)
+        return fail(TODE_E_UNSUPPORTED, "the network's kernels take 1 to %d features and 1 to %d hidden units, got %d and %d", MLP_F, MLP_H, p->n_features, p->n_hidden);
+    if (p->batch < 0 || p->batch > (1ll << 40)) return fail(TODE_E_INVALID, "batch %lld", (long long)p->batch);
+    if (p->splits < 1 || p->splits > TODE_MLP_MAX_SPLITS) return fail(TODE_E_INVALID, "splits %d", p->splits);
+    if (p->batch > 0 && (!p->packed || !p->packed_reverse || !p->t || !p->dt || !p->y || !p->k0 || !p->k || !p->stage_inputs || !p->stage_times || !p->hidden ||
+                         !p->g_k || !p->g_y || !p->g_y1 || !p->g_t || !p->g_dt))
+        return fail(TODE_E_INVALID, "null pointer");
+    if (!p->hidden_cotangents != !p->sums) return fail(TODE_E_INVALID, "hidden_cotangents and sums go together");
+    return TODE_OK;
+}
+
+// A workgroup of the reverse kernel fills its compute unit (one wavefront per SIMD), of the stages' kernel half of one:
+// beyond that they take several tiles each and load the weights once (133 KB per workgroup, as long as a stage takes).
+static unsigned mlp_tiles_grid(const tode_mlp_reverse &p, int per_unit) {
+    const long long tiles = (p.batch + MLP_TILE - 1) / MLP_TILE;
+    return (unsigned)(tiles < 256ll * per_unit ? tiles : 256ll * per_unit);
+}
+
+}  // namespace tode
+
+extern "C" {
+
+int tode_mlp_pack_weights_reverse(const void *raw, int64_t n_raw, int32_t n_features, void *packed, void *stream) {
+    using namespace tode;
+    static_assert(TODE_MLP_REVERSE_PACKED_SIZE == MLP_REVERSE_REGS * 256 && TODE_MLP_SUMS_SIZE == MLP_SUMS, "sizes");
+    if (!raw || !packed) return fail(TODE_E_INVALID, "null pointer");
+    const long long FR = n_features;
+    if (FR < 1 || FR > MLP_F) return fail(TODE_E_UNSUPPORTED, "the network's kernels take 1 to %d features, got %lld", MLP_F, FR);
+    const long long H = (n_raw - FR) / (2 * FR + 2);
+    if (n_raw < FR || H * (2 * FR + 2) + FR != n_raw || H < 1 || H > MLP_H) return fail(TODE_E_UNSUPPORTED, "%lld weights do not make a network of up to %d hidden units", (long long)n_raw, MLP_H);
+    hipLaunchKernelGGL(mlp_pack_reverse_kernel, dim3(MLP_REVERSE_REGS), dim3(256), 0, (hipStream_t)stream, (const float *)raw, (float *)packed, (int)H, (int)FR);
+    return check_hip(hipGetLastError(), "tode_mlp_pack_weights_reverse");
+}
+
+int tode_mlp_stages(const tode_mlp_reverse *p, void *stream) {
+    using namespace tode;
+    const int rc = check_mlp_reverse(p);
+    if (rc || p->batch == 0) return rc;
+    const dim3 grid(mlp_tiles_grid(*p, 2));
+    if (p->method == TODE_TSIT5) hipLaunchKernelGGL((mlp_stages_kernel<1>), grid, dim3(256), 0, (hipStream_t)stream, *p);
+    else hipLaunchKernelGGL((mlp_stages_kernel<0>), grid, dim3(256), 0, (hipStream_t)stream, *p);
+    return check_hip(hipGetLastError(), "tode_mlp_stages");
+}
+
+int tode_mlp_stages_backward(const tode_mlp_reverse *p, int32_t accumulate, void *stream) {
+    using namespace tode;
+    const int rc = check_mlp_reverse(p);
+    if (rc || p->batch == 0) return rc;
+    const dim3 grid(mlp_tiles_grid(*p, 1));
+    if (p->method == TODE_TSIT5) hipLaunchKernelGGL((mlp_stages_backward_kernel<1>), grid, dim3(256), 0, (hipStream_t)stream, *p);
+    else hipLaunchKernelGGL((mlp_stages_backward_kernel<0>), grid, dim3(256), 0, (hipStream_t)stream, *p);
+    if (p->sums) {
+        const long long rows = 6 * p->batch, per_split = ((rows + p->splits - 1) / p->splits + 3) / 4 * 4;
+        hipLaunchKernelGGL(mlp_weight_gradient_kernel, dim3(p->splits), dim3(256), 0, (hipStream_t)stream, *p, per_split, accumulate);
+    }
+    return check_hip(hipGetLastError(), "tode_mlp_stages_backward");
+}
+
+int tode_mlp_weight_gradients(const tode_mlp_reverse *p, void *out, void *stream) {
+    using namespace tode;
+    const int rc = check_mlp_reverse(p);
+    if (rc) return rc;
+    if (!p->sums || !out) return fail(TODE_E_INVALID, "null pointer");
+    hipLaunchKernelGGL(mlp_weight_gradient_sum_kernel, dim3((MLP_SUMS + 255) / 256), dim3(256), 0, (hipStream_t)stream, (const float *)p->sums, p->splits, p->n_hidden,
+                       p->n_features, (float *)out);
+    return check_hip(hipGetLastError(), "tode_mlp_weight_gradients");
+}
+
+}  // extern "C"
