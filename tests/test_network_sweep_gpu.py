@@ -51,3 +51,29 @@ def test_a_hook_on_the_network_is_called():
     got, want = (_gradients(17, 8, 16, 4, to.Dopri5, lambda: to.IntegralController(1e-5, 1e-3), False, network, hook=True) for network in (True, False))
     for a, b in zip(got, want):
         assert torch.equal(a, b)
+
+
+@pytest.mark.parametrize("B, F, H", [(1, 3, 5), (50, 64, 256)])
+def test_a_solve_of_more_steps_than_the_first_record_holds(B, F, H):
+    """Tight tolerances: more iterations than the record's first size, so the first solve is repeated with a longer one and
+    the next solve of the same solver fits at once; every pass returns the same bits, and the gradients are those of the
+    per-step path with torch's products.  (At these tolerances the error estimate is float32 rounding, so the two may take
+    other steps: each is within 2^-24 times the some hundred roundings per step of 10 to 100 steps, 6e-4, of the same solution.)"""
+    g = torch.Generator("cuda").manual_seed(B)
+    rand = lambda *shape: (math.sqrt(6.0 / sum(shape)) * (2 * torch.rand(shape, generator=g, device="cuda") - 1)).requires_grad_()
+    weights = [rand(H, F + 1), rand(H), rand(F, H), rand(F)]
+    y0, cotangent = rand(B, F), rand(B, 6, F).detach()
+    t_eval = torch.linspace(0, 3, 6, device="cuda").repeat(B, 1)
+    results = {}
+    for network in (True, False):
+        solver = to.AutoDiffAdjoint(to.Tsit5(), to.IntegralController(1e-8, 1e-7), backprop_through_step_size_control=False)
+        solver.backward_network_kernels = network
+        for attempt in range(2):
+            sol = solver.solve(to.InitialValueProblem(y0, t_eval=t_eval), to.ODETerm(to.MLPField(*weights)))
+            assert int(sol.status.abs().sum()) == 0 and int(sol.stats["n_steps"].max()) > 8
+            results[network, attempt] = torch.autograd.grad(sol.ys, [y0, *weights], cotangent)
+        if network:
+            assert list(solver._record_entries.values()) == [int(sol.stats["n_steps"].max()) + 5]
+    for a, b, c in zip(results[True, 0], results[True, 1], results[False, 0]):
+        assert torch.equal(a, b)
+        assert float((a.double() - c.double()).norm()) <= 1e-3 * float(c.double().norm())

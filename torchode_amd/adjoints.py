@@ -575,7 +575,12 @@ class AutoDiffAdjoint(nn.Module):
         lib = _lib.load()
         f: BuiltinTerm = _sub(term, "f")
         if record is not None and f.builtin_kind not in _lib.GENERAL_TERMS:
-            return None  # (the record is written for the three small systems: the grid and MLP terms record on the per-step path)
+            # (the record is written for the three small systems and for the network whose reverse sweep has kernels of its own:
+            # the grid term and other networks record on the per-step path)
+            from .autodiff import NetworkSweep
+
+            if f.builtin_kind != _lib.TERM_MLP or problem.n_evaluation_points == 0 or not self.use_fast_path or not NetworkSweep.takes(self, term, problem.y0, problem.t_start):
+                return None
         method_id, controller = _sub(self, "step_method").method_id, _sub(self, "step_size_controller")
         # What depends on the problem's tensors alone is worked out once per problem object and kept on it (checked by
         # identity, since the attributes of a problem may be reassigned, and by the tensors' version counters, since
@@ -605,7 +610,7 @@ class AutoDiffAdjoint(nn.Module):
             dtype != torch.float32 or not 1 <= F <= 64 or f.W1.shape[1] != F + 1 or not 1 <= f.W1.shape[0] <= 256
         ):
             return None  # the matrix-core kernel takes up to 64 features and up to 256 hidden units: the caller takes another path
-        shared = f.builtin_packed(dev, dtype) if mlp else None
+        shared = f.builtin_packed(dev, dtype, fresh=record is not None) if mlp else None
         ttype = t_start.dtype
         dt0_ = None if dt0 is None else dt0.to(ttype).contiguous()
 
@@ -646,7 +651,7 @@ class AutoDiffAdjoint(nn.Module):
             # takes more iterations than the record holds, goes the long way below.
             solution = self._solve_recording_in_one_kernel(lib, a, ctrl, out, stream, record, dict(
                 B=B, E=E, F=F, dtype=dtype, ttype=ttype, dev=dev, ts=ts, ys=ys, has_dt0=dt0 is not None, with_stats=term.with_stats))  # fmt: skip
-            if solution is not None:
+            if solution is not None or mlp:
                 return solution
         workspace = torch.empty(held["workspace_bytes"], dtype=torch.uint8, device=dev)
         iterations = _lib.C.c_int64(0)
@@ -704,9 +709,12 @@ class AutoDiffAdjoint(nn.Module):
         setting outside that kernel's case, a batch that leaves it, or a record that came out too short."""
         shape = (q["B"], q["F"], q["E"], q["dtype"], a.term)
         n = getattr(self, "_record_entries", {}).get(shape)
+        mlp = a.term == _lib.TERM_MLP
+        if n is None and mlp:
+            n = 8  # (a smooth network takes a handful of steps; where it takes more, the first launch says how many)
         if n is None or not getattr(self, "record_in_one_kernel", True) or not self.use_fast_path:
             return None
-        if q["E"] == 0 or q["dtype"] != q["ttype"] or a.term in (_lib.TERM_REACTION_DIFFUSION, _lib.TERM_MLP):
+        if q["E"] == 0 or q["dtype"] != q["ttype"] or a.term == _lib.TERM_REACTION_DIFFUSION:
             return None
         B = q["B"]
         fields, rec = self._record_arrays(n, B, q["F"], q["dtype"], q["ttype"], q["dev"])
@@ -719,6 +727,10 @@ class AutoDiffAdjoint(nn.Module):
             return None
         _lib.check(rc, "tode_solve_builtin_fast_sync")
         if fl[_lib.FLAG_NEEDS_GENERAL]:
+            needed = fl[_lib.FLAG_MAX_ITERATIONS] + 1
+            if mlp and needed > n:  # too short: once more with a record of that length (a batch that leaves the kernel's case for another reason goes on)
+                self._remember_record_entries(shape, needed + 4)
+                return self._solve_recording_in_one_kernel(lib, a, ctrl, out, stream, record, q)
             return None
         L = fl[_lib.FLAG_MAX_ITERATIONS]
         record.iterations, record.arrays = L, fields

@@ -559,7 +559,9 @@ class NetworkSweep:
         _lib.check(self.lib.tode_mlp_stages(self.ref, self.stream), "tode_mlp_stages")
         return [state["k0"], *self.k.unbind(0)], self.inputs[5]
 
-    def stages_backward(self):
+    def stages_backward(self, g_k, g_y, g_t, g_dt):
+        a = self.args
+        a.g_k, a.g_y, a.g_t, a.g_dt = g_k.data_ptr(), g_y.data_ptr(), g_t.data_ptr(), g_dt.data_ptr()
         _lib.check(self.lib.tode_mlp_stages_backward(self.ref, int(self.started), self.stream), "tode_mlp_stages_backward")
         self.started = True
 
@@ -576,7 +578,7 @@ class NetworkSweep:
         return list(torch.autograd.grad([x for x, _ in pairs], params, [g for _, g in pairs], allow_unused=True, retain_graph=True))
 
 
-def reverse_sweep_kernels(adjoint, replay: Replay, term, args, problem, dt0_given, dt0, states, hits, grad_ys, params, params_given):
+def reverse_sweep_kernels(adjoint, replay: Replay, term, args, problem, dt0_given, dt0, states, hits, grad_ys, params, params_given, arrays=None):
     """The iterations in reverse through the library's reverse kernels (tode_step_finish_backward,
     tode_step_stage_backward): per iteration the stage values are recomputed by the forward stage kernel and ``f``
     (six evaluations under grad mode, each a small graph of its own), the finish kernel is reversed in one launch,
@@ -602,7 +604,13 @@ def reverse_sweep_kernels(adjoint, replay: Replay, term, args, problem, dt0_give
 
     # which iteration wrote which evaluation point
     hit_iteration = None
-    if E > 0:
+    if hits is None:  # (a record in arrays, of a batch in the whole-solve kernel's case: times that run in the solve's direction)
+        direction = replay.direction.detach()
+        reached = direction[None, :, None] * arrays["t"][1 : n_iterations + 1, :, None] >= (direction[:, None] * t_eval)[None]
+        hit_iteration = n_iterations - reached.sum(0, dtype=torch.int32)
+        hit_iteration = torch.where(hit_iteration < n_iterations, hit_iteration, -1).to(torch.int32)
+        hit_iteration[:, 0] = torch.where(t_eval[:, 0] == t_start, -1, hit_iteration[:, 0])
+    elif E > 0:
         hit_iteration = torch.full((B, E), -1, dtype=torch.int32, device=dev)
         for n, h in enumerate(hits):
             if h is not None:
@@ -647,7 +655,7 @@ def reverse_sweep_kernels(adjoint, replay: Replay, term, args, problem, dt0_give
 
     f, with_args = term.f, term.with_args
     network = None
-    if NetworkSweep.takes(adjoint, term, y0, t_start):
+    if NetworkSweep.takes(adjoint, term, y0, t_start):  # (always so where `arrays` are given)
         network = NetworkSweep(lib, method.method_id, f, B, F, g_k, g_y, g_y1, g_t, g_dt, stream)
 
     def rhs(tt, yy):
@@ -659,7 +667,33 @@ def reverse_sweep_kernels(adjoint, replay: Replay, term, args, problem, dt0_give
     adj = None  # cotangents of the state after the iteration at hand: (y, k0, t, dt, prev, pprev) or None for zeros
     grad_params = [None] * len(params)
     last = n_iterations - 1
+    if arrays is not None:
+        # (the decisions of all iterations in two launches, and two sets of cotangents that take turns instead of copies)
+        moved_all = (arrays["n_accepted"][1:] > arrays["n_accepted"][:-1]).to(torch.int32)
+        running_all = (arrays["running"][1:] != 0).to(torch.int32)
+        spare = (new(7, B, F), new(B, F), new(B, dt=ttype), new(B, dt=ttype), new(2, B))
+        sets = [(g_k, g_y, g_t, g_dt, g_hist), spare]
     for n in range(last, -1, -1):
+        if arrays is not None:
+            now = states[n]
+            g_k, g_y, g_t, g_dt, g_hist = sets[n % 2]
+            for i in range(7):
+                ad.g_k[i] = g_k[i].data_ptr()
+            ad.g_y, ad.g_t, ad.g_dt, ad.g_prev, ad.g_pprev = (x.data_ptr() for x in (g_y, g_t, g_dt, g_hist[0], g_hist[1]))
+            ks, y1 = network.stages(now)
+            ad.iteration, ad.end_point = n, 0
+            ad.t, ad.dt, ad.y = (now[k].data_ptr() for k in ("t", "dt", "y"))
+            ad.ratio_prev, ad.ratio_pprev = now["prev"].data_ptr(), now["pprev"].data_ptr()
+            ad.moved, ad.running_next = moved_all[n].data_ptr(), running_all[n].data_ptr()
+            for i in range(7):
+                ad.k[i] = ks[i].data_ptr()
+            ad.y1 = y1.data_ptr()
+            for name, value in zip(("a_y", "a_k0", "a_t", "a_dt", "a_prev", "a_pprev"), adj or [None] * 6):
+                setattr(ad, name, _lib.ptr(value))
+            _lib.check(lib.tode_step_finish_backward(aref, cref, stream), "tode_step_finish_backward")
+            network.stages_backward(g_k, g_y, g_t, g_dt)
+            adj = (g_y, g_k[0], g_t, g_dt, g_hist[0], g_hist[1])
+            continue
         has_hits = hits[n] is not None if E > 0 else n == last
         if adj is None and not has_hits:
             continue
@@ -701,7 +735,7 @@ def reverse_sweep_kernels(adjoint, replay: Replay, term, args, problem, dt0_give
         _lib.check(lib.tode_step_finish_backward(aref, cref, stream), "tode_step_finish_backward")
         # ---- the stages reversed: f's vector-Jacobian products by autograd, the sums by the kernel ----
         if network is not None:
-            network.stages_backward()
+            network.stages_backward(g_k, g_y, g_t, g_dt)
         for i in range(6 if network is None else 0, 0, -1):
             yi, ti, ki = inputs[i]
             if ki.requires_grad:
@@ -811,6 +845,7 @@ class SolveThroughLoop(torch.autograd.Function):
             use_kernels
             and getattr(adjoint, "backward_whole_kernel", True)
             and getattr(ctx.record, "arrays", None) is not None
+            and getattr(term.f, "builtin_kind", None) in _lib.GENERAL_TERMS
             and problem.time_dtype == problem.data_dtype
             and not term.with_args
         )
@@ -822,9 +857,13 @@ class SolveThroughLoop(torch.autograd.Function):
         else:
             LAST_SWEEP = "kernels" if use_kernels else "torch"
             states = ctx.record.trimmed(ctx.record.iterations)
-            hits = simulate_hits(replay, states, E)
+            # (a record in arrays that no sweep of one kernel takes is the network's: the other long-row term leaves none)
+            arrays = ctx.record.arrays if use_kernels and E > 0 and NetworkSweep.takes(adjoint, term, y0, problem.t_start) else None
+            hits = simulate_hits(replay, states, E) if arrays is None else None
             if use_kernels:
-                adj, grad_params = reverse_sweep_kernels(adjoint, replay, term, args, problem, ctx.dt0, dt0, states, hits, grad_ys, params, list(ctx.params))
+                adj, grad_params = reverse_sweep_kernels(
+                    adjoint, replay, term, args, problem, ctx.dt0, dt0, states, hits, grad_ys, params, list(ctx.params), arrays
+                )
             else:
                 adj, grad_params = reverse_sweep_torch(replay, states, hits, grad_ys, params)
 

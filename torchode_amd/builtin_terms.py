@@ -168,15 +168,15 @@ class MLPField(BuiltinTerm):
         """W1 | b1 | W2 | b2, row-major and concatenated."""
         return torch.cat([w.reshape(-1) for w in (self.W1, self.b1, self.W2, self.b2)]).contiguous()
 
-    def builtin_packed(self, device, dtype) -> torch.Tensor:
+    def builtin_packed(self, device, dtype, fresh: bool = False) -> torch.Tensor:
         """The weights in the order the whole-solve kernel loads them into registers (a device
         tensor).  Packed once, and again whenever a weight tensor has been replaced or written
-        in place."""
+        in place; ``fresh``: for this call, whatever was kept (a training step changes its weights every time)."""
         from . import _lib
 
         weights = (self.W1, self.b1, self.W2, self.b2)
         key = (tuple((w.data_ptr(), w._version) for w in weights), device, dtype, self.matrix_inputs)
-        if getattr(self, "_packed_key", None) != key:
+        if fresh or getattr(self, "_packed_key", None) != key:
             raw = self.builtin_shared().to(device=device, dtype=dtype)
             packed = torch.empty(_lib.MLP_PACKED_SIZE[self.matrix_inputs], dtype=dtype, device=device)
             rc = _lib.load().tode_mlp_pack_weights_for(

@@ -292,8 +292,8 @@ int tode_solve_builtin_fast(const tode_solve_args *a, const tode_controller *c, 
     hipStream_t s = (hipStream_t)stream;
     if (!known_dtype(a->dtype)) return fail(TODE_E_INVALID, "unknown dtype %d", a->dtype);
     if (a->dtype & TODE_DTYPE_PAIR) return fail(TODE_E_UNSUPPORTED, "the fast entry point is built for time and data in one dtype");
-    if (a->record && (a->term == TODE_TERM_REACTION_DIFFUSION || a->term == TODE_TERM_MLP))
-        return fail(TODE_E_UNSUPPORTED, "a record of the loop state is written for the small systems only");
+    if (a->record && a->term == TODE_TERM_REACTION_DIFFUSION)
+        return fail(TODE_E_UNSUPPORTED, "a record of the loop state is written for the small systems and the network only");
     if (a->term == TODE_TERM_REACTION_DIFFUSION) {
         return a->dtype == TODE_F32 ? solve_grid_f32(*a, *c, ns, na, ni, st, s) : solve_grid_f64(*a, *c, ns, na, ni, st, s);
     }

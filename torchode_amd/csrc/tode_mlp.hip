@@ -56,7 +56,12 @@ static __global__ void mlp_pack_kernel(const float *raw, float *packed, int H, i
 
 // FULL: all 64 state values are the problem's and evaluation points are given (the feature count and the end-point mode are
 // constants and their tests fold away).
-template <int METHOD, int CTRL, typename Weights, bool FULL>
+// RECORD: the loop state before every iteration of the workgroup goes to p.rec_* (tode_solve_record), and the state its samples
+// are left in fills the record up to its capacity with `running` 0, as in the small systems' kernels; a record that is too
+// short raises TODE_FLAG_NEEDS_GENERAL (TODE_FLAG_MAX_ITERATIONS says how long it has to be).  For gradients: f there takes the
+// math library's tanh, since it stands where torch's evaluations of the network stood.  Network of 64 and 256 at B = 4096:
+// solve and record in 0.12 ms, where the per-step kernels around torch's products took 2.6 ms.
+template <int METHOD, int CTRL, typename Weights, bool FULL, bool RECORD>
 __global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2, 2))) solve_mlp_kernel(const SolveParams<float> p, const float *packed, const MlpOut o) {
     using T = float;
     using Tab = typename std::conditional<METHOD == 1, Tsit5Tab, Dopri5Tab>::type;
@@ -122,7 +127,11 @@ __global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2, 2))
     int cursor = 0, n_steps = 0, n_acc = 0;
 
     // ---- first step size (step_size_controllers.py:431-490, 776-835) ----
-    mlp_rhs(sh, W, ts, y, k[0]);
+    const auto rhs = [&](float tn, const float (&yi)[4], float (&out)[4]) {
+        if constexpr (RECORD) mlp_rhs<true>(sh, W, tn, yi, out);
+        else mlp_rhs(sh, W, tn, yi, out);
+    };
+    rhs(ts, y, k[0]);
     if (p.dt0) {
         dt = p.dt0[bs];
     } else {
@@ -140,7 +149,7 @@ __global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2, 2))
         const T h0 = tmin(h, abs_(te - ts));
 #pragma unroll
         for (int r = 0; r < 4; ++r) y1[r] = fma_(dir * h0, k[0][r], y[r]);
-        mlp_rhs(sh, W, fma_(dir, h0, ts), y1, f1);
+        rhs(fma_(dir, h0, ts), y1, f1);
 #pragma unroll
         for (int r = 0; r < 4; ++r) {
             const T x2 = ((f1[r] - k[0][r]) * inv[r]) / sf;
@@ -163,7 +172,22 @@ __global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2, 2))
     // iterations with the clamped step t_end - t, which is seen only in the status of that step: the sample sits
     // through one more iteration here, inactive, and the status of its step is looked at.
     bool idle = false, idle_done = false;
+    long long iteration = 0;  // (RECORD) of this workgroup, so far
+    auto keep = [&](bool running) {
+        if (iteration >= p.rec_capacity || !live) return;
+        const long long at = iteration * p.batch + bs;
+        put(p.rec_y + at * FR, y);
+        put(p.rec_k0 + at * FR, k[0]);
+        if (w == 0 && q == 0) {
+            p.rec_t[at] = t, p.rec_dt[at] = dt, p.rec_prev[at] = prev, p.rec_pprev[at] = pprev;
+            p.rec_running[at] = running ? 1 : 0, p.rec_n_accepted[at] = n_acc;
+        }
+    };
     while (state == 1) {
+        if (RECORD) {
+            keep(active);
+            ++iteration;
+        }
         // ---- stages (runge_kutta.py:255-263) ----
         const T t0 = t;
         T y1[4];
@@ -177,7 +201,7 @@ __global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2, 2))
                 for (int j = 0; j < i; ++j) s = fma_((T)Tab::a[i][j], k[j][r], s);
                 yi[r] = fma_(dt, s, y[r]);
             }
-            mlp_rhs(sh, W, fma_((T)Tab::c[i], dt, t0), yi, k[i]);
+            rhs(fma_((T)Tab::c[i], dt, t0), yi, k[i]);
             if (i == 6) {
 #pragma unroll
                 for (int r = 0; r < 4; ++r) y1[r] = yi[r];
@@ -269,6 +293,10 @@ __global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2, 2))
         bail = (state & 2) != 0;
     }
 
+    if (RECORD) {
+        bail = bail || iteration >= p.rec_capacity;  // (the state after the last iteration is an entry as well)
+        for (; iteration < p.rec_capacity; ++iteration) keep(false);
+    }
     if (end_only && live && !idle_done) put(p.y_idle + bs * FR, y);  // the final state
     if (w == 0) {
         if (q == 0 && live) {
@@ -297,10 +325,14 @@ template <int METHOD, int CTRL, typename Weights> static int launch_mlp(const to
     const size_t lds = (size_t)MLP_TILE * (a.n_eval > 0 ? a.n_eval : 1) * sizeof(float);
     const unsigned blocks = (unsigned)((a.batch + MLP_TILE - 1) / MLP_TILE);
     timing_before(stream, std::is_same<Weights, MlpWeightsBf16>::value ? "tode::solve_mlp_kernel (bfloat16 matrix inputs)" : "tode::solve_mlp_kernel");
-    if (o.n_features == MLP_F && a.n_eval > 0)
-        hipLaunchKernelGGL((solve_mlp_kernel<METHOD, CTRL, Weights, true>), dim3(blocks), dim3(256), lds, stream, p, (const float *)a.shared_params, o);
-    else
-        hipLaunchKernelGGL((solve_mlp_kernel<METHOD, CTRL, Weights, false>), dim3(blocks), dim3(256), lds, stream, p, (const float *)a.shared_params, o);
+    const bool full = o.n_features == MLP_F && a.n_eval > 0;
+    const auto launch = [&](auto kernel) { hipLaunchKernelGGL(kernel, dim3(blocks), dim3(256), lds, stream, p, (const float *)a.shared_params, o); };
+    if constexpr (std::is_same<Weights, MlpWeights>::value) {
+        if (a.record && full) launch(solve_mlp_kernel<METHOD, CTRL, Weights, true, true>);
+        else if (a.record) launch(solve_mlp_kernel<METHOD, CTRL, Weights, false, true>);
+    }
+    if (!a.record && full) launch(solve_mlp_kernel<METHOD, CTRL, Weights, true, false>);
+    else if (!a.record) launch(solve_mlp_kernel<METHOD, CTRL, Weights, false, false>);
     timing_after(stream);
     return check_hip(hipGetLastError(), "tode_solve_builtin_fast launch");
 }
@@ -321,6 +353,12 @@ int solve_mlp_f32(const tode_solve_args &a, const tode_controller &c, int64_t *n
                     "(%d or %d values); got F=%d and %lld shared parameters", TODE_MLP_PACKED_SIZE, TODE_MLP_PACKED_SIZE_BF16, a.n_features,
                     (long long)a.n_shared_params);
     if (!a.shared_params) return fail(TODE_E_INVALID, "null shared_params");
+    if (a.record) {
+        const tode_solve_record &r = *a.record;
+        if (bf16 || a.n_eval == 0) return fail(TODE_E_UNSUPPORTED, "the MLP kernel writes a record for float32 matrix inputs and evaluation points only");
+        if (r.capacity < 1 || !r.t || !r.dt || !r.y || !r.k0 || !r.prev || !r.pprev || !r.running || !r.n_accepted)
+            return fail(TODE_E_INVALID, "tode_solve_record: capacity %lld, or a null array", (long long)r.capacity);
+    }
     if (a.n_eval > 512) return fail(TODE_E_UNSUPPORTED, "n_eval=%d is too large for the MLP kernel", a.n_eval);
     if (a.batch > (long long)INT_MAX * MLP_TILE) return fail(TODE_E_UNSUPPORTED, "batch too large");
     MlpOut o{ns, na, ni, st, a.n_features};
