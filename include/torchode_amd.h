@@ -125,7 +125,8 @@ typedef struct tode_controller {
  * tode_finalize_stats.
  */
 /*
- * Optional record of the loop state, written by tode_solve_builtin (the general kernel) and, for the three small
+ * Optional record of the loop state, written by tode_solve_builtin (the general kernel) and, for the network (float32
+ * matrix inputs, evaluation points) and the three small
  * systems with evaluation points, by tode_solve_builtin_fast and its _sync / _static forms (the two-wavefront or the
  * single-wavefront kernel: the solve and its record in one launch) when tode_solve_args.record points to one: entry i
  * holds what the reference's loop variables hold before iteration i
@@ -426,6 +427,18 @@ typedef struct tode_mlp_reverse {
 int tode_mlp_pack_weights_reverse(const void *raw, int64_t n_raw, int32_t n_features, void *packed, void *stream);
 int tode_mlp_stages(const tode_mlp_reverse *p, void *stream);
 int tode_mlp_stages_backward(const tode_mlp_reverse *p, int32_t accumulate, void *stream);
+/*
+ * The start of the loop reversed (y = y0, k0 = f(t_start, y0), the start rule's first step clamped to the time range; the times
+ * are constants): p->t, y, k0 are the record's first entry, p->g_y receives the cotangent of y0; the weights' share is
+ * added as by tode_mlp_stages_backward, ahead of tode_mlp_weight_gradients.
+ */
+typedef struct tode_mlp_start {
+    const void *t_end;                /* [B] */
+    const void *a_y, *a_k0, *a_dt;    /* [B,F], [B,F], [B] cotangents of that first loop state */
+    int32_t through_rule;             /* the first step is a function of y0 and the weights (no step of the user's, gradients
+                                         through the step sizes) */
+} tode_mlp_start;
+int tode_mlp_start_backward(const tode_mlp_reverse *p, const tode_mlp_start *start, const tode_controller *c, int32_t accumulate, void *stream);
 int tode_mlp_weight_gradients(const tode_mlp_reverse *p, void *out, void *stream);
 
 /* ------------------------------------------------------------------------- */

@@ -49,6 +49,7 @@ EXPORTS = (
     "tode_mlp_pack_weights_reverse",
     "tode_mlp_stages",
     "tode_mlp_stages_backward",
+    "tode_mlp_start_backward",
     "tode_mlp_weight_gradients",
     "tode_select_end_point",
     "tode_step_begin",
@@ -214,6 +215,12 @@ class MlpReverse(C.Structure):
     ]  # fmt: skip
 
 
+class MlpStart(C.Structure):
+    """struct tode_mlp_start"""
+
+    _fields_ = [(name, C.c_void_p) for name in ("t_end", "a_y", "a_k0", "a_dt")] + [("through_rule", C.c_int32)]
+
+
 class StepAdjoint(C.Structure):
     """struct tode_step_adjoint"""
 
@@ -354,6 +361,8 @@ def load():
         lib.tode_mlp_stages.argtypes = [C.POINTER(MlpReverse), C.c_void_p]
         lib.tode_mlp_stages_backward.restype = C.c_int
         lib.tode_mlp_stages_backward.argtypes = [C.POINTER(MlpReverse), C.c_int32, C.c_void_p]
+        lib.tode_mlp_start_backward.restype = C.c_int
+        lib.tode_mlp_start_backward.argtypes = [C.POINTER(MlpReverse), C.POINTER(MlpStart), C.POINTER(Controller), C.c_int32, C.c_void_p]
         lib.tode_mlp_weight_gradients.restype = C.c_int
         lib.tode_mlp_weight_gradients.argtypes = [C.POINTER(MlpReverse), C.c_void_p, C.c_void_p]
         lib.tode_solve_builtin_fast_static.restype = C.c_int

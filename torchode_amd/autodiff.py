@@ -565,6 +565,15 @@ class NetworkSweep:
         _lib.check(self.lib.tode_mlp_stages_backward(self.ref, int(self.started), self.stream), "tode_mlp_stages_backward")
         self.started = True
 
+    def start_backward(self, controller, state, t_end, a_y, a_k0, a_dt, g_k, g_y, through_rule):
+        """The start of the loop reversed; ``g_y`` becomes the cotangent of ``y0`` (``g_k``: room for those of the derivatives)."""
+        a = self.args
+        a.t, a.dt, a.y, a.k0 = (state[k].data_ptr() for k in ("t", "dt", "y", "k0"))
+        a.g_k, a.g_y = g_k.data_ptr(), g_y.data_ptr()
+        start = _lib.MlpStart(t_end.data_ptr(), a_y.data_ptr(), a_k0.data_ptr(), a_dt.data_ptr(), int(bool(through_rule)))
+        _lib.check(self.lib.tode_mlp_start_backward(self.ref, _lib.C.byref(start), controller, int(self.started), self.stream), "tode_mlp_start_backward")
+        self.started = True
+
     def weight_gradients(self, params):
         """The gradients of ``params`` through the weights: autograd carries those of the held tensors on to the leaves."""
         f = self.f
@@ -751,6 +760,13 @@ def reverse_sweep_kernels(adjoint, replay: Replay, term, args, problem, dt0_give
                 grad_params[j] = _add(grad_params[j], g)
         adj = (g_y.clone(), g_k[0].clone(), g_t.clone(), g_dt.clone(), g_hist[0].clone(), g_hist[1].clone())
 
+    through_start = False
+    if arrays is not None and not any(wants(x) for x in (replay.t_start, replay.t_end, replay.t_eval, dt0)):
+        # the start of the loop in kernels as well (they take its times as constants): what comes back is the cotangent of y0
+        a_y, a_k0, _, a_dt = adj[:4]
+        g_k, g_y = sets[1][:2]
+        network.start_backward(cref, states[0], t_end, a_y, a_k0, a_dt, g_k, g_y, dt0_given is None and replay.through_control)
+        adj, through_start = (g_y, *adj[1:]), True
     if network is not None:
         grad_params = network.weight_gradients(params)
 
@@ -765,7 +781,7 @@ def reverse_sweep_kernels(adjoint, replay: Replay, term, args, problem, dt0_give
                 break
     out = {k: None for k in STATE_NAMES}
     if adj is not None:
-        out = dict(zip(STATE_NAMES, adj))
+        out = dict(zip(STATE_NAMES, adj), through_start=through_start)
     return out, grad_params
 
 

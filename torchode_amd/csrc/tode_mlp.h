@@ -277,7 +277,7 @@ __device__ __forceinline__ void mlp_load(MlpWeightsBf16 &W, const float *packed,
 
 // Per-sample sums over the 64 features of two quantities at once: the lane's four features, the
 // four lane groups of a wavefront by shuffles, the four wavefronts through LDS.
-__device__ __forceinline__ void mlp_sum2(MlpShared &sh, int &slot, const float (&a)[4], const float (&b)[4], float &A, float &B) {
+template <typename Shared> __device__ __forceinline__ void mlp_sum2(Shared &sh, int &slot, const float (&a)[4], const float (&b)[4], float &A, float &B) {
     const int lane = threadIdx.x & 63, w = threadIdx.x >> 6, q = lane >> 4, c = lane & 15;
     float u = (a[0] + a[1]) + (a[2] + a[3]), v = (b[0] + b[1]) + (b[2] + b[3]);
 #pragma unroll

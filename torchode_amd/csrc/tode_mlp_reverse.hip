@@ -107,8 +107,87 @@ template <int METHOD> __global__ void __launch_bounds__(256) __attribute__((amdg
 struct __align__(16) MlpReverseShared {
     float g[MLP_TILE * MLP_XS];   // cotangent of the stage derivative: [sample][feature]
     float part[4][4][64][4];      // [16 inputs][wavefront it comes from][lane][4 inputs]
-    float red[4][MLP_TILE][2];
+    float red[2][4][MLP_TILE][2]; // sums over a sample's features (mlp_sum2)
 };
+
+struct MlpReverseWeights {
+    float w2t[16][4];   // W2[16q + kk][64w + 16 tile + c]
+    float w1t[4][16];   // W1[64w + 16 tile + 4q + r][16 it + c]
+    float wt[16];       // W1[64w + 16 tile + 4q + r][time]
+};
+
+__device__ __forceinline__ void mlp_load(MlpReverseWeights &W, const float *packed, int tid) {
+    const float4 *src = reinterpret_cast<const float4 *>(packed) + tid;
+#pragma unroll
+    for (int i = 0; i < MLP_REVERSE_REGS / 4; ++i) {
+        const float4 u = src[i * 256];
+        const float v[4] = {u.x, u.y, u.z, u.w};
+#pragma unroll
+        for (int r = 0; r < 4; ++r) {
+            if (i < 16) W.w2t[i][r] = v[r];
+            else if (i < 32) W.w1t[(i - 16) / 4][4 * ((i - 16) % 4) + r] = v[r];
+            else W.wt[4 * (i - 32) + r] = v[r];
+        }
+    }
+}
+
+// The network's vector-Jacobian product for the lane's sample: g (cotangent of f, the lane's four features) to gi (of y) and
+// gt (of t: this lane's share, to be summed over the sample's lanes).  hidden: the sample's row of hidden activations;
+// cotangents: its row of the cotangents in front of tanh, to be written, or null.
+__device__ __forceinline__ void mlp_vjp(MlpReverseShared &sh, const MlpReverseWeights &W, const float (&gf)[4], const float *hidden, float *cotangents, float (&gi)[4], float &gt) {
+    const int lane = threadIdx.x & 63, w = threadIdx.x >> 6, q = lane >> 4, c = lane & 15;
+    *reinterpret_cast<float4 *>(sh.g + c * MLP_XS + 16 * w + 4 * q) = make_float4(gf[0], gf[1], gf[2], gf[3]);
+    float4 h[4];
+#pragma unroll
+    for (int u = 0; u < 4; ++u) h[u] = *reinterpret_cast<const float4 *>(hidden + 64 * w + 16 * u + 4 * q);
+    lds_barrier();
+    float g[16];
+    {
+        const float4 *at = reinterpret_cast<const float4 *>(sh.g + c * MLP_XS + 16 * q);
+#pragma unroll
+        for (int j = 0; j < 4; ++j) {
+            const float4 v = at[j];
+            g[4 * j] = v.x, g[4 * j + 1] = v.y, g[4 * j + 2] = v.z, g[4 * j + 3] = v.w;
+        }
+    }
+    mfma_acc d[4];
+#pragma unroll
+    for (int u = 0; u < 4; ++u) d[u] = {0.0f, 0.0f, 0.0f, 0.0f};
+#pragma unroll
+    for (int kk = 0; kk < 16; ++kk)
+#pragma unroll
+        for (int u = 0; u < 4; ++u) d[u] = __builtin_amdgcn_mfma_f32_16x16x4f32(W.w2t[kk][u], g[kk], d[u], 0, 0, 0);
+    gt = 0;
+#pragma unroll
+    for (int u = 0; u < 4; ++u) {
+        const float hv[4] = {h[u].x, h[u].y, h[u].z, h[u].w};
+#pragma unroll
+        for (int r = 0; r < 4; ++r) {
+            d[u][r] = d[u][r] * fma_(-hv[r], hv[r], 1.0f);
+            gt = fma_(W.wt[4 * u + r], d[u][r], gt);
+        }
+        if (cotangents) *reinterpret_cast<float4 *>(cotangents + 64 * w + 16 * u + 4 * q) = make_float4(d[u][0], d[u][1], d[u][2], d[u][3]);
+    }
+    mfma_acc acc[4];
+#pragma unroll
+    for (int it = 0; it < 4; ++it) acc[it] = {0.0f, 0.0f, 0.0f, 0.0f};
+#pragma unroll
+    for (int u = 0; u < 4; ++u)
+#pragma unroll
+        for (int r = 0; r < 4; ++r)
+#pragma unroll
+            for (int it = 0; it < 4; ++it) acc[it] = __builtin_amdgcn_mfma_f32_16x16x4f32(W.w1t[it][4 * u + r], d[u][r], acc[it], 0, 0, 0);
+#pragma unroll
+    for (int it = 0; it < 4; ++it) *reinterpret_cast<float4 *>(sh.part[it][w][lane]) = make_float4(acc[it][0], acc[it][1], acc[it][2], acc[it][3]);
+    lds_barrier();
+    float4 v[4];
+#pragma unroll
+    for (int from = 0; from < 4; ++from) v[from] = *reinterpret_cast<const float4 *>(sh.part[w][from][lane]);
+    gi[0] = (v[0].x + v[1].x) + (v[2].x + v[3].x);
+    gi[1] = (v[0].y + v[1].y) + (v[2].y + v[3].y);
+    gi[2] = (v[0].z + v[1].z) + (v[2].z + v[3].z);
+    gi[3] = (v[0].w + v[1].w) + (v[2].w + v[3].w);
+}
 
 // One wavefront per SIMD: 144 registers of weights, 28 + 24 of stage derivatives and their cotangents.  A workgroup takes
 // several tiles where the batch has more than the grid, so that the weights are loaded once.
@@ -117,21 +196,9 @@ template <int METHOD> __global__ void __launch_bounds__(256) __attribute__((amdg
     __shared__ MlpReverseShared sh;
     const int tid = threadIdx.x, lane = tid & 63, w = tid >> 6, q = lane >> 4, c = lane & 15, FR = p.n_features, f0 = 16 * w + 4 * q;
     const long long B = p.batch, tiles = (B + MLP_TILE - 1) / MLP_TILE;
-    float w2t[16][4], w1t[4][16], wt[16];
-    {
-        const float4 *src = reinterpret_cast<const float4 *>(p.packed_reverse) + tid;
-#pragma unroll
-        for (int i = 0; i < MLP_REVERSE_REGS / 4; ++i) {
-            const float4 u = src[i * 256];
-            const float v[4] = {u.x, u.y, u.z, u.w};
-#pragma unroll
-            for (int r = 0; r < 4; ++r) {
-                if (i < 16) w2t[i][r] = v[r];
-                else if (i < 32) w1t[(i - 16) / 4][4 * ((i - 16) % 4) + r] = v[r];
-                else wt[4 * (i - 32) + r] = v[r];
-            }
-        }
-    }
+    MlpReverseWeights W;
+    mlp_load(W, (const float *)p.packed_reverse, tid);
+    int slot = 0;
     for (long long tile = blockIdx.x; tile < tiles; tile += gridDim.x) {
         const bool live = tile * MLP_TILE + c < B;
         const long long b = live ? tile * MLP_TILE + c : B - 1;
@@ -147,59 +214,11 @@ template <int METHOD> __global__ void __launch_bounds__(256) __attribute__((amdg
 #pragma unroll
         for (int s = 6; s >= 1; --s) {
             const long long row = (s - 1) * B + b;
-            *reinterpret_cast<float4 *>(sh.g + c * MLP_XS + f0) = make_float4(gk[s][0], gk[s][1], gk[s][2], gk[s][3]);
             if (s < 6 && live) mlp_put((float *)p.g_k + (s * B + b) * FR, f0, FR, gk[s]);  // (final: the weights' gradients read it)
-            float4 h[4];
-#pragma unroll
-            for (int u = 0; u < 4; ++u) h[u] = *reinterpret_cast<const float4 *>((const float *)p.hidden + row * MLP_H + 64 * w + 16 * u + 4 * q);
-            lds_barrier();
-            float g[16];
-            {
-                const float4 *at = reinterpret_cast<const float4 *>(sh.g + c * MLP_XS + 16 * q);
-#pragma unroll
-                for (int j = 0; j < 4; ++j) {
-                    const float4 v = at[j];
-                    g[4 * j] = v.x, g[4 * j + 1] = v.y, g[4 * j + 2] = v.z, g[4 * j + 3] = v.w;
-                }
-            }
-            mfma_acc d[4];
-#pragma unroll
-            for (int u = 0; u < 4; ++u) d[u] = {0.0f, 0.0f, 0.0f, 0.0f};
-#pragma unroll
-            for (int kk = 0; kk < 16; ++kk)
-#pragma unroll
-                for (int u = 0; u < 4; ++u) d[u] = __builtin_amdgcn_mfma_f32_16x16x4f32(w2t[kk][u], g[kk], d[u], 0, 0, 0);
-            float gt = 0;
-#pragma unroll
-            for (int u = 0; u < 4; ++u) {
-                const float hv[4] = {h[u].x, h[u].y, h[u].z, h[u].w};
-#pragma unroll
-                for (int r = 0; r < 4; ++r) {
-                    d[u][r] = d[u][r] * fma_(-hv[r], hv[r], 1.0f);
-                    gt = fma_(wt[4 * u + r], d[u][r], gt);
-                }
-                if (live && p.hidden_cotangents)
-                    *reinterpret_cast<float4 *>((float *)p.hidden_cotangents + row * MLP_H + 64 * w + 16 * u + 4 * q) = make_float4(d[u][0], d[u][1], d[u][2], d[u][3]);
-            }
+            float gi[4], gt;
+            mlp_vjp(sh, W, gk[s], (const float *)p.hidden + row * MLP_H, live && p.hidden_cotangents ? (float *)p.hidden_cotangents + row * MLP_H : nullptr, gi, gt);
             g_t += gt;
             g_dt = fma_((float)Tab::c[s], gt, g_dt);
-            mfma_acc acc[4];
-#pragma unroll
-            for (int it = 0; it < 4; ++it) acc[it] = {0.0f, 0.0f, 0.0f, 0.0f};
-#pragma unroll
-            for (int u = 0; u < 4; ++u)
-#pragma unroll
-                for (int r = 0; r < 4; ++r)
-#pragma unroll
-                    for (int it = 0; it < 4; ++it) acc[it] = __builtin_amdgcn_mfma_f32_16x16x4f32(w1t[it][4 * u + r], d[u][r], acc[it], 0, 0, 0);
-#pragma unroll
-            for (int it = 0; it < 4; ++it) *reinterpret_cast<float4 *>(sh.part[it][w][lane]) = make_float4(acc[it][0], acc[it][1], acc[it][2], acc[it][3]);
-            lds_barrier();
-            float4 v[4];
-#pragma unroll
-            for (int from = 0; from < 4; ++from) v[from] = *reinterpret_cast<const float4 *>(sh.part[w][from][lane]);
-            float gi[4] = {(v[0].x + v[1].x) + (v[2].x + v[3].x), (v[0].y + v[1].y) + (v[2].y + v[3].y), (v[0].z + v[1].z) + (v[2].z + v[3].z),
-                           (v[0].w + v[1].w) + (v[2].w + v[3].w)};
             // the stage's sum reversed (stage_backward_sample)
 #pragma unroll
             for (int r = 0; r < 4; ++r) {
@@ -214,19 +233,184 @@ template <int METHOD> __global__ void __launch_bounds__(256) __attribute__((amdg
                 g_dt = fma_(gi[r], sum, g_dt);
             }
         }
-        // the sample's shares of the cotangents of t and dt: four lane groups of four wavefronts
-#pragma unroll
-        for (int off = 16; off < 64; off <<= 1) g_t += __shfl_xor(g_t, off), g_dt += __shfl_xor(g_dt, off);
-        if (q == 0) sh.red[w][c][0] = g_t, sh.red[w][c][1] = g_dt;
-        lds_barrier();  // (the next tile's sums come behind its own barriers, so one set of words is enough)
+        const float share_t[4] = {g_t, 0, 0, 0}, share_dt[4] = {g_dt, 0, 0, 0};
+        mlp_sum2(sh, slot, share_t, share_dt, g_t, g_dt);
         if (live) {
             mlp_put((float *)p.g_y + b * FR, f0, FR, gy);
             mlp_put((float *)p.g_k + b * FR, f0, FR, gk[0]);
             if (w == 0 && q == 0) {
-                ((float *)p.g_t)[b] += (sh.red[0][c][0] + sh.red[1][c][0]) + (sh.red[2][c][0] + sh.red[3][c][0]);
-                ((float *)p.g_dt)[b] += (sh.red[0][c][1] + sh.red[1][c][1]) + (sh.red[2][c][1] + sh.red[3][c][1]);
+                ((float *)p.g_t)[b] += g_t;
+                ((float *)p.g_dt)[b] += g_dt;
             }
         }
+    }
+}
+
+// The start of the loop (y = y0, k0 = f(t_start, y0) and, with THROUGH, the step of the start rule clamped to the time range,
+// step_size_controllers.py:431-490 / 776-835, adjoints.py:86-107), its evaluations of the network again: slot 0 of the stage
+// buffers f(t_start, y0), slot 1 (THROUGH) the start rule's probe, whose value goes to p.k.
+__device__ __forceinline__ void mlp_start_scale(const CtrlParams<float> &cp, int f0, int FR, float sf, const float (&y)[4], const float (&k0)[4], float (&inv)[4], float (&a0)[4],
+                                                float (&a1)[4]) {
+#pragma unroll
+    for (int r = 0; r < 4; ++r) {
+        inv[r] = f0 + r < FR ? 1.0f / fma_(cp.rtol, abs_(y[r]), cp.atol) : 0.0f;  // (features beyond the problem's add nothing to the norms)
+        const float u = (y[r] * inv[r]) / sf, v = (k0[r] * inv[r]) / sf;
+        a0[r] = u * u, a1[r] = v * v;
+    }
+}
+
+__device__ __forceinline__ float mlp_start_probe_step(float d0, float d1, float span, bool &small, float &h0a) {
+    small = d0 < 1e-5f || d1 < 1e-5f;
+    h0a = small ? 1e-6f : (0.01f * d0) / d1;
+    return tmin(h0a, span);
+}
+
+template <bool THROUGH>
+__global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2, 2))) mlp_start_kernel(const tode_mlp_reverse p, const tode_mlp_start st, const CtrlParams<float> cp) {
+    __shared__ MlpShared sh;
+    const int tid = threadIdx.x, lane = tid & 63, w = tid >> 6, q = lane >> 4, c = lane & 15, FR = p.n_features, f0 = 16 * w + 4 * q;
+    const long long B = p.batch, tiles = (B + MLP_TILE - 1) / MLP_TILE;
+    const float sf = (float)__builtin_sqrt((double)FR);
+    MlpWeights W;
+    mlp_load(W, (const float *)p.packed, tid);
+    for (int i = tid; i < MLP_TILE * MLP_XS; i += 256) sh.x[i] = 0.0f;
+    __syncthreads();
+    int slot = 0;
+    for (long long tile = blockIdx.x; tile < tiles; tile += gridDim.x) {
+        const bool live = tile * MLP_TILE + c < B;
+        const long long b = live ? tile * MLP_TILE + c : B - 1;
+        float y[4], k0[4], out[4];
+        mlp_get((const float *)p.y + b * FR, f0, FR, y);
+        mlp_get((const float *)p.k0 + b * FR, f0, FR, k0);
+        const auto evaluate = [&](int at, float t, const float (&x)[4]) {
+            const long long row = at * B + b;
+            if (live) {
+                mlp_put((float *)p.stage_inputs + row * FR, f0, FR, x);
+                if (w == 0 && q == 0) ((float *)p.stage_times)[row] = t;
+            }
+            mlp_rhs<true>(sh, W, t, x, out, live ? (float *)p.hidden + row * MLP_H : nullptr);
+        };
+        const float ts = ((const float *)p.t)[b], te = ((const float *)st.t_end)[b];
+        evaluate(0, ts, y);
+        if (THROUGH) {
+            float inv[4], a0[4], a1[4], d0, d1, h0a, y1[4];
+            mlp_start_scale(cp, f0, FR, sf, y, k0, inv, a0, a1);
+            mlp_sum2(sh, slot, a0, a1, d0, d1);
+            bool small;
+            const float dir = te > ts ? 1.0f : -1.0f, h0 = mlp_start_probe_step(sqrt_(d0), sqrt_(d1), abs_(te - ts), small, h0a);
+#pragma unroll
+            for (int r = 0; r < 4; ++r) y1[r] = fma_(dir * h0, k0[r], y[r]);
+            evaluate(1, fma_(dir, h0, ts), y1);
+            if (live) mlp_put((float *)p.k + b * FR, f0, FR, out);
+        }
+    }
+}
+
+// The same reversed: the cotangents a_y, a_k0, a_dt of the first loop state to that of y0 (p.g_y), those of the two evaluations of
+// the network left in slots 1 and 2 of p.g_k for the weights' gradients.  The times are constants here.  (start_backward of
+// the small systems, a sample's row spread over sixteen lanes; a term that a sample does not have is selected away, since
+// all lanes meet at the barriers of the sums and products.)
+template <bool THROUGH>
+__global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(1, 1))) mlp_start_backward_kernel(const tode_mlp_reverse p, const tode_mlp_start st, const CtrlParams<float> cp,
+                                                                                                           const bool integral) {
+    __shared__ MlpReverseShared sh;
+    const int tid = threadIdx.x, lane = tid & 63, w = tid >> 6, q = lane >> 4, c = lane & 15, FR = p.n_features, f0 = 16 * w + 4 * q;
+    const long long B = p.batch, tiles = (B + MLP_TILE - 1) / MLP_TILE;
+    const float sf = (float)__builtin_sqrt((double)FR);
+    const auto share_of_min = [](float a, float b) { return a < b ? 1.0f : (a == b ? 0.5f : 0.0f); };
+    const auto share_of_max = [](float a, float b) { return a > b ? 1.0f : (a == b ? 0.5f : 0.0f); };
+    MlpReverseWeights W;
+    mlp_load(W, (const float *)p.packed_reverse, tid);
+    int slot = 0;
+    for (long long tile = blockIdx.x; tile < tiles; tile += gridDim.x) {
+        const bool live = tile * MLP_TILE + c < B;
+        const long long b = live ? tile * MLP_TILE + c : B - 1;
+        float g_y0[4], g_k0[4], gi[4], gt;
+        mlp_get((const float *)st.a_y + b * FR, f0, FR, g_y0);
+        mlp_get((const float *)st.a_k0 + b * FR, f0, FR, g_k0);
+        const auto product = [&](int at, const float (&g)[4]) {
+            const long long row = at * B + b;
+            if (live) mlp_put((float *)p.g_k + (B + row) * FR, f0, FR, g);
+            mlp_vjp(sh, W, g, (const float *)p.hidden + row * MLP_H, live && p.hidden_cotangents ? (float *)p.hidden_cotangents + row * MLP_H : nullptr, gi, gt);
+        };
+        if (THROUGH) {
+            // ---- forward values ----
+            float y[4], k0[4], f1[4], inv[4], a0[4], a1[4], a2[4], none[4] = {0, 0, 0, 0}, A0, A1, A2, unused;
+            mlp_get((const float *)p.y + b * FR, f0, FR, y);
+            mlp_get((const float *)p.k0 + b * FR, f0, FR, k0);
+            mlp_get((const float *)p.k + b * FR, f0, FR, f1);
+            const float ts = ((const float *)p.t)[b], te = ((const float *)st.t_end)[b], a_dt = ((const float *)st.a_dt)[b];
+            mlp_start_scale(cp, f0, FR, sf, y, k0, inv, a0, a1);
+#pragma unroll
+            for (int r = 0; r < 4; ++r) {
+                const float x = ((f1[r] - k0[r]) * inv[r]) / sf;
+                a2[r] = x * x;
+            }
+            mlp_sum2(sh, slot, a0, a1, A0, A1);
+            mlp_sum2(sh, slot, a2, none, A2, unused);
+            const float d0 = sqrt_(A0), d1 = sqrt_(A1), r2 = sqrt_(A2), dir = te > ts ? 1.0f : -1.0f, span = abs_(te - ts);
+            bool small;
+            float h0a;
+            const float h0 = mlp_start_probe_step(d0, d1, span, small, h0a), dh = dir * h0;
+            const bool blocked = integral && h0 == 0.0f;  // (the integral controller's copy of the rule: d2 = inf)
+            const float d2 = blocked ? __builtin_huge_valf() : r2 / h0, m = tmax(d1, d2);
+            const bool tiny = m <= 1e-15f;
+            const float rm = 1.0f / m, z = rm * 0.01f;
+            const float h1 = tiny ? tmax(1e-6f, h0 * 1e-3f) : rpow<float>(z, 1.0 / 5.0);
+            const float first = dir * tmin(100.0f * h0, h1), lo = tmin(ts, te) - ts, hi = tmax(te, ts) - ts;
+            // ---- reversed ----
+            const bool on = a_dt != 0.0f;
+            const float g_min = (on && first >= lo && first <= hi) ? a_dt * dir : 0.0f;
+            float g_h0 = 100.0f * (g_min * share_of_min(100.0f * h0, h1)), g_d1 = 0, g_d2 = 0;
+            const float g_h1 = g_min * share_of_min(h1, 100.0f * h0);
+            if (on && tiny) g_h0 += (h0 * 1e-3f >= 1e-6f) ? g_h1 * 1e-3f : 0.0f;
+            if (on && !tiny) {
+                const float g_z = g_h1 * (0.2f * rpow<float>(z, 1.0 / 5.0 - 1.0)), g_m = -(g_z * 0.01f) * rm * rm;
+                g_d1 = g_m * share_of_max(d1, d2), g_d2 = g_m * share_of_max(d2, d1);
+            }
+            const bool probe = on && !blocked && g_d2 != 0.0f;
+            float g_inv[4], g_f1[4], g_step[4];
+            const float g_r2 = probe ? g_d2 / h0 : 0.0f;
+            if (probe) g_h0 += -g_d2 * r2 / (h0 * h0);
+#pragma unroll
+            for (int r = 0; r < 4; ++r) {
+                const float diff = f1[r] - k0[r], g_w = (probe && r2 != 0.0f) ? (g_r2 * (((diff * inv[r]) / sf) / r2)) / sf : 0.0f;
+                g_f1[r] = probe ? g_w * inv[r] : 0.0f;
+                g_inv[r] = probe ? g_w * diff : 0.0f;
+                g_k0[r] -= g_f1[r];
+            }
+            product(1, g_f1);
+#pragma unroll
+            for (int r = 0; r < 4; ++r) {
+                g_y0[r] += probe ? gi[r] : 0.0f;
+                g_k0[r] += probe ? gi[r] * dh : 0.0f;
+                g_step[r] = probe ? gi[r] * k0[r] : 0.0f;
+            }
+            g_step[0] += probe ? gt : 0.0f;  // (the probe's time moves with its step as well)
+            float steps;
+            mlp_sum2(sh, slot, g_step, none, steps, unused);
+            g_h0 += steps * dir;
+            const float g_h0a = on ? g_h0 * share_of_min(h0a, span) : 0.0f;
+            float g_d0 = 0;
+            if (on && !small) {
+                g_d1 += -g_h0a * (0.01f * d0) / (d1 * d1);
+                g_d0 = 0.01f * (g_h0a / d1);
+            }
+#pragma unroll
+            for (int r = 0; r < 4; ++r) {
+                const float g_u = (on && !small && d0 != 0.0f) ? (g_d0 * (((y[r] * inv[r]) / sf) / d0)) / sf : 0.0f;
+                const float g_v = (on && d1 != 0.0f) ? (g_d1 * (((k0[r] * inv[r]) / sf) / d1)) / sf : 0.0f;
+                g_y0[r] += on ? g_u * inv[r] : 0.0f;
+                g_k0[r] += on ? g_v * inv[r] : 0.0f;
+                g_inv[r] += on ? g_u * y[r] + g_v * k0[r] : 0.0f;
+                const float sign = y[r] > 0.0f ? 1.0f : (y[r] < 0.0f ? -1.0f : 0.0f);
+                g_y0[r] += on ? (-g_inv[r] * inv[r] * inv[r]) * cp.rtol * sign : 0.0f;
+            }
+        }
+        product(0, g_k0);
+#pragma unroll
+        for (int r = 0; r < 4; ++r) g_y0[r] += gi[r];
+        if (live) mlp_put((float *)p.g_y + b * FR, f0, FR, g_y0);
     }
 }
 
@@ -258,9 +442,9 @@ __device__ __forceinline__ MlpOuterRows mlp_outer_rows(const tode_mlp_reverse &p
 // every workgroup takes a share of the rows and holds all sums of it in registers (wavefront w: units 64w .. 64w + 63, 128
 // accumulators), 32 matrix instructions per four rows with the next four rows' operands on their way.  The sums of a
 // share go to the workgroup's own slot, added to those of the iterations before (`accumulate`).
-__global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2, 2))) mlp_weight_gradient_kernel(const tode_mlp_reverse p, long long rows_per_split, int accumulate) {
+__global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2, 2))) mlp_weight_gradient_kernel(const tode_mlp_reverse p, long long rows, long long rows_per_split, int accumulate) {
     const int tid = threadIdx.x, lane = tid & 63, w = tid >> 6, q = lane >> 4, c = lane & 15;
-    const long long rows = 6 * p.batch, first = (long long)blockIdx.x * rows_per_split, end = min(rows, first + rows_per_split);
+    const long long first = (long long)blockIdx.x * rows_per_split, end = min(rows, first + rows_per_split);
     mfma_acc a2[4][4], a1[4][4];
     float at[4], ab[4], ag[4];
 #pragma unroll
@@ -344,6 +528,11 @@ static int check_mlp_reverse(const tode_mlp_reverse *p) {
     return TODE_OK;
 }
 
+static void launch_weight_gradient(const tode_mlp_reverse &p, long long rows, int accumulate, hipStream_t s) {
+    const long long per_split = ((rows + p.splits - 1) / p.splits + 3) / 4 * 4;
+    hipLaunchKernelGGL(mlp_weight_gradient_kernel, dim3(p.splits), dim3(256), 0, s, p, rows, per_split, accumulate);
+}
+
 // A workgroup of the reverse kernel fills its compute unit (one wavefront per SIMD), of the stages' kernel half of one:
 // beyond that they take several tiles each and load the weights once (133 KB per workgroup, as long as a stage takes).
 static unsigned mlp_tiles_grid(const tode_mlp_reverse &p, int per_unit) {
@@ -384,11 +573,29 @@ int tode_mlp_stages_backward(const tode_mlp_reverse *p, int32_t accumulate, void
     const dim3 grid(mlp_tiles_grid(*p, 1));
     if (p->method == TODE_TSIT5) hipLaunchKernelGGL((mlp_stages_backward_kernel<1>), grid, dim3(256), 0, (hipStream_t)stream, *p);
     else hipLaunchKernelGGL((mlp_stages_backward_kernel<0>), grid, dim3(256), 0, (hipStream_t)stream, *p);
-    if (p->sums) {
-        const long long rows = 6 * p->batch, per_split = ((rows + p->splits - 1) / p->splits + 3) / 4 * 4;
-        hipLaunchKernelGGL(mlp_weight_gradient_kernel, dim3(p->splits), dim3(256), 0, (hipStream_t)stream, *p, per_split, accumulate);
-    }
+    if (p->sums) launch_weight_gradient(*p, 6 * p->batch, accumulate, (hipStream_t)stream);
     return check_hip(hipGetLastError(), "tode_mlp_stages_backward");
+}
+
+int tode_mlp_start_backward(const tode_mlp_reverse *p, const tode_mlp_start *start, const tode_controller *c, int32_t accumulate, void *stream) {
+    using namespace tode;
+    const int rc = check_mlp_reverse(p);
+    if (rc || p->batch == 0) return rc;
+    if (!start || !c || !start->t_end || !start->a_y || !start->a_k0 || !start->a_dt) return fail(TODE_E_INVALID, "null pointer");
+    if (c->kind != TODE_CTRL_INTEGRAL && c->kind != TODE_CTRL_PID) return fail(TODE_E_INVALID, "unknown controller kind %d", c->kind);
+    const CtrlParams<float> cp = make_ctrl<float>(*c);
+    const bool integral = c->kind == TODE_CTRL_INTEGRAL;
+    const dim3 grid(mlp_tiles_grid(*p, 2)), grid_back(mlp_tiles_grid(*p, 1));
+    hipStream_t s = (hipStream_t)stream;
+    if (start->through_rule) {
+        hipLaunchKernelGGL((mlp_start_kernel<true>), grid, dim3(256), 0, s, *p, *start, cp);
+        hipLaunchKernelGGL((mlp_start_backward_kernel<true>), grid_back, dim3(256), 0, s, *p, *start, cp, integral);
+    } else {
+        hipLaunchKernelGGL((mlp_start_kernel<false>), grid, dim3(256), 0, s, *p, *start, cp);
+        hipLaunchKernelGGL((mlp_start_backward_kernel<false>), grid_back, dim3(256), 0, s, *p, *start, cp, integral);
+    }
+    if (p->sums) launch_weight_gradient(*p, (start->through_rule ? 2 : 1) * p->batch, accumulate, s);
+    return check_hip(hipGetLastError(), "tode_mlp_start_backward");
 }
 
 int tode_mlp_weight_gradients(const tode_mlp_reverse *p, void *out, void *stream) {
