@@ -398,8 +398,9 @@ int tode_mlp_pack_weights_for(const void *raw, int64_t n_raw, int32_t n_features
  * Reverse sweep with the perceptron as right-hand side (float32, n_features = 1 ... 64, n_hidden = 1 ... 256): what
  * surrounds tode_step_finish_backward for one recorded iteration.  Per iteration: tode_mlp_stages forms the six stages
  * again from the recorded t, dt, y, k0 (y1 is the last stage input); tode_step_finish_backward leaves the cotangents g_*;
- * tode_mlp_stages_backward takes them through the stages and, where `sums` is not null, adds the iteration's share to the
- * weights' gradients (accumulate = 0: the sweep's first call, which sets them).  After the last iteration
+ * tode_mlp_stages_backward takes them through the stages.  Where the weights want gradients the stage buffers of several
+ * iterations lie one behind the other (the caller moves the pointers on) and tode_mlp_outer_products adds the first `rows`
+ * rows of them to `sums` (accumulate = 0: the sweep's first call, which sets them).  At the end
  * tode_mlp_weight_gradients adds up the splits: out = W1 [n_hidden x (n_features + 1)] | b1 | W2 | b2.
  * tode_mlp_pack_weights_reverse packs the same raw weights as tode_mlp_pack_weights_for for the way back.
  */
@@ -419,6 +420,7 @@ typedef struct tode_mlp_reverse {
     void *stage_times;           /* [6,B] */
     void *hidden;                /* [6,B,256] */
     void *hidden_cotangents;     /* [6,B,256], null where no weight wants a gradient */
+    void *stage_cotangents;      /* [6,B,F], likewise: the cotangents of the evaluations' results */
     void *g_k;                   /* [7,B,F] in and out */
     void *g_y, *g_y1;            /* [B,F] in (and out: g_y) */
     void *g_t, *g_dt;            /* [B] in and out */
@@ -426,11 +428,12 @@ typedef struct tode_mlp_reverse {
 } tode_mlp_reverse;
 int tode_mlp_pack_weights_reverse(const void *raw, int64_t n_raw, int32_t n_features, void *packed, void *stream);
 int tode_mlp_stages(const tode_mlp_reverse *p, void *stream);
-int tode_mlp_stages_backward(const tode_mlp_reverse *p, int32_t accumulate, void *stream);
+int tode_mlp_stages_backward(const tode_mlp_reverse *p, void *stream);
+int tode_mlp_outer_products(const tode_mlp_reverse *p, int64_t rows, int32_t accumulate, void *stream);
 /*
  * The start of the loop reversed (y = y0, k0 = f(t_start, y0), the start rule's first step clamped to the time range; the times
- * are constants): p->t, y, k0 are the record's first entry, p->g_y receives the cotangent of y0; the weights' share is
- * added as by tode_mlp_stages_backward, ahead of tode_mlp_weight_gradients.
+ * are constants): p->t, y, k0 are the record's first entry, p->g_y receives the cotangent of y0; its two evaluations of the
+ * network (one without through_rule) take 2 B (B) rows of the stage buffers.
  */
 typedef struct tode_mlp_start {
     const void *t_end;                /* [B] */
@@ -438,7 +441,7 @@ typedef struct tode_mlp_start {
     int32_t through_rule;             /* the first step is a function of y0 and the weights (no step of the user's, gradients
                                          through the step sizes) */
 } tode_mlp_start;
-int tode_mlp_start_backward(const tode_mlp_reverse *p, const tode_mlp_start *start, const tode_controller *c, int32_t accumulate, void *stream);
+int tode_mlp_start_backward(const tode_mlp_reverse *p, const tode_mlp_start *start, const tode_controller *c, void *stream);
 int tode_mlp_weight_gradients(const tode_mlp_reverse *p, void *out, void *stream);
 
 /* ------------------------------------------------------------------------- */

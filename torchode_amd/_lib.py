@@ -50,6 +50,7 @@ EXPORTS = (
     "tode_mlp_stages",
     "tode_mlp_stages_backward",
     "tode_mlp_start_backward",
+    "tode_mlp_outer_products",
     "tode_mlp_weight_gradients",
     "tode_select_end_point",
     "tode_step_begin",
@@ -210,7 +211,7 @@ class MlpReverse(C.Structure):
 
     _fields_ = [(name, C.c_int32) for name in ("method", "n_features", "n_hidden", "splits")] + [("batch", C.c_int64)] + [
         (name, C.c_void_p)
-        for name in ("packed", "packed_reverse", "t", "dt", "y", "k0", "k", "stage_inputs", "stage_times", "hidden", "hidden_cotangents",
+        for name in ("packed", "packed_reverse", "t", "dt", "y", "k0", "k", "stage_inputs", "stage_times", "hidden", "hidden_cotangents", "stage_cotangents",
                      "g_k", "g_y", "g_y1", "g_t", "g_dt", "sums")
     ]  # fmt: skip
 
@@ -360,9 +361,11 @@ def load():
         lib.tode_mlp_stages.restype = C.c_int
         lib.tode_mlp_stages.argtypes = [C.POINTER(MlpReverse), C.c_void_p]
         lib.tode_mlp_stages_backward.restype = C.c_int
-        lib.tode_mlp_stages_backward.argtypes = [C.POINTER(MlpReverse), C.c_int32, C.c_void_p]
+        lib.tode_mlp_stages_backward.argtypes = [C.POINTER(MlpReverse), C.c_void_p]
+        lib.tode_mlp_outer_products.restype = C.c_int
+        lib.tode_mlp_outer_products.argtypes = [C.POINTER(MlpReverse), C.c_int64, C.c_int32, C.c_void_p]
         lib.tode_mlp_start_backward.restype = C.c_int
-        lib.tode_mlp_start_backward.argtypes = [C.POINTER(MlpReverse), C.POINTER(MlpStart), C.POINTER(Controller), C.c_int32, C.c_void_p]
+        lib.tode_mlp_start_backward.argtypes = [C.POINTER(MlpReverse), C.POINTER(MlpStart), C.POINTER(Controller), C.c_void_p]
         lib.tode_mlp_weight_gradients.restype = C.c_int
         lib.tode_mlp_weight_gradients.argtypes = [C.POINTER(MlpReverse), C.c_void_p, C.c_void_p]
         lib.tode_solve_builtin_fast_static.restype = C.c_int

@@ -531,7 +531,7 @@ class NetworkSweep:
             and y0.shape[0] > 0
         )
 
-    def __init__(self, lib, method_id, f, B, F, g_k, g_y, g_y1, g_t, g_dt, stream):
+    def __init__(self, lib, method_id, f, B, F, iterations, g_k, g_y, g_y1, g_t, g_dt, stream):
         dev, H = g_k.device, f.W2.shape[1]
         new = lambda *shape: torch.empty(shape, dtype=torch.float32, device=dev)
         self.lib, self.stream, self.f, self.started = lib, stream, f, False
@@ -541,44 +541,75 @@ class NetworkSweep:
         packed, packed_reverse = new(_lib.MLP_PACKED_SIZE["float32"]), new(_lib.MLP_REVERSE_PACKED_SIZE)
         _lib.check(lib.tode_mlp_pack_weights_for(raw.data_ptr(), raw.numel(), F, _lib.MLP_INPUTS["float32"], packed.data_ptr(), stream), "tode_mlp_pack_weights_for")
         _lib.check(lib.tode_mlp_pack_weights_reverse(raw.data_ptr(), raw.numel(), F, packed_reverse.data_ptr(), stream), "tode_mlp_pack_weights_reverse")
-        # One share of the 6 B rows per compute unit and at least 64 rows each: a share ends with 133 KB of sums.
-        splits = max(1, min(256, (6 * B) // 64))
-        self.k, self.inputs, self.times, self.hidden = new(6, B, F), new(6, B, F), new(6, B), new(6, B, 256)
-        self.cotangents = new(6, B, 256) if wanted else None
+        # The weights' gradients are sums over the rows of all evaluations.  A call for them ends with 133 KB of sums per
+        # share of the rows (one per compute unit, at least 64 rows each), so the evaluations of several iterations are
+        # kept for one call, as far as they fit into ROOM.
+        per_evaluation = 4 * B * (2 * 256 + 2 * F + 1)
+        self.room = max(6, min(6 * iterations + 2, self.ROOM // per_evaluation)) if wanted else 6
+        splits = max(1, min(256, (self.room * B) // 64))
+        self.held, self.B, self.k = 0, B, new(6, B, F)
+        rows = lambda *last: new(self.room, B, *last)
+        self.inputs, self.times, self.hidden = rows(F), rows(), rows(256)
+        self.cotangents, self.derivatives = (rows(256), rows(F)) if wanted else (None, None)
         self.sums = new(splits, _lib.MLP_SUMS_SIZE) if wanted else None
-        self.keep = (raw, packed, packed_reverse, g_k, g_y, g_y1, g_t, g_dt)
-        self.args = _lib.MlpReverse(
-            method_id, F, H, splits, B, packed.data_ptr(), packed_reverse.data_ptr(), None, None, None, None, self.k.data_ptr(), self.inputs.data_ptr(),
-            self.times.data_ptr(), self.hidden.data_ptr(), _lib.ptr(self.cotangents), *(x.data_ptr() for x in (g_k, g_y, g_y1, g_t, g_dt)), _lib.ptr(self.sums),
-        )  # fmt: skip
-        self.ref = _lib.C.byref(self.args)
+        self.keep = (raw, packed, packed_reverse, g_y1)
+        self.args = _lib.MlpReverse(method_id, F, H, splits, B)
+        a = self.args
+        a.packed, a.packed_reverse, a.k, a.g_y1, a.sums = packed.data_ptr(), packed_reverse.data_ptr(), self.k.data_ptr(), g_y1.data_ptr(), _lib.ptr(self.sums)
+        a.g_k, a.g_y, a.g_t, a.g_dt = (x.data_ptr() for x in (g_k, g_y, g_t, g_dt))
+        self.ref = _lib.C.byref(a)
 
-    def stages(self, state):
+    ROOM = 1 << 30  # bytes
+
+    def _at(self, state, evaluations):
+        """The state an iteration starts from, and room for that many evaluations' rows."""
         a = self.args
         a.t, a.dt, a.y, a.k0 = (state[k].data_ptr() for k in ("t", "dt", "y", "k0"))
+        if self.sums is None:
+            self.held = 0
+        elif self.held + evaluations > self.room:
+            self._add_rows()
+        at = self.held
+        a.stage_inputs, a.stage_times, a.hidden = (x[at].data_ptr() for x in (self.inputs, self.times, self.hidden))
+        if self.sums is not None:
+            a.hidden_cotangents, a.stage_cotangents = self.cotangents[at].data_ptr(), self.derivatives[at].data_ptr()
+        self.held += evaluations
+        return self.inputs[at + evaluations - 1]
+
+    def _add_rows(self):
+        """The outer products of the rows held so far."""
+        if self.held == 0:
+            return
+        a = self.args
+        a.stage_inputs, a.stage_times, a.hidden = (x.data_ptr() for x in (self.inputs, self.times, self.hidden))
+        a.hidden_cotangents, a.stage_cotangents = self.cotangents.data_ptr(), self.derivatives.data_ptr()
+        _lib.check(self.lib.tode_mlp_outer_products(self.ref, self.held * self.B, int(self.started), self.stream), "tode_mlp_outer_products")
+        self.held, self.started = 0, True
+
+    def stages(self, state):
+        y1 = self._at(state, 6)
         _lib.check(self.lib.tode_mlp_stages(self.ref, self.stream), "tode_mlp_stages")
-        return [state["k0"], *self.k.unbind(0)], self.inputs[5]
+        return [state["k0"], *self.k.unbind(0)], y1
 
     def stages_backward(self, g_k, g_y, g_t, g_dt):
         a = self.args
         a.g_k, a.g_y, a.g_t, a.g_dt = g_k.data_ptr(), g_y.data_ptr(), g_t.data_ptr(), g_dt.data_ptr()
-        _lib.check(self.lib.tode_mlp_stages_backward(self.ref, int(self.started), self.stream), "tode_mlp_stages_backward")
-        self.started = True
+        _lib.check(self.lib.tode_mlp_stages_backward(self.ref, self.stream), "tode_mlp_stages_backward")
 
-    def start_backward(self, controller, state, t_end, a_y, a_k0, a_dt, g_k, g_y, through_rule):
-        """The start of the loop reversed; ``g_y`` becomes the cotangent of ``y0`` (``g_k``: room for those of the derivatives)."""
-        a = self.args
-        a.t, a.dt, a.y, a.k0 = (state[k].data_ptr() for k in ("t", "dt", "y", "k0"))
-        a.g_k, a.g_y = g_k.data_ptr(), g_y.data_ptr()
+    def start_backward(self, controller, state, t_end, a_y, a_k0, a_dt, g_y, through_rule):
+        """The start of the loop reversed; ``g_y`` becomes the cotangent of ``y0``."""
+        self._at(state, 2 if through_rule else 1)
+        self.args.g_y = g_y.data_ptr()
         start = _lib.MlpStart(t_end.data_ptr(), a_y.data_ptr(), a_k0.data_ptr(), a_dt.data_ptr(), int(bool(through_rule)))
-        _lib.check(self.lib.tode_mlp_start_backward(self.ref, _lib.C.byref(start), controller, int(self.started), self.stream), "tode_mlp_start_backward")
-        self.started = True
+        _lib.check(self.lib.tode_mlp_start_backward(self.ref, _lib.C.byref(start), controller, self.stream), "tode_mlp_start_backward")
 
     def weight_gradients(self, params):
         """The gradients of ``params`` through the weights: autograd carries those of the held tensors on to the leaves."""
         f = self.f
         weights = (f.W1, f.b1, f.W2, f.b2)
-        if self.sums is None or not self.started or not params:
+        if self.sums is not None:
+            self._add_rows()
+        if not self.started or not params:
             return [None] * len(params)
         out = torch.empty(sum(x.numel() for x in weights), dtype=torch.float32, device=self.sums.device)
         _lib.check(self.lib.tode_mlp_weight_gradients(self.ref, out.data_ptr(), self.stream), "tode_mlp_weight_gradients")
@@ -665,7 +696,7 @@ def reverse_sweep_kernels(adjoint, replay: Replay, term, args, problem, dt0_give
     f, with_args = term.f, term.with_args
     network = None
     if NetworkSweep.takes(adjoint, term, y0, t_start):  # (always so where `arrays` are given)
-        network = NetworkSweep(lib, method.method_id, f, B, F, g_k, g_y, g_y1, g_t, g_dt, stream)
+        network = NetworkSweep(lib, method.method_id, f, B, F, n_iterations, g_k, g_y, g_y1, g_t, g_dt, stream)
 
     def rhs(tt, yy):
         out = f(tt, yy, args) if with_args else f(tt, yy)
@@ -764,8 +795,8 @@ def reverse_sweep_kernels(adjoint, replay: Replay, term, args, problem, dt0_give
     if arrays is not None and not any(wants(x) for x in (replay.t_start, replay.t_end, replay.t_eval, dt0)):
         # the start of the loop in kernels as well (they take its times as constants): what comes back is the cotangent of y0
         a_y, a_k0, _, a_dt = adj[:4]
-        g_k, g_y = sets[1][:2]
-        network.start_backward(cref, states[0], t_end, a_y, a_k0, a_dt, g_k, g_y, dt0_given is None and replay.through_control)
+        g_y = sets[1][1]
+        network.start_backward(cref, states[0], t_end, a_y, a_k0, a_dt, g_y, dt0_given is None and replay.through_control)
         adj, through_start = (g_y, *adj[1:]), True
     if network is not None:
         grad_params = network.weight_gradients(params)

@@ -7,7 +7,8 @@
 //                               the whole-solve kernel), keeping stage inputs, derivatives and hidden activations;
 //   mlp_stages_backward_kernel  the six stages in reverse: the network's vector-Jacobian product and the stage sums' reverse,
 //                               the cotangents of all stage derivatives in registers between them;
-//   mlp_weight_gradient_kernel  the two outer products over all 6 B rows of the iteration, split over the rows;
+//   mlp_weight_gradient_kernel  the two outer products over the rows of all evaluations of several iterations, split over
+//                               the rows;
 //   mlp_weight_gradient_sum_kernel  the splits' sums added in order, once per sweep.
 //
 // All products are on v_mfma_f32_16x16x4_f32.  For the vector-Jacobian product the weights are packed a second time,
@@ -214,7 +215,7 @@ template <int METHOD> __global__ void __launch_bounds__(256) __attribute__((amdg
 #pragma unroll
         for (int s = 6; s >= 1; --s) {
             const long long row = (s - 1) * B + b;
-            if (s < 6 && live) mlp_put((float *)p.g_k + (s * B + b) * FR, f0, FR, gk[s]);  // (final: the weights' gradients read it)
+            if (live && p.stage_cotangents) mlp_put((float *)p.stage_cotangents + row * FR, f0, FR, gk[s]);  // (final: the weights' gradients read it)
             float gi[4], gt;
             mlp_vjp(sh, W, gk[s], (const float *)p.hidden + row * MLP_H, live && p.hidden_cotangents ? (float *)p.hidden_cotangents + row * MLP_H : nullptr, gi, gt);
             g_t += gt;
@@ -307,7 +308,7 @@ __global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2, 2))
 }
 
 // The same reversed: the cotangents a_y, a_k0, a_dt of the first loop state to that of y0 (p.g_y), those of the two evaluations of
-// the network left in slots 1 and 2 of p.g_k for the weights' gradients.  The times are constants here.  (start_backward of
+// the network left in p.stage_cotangents for the weights' gradients.  The times are constants here.  (start_backward of
 // the small systems, a sample's row spread over sixteen lanes; a term that a sample does not have is selected away, since
 // all lanes meet at the barriers of the sums and products.)
 template <bool THROUGH>
@@ -330,7 +331,7 @@ __global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(1, 1))
         mlp_get((const float *)st.a_k0 + b * FR, f0, FR, g_k0);
         const auto product = [&](int at, const float (&g)[4]) {
             const long long row = at * B + b;
-            if (live) mlp_put((float *)p.g_k + (B + row) * FR, f0, FR, g);
+            if (live && p.stage_cotangents) mlp_put((float *)p.stage_cotangents + row * FR, f0, FR, g);
             mlp_vjp(sh, W, g, (const float *)p.hidden + row * MLP_H, live && p.hidden_cotangents ? (float *)p.hidden_cotangents + row * MLP_H : nullptr, gi, gt);
         };
         if (THROUGH) {
@@ -414,7 +415,9 @@ __global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(1, 1))
     }
 }
 
-// The operands of four rows (k of the matrix instructions) for one wavefront: lane (q, c) holds row 4 step + q.
+// The operands of four rows (k of the matrix instructions) for one wavefront: lane (q, c) holds row 4 step + q.  Rows past
+// the end repeat the last one with cotangents of zero.
+constexpr int MLP_OUTER_AHEAD = 3;
 struct MlpOuterRows {
     float h[4], d[4], g[4], x[4], t;
 };
@@ -429,7 +432,7 @@ __device__ __forceinline__ MlpOuterRows mlp_outer_rows(const tode_mlp_reverse &p
         v.h[u] = ((const float *)p.hidden)[at * MLP_H + 64 * w + 16 * u + c];
         v.d[u] = ((const float *)p.hidden_cotangents)[at * MLP_H + 64 * w + 16 * u + c];
         const int f = 16 * u + c;
-        v.g[u] = f < FR ? ((const float *)p.g_k)[(p.batch + at) * FR + f] : 0.0f;
+        v.g[u] = f < FR ? ((const float *)p.stage_cotangents)[at * FR + f] : 0.0f;
         v.x[u] = f < FR ? ((const float *)p.stage_inputs)[at * FR + f] : 0.0f;
         v.d[u] = in ? v.d[u] : 0.0f;
         v.g[u] = in ? v.g[u] : 0.0f;
@@ -440,9 +443,10 @@ __device__ __forceinline__ MlpOuterRows mlp_outer_rows(const tode_mlp_reverse &p
 
 // dW2[f][u] = sum over rows g[f] h[u],  dW1[u][i] = sum over rows d[u] x[i],  and the biases' and the time column's sums:
 // every workgroup takes a share of the rows and holds all sums of it in registers (wavefront w: units 64w .. 64w + 63, 128
-// accumulators), 32 matrix instructions per four rows with the next four rows' operands on their way.  The sums of a
-// share go to the workgroup's own slot, added to those of the iterations before (`accumulate`).
-__global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2, 2))) mlp_weight_gradient_kernel(const tode_mlp_reverse p, long long rows, long long rows_per_split, int accumulate) {
+// accumulators), 32 matrix instructions (0.45 us) per four rows with the operands of the next three such steps on their way:
+// one wavefront per SIMD has nothing else to cover the memory's latency with.  The sums of a share go to the workgroup's
+// own slot, added to those of earlier calls (`accumulate`).
+__global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(1, 2))) mlp_weight_gradient_kernel(const tode_mlp_reverse p, long long rows, long long rows_per_split, int accumulate) {
     const int tid = threadIdx.x, lane = tid & 63, w = tid >> 6, q = lane >> 4, c = lane & 15;
     const long long first = (long long)blockIdx.x * rows_per_split, end = min(rows, first + rows_per_split);
     mfma_acc a2[4][4], a1[4][4];
@@ -454,21 +458,26 @@ __global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2, 2))
         for (int u = 0; u < 4; ++u) a2[i][u] = {0.0f, 0.0f, 0.0f, 0.0f}, a1[i][u] = {0.0f, 0.0f, 0.0f, 0.0f};
     }
     if (first < end) {
-        MlpOuterRows here = mlp_outer_rows(p, first + q, end, w, c);
-        for (long long row = first; row < end; row += 4) {
-            const MlpOuterRows next = mlp_outer_rows(p, row + 4 + q, end, w, c);
+        MlpOuterRows ring[MLP_OUTER_AHEAD];
 #pragma unroll
-            for (int u = 0; u < 4; ++u) {
+        for (int n = 0; n < MLP_OUTER_AHEAD; ++n) ring[n] = mlp_outer_rows(p, first + 4 * n + q, end, w, c);
+        for (long long row = first; row < end; row += 4 * MLP_OUTER_AHEAD) {
 #pragma unroll
-                for (int i = 0; i < 4; ++i) {
-                    a2[i][u] = __builtin_amdgcn_mfma_f32_16x16x4f32(here.g[i], here.h[u], a2[i][u], 0, 0, 0);
-                    a1[i][u] = __builtin_amdgcn_mfma_f32_16x16x4f32(here.x[i], here.d[u], a1[i][u], 0, 0, 0);
+            for (int n = 0; n < MLP_OUTER_AHEAD; ++n) {
+                const MlpOuterRows here = ring[n];
+                ring[n] = mlp_outer_rows(p, row + 4 * (MLP_OUTER_AHEAD + n) + q, end, w, c);
+#pragma unroll
+                for (int u = 0; u < 4; ++u) {
+#pragma unroll
+                    for (int i = 0; i < 4; ++i) {
+                        a2[i][u] = __builtin_amdgcn_mfma_f32_16x16x4f32(here.g[i], here.h[u], a2[i][u], 0, 0, 0);
+                        a1[i][u] = __builtin_amdgcn_mfma_f32_16x16x4f32(here.x[i], here.d[u], a1[i][u], 0, 0, 0);
+                    }
+                    at[u] = fma_(here.t, here.d[u], at[u]);
+                    ab[u] += here.d[u];
+                    ag[u] += here.g[u];
                 }
-                at[u] = fma_(here.t, here.d[u], at[u]);
-                ab[u] += here.d[u];
-                ag[u] += here.g[u];
             }
-            here = next;
         }
     }
     float *out = (float *)p.sums + (long long)blockIdx.x * MLP_SUMS;
@@ -493,10 +502,23 @@ __global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2, 2))
     }
 }
 
-// One thread per sum, the splits in order; out in the order of the weights: W1 [H x (F + 1)] | b1 | W2 [F x H] | b2.
+// The splits of 64 sums per workgroup, a quarter of the splits per wavefront with eight loads in flight (one thread per sum
+// over all splits waited for memory 64 times in a row: 68 us for 34 MB); always in the same order.  out in the order of
+// the weights: W1 [H x (F + 1)] | b1 | W2 [F x H] | b2.
 static __global__ void __launch_bounds__(256) mlp_weight_gradient_sum_kernel(const float *sums, int splits, int H, int FR, float *out) {
-    const int i = blockIdx.x * 256 + threadIdx.x;
-    if (i >= MLP_SUMS) return;
+    __shared__ float part[4][64];
+    const int lane = threadIdx.x & 63, w = threadIdx.x >> 6, i = blockIdx.x * 64 + lane;
+    const int share = (splits + 3) / 4, first = w * share, end = min(splits, first + share);
+    float s[8] = {0, 0, 0, 0, 0, 0, 0, 0};
+    if (i < MLP_SUMS) {
+        for (int k = first; k < end; k += 8)
+#pragma unroll
+            for (int j = 0; j < 8; ++j)
+                if (k + j < end) s[j] += sums[(long long)(k + j) * MLP_SUMS + i];
+    }
+    part[w][lane] = ((s[0] + s[1]) + (s[2] + s[3])) + ((s[4] + s[5]) + (s[6] + s[7]));
+    __syncthreads();
+    if (w != 0 || i >= MLP_SUMS) return;
     const long long o_b1 = (long long)H * (FR + 1), o_w2 = o_b1 + H, o_b2 = o_w2 + (long long)FR * H;
     long long to = -1;
     const int row = i / MLP_H, unit = i % MLP_H;  // (of the first part; the others start at multiples of MLP_H as well)
@@ -505,13 +527,7 @@ static __global__ void __launch_bounds__(256) mlp_weight_gradient_sum_kernel(con
     else if (i < MLP_SUM_W2) to = unit < H ? o_b1 + unit : -1;
     else if (i < MLP_SUM_B2) to = (unit < H && row - MLP_F - 2 < FR) ? o_w2 + (long long)(row - MLP_F - 2) * H + unit : -1;
     else to = i - MLP_SUM_B2 < FR ? o_b2 + (i - MLP_SUM_B2) : -1;
-    if (to < 0) return;
-    float s[4] = {0, 0, 0, 0};
-    for (int k = 0; k < splits; k += 4)
-#pragma unroll
-        for (int j = 0; j < 4; ++j)
-            if (k + j < splits) s[j] += sums[(long long)(k + j) * MLP_SUMS + i];
-    out[to] = (s[0] + s[1]) + (s[2] + s[3]);
+    if (to >= 0) out[to] = (part[0][lane] + part[1][lane]) + (part[2][lane] + part[3][lane]);
 }
 
 static int check_mlp_reverse(const tode_mlp_reverse *p) {
@@ -524,13 +540,8 @@ static int check_mlp_reverse(const tode_mlp_reverse *p) {
     if (p->batch > 0 && (!p->packed || !p->packed_reverse || !p->t || !p->dt || !p->y || !p->k0 || !p->k || !p->stage_inputs || !p->stage_times || !p->hidden ||
                          !p->g_k || !p->g_y || !p->g_y1 || !p->g_t || !p->g_dt))
         return fail(TODE_E_INVALID, "null pointer");
-    if (!p->hidden_cotangents != !p->sums) return fail(TODE_E_INVALID, "hidden_cotangents and sums go together");
+    if (!p->hidden_cotangents != !p->sums || !p->stage_cotangents != !p->sums) return fail(TODE_E_INVALID, "hidden_cotangents, stage_cotangents and sums go together");
     return TODE_OK;
-}
-
-static void launch_weight_gradient(const tode_mlp_reverse &p, long long rows, int accumulate, hipStream_t s) {
-    const long long per_split = ((rows + p.splits - 1) / p.splits + 3) / 4 * 4;
-    hipLaunchKernelGGL(mlp_weight_gradient_kernel, dim3(p.splits), dim3(256), 0, s, p, rows, per_split, accumulate);
 }
 
 // A workgroup of the reverse kernel fills its compute unit (one wavefront per SIMD), of the stages' kernel half of one:
@@ -566,18 +577,17 @@ int tode_mlp_stages(const tode_mlp_reverse *p, void *stream) {
     return check_hip(hipGetLastError(), "tode_mlp_stages");
 }
 
-int tode_mlp_stages_backward(const tode_mlp_reverse *p, int32_t accumulate, void *stream) {
+int tode_mlp_stages_backward(const tode_mlp_reverse *p, void *stream) {
     using namespace tode;
     const int rc = check_mlp_reverse(p);
     if (rc || p->batch == 0) return rc;
     const dim3 grid(mlp_tiles_grid(*p, 1));
     if (p->method == TODE_TSIT5) hipLaunchKernelGGL((mlp_stages_backward_kernel<1>), grid, dim3(256), 0, (hipStream_t)stream, *p);
     else hipLaunchKernelGGL((mlp_stages_backward_kernel<0>), grid, dim3(256), 0, (hipStream_t)stream, *p);
-    if (p->sums) launch_weight_gradient(*p, 6 * p->batch, accumulate, (hipStream_t)stream);
     return check_hip(hipGetLastError(), "tode_mlp_stages_backward");
 }
 
-int tode_mlp_start_backward(const tode_mlp_reverse *p, const tode_mlp_start *start, const tode_controller *c, int32_t accumulate, void *stream) {
+int tode_mlp_start_backward(const tode_mlp_reverse *p, const tode_mlp_start *start, const tode_controller *c, void *stream) {
     using namespace tode;
     const int rc = check_mlp_reverse(p);
     if (rc || p->batch == 0) return rc;
@@ -594,8 +604,18 @@ int tode_mlp_start_backward(const tode_mlp_reverse *p, const tode_mlp_start *sta
         hipLaunchKernelGGL((mlp_start_kernel<false>), grid, dim3(256), 0, s, *p, *start, cp);
         hipLaunchKernelGGL((mlp_start_backward_kernel<false>), grid_back, dim3(256), 0, s, *p, *start, cp, integral);
     }
-    if (p->sums) launch_weight_gradient(*p, (start->through_rule ? 2 : 1) * p->batch, accumulate, s);
     return check_hip(hipGetLastError(), "tode_mlp_start_backward");
+}
+
+int tode_mlp_outer_products(const tode_mlp_reverse *p, int64_t rows, int32_t accumulate, void *stream) {
+    using namespace tode;
+    const int rc = check_mlp_reverse(p);
+    if (rc || p->batch == 0) return rc;
+    if (!p->sums) return fail(TODE_E_INVALID, "null pointer");
+    if (rows < 0) return fail(TODE_E_INVALID, "rows %lld", (long long)rows);
+    const long long per_split = ((rows + p->splits - 1) / p->splits + 3) / 4 * 4;
+    hipLaunchKernelGGL(mlp_weight_gradient_kernel, dim3(p->splits), dim3(256), 0, (hipStream_t)stream, *p, (long long)rows, per_split, accumulate);
+    return check_hip(hipGetLastError(), "tode_mlp_outer_products");
 }
 
 int tode_mlp_weight_gradients(const tode_mlp_reverse *p, void *out, void *stream) {
@@ -603,7 +623,7 @@ int tode_mlp_weight_gradients(const tode_mlp_reverse *p, void *out, void *stream
     const int rc = check_mlp_reverse(p);
     if (rc) return rc;
     if (!p->sums || !out) return fail(TODE_E_INVALID, "null pointer");
-    hipLaunchKernelGGL(mlp_weight_gradient_sum_kernel, dim3((MLP_SUMS + 255) / 256), dim3(256), 0, (hipStream_t)stream, (const float *)p->sums, p->splits, p->n_hidden,
+    hipLaunchKernelGGL(mlp_weight_gradient_sum_kernel, dim3((MLP_SUMS + 63) / 64), dim3(256), 0, (hipStream_t)stream, (const float *)p->sums, p->splits, p->n_hidden,
                        p->n_features, (float *)out);
     return check_hip(hipGetLastError(), "tode_mlp_weight_gradients");
 }
