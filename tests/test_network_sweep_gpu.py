@@ -77,3 +77,48 @@ def test_a_solve_of_more_steps_than_the_first_record_holds(B, F, H):
     for a, b, c in zip(results[True, 0], results[True, 1], results[False, 0]):
         assert torch.equal(a, b)
         assert float((a.double() - c.double()).norm()) <= 1e-3 * float(c.double().norm())
+
+
+def test_gradient_of_y0_alone():
+    """No weight wants a gradient: no outer products, and the same bits for y0."""
+    g = torch.Generator("cuda").manual_seed(5)
+    rand = lambda *shape: 2 * torch.rand(shape, generator=g, device="cuda") - 1
+    B, F, H = 19, 10, 24
+    weights = [rand(H, F + 1), rand(H), rand(F, H), rand(F)]
+    y0, t_eval, cotangent = rand(B, F).requires_grad_(), torch.linspace(0, 1, 5, device="cuda").repeat(B, 1), rand(B, 5, F)
+    results = []
+    for wanted in (False, True):
+        f = to.MLPField(*(w.clone().requires_grad_(wanted) for w in weights))
+        solver = to.AutoDiffAdjoint(to.Tsit5(), to.IntegralController(1e-5, 1e-3))
+        sol = solver.solve(to.InitialValueProblem(y0, t_eval=t_eval), to.ODETerm(f))
+        results.append(torch.autograd.grad(sol.ys, y0, cotangent)[0])
+    assert torch.equal(*results) and float(results[0].abs().max()) > 0
+
+
+@pytest.mark.parametrize("times", [False, True], ids=["constant-times", "time-gradients"])
+@pytest.mark.parametrize("F, E", [(64, 63), (64, 65), (100, 130), (64, 0)])
+@pytest.mark.parametrize("method", [to.Dopri5, to.Tsit5], ids=["dopri5", "tsit5"])
+def test_points_of_long_rows_as_sums(method, F, E, times):
+    """The dense output's reverse on rows of a wavefront each, its marks looked at 64 at a time: fewer and more points than
+    that, a row that is no multiple of 64, no points; against the sweep in torch operations (float64, the bound of the other
+    comparisons of the two with the steps held constant)."""
+    g = torch.Generator("cuda").manual_seed(F + E)
+    rand = lambda *shape: torch.rand(shape, generator=g, dtype=torch.float64, device="cuda")
+    B = 3
+    rate, y0 = (0.5 + rand(F)).requires_grad_(), rand(B, F).requires_grad_()
+    t1 = 0.5 + rand(B)
+    if E:
+        given = dict(t_eval=t1[:, None] * torch.linspace(0, 1, E, dtype=torch.float64, device="cuda")[None, :])
+    else:
+        given = dict(t_start=torch.zeros_like(t1), t_end=t1)
+    given = {k: v.clone().requires_grad_(times) for k, v in given.items()}
+    wrt = [rate, y0, *(given.values() if times else ())]
+    cotangent = rand(B, max(E, 1), F)
+    results = []
+    for kernels in (True, False):
+        solver = to.AutoDiffAdjoint(method(), to.IntegralController(1e-6, 1e-4), backprop_through_step_size_control=False)
+        solver.backward_kernels = kernels
+        sol = solver.solve(to.InitialValueProblem(y0, **given), to.ODETerm(lambda t, y: -rate * y * y + torch.sin(t)[:, None]))
+        results.append(torch.autograd.grad(sol.ys, wrt, cotangent))
+    for got, want in zip(*results):
+        assert float((got - want).abs().max()) <= 1e-9 * float(want.abs().max())
