@@ -60,7 +60,7 @@ static __global__ void mlp_pack_kernel(const float *raw, float *packed, int H, i
 // are left in fills the record up to its capacity with `running` 0, as in the small systems' kernels; a record that is too
 // short raises TODE_FLAG_NEEDS_GENERAL (TODE_FLAG_MAX_ITERATIONS says how long it has to be).  For gradients: f there takes the
 // math library's tanh, since it stands where torch's evaluations of the network stood.  Network of 64 and 256 at B = 4096:
-// solve and record in 0.12 ms, where the per-step kernels around torch's products took 2.6 ms.
+// solve and record in 0.105 ms, where the per-step kernels around torch's products took 2.6 ms.
 template <int METHOD, int CTRL, typename Weights, bool FULL, bool RECORD>
 __global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2, 2))) solve_mlp_kernel(const SolveParams<float> p, const float *packed, const MlpOut o) {
     using T = float;

@@ -11,6 +11,12 @@
 //                               the rows;
 //   mlp_weight_gradient_sum_kernel  the splits' sums added in order, once per sweep.
 //
+// What bounds them, network of 64 and 256 at B = 4096 (one workgroup per compute unit, one wavefront per SIMD): six
+// evaluations forward 32 us, back 30 us, of which the matrix cores are busy 10.6 and 10.2 us -- the rest are the round trips
+// through LDS between two products, tanh, the stage sums and 150 KB of weights loaded per workgroup; the outer products of 20
+// evaluations 91 us (35 us of matrix instructions, 200 MB of rows at 2.2 TB/s; four calls of an iteration each with one step
+// of loads ahead took 215 us).  A solve and its backward pass: 9.75 ms through autograd, 1.27 ms.
+//
 // All products are on v_mfma_f32_16x16x4_f32.  For the vector-Jacobian product the weights are packed a second time,
 // transposed (tode_mlp_pack_weights_reverse), so that the same two facts hold as in the forward kernel: every lane keeps its
 // A operands in registers, and the first product's result, lane (q, c) holding the cotangents of hidden units 4q..4q+3 of
