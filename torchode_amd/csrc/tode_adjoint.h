@@ -205,54 +205,50 @@ __device__ __forceinline__ void finish_backward_sample(const AdjointParams<TT, T
     if (flat) den = (TT)1;
     const int n_points = E > 0 ? (n_listed >= 0 ? n_listed : E) : (p.end_point ? 1 : 0);
     // The output at a point is a polynomial in the point's position x, and its cotangent g enters all results through the
-    // sums of g, g x, .. g x^4 over the points: five sums per feature, and the stages' shares once per iteration instead of
-    // once per point.  (A point's own gradient, where t_eval wants one, is formed point by point.)
+    // sums of g, g x, .. g x^4 over the points.  Rows of a wavefront each take the sums first, five per feature, and the
+    // stages' shares once per iteration (point by point, every point read, changed and wrote the cotangents of all seven
+    // stages in memory, and every lane looked at every mark: finish_backward_kernel at B = 4096, F = 64, E = 20 took 56 us
+    // instead of 19).  A row of one thread adds point by point, in the order of the points: its gradients go through
+    // powers of error ratios near rounding, where another order of the same sums moves a sample's result by percents.
+    // (A point's own gradient, where t_eval wants one, is formed point by point in both.)
     const bool own_gradients = E > 0 && p.g_t_eval;
-    constexpr bool SUMS = WAVE || FC > 0;
-    // the shares of one feature from its sums; `any`: some cotangent was not zero (a state that is not finite adds nothing then)
-    const auto spread = [&](int f, const T (&G)[5], bool any) {
-        if (!any) return;
-        const long long i = b * F + f;
-        T ks[7], q[5][1];
-#pragma unroll
-        for (int s = 0; s < 7; ++s) ks[s] = p.k[s][i];
-        quartic_elem<T, METHOD>(h, y[f], y1[f], ks, true, q);
-        const T gx = G[0] * q[1][0] + (T)2 * (G[1] * q[2][0]) + (T)3 * (G[2] * q[3][0]) + (T)4 * (G[3] * q[4][0]);
-        const T gxx = G[1] * q[1][0] + (T)2 * (G[2] * q[2][0]) + (T)3 * (G[3] * q[3][0]) + (T)4 * (G[4] * q[4][0]);
-        g_points += gx, g_points_x += gxx;
-        if (METHOD == 1) {
-            p.g_y[i] += G[0];
-            p.g_k[0][i] += G[1] * h;
-            g_h += G[1] * ks[0];
-#pragma unroll
-            for (int s = 0; s < 7; ++s) {
-                const T w = G[2] * (T)Tsit5Tab::w[0][s] + G[3] * (T)Tsit5Tab::w[1][s] + G[4] * (T)Tsit5Tab::w[2][s];
-                p.g_k[s][i] += w * h;
-                g_h += w * ks[s];
-            }
-        } else {
-            const T g_f0 = (T)-2 * G[4] + (T)5 * G[3] - (T)4 * G[2] + G[1], g_f1 = (T)2 * G[4] - (T)3 * G[3] + G[2];
-            const T g_mid = (T)16 * G[4] - (T)32 * G[3] + (T)16 * G[2];
-            p.g_y[i] += (T)-8 * G[4] + (T)18 * G[3] - (T)11 * G[2] + G[0] + g_mid;
-            p.g_y1[i] += (T)-8 * G[4] + (T)14 * G[3] - (T)5 * G[2];
-            p.g_k[0][i] += g_f0 * h;
-            p.g_k[6][i] += g_f1 * h;
-            g_h += g_f0 * ks[0] + g_f1 * ks[6];
-#pragma unroll
-            for (int s = 0; s < 7; ++s) {
-                p.g_k[s][i] += g_mid * (h * (T)Dopri5Tab::w[0][s]);
-                g_h += g_mid * (T)Dopri5Tab::w[0][s] * ks[s];
-            }
-        }
-    };
-    const auto add = [](T (&G)[5], bool &any, T g, T x) {
-        any = any || g != (T)0;
-#pragma unroll
-        for (int n = 0; n < 5; ++n) G[n] += g, g = g * x;
-    };
-    const auto position = [&](int e) { return (T)(((E > 0 ? p.t_eval[b * E + e] : te) - t0) / den); };
-    const auto cotangent = [&](int e, int f) { return p.grad_ys[(b * (long long)(E > 0 ? E : 1) + e) * F + f]; };
     if constexpr (WAVE) {
+        // the shares of one feature from its sums; `any`: some cotangent was not zero (a state that is not finite adds nothing then)
+        const auto spread = [&](int f, const T (&G)[5], bool any) {
+            if (!any) return;
+            const long long i = b * F + f;
+            T ks[7], q[5][1];
+#pragma unroll
+            for (int s = 0; s < 7; ++s) ks[s] = p.k[s][i];
+            quartic_elem<T, METHOD>(h, y[f], y1[f], ks, true, q);
+            const T gx = G[0] * q[1][0] + (T)2 * (G[1] * q[2][0]) + (T)3 * (G[2] * q[3][0]) + (T)4 * (G[3] * q[4][0]);
+            const T gxx = G[1] * q[1][0] + (T)2 * (G[2] * q[2][0]) + (T)3 * (G[3] * q[3][0]) + (T)4 * (G[4] * q[4][0]);
+            g_points += gx, g_points_x += gxx;
+            if (METHOD == 1) {
+                p.g_y[i] += G[0];
+                p.g_k[0][i] += G[1] * h;
+                g_h += G[1] * ks[0];
+#pragma unroll
+                for (int s = 0; s < 7; ++s) {
+                    const T w = G[2] * (T)Tsit5Tab::w[0][s] + G[3] * (T)Tsit5Tab::w[1][s] + G[4] * (T)Tsit5Tab::w[2][s];
+                    p.g_k[s][i] += w * h;
+                    g_h += w * ks[s];
+                }
+            } else {
+                const T g_f0 = (T)-2 * G[4] + (T)5 * G[3] - (T)4 * G[2] + G[1], g_f1 = (T)2 * G[4] - (T)3 * G[3] + G[2];
+                const T g_mid = (T)16 * G[4] - (T)32 * G[3] + (T)16 * G[2];
+                p.g_y[i] += (T)-8 * G[4] + (T)18 * G[3] - (T)11 * G[2] + G[0] + g_mid;
+                p.g_y1[i] += (T)-8 * G[4] + (T)14 * G[3] - (T)5 * G[2];
+                p.g_k[0][i] += g_f0 * h;
+                p.g_k[6][i] += g_f1 * h;
+                g_h += g_f0 * ks[0] + g_f1 * ks[6];
+#pragma unroll
+                for (int s = 0; s < 7; ++s) {
+                    p.g_k[s][i] += g_mid * (h * (T)Dopri5Tab::w[0][s]);
+                    g_h += g_mid * (T)Dopri5Tab::w[0][s] * ks[s];
+                }
+            }
+        };
         // the marks of 64 points at a time, one per lane
         for (int f = f_first; f - f_first < F; f += f_step) {  // (every lane takes every turn: the marks are voted on)
             T G[5] = {0, 0, 0, 0, 0};
@@ -263,38 +259,23 @@ __device__ __forceinline__ void finish_backward_sample(const AdjointParams<TT, T
                 while (marks) {
                     const int e = base + __builtin_ctzll(marks);
                     marks &= marks - 1;
-                    if (f < F) add(G, any, cotangent(e, f), position(e));
+                    if (f >= F) continue;
+                    const T x = (T)(((E > 0 ? p.t_eval[b * E + e] : te) - t0) / den);
+                    T g = p.grad_ys[(b * (long long)(E > 0 ? E : 1) + e) * F + f];
+                    any = any || g != (T)0;
+#pragma unroll
+                    for (int n = 0; n < 5; ++n) G[n] += g, g = g * x;
                 }
             }
             if (f < F) spread(f, G, any);
         }
-    } else if constexpr (FC > 0) {
-        T G[FC > 0 ? FC : 1][5];
-        bool any[FC > 0 ? FC : 1];
-#pragma unroll
-        for (int f = 0; f < FC; ++f) {
-            any[f] = false;
-#pragma unroll
-            for (int n = 0; n < 5; ++n) G[f][n] = 0;
-        }
-        for (int idx = 0; idx < n_points; ++idx) {
-            const int e = (E > 0 && n_listed >= 0) ? points[idx] : idx;
-            if (E > 0 && n_listed < 0 && p.hit_iteration[b * E + e] != p.iteration) continue;
-            const T x = position(e);
-#pragma unroll
-            for (int f = 0; f < FC; ++f) add(G[f], any[f], cotangent(e, f), x);
-        }
-#pragma unroll
-        for (int f = 0; f < FC; ++f) spread(f, G[f], any[f]);
-    }
-    if constexpr (SUMS) {
         // x = (at - t0) / ((t0 + dt) - t0)
         const TT gx = (TT)row_sum<WAVE>(g_points), gxx = (TT)row_sum<WAVE>(g_points_x);
         if (E == 0 && p.g_t_end && scalar_lane) p.g_t_end[b] += gx / den;
         g_t -= gx / den;
         if (!flat) g_dt -= gxx / den;
     }
-    for (int idx = 0; idx < ((SUMS && !own_gradients) ? 0 : n_points); ++idx) {
+    for (int idx = 0; idx < ((WAVE && !own_gradients) ? 0 : n_points); ++idx) {
         const int e = (E > 0 && n_listed >= 0) ? points[idx] : idx;
         if (E > 0 && n_listed < 0 && p.hit_iteration[b * E + e] != p.iteration) continue;
         const TT at = E > 0 ? p.t_eval[b * E + e] : te;
@@ -312,7 +293,7 @@ __device__ __forceinline__ void finish_backward_sample(const AdjointParams<TT, T
             T q[5][1];
             quartic_elem<T, METHOD>(h, y[f], y1[f], ks, true, q);
             g_x += g * (q[1][0] + x * ((T)2 * q[2][0] + x * ((T)3 * q[3][0] + x * (T)4 * q[4][0])));
-            if (SUMS) continue;
+            if (WAVE) continue;
             const T g0 = g, g1 = g * x, g2 = g1 * x, g3 = g2 * x, g4 = g3 * x;
             if (METHOD == 1) {
                 p.g_y[i] += g0;
@@ -346,7 +327,7 @@ __device__ __forceinline__ void finish_backward_sample(const AdjointParams<TT, T
         } else if (p.g_t_end && scalar_lane) {
             p.g_t_end[b] += gx / den;
         }
-        if (SUMS) continue;
+        if (WAVE) continue;
         g_t -= gx / den;
         if (!flat) g_dt -= gx * (TT)x / den;
     }
