@@ -197,6 +197,26 @@ def test_more_evaluation_points_than_fit_on_chip(dtype, n_eval):
     assert _lib.last_solve_kernel_name() == "tode::solve_kernel"
 
 
+@pytest.mark.parametrize("fast", ["one", True], ids=["fast1", "automatic"])
+@pytest.mark.parametrize("dtype, largest", [(F32, 3.4e38), (F64, 1.79e308)], ids=["f32", "f64"])
+@pytest.mark.parametrize("features", [1, 2])
+def test_a_time_range_beyond_the_largest_value(features, dtype, largest, fast):
+    """t_end - t_start overflows for two samples among ordinary ones, forwards and backwards, and their derivative is zero: the
+    step grows to infinity.  The batch goes to the general kernel; what the fast kernels write before that ends with the
+    last evaluation point."""
+    B = 70
+    f = to.LinearDecay(torch.full((B, features), 0.5, dtype=dtype))
+    y0 = torch.linspace(1, 2, B * features, dtype=torch.float64).reshape(B, features).to(dtype)
+    t_eval = torch.tensor([0.0, 0.5, 1.0], dtype=dtype).repeat(B, 1)
+    for b, sign in ((3, 1), (65, -1)):
+        f.k[b] = 0.0
+        t_eval[b] = sign * torch.tensor([-largest, 0.0, largest], dtype=dtype)
+    spec = dict(kind="integral", atol=1e-6, rtol=1e-4)
+    for method in ("dopri5", "tsit5"):
+        ref = c_oracle_solve(f, y0, t_eval, method, spec)
+        assert_identical(gpu_solve(f, y0, t_eval, method, spec, fast=fast), ref)
+
+
 def test_user_dt0_skips_start_step():
     w = to.workloads.make("lorenz", batch=256, dtype=F32)
     dt0 = torch.full((256,), 0.01, dtype=F32)

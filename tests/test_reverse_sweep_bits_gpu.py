@@ -7,7 +7,7 @@ bits to compare with (torch sums the same terms in another order), hence the sto
 
     python tests/test_reverse_sweep_bits_gpu.py
 
-writes tests/golden/reverse_sweep_gradients.json on a machine with a GPU (float.hex of every value)."""
+writes tests/stored/reverse_sweep_gradients.json on a machine with a GPU (float.hex of every value)."""
 import json
 import os
 import sys
@@ -17,7 +17,7 @@ import torch
 
 if __name__ != "__main__":
     pytestmark = pytest.mark.gpu
-GOLDEN = os.path.join(os.path.dirname(os.path.abspath(__file__)), "golden", "reverse_sweep_gradients.json")
+GOLDEN = os.path.join(os.path.dirname(os.path.abspath(__file__)), "stored", "reverse_sweep_gradients.json")
 
 # (system, features, method, controller, dtype, evaluation points)
 CASES = {
