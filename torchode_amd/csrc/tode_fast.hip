@@ -84,9 +84,10 @@ __global__ void __launch_bounds__(64, fast_wavefronts(sizeof(T), Term::F, NHIST,
     const T tlo = tmin(ts, te), thi = tmax(te, ts);
 
     // From here on times are multiplied by the sample's direction (+-1: exact), so that "a has reached b" is dir * a >= dir * b
-    // in either direction; behind the last evaluation point lies one that no step reaches (not as another row in LDS: at 20
-    // points a workgroup's rows fill exactly the 1/32 of LDS that eight wavefronts per SIMD leave it).
-    const T never = (T)__builtin_huge_val();
+    // in either direction; behind the last evaluation point lies one that no time reaches, not even the infinite one that a step
+    // without a finite result may lead to: not a number (not as another row in LDS: at 20 points a workgroup's rows fill
+    // exactly the 1/32 of LDS that eight wavefronts per SIMD leave it).
+    const T never = nan_<T>();
     bool bail = false;
     const T te_first = te_s[lane];
     {

@@ -274,8 +274,9 @@ __global__ void __launch_bounds__(128) solve_pair_kernel(const SolveParams<T> p,
         }
         // (LDS accesses of one wavefront complete in order; te_s is private to this wave)
         // From here on times are multiplied by the sample's direction (exact), and behind the last point lies one that no
-        // step reaches: whether a step has passed the next point is one comparison.
-        const T never = (T)__builtin_huge_val();
+        // time reaches, not even the infinite one that a step without a finite result may lead to: not a number.  Whether a
+        // step has passed the next point is one comparison.
+        const T never = nan_<T>();
         bool bail = false;
         const T te_first = end_only ? te : (STAGE_TE ? te_s[group] : tev_g[0]);
         if (!end_only) {
