@@ -67,3 +67,12 @@ def test_a_time_range_beyond_the_largest_value(program, kernel, method, sign, dt
     batch is handed to the general kernel."""
     flag, _, initialized, value = program(kernel, dtype, method, 0.0, 1.0, -sign * largest, 0.0, sign * largest)
     assert flag == 1 and initialized <= 1
+
+
+@pytest.mark.parametrize("dtype, far", [("f32", -3e38), ("f32", -1e30), ("f64", -1e308)])
+@pytest.mark.parametrize("kernel, method", KERNELS)
+def test_a_point_far_in_front_of_the_start(program, kernel, method, dtype, far):
+    """A point so far in front of t_start that its position in units of the first step overflows: extrapolated to an infinity, as
+    by the division (the product with the step's reciprocal made it an infinity less an infinity)."""
+    flag, _, initialized, value = program(kernel, dtype, method, 1.0, 1.0, 1.0, far, 2.0)
+    assert (flag, initialized) == (0, 1) and abs(value) == float("inf")

@@ -217,6 +217,21 @@ def test_a_time_range_beyond_the_largest_value(features, dtype, largest, fast):
         assert_identical(gpu_solve(f, y0, t_eval, method, spec, fast=fast), ref)
 
 
+@pytest.mark.parametrize("fast", ["one", True], ids=["fast1", "automatic"])
+@pytest.mark.parametrize("dtype, far", [(F32, -3e38), (F64, -1e308)], ids=["f32", "f64"])
+def test_a_point_far_in_front_of_t_start(dtype, far, fast):
+    """Evaluation points in front of t_start are extrapolated in the first step: one whose position in units of that step is no
+    longer finite, next to ordinary samples."""
+    w = to.workloads.make("vdp", batch=70, dtype=dtype)
+    t_start = torch.full((70,), 0.5, dtype=dtype)
+    t_eval = t_start[:, None] + torch.tensor([0.0, 0.5, 1.0], dtype=dtype)[None, :]
+    t_eval[7, 0] = far
+    for method in ("dopri5", "tsit5"):
+        ref = c_oracle_solve(w.f, w.y0, t_eval, method, w.controller, t_start=t_start)
+        assert not bool(ref["ys"][7, 0].isfinite().any())
+        assert_identical(gpu_solve(w.f, w.y0, t_eval, method, w.controller, t_start=t_start, fast=fast), ref)
+
+
 def test_user_dt0_skips_start_step():
     w = to.workloads.make("lorenz", batch=256, dtype=F32)
     dt0 = torch.full((256,), 0.01, dtype=F32)

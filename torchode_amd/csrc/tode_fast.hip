@@ -205,7 +205,7 @@ __global__ void __launch_bounds__(64, fast_wavefronts(sizeof(T), Term::F, NHIST,
         if (holds(active) && dt_new >= dte_next) {
             T q[5][F];
             quartic<T, F, METHOD, true>(dt, y, y1, k, q);
-            const StepPosition<T> position(t0, dt);
+            const StepPosition<T> position(t0, dt, dir, dte_next);
             auto write_points = [&](auto plain) {
                 do {
                     T out[F];

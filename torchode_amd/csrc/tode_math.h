@@ -676,14 +676,17 @@ template <typename T, int F, typename TT = T> __device__ __forceinline__ void qu
 // one step: the step's reciprocal is formed once and a point costs a product and a correction (quotient_with) where
 // `plain` says that the operands are in the range of that form.  A point in [t0, t0 + dt] is t0 itself or at least
 // 2^-25 |t0| away, so |t0| >= 2^-30 |den| puts the quotient above 2^-55; the step before that (t0 = 0 or near it) divides.
+// Points in front of t_start are extrapolated in the first step, from any distance: `first`, the pass's first point and the
+// one furthest from t0, is held below 2^80, so that no product overflows where the quotient is an infinity.
 template <typename T> struct StepPosition {
     T t0, den, r;
     lanes_t plain;
-    __device__ __forceinline__ StepPosition(T t0_, T dt) : t0(t0_) {
+    __device__ __forceinline__ StepPosition(T t0_, T dt, T dir, T first) : t0(t0_) {
         const T t1 = t0 + dt, d = t1 - t0;
         den = abs_(d) > (T)0 ? d : (T)1;
         r = reciprocal_estimate(den);
-        plain = lanes_where(abs_(den) >= (T)0x1p-40) & lanes_where(abs_(den) <= (T)0x1p+40) & lanes_where(abs_(t0) >= abs_(den) * (T)0x1p-30);
+        plain = lanes_where(abs_(den) >= (T)0x1p-40) & lanes_where(abs_(den) <= (T)0x1p+40) & lanes_where(abs_(t0) >= abs_(den) * (T)0x1p-30) &
+                lanes_where(abs_(fma_(dir, first, -t0)) <= (T)0x1p+80);
     }
     // t = dir * dte with dir = +-1 (an exact product)
     template <bool PLAIN> __device__ __forceinline__ T at(T dir, T dte) const {

@@ -327,7 +327,7 @@ __global__ void __launch_bounds__(128) solve_pair_kernel(const SolveParams<T> p,
 #pragma unroll
                     for (int f = 0; f < K; ++f) k[s][f] = r[(3 + 2 * K + s * K + f) * 64];
                 quartic<T, K, METHOD, true>(dt, y, y1, k, q);
-                const StepPosition<T> position(t0, dt);
+                const StepPosition<T> position(t0, dt, dir, dte_next);
                 auto write_points = [&](auto plain) {
                     do {
                         T out[K];
