@@ -122,3 +122,22 @@ def test_points_of_long_rows_as_sums(method, F, E, times):
         results.append(torch.autograd.grad(sol.ys, wrt, cotangent))
     for got, want in zip(*results):
         assert float((got - want).abs().max()) <= 1e-9 * float(want.abs().max())
+
+
+@pytest.mark.parametrize("method", [to.Dopri5, to.Tsit5], ids=["dopri5", "tsit5"])
+def test_points_of_long_rows_are_added_up_in_the_time_type(method):
+    """float64 times and float32 data, a step with 100 000 points and the same cotangent at each: the gradient of t_start is
+    -sum(g f) exactly, f being constant.  Added up in float32 it would be off by some 2^-24 per added point in one
+    direction; the interpolant's coefficients (weights of up to 30, rounded to float32, where all but one should be zero)
+    leave 30 * 2^-24 times a few."""
+    E, F = 100_000, 64
+    c = torch.arange(64, 64 + F, device="cuda") / 64
+    t_eval = torch.linspace(0.001, 0.999, E, dtype=torch.float64, device="cuda").repeat(2, 1)
+    t_start = torch.zeros(2, dtype=torch.float64, device="cuda", requires_grad=True)
+    t_end, dt0 = torch.full_like(t_start, 2.0).detach(), torch.ones_like(t_start).detach()
+    solver = to.AutoDiffAdjoint(method(), to.IntegralController(1e-5, 1e-3), backprop_through_step_size_control=False)
+    y0 = torch.zeros(2, F, device="cuda")
+    sol = solver.solve(to.InitialValueProblem(y0, t_start, t_end, t_eval), to.ODETerm(lambda t, y: c + 0 * y), dt0=dt0)
+    (got,) = torch.autograd.grad(sol.ys, t_start, torch.full_like(sol.ys, 0.1))
+    want = -float(torch.tensor(0.1)) * E * float(c.double().sum())
+    assert float((got / want - 1).abs().max()) <= 1e-5

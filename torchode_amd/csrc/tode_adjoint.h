@@ -164,7 +164,9 @@ __device__ __forceinline__ void finish_backward_sample(const AdjointParams<TT, T
     const T tiny = (T)1e-38;
     const T g_r = r > tiny ? g_ratio : (r == tiny ? g_ratio / (T)2 : (T)0);
     T g_h = 0;  // (this lane's share; summed over the row at the end)
-    T g_points = 0, g_points_x = 0;  // likewise: cotangents of the points' positions, and those times the positions
+    // likewise, in the wider of the two types: cotangents of the points' positions, and those times the positions
+    using Wide = typename std::conditional<(sizeof(TT) > sizeof(T)), TT, T>::type;
+    Wide g_points = 0, g_points_x = 0;
 #pragma unroll
     for (int f = f_first; f < F; f += f_step) {
         const long long i = b * F + f;
@@ -210,20 +212,24 @@ __device__ __forceinline__ void finish_backward_sample(const AdjointParams<TT, T
     // stages in memory, and every lane looked at every mark: finish_backward_kernel at B = 4096, F = 64, E = 20 took 56 us
     // instead of 19).  A row of one thread adds point by point, in the order of the points: its gradients go through
     // powers of error ratios near rounding, where another order of the same sums moves a sample's result by percents.
-    // (A point's own gradient, where t_eval wants one, is formed point by point in both.)
+    // (A point's own gradient, where t_eval wants one, is formed point by point in both.)  Where times have more bits than the
+    // data, the cotangents of t0 and dt add up in theirs, point by point: POINTWISE.
     const bool own_gradients = E > 0 && p.g_t_eval;
+    constexpr bool POINTWISE = sizeof(TT) > sizeof(T);
     if constexpr (WAVE) {
         // the shares of one feature from its sums; `any`: some cotangent was not zero (a state that is not finite adds nothing then)
         const auto spread = [&](int f, const T (&G)[5], bool any) {
             if (!any) return;
             const long long i = b * F + f;
-            T ks[7], q[5][1];
+            T ks[7];
 #pragma unroll
             for (int s = 0; s < 7; ++s) ks[s] = p.k[s][i];
-            quartic_elem<T, METHOD>(h, y[f], y1[f], ks, true, q);
-            const T gx = G[0] * q[1][0] + (T)2 * (G[1] * q[2][0]) + (T)3 * (G[2] * q[3][0]) + (T)4 * (G[3] * q[4][0]);
-            const T gxx = G[1] * q[1][0] + (T)2 * (G[2] * q[2][0]) + (T)3 * (G[3] * q[3][0]) + (T)4 * (G[4] * q[4][0]);
-            g_points += gx, g_points_x += gxx;
+            if (!POINTWISE) {
+                T q[5][1];
+                quartic_elem<T, METHOD>(h, y[f], y1[f], ks, true, q);
+                g_points += (Wide)(G[0] * q[1][0] + (T)2 * (G[1] * q[2][0]) + (T)3 * (G[2] * q[3][0]) + (T)4 * (G[3] * q[4][0]));
+                g_points_x += (Wide)(G[1] * q[1][0] + (T)2 * (G[2] * q[2][0]) + (T)3 * (G[3] * q[3][0]) + (T)4 * (G[4] * q[4][0]));
+            }
             if (METHOD == 1) {
                 p.g_y[i] += G[0];
                 p.g_k[0][i] += G[1] * h;
@@ -251,8 +257,14 @@ __device__ __forceinline__ void finish_backward_sample(const AdjointParams<TT, T
         };
         // the marks of 64 points at a time, one per lane
         for (int f = f_first; f - f_first < F; f += f_step) {  // (every lane takes every turn: the marks are voted on)
-            T G[5] = {0, 0, 0, 0, 0};
+            T G[5] = {0, 0, 0, 0, 0}, q[5][1];
             bool any = false;
+            if (POINTWISE && f < F) {
+                T ks[7];
+#pragma unroll
+                for (int s = 0; s < 7; ++s) ks[s] = p.k[s][b * F + f];
+                quartic_elem<T, METHOD>(h, y[f], y1[f], ks, true, q);
+            }
             for (int base = 0; base < n_points; base += 64) {
                 const int mine = base + f_first;
                 unsigned long long marks = __ballot(mine < n_points && (E == 0 || p.hit_iteration[b * E + mine] == p.iteration));
@@ -263,6 +275,10 @@ __device__ __forceinline__ void finish_backward_sample(const AdjointParams<TT, T
                     const T x = (T)(((E > 0 ? p.t_eval[b * E + e] : te) - t0) / den);
                     T g = p.grad_ys[(b * (long long)(E > 0 ? E : 1) + e) * F + f];
                     any = any || g != (T)0;
+                    if (POINTWISE && g != (T)0) {
+                        const Wide g_x = (Wide)(g * (q[1][0] + x * ((T)2 * q[2][0] + x * ((T)3 * q[3][0] + x * (T)4 * q[4][0]))));
+                        g_points += g_x, g_points_x += g_x * (Wide)x;
+                    }
 #pragma unroll
                     for (int n = 0; n < 5; ++n) G[n] += g, g = g * x;
                 }
