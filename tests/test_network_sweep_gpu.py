@@ -141,3 +141,23 @@ def test_points_of_long_rows_are_added_up_in_the_time_type(method):
     (got,) = torch.autograd.grad(sol.ys, t_start, torch.full_like(sol.ys, 0.1))
     want = -float(torch.tensor(0.1)) * E * float(c.double().sum())
     assert float((got / want - 1).abs().max()) <= 1e-5
+
+
+@pytest.mark.parametrize("method", [to.Dopri5, to.Tsit5], ids=["dopri5", "tsit5"])
+def test_a_point_without_a_cotangent_adds_nothing(method):
+    """A point so far in front of t_start that its position in the step is an infinity, and no cotangent at it, next to one
+    that has one in the same step: gradients
+    are those of the problem without the point."""
+    B, F = 3, 70
+    rate = torch.linspace(0.5, 1.5, F, device="cuda").requires_grad_()
+    y0, t_start = torch.linspace(1, 2, B * F, device="cuda").reshape(B, F).requires_grad_(), torch.ones(B, device="cuda")
+    points = torch.tensor([-3e38, 1.0001, 1.7, 2.0], device="cuda").repeat(B, 1)
+    results = []
+    for first in (0, 1):
+        solver = to.AutoDiffAdjoint(method(), to.IntegralController(1e-5, 1e-3))
+        sol = solver.solve(to.InitialValueProblem(y0, t_start, points[:, 3].contiguous(), points[:, first:].contiguous()), to.ODETerm(lambda t, y: -rate * y))
+        cotangent = torch.ones_like(sol.ys)
+        cotangent[:, : 1 - first] = 0
+        results.append(torch.autograd.grad(sol.ys, [y0, rate], cotangent))
+    for got, want in zip(*results):
+        assert bool(want.isfinite().all()) and torch.equal(got, want)

@@ -274,8 +274,9 @@ __device__ __forceinline__ void finish_backward_sample(const AdjointParams<TT, T
                     if (f >= F) continue;
                     const T x = (T)(((E > 0 ? p.t_eval[b * E + e] : te) - t0) / den);
                     T g = p.grad_ys[(b * (long long)(E > 0 ? E : 1) + e) * F + f];
-                    any = any || g != (T)0;
-                    if (POINTWISE && g != (T)0) {
+                    if (g == (T)0) continue;  // (adds nothing, wherever the point lies: its position may be an infinity)
+                    any = true;
+                    if (POINTWISE) {
                         const Wide g_x = (Wide)(g * (q[1][0] + x * ((T)2 * q[2][0] + x * ((T)3 * q[3][0] + x * (T)4 * q[4][0]))));
                         g_points += g_x, g_points_x += g_x * (Wide)x;
                     }
