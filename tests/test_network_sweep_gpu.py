@@ -161,3 +161,33 @@ def test_a_point_without_a_cotangent_adds_nothing(method):
         results.append(torch.autograd.grad(sol.ys, [y0, rate], cotangent))
     for got, want in zip(*results):
         assert bool(want.isfinite().all()) and torch.equal(got, want)
+
+
+def test_a_record_that_just_fits():
+    """As many entries as the solve has iterations, and one for the state after them, are enough also where the sample with the
+    most steps has landed past t_end and sits through one more iteration: the record is kept and the same."""
+    g = torch.Generator("cuda").manual_seed(3)
+    rand = lambda *shape: 2 * torch.rand(shape, generator=g, device="cuda") - 1
+    B, F, H, E = 200, 8, 16, 5
+    weights = [rand(H, F + 1), rand(H), rand(F, H), rand(F)]
+    y0 = rand(B, F).requires_grad_()
+    t_start, t_end = -0.3 - 0.1 * torch.rand(B, generator=g, device="cuda"), 1e-3 + 1e-3 * torch.rand(B, generator=g, device="cuda")
+    t_eval = t_start[:, None] + (t_end - t_start)[:, None] * torch.linspace(0, 0.9, E, device="cuda")[None, :]
+    solver = to.AutoDiffAdjoint(to.Dopri5(), to.IntegralController(1e-5, 1e-3))
+    kept, real = [], solver._solve_recording_in_one_kernel
+    solver._solve_recording_in_one_kernel = lambda *args: kept.append((real(*args), args[5])) or kept[-1][0]
+    grads = []
+    for attempt in range(2):
+        sol = solver.solve(to.InitialValueProblem(y0, t_start, t_end, t_eval), to.ODETerm(to.MLPField(*weights)))
+        grads.append(torch.autograd.grad(sol.ys, y0, torch.ones_like(sol.ys))[0])
+        n = int(sol.stats["n_steps"].max())
+        ((shape, entries),) = solver._record_entries.items()
+        assert entries == n + 5
+        solver._record_entries[shape] = n + 1
+    assert [solution is not None for solution, _ in kept] == [True, True]
+    record = kept[1][1].arrays
+    assert record["t"].shape[0] == n + 1
+    assert bool((record["t"][n] > t_end)[sol.stats["n_steps"] == n].any())  # (the case meant)
+    for name, x in record.items():
+        assert torch.equal(x, kept[0][1].arrays[name][: n + 1]), name
+    assert torch.equal(*grads)

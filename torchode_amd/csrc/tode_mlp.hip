@@ -165,14 +165,15 @@ __global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2, 2))
         cursor = 1;
     }
     int vslot = 0;
-    // bit 1: some sample needs the general kernel; bit 0: some sample still runs
-    int state = block_or(sh, vslot, (bail ? 2 : 0) | (active ? 1 : 0));
+    // bit 1: some sample needs the general kernel; bit 0: some sample still runs or sits through its last iteration; bit 2
+    // (RECORD): some sample still runs
+    int state = block_or(sh, vslot, (bail ? 2 : 0) | (active ? (RECORD ? 5 : 1) : 0));
     bail = (state & 2) != 0;
     // A sample that has landed past t_end (t + (t_end - t) rounded upwards) keeps stepping in the reference's later
     // iterations with the clamped step t_end - t, which is seen only in the status of that step: the sample sits
     // through one more iteration here, inactive, and the status of its step is looked at.
     bool idle = false, idle_done = false;
-    long long iteration = 0;  // (RECORD) of this workgroup, so far
+    long long iteration = 0, counted = 0;  // (RECORD) of this workgroup, so far; those of them that some sample ran in
     auto keep = [&](bool running) {
         if (iteration >= p.rec_capacity || !live) return;
         const long long at = iteration * p.batch + bs;
@@ -183,10 +184,11 @@ __global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2, 2))
             p.rec_running[at] = running ? 1 : 0, p.rec_n_accepted[at] = n_acc;
         }
     };
-    while (state == 1) {
+    while ((RECORD ? state & 3 : state) == 1) {
         if (RECORD) {
             keep(active);
             ++iteration;
+            counted += state >> 2;
         }
         // ---- stages (runge_kutta.py:255-263) ----
         const T t0 = t;
@@ -289,12 +291,14 @@ __global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2, 2))
         bail = bail || failed || (finished && nonfinite);
         idle = finished && !nonfinite && !(t == te);
         active = active && !failed && running_new;
-        state = block_or(sh, vslot, (bail ? 2 : 0) | ((active || idle) ? 1 : 0));
+        state = block_or(sh, vslot, (bail ? 2 : 0) | ((active || idle) ? 1 : 0) | ((RECORD && active) ? 4 : 0));
         bail = (state & 2) != 0;
     }
 
     if (RECORD) {
-        bail = bail || iteration >= p.rec_capacity;  // (the state after the last iteration is an entry as well)
+        // (the state after the last counted iteration is an entry as well: an iteration that samples sit through behind it is not
+        // one of the solve's, and has written that entry where it ran)
+        bail = bail || counted >= p.rec_capacity;
         for (; iteration < p.rec_capacity; ++iteration) keep(false);
     }
     if (end_only && live && !idle_done) put(p.y_idle + bs * FR, y);  // the final state
