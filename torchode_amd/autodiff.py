@@ -645,10 +645,10 @@ def reverse_sweep_kernels(adjoint, replay: Replay, term, args, problem, dt0_give
     # which iteration wrote which evaluation point
     hit_iteration = None
     if hits is None:  # (a record in arrays, of a batch in the whole-solve kernel's case: times that run in the solve's direction)
-        direction = replay.direction.detach()
-        reached = direction[None, :, None] * arrays["t"][1 : n_iterations + 1, :, None] >= (direction[:, None] * t_eval)[None]
-        hit_iteration = n_iterations - reached.sum(0, dtype=torch.int32)
-        hit_iteration = torch.where(hit_iteration < n_iterations, hit_iteration, -1).to(torch.int32)
+        direction = replay.direction.detach().to(ttype)
+        new_times = (direction[None, :] * arrays["t"][1 : n_iterations + 1]).t().contiguous()  # [B, iterations], ascending
+        hit_iteration = torch.searchsorted(new_times, direction[:, None] * t_eval, out_int32=True)
+        hit_iteration = torch.where(hit_iteration < n_iterations, hit_iteration, -1)
         hit_iteration[:, 0] = torch.where(t_eval[:, 0] == t_start, -1, hit_iteration[:, 0])
     elif E > 0:
         hit_iteration = torch.full((B, E), -1, dtype=torch.int32, device=dev)
