@@ -215,3 +215,24 @@ def test_memory_of_the_points_iterations(monkeypatch):
         torch.cuda.reset_peak_memory_stats()
         torch.autograd.grad(sol.ys, weights[0], torch.ones_like(sol.ys))
         assert torch.cuda.max_memory_allocated() - held < 40e6
+
+
+def test_rows_that_do_not_fit_into_memory(monkeypatch):
+    """Where the rows of all evaluations cannot be had the sweep takes those of one iteration at a time: the same gradient of y0,
+    and the weights' with their rows added up in other shares (the bound of the comparison with autograd)."""
+    case = (300, 64, 256, 9, to.Dopri5, lambda: to.IntegralController(1e-5, 1e-3), False, True)
+    want = _gradients(*case)
+    real, refused = torch.empty, []
+
+    def empty(*args, **kwargs):
+        shape = args[0] if args and isinstance(args[0], tuple) else ()
+        if len(shape) == 3 and shape[0] > 7 and shape[1:] == (300, 256):  # (more than an iteration's evaluations of hidden units)
+            refused.append(shape)
+            raise torch.cuda.OutOfMemoryError("no room")
+        return real(*args, **kwargs)
+
+    monkeypatch.setattr(torch, "empty", empty)
+    got = _gradients(*case)
+    assert len(refused) == 1 and torch.equal(got[0], want[0])
+    for a, b in zip(got, want):
+        assert float((a.double() - b.double()).norm()) <= 2e-5 * float(b.double().norm())

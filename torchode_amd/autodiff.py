@@ -545,13 +545,14 @@ class NetworkSweep:
         # share of the rows (one per compute unit, at least 64 rows each), so the evaluations of several iterations are
         # kept for one call, as far as they fit into ROOM.
         per_evaluation = 4 * B * (2 * 256 + 2 * F + 1)
-        self.room = max(6, min(6 * iterations + 2, self.ROOM // per_evaluation)) if wanted else 6
-        splits = max(1, min(256, (self.room * B) // 64))
+        room = max(6, min(6 * iterations + 2, self.ROOM // per_evaluation)) if wanted else 6
         self.held, self.B, self.k = 0, B, new(6, B, F)
-        rows = lambda *last: new(self.room, B, *last)
-        self.inputs, self.times, self.hidden = rows(F), rows(), rows(256)
-        self.cotangents, self.derivatives = (rows(256), rows(F)) if wanted else (None, None)
-        self.sums = new(splits, _lib.MLP_SUMS_SIZE) if wanted else None
+        try:
+            splits = self._allocate(room, new, F, wanted)
+        except torch.cuda.OutOfMemoryError:  # (what one iteration takes has to be there)
+            if room == 6:
+                raise
+            splits = self._allocate(6, new, F, wanted)
         self.keep = (raw, packed, packed_reverse, g_y1)
         self.args = _lib.MlpReverse(method_id, F, H, splits, B)
         a = self.args
@@ -559,7 +560,18 @@ class NetworkSweep:
         a.g_k, a.g_y, a.g_t, a.g_dt = (x.data_ptr() for x in (g_k, g_y, g_t, g_dt))
         self.ref = _lib.C.byref(a)
 
-    ROOM = 1 << 30  # bytes
+    # bytes, freed with the sweep (solve and backward pass at B = 12 000, 30 points: 1.87 ms, a half of it 1.93, a quarter 1.97)
+    ROOM = 1 << 30
+
+    def _allocate(self, room, new, F, wanted) -> int:
+        """The rows of ``room`` evaluations and the shares' sums; returns the number of shares."""
+        self.room, splits = room, max(1, min(256, (room * self.B) // 64))
+        self.inputs = self.times = self.hidden = self.cotangents = self.derivatives = self.sums = None
+        rows = lambda *last: new(room, self.B, *last)
+        self.inputs, self.times, self.hidden = rows(F), rows(), rows(256)
+        if wanted:
+            self.cotangents, self.derivatives, self.sums = rows(256), rows(F), new(splits, _lib.MLP_SUMS_SIZE)
+        return splits
 
     def _at(self, state, evaluations):
         """The state an iteration starts from, and room for that many evaluations' rows."""
