@@ -58,3 +58,18 @@ def test_last_batch_size_of_the_form(name, dtype, last):
     after = lanes_solve(f, y0, t_eval, "tsit5", PID)  # (one sample more is not covered: the call goes to the general kernel)
     assert _lib.last_solve_kernel_name() == "tode::solve_kernel"
     assert torch.equal(after.ys, ref.ys)
+
+
+# Evaluation points of 32 samples (lanes) or 64 (one sample per lane) per workgroup, beside step records of 6 to 21 KB in LDS: numbers of
+# points that a small batch keeps there too, with 64 KB and up to the last byte of its budget, and the next one, which
+# is read from memory.
+@pytest.mark.parametrize("form, dtype, n_eval", [
+    ("lanes", torch.float32, 700), ("lanes", torch.float32, 1226), ("lanes", torch.float32, 1227), ("lanes", torch.float64, 588), ("lanes", torch.float64, 589),
+    ("two", torch.float32, 300), ("two", torch.float32, 594), ("two", torch.float32, 595), ("two", torch.float64, 275), ("two", torch.float64, 276),
+], ids=str)  # fmt: skip
+def test_evaluation_points_up_to_the_size_of_lds(form, dtype, n_eval):
+    f, y0, t_eval = problem("vdp", 70, dtype, n_eval)
+    solve = lanes_solve if form == "lanes" else lambda *args: gpu_solve(*args, fast="two")
+    for method, spec in (("tsit5", PID), ("dopri5", dict(kind="integral", atol=1e-5, rtol=1e-3))):
+        assert_identical(solve(f, y0, t_eval, method, spec), c_oracle_solve(f, y0, t_eval, method, spec))
+        assert _lib.last_solve_kernel_name() == "tode::solve_pair_kernel"
