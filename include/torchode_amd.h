@@ -567,6 +567,14 @@ int tode_step_stats(const tode_step_state *state, int64_t *out_n_steps, int64_t 
 int tode_set_fast_kernel_variant(int variant);
 
 /*
+ * A hook for tests: the short forms of division and square root in the small systems' kernels against the compiler's.  Adds the
+ * number of results that differ to `mismatches` (one int32 in device memory).  form 0 ... 3: float32 reciprocal, square
+ * root, division by the square root of 2 and of 3, over every value of their ranges; 4: float32 quotient, of `samples`
+ * pseudo-random pairs; 5 ... 9: the same five in float64, of `samples` pseudo-random operands.
+ */
+int tode_check_short_forms(int32_t form, int64_t samples, void *mismatches, void *stream);
+
+/*
  * Kernel timing for benchmarks and profiling; no counterpart in the reference.
  * While enabled (per host thread), tode_solve_builtin and tode_solve_builtin_fast record a HIP event on
  * `stream` directly before and directly after its solve kernel.

@@ -1,5 +1,6 @@
-"""The loops of the whole-solve kernels of the small systems, compiled for the host with the address sanitizer, one lane per
-wavefront (tests/host_wavefront): what they do on inputs whose times or states leave the range of the type."""
+"""The whole-solve kernels of the small systems, compiled for the host (tests/host_wavefront): with the address sanitizer and
+one lane per wavefront, what their loops do on inputs whose times leave the range of the type; and their short form of
+the division."""
 import os
 import re
 import shutil
@@ -14,7 +15,8 @@ OPERATIONS = {"v_max": "fmax", "v_min": "fmin"}
 
 
 @pytest.fixture(scope="module")
-def program(tmp_path_factory):
+def sources(tmp_path_factory):
+    """A copy of the kernels' sources that the host's compiler takes; returns the compiler's command up to its file."""
     if shutil.which("g++") is None:
         pytest.skip("no g++ here")
     build = tmp_path_factory.mktemp("host_wavefront")
@@ -33,9 +35,14 @@ def program(tmp_path_factory):
         text = re.sub(r'asm volatile\(""[^;]*;', "", text)
         text = text.replace("extern __shared__ __align__(16) unsigned char smem_raw[];", "unsigned char *const smem_raw = host::lds;")
         open(path, "w").write(text)
+    return str(build), ["g++", "-std=c++17", "-w", "-ffp-contract=off", "-pthread", f"-I{os.path.join(HERE, 'host_wavefront')}", f"-I{csrc}"]
+
+
+@pytest.fixture(scope="module")
+def program(sources):
+    build, compiler = sources
     out = os.path.join(build, "main")
-    subprocess.run(["g++", "-std=c++17", "-O1", "-g", "-w", "-ffp-contract=off", "-fsanitize=address", "-pthread", f"-I{os.path.join(HERE, 'host_wavefront')}",
-                    f"-I{csrc}", os.path.join(HERE, "host_wavefront", "main.cpp"), "-o", out], check=True, timeout=600)  # fmt: skip
+    subprocess.run([*compiler, "-O1", "-g", "-fsanitize=address", os.path.join(HERE, "host_wavefront", "main.cpp"), "-o", out], check=True, timeout=600)
 
     def run(*args):
         env = dict(os.environ, ASAN_OPTIONS="verify_asan_link_order=0")
@@ -76,3 +83,13 @@ def test_a_point_far_in_front_of_the_start(program, kernel, method, dtype, far):
     by the division (the product with the step's reciprocal made it an infinity less an infinity)."""
     flag, _, initialized, value = program(kernel, dtype, method, 1.0, 1.0, 1.0, far, 2.0)
     assert (flag, initialized) == (0, 1) and abs(value) == float("inf")
+
+
+def test_quotients_next_to_a_rounding_boundary(sources):
+    """The short form of the float32 quotient, given the correctly rounded reciprocal, on all 46 517 418 pairs of mantissas
+    whose quotient lies so close to a boundary that the form's error could take it to the other side."""
+    build, compiler = sources
+    out = os.path.join(build, "quotients")
+    subprocess.run([*compiler, "-O2", "-march=native", os.path.join(HERE, "host_wavefront", "quotients.cpp"), "-o", out], check=True, timeout=600)
+    r = subprocess.run([out], capture_output=True, text=True, timeout=600, check=True)
+    assert r.stdout.split() == ["46517418", "0"]

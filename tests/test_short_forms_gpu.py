@@ -49,3 +49,14 @@ def test_scaled_errors_of_every_size(features, dtype):
         ref = c_oracle_solve(f, y0, t_eval, method, spec)
         for fast in ("one", True):
             assert_identical(gpu_solve(f, y0, t_eval, method, spec, fast=fast), ref)
+
+
+@pytest.mark.parametrize("form", range(10), ids=[f"{name}-{dtype}" for dtype in ("f32", "f64") for name in ("reciprocal", "root", "over-root-2", "over-root-3", "quotient")])
+def test_forms_against_the_compilers(form):
+    """float32 over every value of the form's range, float64 and quotients on 2^28 pseudo-random operands: not one result
+    that differs from the division's or the square root's (ids in the order of the library's forms)."""
+    from torchode_amd import _lib
+
+    mismatches = torch.zeros(1, dtype=torch.int32, device="cuda")
+    _lib.check(_lib.load().tode_check_short_forms(form, 1 << 28, mismatches.data_ptr(), _lib.stream_of(mismatches)), "tode_check_short_forms")
+    assert int(mismatches) == 0

@@ -61,6 +61,7 @@ EXPORTS = (
     "tode_step_stats",
     "tode_finalize_stats",
     "tode_set_fast_kernel_variant",
+    "tode_check_short_forms",
     "tode_set_kernel_timing",
     "tode_last_solve_kernel_ms",
     "tode_last_solve_kernel_name",
@@ -394,6 +395,8 @@ def load():
         lib.tode_step_stats.argtypes = [C.POINTER(StepState)] + [C.c_void_p] * 5
         lib.tode_finalize_stats.restype = C.c_int
         lib.tode_finalize_stats.argtypes = [C.c_int64, C.c_int64] + [C.c_void_p] * 9 + [C.c_int32] * 3 + [C.c_void_p] * 3
+        lib.tode_check_short_forms.restype = C.c_int
+        lib.tode_check_short_forms.argtypes = [C.c_int32, C.c_int64, C.c_void_p, C.c_void_p]
         lib.tode_set_fast_kernel_variant.restype = C.c_int
         lib.tode_set_fast_kernel_variant.argtypes = [C.c_int]
         lib.tode_set_kernel_timing.restype = C.c_int

@@ -64,6 +64,7 @@ UNITS = [
     ("tode_grid.hip", "tode_grid.o", []),
     ("tode_mlp.hip", "tode_mlp.o", []),
     ("tode_mlp_reverse.hip", "tode_mlp_reverse.o", []),
+    ("tode_checks.hip", "tode_checks.o", []),
 ]
 
 

@@ -124,13 +124,14 @@ template <typename T> __device__ __forceinline__ T ldexp2k(T d, int e) { return 
 // iteration of the small systems holds three to four divisions, a square root and two powers, and
 // runs at the rate at which a SIMD issues vector instructions: 11 -> 6 instructions per float32
 // division, 11 -> 3 for the logarithm's reciprocal, 17 -> 5 per square root, 7 -> 1 per power of two.
-// Same values, by proof or exhaustively:
-//  * float32 reciprocal, square root: equal to 1 / x and sqrt(x) for every mantissa (1 <= x < 4, checked on
-//    the hardware; both scale exactly with even powers of two while nothing underflows);
+// The sequences are Newton's iteration for the reciprocal with Markstein's correction of the quotient, and Goldschmidt's for the
+// square root, in the forms in which AMD's open compiler (LLVM) lowers the two in float64.  Same values, by proof or
+// exhaustively (tode_checks.hip runs the forms against the compiler's on the device):
+//  * float32 reciprocal, square root: equal to 1 / x and sqrt(x) for every x of the ranges below, on the hardware;
 //  * float32 quotient: r is the correctly rounded reciprocal, n * r is less than two units off, and the
 //    corrected quotient errs by less than 2^-22 units before its rounding.  The mantissa pairs whose
 //    quotient lies that close to a rounding boundary are those with 2^k n = (2j + 1) d + s, |s| <= 8:
-//    all of them (to |s| = 32) were enumerated, none is rounded to the wrong side;
+//    tests/host_wavefront/quotients.cpp enumerates all of them, none is rounded to the wrong side;
 //  * float64: the iterations that the general forms run on operands they do not have to scale.
 // Measured with the lane conditions below, on whole solves: Van der Pol float32 B = 65536 (tode_pair.hip) 0.147 -> 0.121 ms,
 // float64 B = 20011 0.175 -> 0.145 ms; Lorenz float32 B = 40009 0.063 -> 0.052 ms, B = 1 048 576 (tode_fast.hip, eight
