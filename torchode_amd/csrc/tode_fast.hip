@@ -27,9 +27,9 @@ template <typename T> struct FastOut {
 };
 
 // Wavefronts per SIMD that the registers are held to: five, 96 registers, so that no kernel of the small rows spills (they take
-// 63 to 83, five to eight wavefronts).  Held to 64 registers for eight wavefronts the forms with more tableau weights or a
-// history spilled into scratch memory: Lorenz float32 B = 1 048 576, Tsit5 551 us -> 542 us, Tsit5 with PID 582 -> 547 us;
-// Dopri5 with the integral controller, which takes 69 registers left to itself, 553 us and 557 us.
+// 64 to 83, six to eight wavefronts).  Held to 64 registers for eight wavefronts the forms with more tableau weights or a
+// history spilled into scratch memory: Lorenz float32 B = 1 048 576, a solve back to back, Tsit5 552 us -> 537 us, Tsit5
+// with PID 572 -> 541 us; Dopri5 with the integral controller takes 64 either way.
 constexpr int fast_wavefronts(size_t size, int features, int nhist, bool record) { return size == 4 && features <= 3 && nhist <= 1 && !record ? 5 : 1; }
 
 // NHIST: how many history factors the controller multiplies in (0 integral, 1 PI, 2 PID).

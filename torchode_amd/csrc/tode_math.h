@@ -134,8 +134,8 @@ template <typename T> __device__ __forceinline__ T ldexp2k(T d, int e) { return 
 //    tests/host_wavefront/quotients.cpp enumerates all of them, none is rounded to the wrong side;
 //  * float64: the iterations that the general forms run on operands they do not have to scale.
 // Measured with the lane conditions below, on whole solves: Van der Pol float32 B = 65536 (tode_pair.hip) 0.147 -> 0.121 ms,
-// float64 B = 20011 0.175 -> 0.145 ms; Lorenz float32 B = 40009 0.063 -> 0.052 ms, B = 1 048 576 (tode_fast.hip, eight
-// wavefronts per SIMD, where additions and products are issued at twice the rate of what was removed) 0.51 -> 0.50 ms.
+// float64 B = 20011 0.175 -> 0.145 ms; Lorenz float32 B = 40009 0.063 -> 0.052 ms.  B = 1 048 576 (tode_fast.hip, eight
+// wavefronts per SIMD): a fifth fewer instructions, 548 and 546 us per solve of changing batches, no difference beyond noise.
 // Ranges: quotient d in [2^-40, 2^124], n = 0 or n / d in [2^-60, 2^60] (remainders exact, no intermediate
 // result subnormal); root in [2^-100, 2^100]; reciprocal in [1, 4).
 // ---------------------------------------------------------------------------
