@@ -73,3 +73,11 @@ def test_evaluation_points_up_to_the_size_of_lds(form, dtype, n_eval):
     for method, spec in (("tsit5", PID), ("dopri5", dict(kind="integral", atol=1e-5, rtol=1e-3))):
         assert_identical(solve(f, y0, t_eval, method, spec), c_oracle_solve(f, y0, t_eval, method, spec))
         assert _lib.last_solve_kernel_name() == "tode::solve_pair_kernel"
+
+
+def test_rows_of_more_than_two_to_the_24_values():
+    """Offsets into a workgroup's block of the output are 32 bits wide: 32 samples of that many values are within them."""
+    f, y0, t_eval = problem("vdp", 2, torch.float32, 2**23 + 1)
+    ref = c_oracle_solve(f, y0, t_eval, "tsit5", PID)
+    assert_identical(gpu_solve(f, y0, t_eval, "tsit5", PID), ref)
+    assert _lib.last_solve_kernel_name() == "tode::solve_pair_kernel"

@@ -295,7 +295,7 @@ __global__ void __launch_bounds__(128) solve_pair_kernel(const SolveParams<T> p,
             if (STAGE_TE) return te_s[e * S + group];
             return e < E ? dir * tev_g[e] : never;
         };
-        // (a workgroup's block of ys is far below 4 GiB: launch_pair)
+        // (a workgroup's block of ys holds fewer than 2^32 values: launch_pair)
         T *ys_block = p.ys + b0 * (long long)E * F;
         const unsigned ys_row = (unsigned)(live ? group : 0) * (unsigned)E;
         int cursor = 0;
@@ -373,7 +373,7 @@ static int launch_pair(const tode_solve_args &a, const tode_controller &c, const
     if (blocks == 0 || a.batch > pair_batch_limit<Term>()) return TODE_OK;
     const size_t rec_bytes = (size_t)2 * NF * 64 * sizeof(T) + 16;
     const size_t te_bytes = a.n_eval > 0 ? ((size_t)a.n_eval + 1) * S * sizeof(T) : 0;
-    if ((size_t)a.n_eval * Term::F >= ((size_t)1 << 24)) return TODE_OK;  // (32-bit offsets into a workgroup's block of ys)
+    if ((size_t)a.n_eval * Term::F * S > 0xffffffffu) return TODE_OK;  // (32-bit offsets into a workgroup's block of ys)
     // LDS: up to four workgroups per compute unit for every 64 samples of theirs, fewer in a batch that does not have them
     const long long per_cu = (blocks + 255) / 256;
     const size_t budget = (size_t)(160 * 1024) / (size_t)(per_cu < 4 * L ? per_cu : 4 * L) - 512;
