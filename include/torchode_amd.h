@@ -667,9 +667,9 @@ typedef struct tode_solve_adjoint {
     const void *grad_ys;           /* [B, max(E,1), F] cotangent of ys */
     const int32_t *points_by_iteration; /* [B,E]: each sample's evaluation points ordered by the iteration that wrote them */
     const int32_t *iterations_sorted;   /* [B,E]: those iterations in the same order, ascending; -1 (first) for a point that
-                                           no iteration wrote.  Both NULL when E == 0 -- or to have the library work
-                                           them out from the record's times (a kernel of its own in front of the sweep,
-                                           into `scratch`) */
+                                           no iteration wrote.  Both NULL when E == 0 -- or to have the sweep tell by
+                                           the record's times (it needs lists only for rows of times in no order, and
+                                           makes them in `scratch`) */
     int64_t iterations;            /* L: iterations of the loop; the record's entries 0..L are read */
     int32_t through_control;       /* as in tode_step_adjoint */
     int32_t through_start;         /* 0: the results are the cotangents of the loop's first state.  1: the kernel also

@@ -725,7 +725,7 @@ def test_whole_sweep_kernel_agrees_with_the_per_iteration_kernels_and_the_torch_
     wrt = [y0, leaf] + ([t_eval] if case == "times" else []) + ([dt0] if case == "dt0" else [])
     results = {}
     # ("whole-lists": the one-kernel sweep with the lists of evaluation points by iteration made by torch operations and
-    # handed in, where "whole" lets the library's two kernels make them: the same bits)
+    # handed in, where "whole" lets the kernel tell by the record's times: the same bits)
     for sweep in ("whole", "whole-lists", "kernels", "torch"):
         solver = to.AutoDiffAdjoint(method(), make_controller(), max_steps=30 if case == "max-steps" else None,
                                     backprop_through_step_size_control=through_control)  # fmt: skip
@@ -763,6 +763,39 @@ def test_whole_sweep_kernel_agrees_with_the_per_iteration_kernels_and_the_torch_
                 else:
                     torch.testing.assert_close(g / scale, ref / scale, rtol=rtol, atol=atol)
     assert all(g is not None and bool(g.isfinite().all()) for g in results["whole"][:2])
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("features,dtype", [(2, torch.float32), (2, torch.float64), (4, torch.float32), (8, torch.float32), (8, torch.float64)])
+@pytest.mark.parametrize("rows", ["ordered", "some-shuffled", "repeated", "beyond-the-end"])
+def test_points_of_the_whole_sweep_against_lists_handed_in(rows, features, dtype):
+    """Which points an iteration wrote, found by walking rows of times (the points held in registers ahead and further ones), or
+    by lists where a wavefront has a row in no order, against lists made by torch operations: the same bits.  150 samples are
+    three wavefronts, of which the middle one alone has shuffled rows; 61 points in a dozen steps are many more than are held;
+    repeated points lie at t_start and on the ends of steps (a point of another row's); points beyond t_end are never reached."""
+    B, E = 150, 61
+    g = torch.Generator().manual_seed(11)
+    k = (0.1 + 3 * torch.rand(B, features, generator=g, dtype=torch.float64)).to(dtype).cuda()
+    y0 = (torch.rand(B, features, generator=g, dtype=torch.float64) * 2 - 1).to(dtype).cuda()
+    t_eval = (torch.rand(B, 1, generator=g, dtype=torch.float64) + torch.linspace(0, 2, E, dtype=torch.float64)[None, :]).to(dtype)
+    t_start, t_end = t_eval[:, 0].clone(), t_eval[:, -1].clone()
+    if rows == "some-shuffled":
+        t_eval[64:128:3, 1:-1] = t_eval[64:128:3, 1:-1][:, torch.randperm(E - 2, generator=g)]
+    if rows == "repeated":
+        t_eval[:, 1:4], t_eval[:, 20:23] = t_eval[:, :1].clone(), t_eval[:, 20:21].clone()
+    if rows == "beyond-the-end":
+        t_end = t_eval[:, 40].clone()
+    cotangent = torch.randn(B, E, features, generator=g, dtype=torch.float64).to(dtype).cuda()
+    results = []
+    for lists in (False, True):
+        leaf, y = k.clone().requires_grad_(), y0.clone().requires_grad_()
+        solver = to.AutoDiffAdjoint(to.Tsit5(), to.PIDController(1e-6, 1e-3, 0.2, 0.5, 0.0))
+        solver.backward_points_in_torch = lists
+        sol = solver.solve(to.InitialValueProblem(y, t_start.cuda(), t_end.cuda(), t_eval.cuda()), to.ODETerm(to.LinearDecay(leaf)))
+        ys = torch.where(sol.ys.detach().isfinite(), sol.ys, torch.zeros_like(sol.ys))
+        results.append(torch.autograd.grad(ys, [y, leaf], cotangent if rows != "beyond-the-end" else cotangent * (torch.arange(E, device="cuda") < 40)[None, :, None]))
+    for a, b in zip(*results):
+        assert bool(a.isfinite().all()) and bool((a != 0).any()) and torch.equal(a, b)
 
 
 @pytest.mark.gpu

@@ -422,9 +422,8 @@ def reverse_sweep_whole(adjoint, replay: Replay, term, problem, dt0, record, gra
     t_eval = None if replay.t_eval is None else contiguous(replay.t_eval)
     L, arrays = record.iterations, record.arrays
 
-    # Which iteration wrote which evaluation point (adjoints.py:215-234: the first whose new time has passed it), and
-    # each sample's points ordered by it: worked out by the library from the record's times, in two kernels in front
-    # of the sweep.  The same in torch operations, handed in, for the tests to hold against that.
+    # Which iteration wrote which evaluation point (adjoints.py:215-234: the first whose new time has passed it): the kernel
+    # tells by the record's times.  The same in torch operations, as lists handed in, for the tests to hold against that.
     iterations_sorted = points_by_iteration = None
     if E > 0 and getattr(adjoint, "backward_points_in_torch", False):
         direction = torch.where(t_end > t_start, 1.0, -1.0).to(dtype)

@@ -1,5 +1,5 @@
-// Reverse of one loop iteration, shared by the per-iteration kernels (tode_stepwise.hip) and the whole-sweep kernel
-// (tode_backward.hip).
+// Reverse of one loop iteration: the per-iteration kernels (tode_stepwise.hip).  The whole-sweep kernel (tode_backward.hip)
+// runs the same operations on rows whose length it knows.
 #pragma once
 #include "tode_solve.h"
 
@@ -59,16 +59,12 @@ template <bool WAVE, typename T> __device__ __forceinline__ T row_sum(T v) {
 }
 
 // (the body of finish_backward_kernel for sample b; f_first / f_step: the features this thread walks)
-// points / n_listed: the evaluation points this iteration wrote, where the caller knows them (n_listed >= 0); else
-// every point of the row is looked at and those with hit_iteration == iteration are taken.
-// FC: the row length where the caller knows it at compile time (0: p.F).  With FC set, b == 0 and every per-sample
-// array a thread-private one, all indices are constants and the arrays can live in registers.
-template <typename TT, typename T, int METHOD, int CTRL, bool WAVE, int FC = 0>
-__device__ __forceinline__ void finish_backward_sample(const AdjointParams<TT, T> &p, const long long b, const int f_first, const int f_step,
-                                                       const int32_t *points = nullptr, const int n_listed = -1) {
+// The evaluation points this iteration wrote are those with hit_iteration == iteration: every point of the row is looked at.
+template <typename TT, typename T, int METHOD, int CTRL, bool WAVE>
+__device__ __forceinline__ void finish_backward_sample(const AdjointParams<TT, T> &p, const long long b, const int f_first, const int f_step) {
     using Tab = typename std::conditional<METHOD == 1, Tsit5Tab, Dopri5Tab>::type;
     const bool scalar_lane = f_first == 0;
-    const int F = FC > 0 ? FC : p.F, E = p.E;
+    const int F = p.F, E = p.E;
     const CtrlParams<T> &cp = p.cp;
     const TT t0 = p.t[b], dt = p.dt[b];
     const T h = (T)dt;
@@ -205,7 +201,7 @@ __device__ __forceinline__ void finish_backward_sample(const AdjointParams<TT, T
     TT den = t1 - t0;
     const bool flat = !(abs_(den) > (TT)0);
     if (flat) den = (TT)1;
-    const int n_points = E > 0 ? (n_listed >= 0 ? n_listed : E) : (p.end_point ? 1 : 0);
+    const int n_points = E > 0 ? E : (p.end_point ? 1 : 0);
     // The output at a point is a polynomial in the point's position x, and its cotangent g enters all results through the
     // sums of g, g x, .. g x^4 over the points.  Rows of a wavefront each take the sums first, five per feature, and the
     // stages' shares once per iteration (point by point, every point read, changed and wrote the cotangents of all seven
@@ -292,9 +288,8 @@ __device__ __forceinline__ void finish_backward_sample(const AdjointParams<TT, T
         g_t -= gx / den;
         if (!flat) g_dt -= gxx / den;
     }
-    for (int idx = 0; idx < ((WAVE && !own_gradients) ? 0 : n_points); ++idx) {
-        const int e = (E > 0 && n_listed >= 0) ? points[idx] : idx;
-        if (E > 0 && n_listed < 0 && p.hit_iteration[b * E + e] != p.iteration) continue;
+    for (int e = 0; e < ((WAVE && !own_gradients) ? 0 : n_points); ++e) {
+        if (E > 0 && p.hit_iteration[b * E + e] != p.iteration) continue;
         const TT at = E > 0 ? p.t_eval[b * E + e] : te;
         const T x = (T)((at - t0) / den);
         T g_x = 0;
@@ -365,11 +360,11 @@ template <typename TT, typename T, int METHOD, int CTRL, bool WAVE> __global__ v
 }
 
 // Stage S reversed.  g_ystage [B,F]: cotangent of the stage input; g_tnode [B] (may be null): of its time.
-template <typename TT, typename T, int METHOD, bool WAVE, int FC = 0>
+template <typename TT, typename T, int METHOD, bool WAVE>
 __device__ __forceinline__ void stage_backward_sample(const AdjointParams<TT, T> &p, const long long b, const int S, const T *g_ystage, const TT *g_tnode,
                                                       const int f_first, const int f_step) {
     using Tab = typename std::conditional<METHOD == 1, Tsit5Tab, Dopri5Tab>::type;
-    const int F = FC > 0 ? FC : p.F;
+    const int F = p.F;
     const T h = (T)p.dt[b];
     T a[7];
 #pragma unroll

@@ -5,28 +5,32 @@
 // iteration (tode_solve_record).  One thread per sample walks its iterations from the last to the first: it forms
 // the six stages again from the recorded state (registers, the right-hand side evaluated in the kernel), pulls the
 // cotangents of the state after the iteration and of the evaluation points the iteration wrote through everything
-// after the stages (finish_backward_sample), then through the stages from the last to the first, with the
+// after the stages, then through the stages from the last to the first, with the
 // right-hand side's own vector-Jacobian product in closed form where the per-iteration path asks autograd for it.
 // Everything a sample's thread works on -- stage derivatives, their cotangents, the cotangents of the state -- is an
-// array private to the thread, indexed by constants once the shared reverse functions are inlined with the row length
-// known (registers): those functions get index 0 and every array in global memory moved forward to the thread's sample.
-// The record of the next iteration down is loaded while the current one is worked on.
+// array private to the thread, indexed by constants (registers).  What an iteration reads is loaded while the one before is
+// worked on: its entry of the record, and the evaluation points it may have written.
 #include "tode_adjoint.h"
 
 namespace tode {
 
 template <typename T> struct WholeBackward {
-    AdjointParams<T, T> base;  // problem and controller; the per-iteration fields and the working arrays are set in the kernel
-    long long iterations;      // L: the record holds entries 0..L
+    long long batch, iterations;  // iterations: L, the record holds entries 0..L
+    int E, through_control;
+    const T *t_start, *t_end, *t_eval, *grad_ys;
+    T *g_t_start, *g_t_end, *g_t_eval;
+    CtrlParams<T> cp;
+    T dt_min, dt_max;
     const T *rec_t, *rec_dt, *rec_y, *rec_k0, *rec_prev, *rec_pprev;
     const int32_t *rec_running, *rec_n_accepted;
     const T *params;
     double scalars[4];
     T *a_y, *a_k0, *a_t, *a_dt, *a_prev, *a_pprev;  // results: cotangents of the state before the first iteration
     T *g_params;  // [B,P] result
-    // the evaluation points of every sample ordered by the iteration that wrote them: [B,E] point indices and, in the
-    // same order, the iterations (-1 first: points no iteration wrote)
+    // the evaluation points of every sample ordered by the iteration that wrote them, where the caller hands them in: [B,E]
+    // point indices and, in the same order, the iterations (-1 first: points no iteration wrote)
     const int32_t *points_by_iteration, *iterations_sorted;
+    int32_t *lists;  // room for both, for wavefronts with a row of times in no order (list_points)
     long long ts_stride, te_stride;  // t_start / t_end: sample b at element b * stride
     int through_start;  // also carry the cotangents through the start of the loop (start_backward)
     int dt0_given;      // the first step was the caller's, not the start rule's
@@ -38,7 +42,7 @@ template <typename T, int F> struct RecordEntry {
 };
 
 template <typename T, int F> __device__ __forceinline__ RecordEntry<T, F> load_entry(const WholeBackward<T> &w, long long entry, long long sample) {
-    const long long at = entry * w.base.batch + sample;
+    const long long at = entry * w.batch + sample;
     RecordEntry<T, F> r;
     r.t = w.rec_t[at], r.dt = w.rec_dt[at], r.prev = w.rec_prev[at], r.pprev = w.rec_pprev[at];
 #pragma unroll
@@ -157,11 +161,41 @@ __device__ __forceinline__ void start_backward(const CtrlParams<T> &cp, const Te
     for (int f = 0; f < F; ++f) a_y[f] = g_y0[f] + g_from_f0[f];
 }
 
+// Which iteration wrote which evaluation point (adjoints.py:215-234: the first whose new time has reached it; none for
+// a point at t_start, which the loop's set-up writes, and for one the solve never reached), for a row of times in no order:
+// a binary search over the sample's recorded times for each point, and the points sorted by insertion (stable: points of one
+// iteration stay in their order).  One thread per sample; rows whose times run in the direction of the solve, nearly all
+// there are, never come here (the sweep meets their points in order).
+template <typename T>
+__device__ __forceinline__ void list_points(const WholeBackward<T> &w, const long long sample, const T ts, const T dir, const T *t_eval, int32_t *its, int32_t *pts) {
+    for (int e = 0; e < w.E; ++e) {
+        const T at = t_eval[e], v = dir * at;
+        long long lo = 0, hi = w.iterations;
+        while (lo < hi) {
+            const long long mid = (lo + hi) / 2;
+            if (dir * w.rec_t[(mid + 1) * w.batch + sample] < v) lo = mid + 1;
+            else hi = mid;
+        }
+        int32_t hit = lo < w.iterations ? (int32_t)lo : -1;
+        if (e == 0 && at == ts) hit = -1;
+        int j = e - 1;
+        for (; j >= 0 && its[j] > hit; --j) its[j + 1] = its[j], pts[j + 1] = pts[j];
+        its[j + 1] = hit, pts[j + 1] = e;
+    }
+}
+
+// What bounds this kernel is one thread's chain: B = 65536 is one wavefront per SIMD, and the slowest sample's 107
+// iterations follow one another.  The evaluation points of an iteration are in registers before the iteration begins: AHEAD
+// of them, from the last one that no iteration has met yet downwards, are loaded as soon as the iteration before has taken
+// its own.  (Looked up in lists that two kernels in front of this one made, an iteration waited for memory two or three
+// times, first for the number of its points, then for each point's index, then for its time and cotangent: Van der Pol float32,
+// B = 65536, 50 points: 0.76 ms and 0.05 ms for the two kernels; 0.66 ms this way.)
 template <typename T, int METHOD, int CTRL, typename Term>
 __global__ void __launch_bounds__(64) whole_backward_kernel(const WholeBackward<T> w) {
     using Tab = typename std::conditional<METHOD == 1, Tsit5Tab, Dopri5Tab>::type;
     constexpr int F = Term::F, P = Term::P;
-    const long long B = w.base.batch;
+    constexpr int AHEAD = F <= 4 ? 4 : 2;  // points held: a step of these systems passes one to four
+    const long long B = w.batch;
     const long long g = (long long)blockIdx.x * 64 + threadIdx.x;  // this thread's sample
     if (g >= B) return;
     Term rhs;
@@ -170,100 +204,319 @@ __global__ void __launch_bounds__(64) whole_backward_kernel(const WholeBackward<
 #pragma unroll
     for (int j = 0; j < P; ++j) gpar[j] = 0;
 
-    // ---- the thread's own arrays; the shared functions reach them through q with index 0 ----
-    T k[7][F], g_k[7][F], y[F], y1[F], g_ystage[F], g_y[F], g_y1[F], a_y[F], a_k0[F];
-    T t0 = 0, dt = 0, prev = 1, pprev = 1, g_t = 0, g_dt = 0, g_prev = 0, g_pprev = 0;
-    T a_t = 0, a_dt = 0, a_prev = 0, a_pprev = 0;  // cotangents of the state after the iteration: zeros behind the last one
-    int32_t moved = 0, running_next = 0;
+    const CtrlParams<T> &cp = w.cp;
+    const int E = w.E;
+    const T ts = w.t_start[g * w.ts_stride], te = w.t_end[g * w.te_stride];
+    const T tlo = tmin(ts, te), thi = tmax(te, ts);
+    const T sf = (T)__builtin_sqrt((double)F);
+    const T *t_eval = E > 0 ? w.t_eval + g * E : nullptr;
+    const T *grad_ys = w.grad_ys + g * (long long)(E > 0 ? E : 1) * F;
+
+    T a_y[F], a_k0[F], a_t = 0, a_dt = 0, a_prev = 0, a_pprev = 0;  // cotangents of the state after the iteration: zeros behind the last one
 #pragma unroll
     for (int f = 0; f < F; ++f) a_y[f] = 0, a_k0[f] = 0;
-    AdjointParams<T, T> q = w.base;
-#pragma unroll
-    for (int s = 0; s < 7; ++s) q.k[s] = k[s], q.g_k[s] = g_k[s];
-    q.t = &t0, q.dt = &dt, q.y = y, q.y1 = y1, q.prev = &prev, q.pprev = &pprev;
-    q.moved = &moved, q.running_next = &running_next;
-    q.g_y = g_y, q.g_y1 = g_y1, q.g_t = &g_t, q.g_dt = &g_dt, q.g_prev = &g_prev, q.g_pprev = &g_pprev;
-    q.a_y = a_y, q.a_k0 = a_k0, q.a_t = &a_t, q.a_dt = &a_dt, q.a_prev = &a_prev, q.a_pprev = &a_pprev;
-    // ---- what lives in global memory, moved forward to this sample ----
-    const int E = q.E;
-    q.t_start += g * w.ts_stride, q.t_end += g * w.te_stride;
-    if (q.t_eval) q.t_eval += g * E;
-    q.grad_ys += g * (long long)(E > 0 ? E : 1) * F;
-    if (q.g_t_start) q.g_t_start += g;
-    if (q.g_t_end) q.g_t_end += g;
-    if (q.g_t_eval) q.g_t_eval += g * E;
-    const int32_t *iterations_sorted = w.iterations_sorted + g * E, *points_by_iteration = w.points_by_iteration + g * E;
 
     const long long L = w.iterations;
-    int cursor = E - 1;  // into the sample's points ordered by iteration, walked from the end as the iterations are
     RecordEntry<T, F> after = load_entry<T, F>(w, L, g), here = load_entry<T, F>(w, L > 0 ? L - 1 : 0, g);
+
+    // ---- the evaluation points, walked from the last to the first as the iterations are ----
+    // Where every row of the wavefront runs in the direction of its solve, a point belongs to the iteration at hand if it
+    // lies behind the time before it: those behind the time after it have been taken.  Elsewhere the lists say.
+    const T dir = te > ts ? (T)1 : (T)-1;
+    const int32_t *its = nullptr, *pts = nullptr;
+    int lowest = 0, cursor = E - 1;
+    if (E > 0) {
+        bool in_order = w.points_by_iteration == nullptr;
+        for (int e = 1; in_order && e < E; ++e) in_order = dir * t_eval[e - 1] <= dir * t_eval[e];  // (false for a time that is not a number)
+        if (lanes_where(!in_order)) {
+            its = w.iterations_sorted + g * E, pts = w.points_by_iteration + g * E;
+            if (w.points_by_iteration == nullptr) {
+                int32_t *const own = w.lists + g * E, *const own_points = own + B * E;
+                list_points<T>(w, g, ts, dir, t_eval, own, own_points);
+                its = own, pts = own_points;
+            }
+        } else {
+            lowest = t_eval[0] == ts ? 1 : 0;  // (written by the loop's set-up)
+            while (cursor >= lowest && dir * after.t < dir * t_eval[cursor]) --cursor;  // (never reached)
+        }
+    }
+    const bool listed = its != nullptr;
+    T at[AHEAD], g_at[AHEAD][F];
+    int32_t written_by[AHEAD];
+    auto load_ahead = [&]() {
+#pragma unroll
+        for (int p = 0; p < AHEAD; ++p) {
+            int e = max(cursor - p, 0);
+            written_by[p] = 0;
+            if (listed) written_by[p] = its[e], e = pts[e];
+            at[p] = t_eval[e];
+#pragma unroll
+            for (int f = 0; f < F; ++f) g_at[p][f] = grad_ys[(long long)e * F + f];
+        }
+    };
+    if (E > 0) {
+        load_ahead();
+    } else {  // (the end point, written by the batch's last iteration)
+        at[0] = te;
+#pragma unroll
+        for (int f = 0; f < F; ++f) g_at[0][f] = grad_ys[f];
+    }
+
     for (long long i = L - 1; i >= 0; --i) {
         const RecordEntry<T, F> before = load_entry<T, F>(w, i > 0 ? i - 1 : 0, g);  // (used by the next pass of this loop)
-        q.iteration = (int)i;
-        q.end_point = (E == 0 && i == L - 1) ? 1 : 0;
+        const bool end_point = E == 0 && i == L - 1;
         // An iteration that none of the wavefront's samples took part in (all had finished before it) changes nothing for
         // them -- no move, no point written, the step and the history kept -- so its reverse hands every cotangent on as
         // it is.  (Without evaluation points the batch's last iteration is the one whose interpolant gives the result.)
-        if (!q.end_point && !__any(here.running != 0)) {
+        if (!end_point && !lanes_where(here.running != 0)) {
             after = here, here = before;
             continue;
         }
-        t0 = here.t, dt = here.dt, prev = here.prev, pprev = here.pprev;
-        moved = (after.n_accepted - here.n_accepted) > 0 ? 1 : 0;
-        running_next = after.running != 0 ? 1 : 0;
+        const T t0 = here.t, dt = here.dt, prev = here.prev, pprev = here.pprev;
+        const bool move = after.n_accepted > here.n_accepted, running_new = after.running != 0;
 
         // ---- the stages again (runge_kutta.py:255-263) ----
+        T k[7][F], y[F], yi[7][F];
 #pragma unroll
         for (int f = 0; f < F; ++f) y[f] = here.y[f], k[0][f] = here.k0[f];
 #pragma unroll
         for (int s = 1; s < 7; ++s) {
-            T yi[F];
 #pragma unroll
             for (int f = 0; f < F; ++f) {
                 T sum = 0;
 #pragma unroll
                 for (int j = 0; j < s; ++j) sum = fma_((T)Tab::a[s][j], k[j][f], sum);
-                yi[f] = fma_(dt, sum, y[f]);
+                yi[s][f] = fma_(dt, sum, y[f]);
             }
-            rhs(fma_((T)Tab::c[s], dt, t0), yi, k[s]);
-            if (s == 6) {
+            rhs(fma_((T)Tab::c[s], dt, t0), yi[s], k[s]);
+        }
+        const T(&y1)[F] = yi[6];
+
+        // ---- everything after the stages, reversed: the operations of finish_backward_sample, in its order ----
+        T acc = 0, err[F];
 #pragma unroll
-                for (int f = 0; f < F; ++f) y1[f] = yi[f];
+        for (int f = 0; f < F; ++f) {
+            err[f] = 0;
+#pragma unroll
+            for (int s = 0; s < 7; ++s) err[f] = fma_(dt * (T)Tab::b_err[s], k[s][f], err[f]);
+            const T m = tmax(abs_(y[f]), abs_(y1[f]));
+            const T x = (abs_(err[f]) / fma_(cp.rtol, m, cp.atol)) / sf;
+            acc = fma_(x, x, acc);
+        }
+        const T r = sqrt_(acc), ratio = tmax(r, (T)1e-38);
+        T F0 = cp.safety * rpow<T>(ratio, cp.e1);
+        if (CTRL == 1) {
+            F0 = F0 * (cp.skip2 ? (T)1 : rpow<T>(prev, cp.e2));
+            F0 = F0 * (cp.skip3 ? (T)1 : rpow<T>(pprev, cp.e3));
+        }
+        const T factor = tclamp(F0, cp.fmin, cp.fmax);
+        const T raw = dt * factor;
+        T dt_next = raw;
+        (void)limit_step<T, T>(cp, w.dt_min, w.dt_max, ratio, dt_next);
+        const T t_new = move ? (t0 + dt) : t0;
+        const T lo = tlo - t_new, hi = thi - t_new;
+        const T dtn = running_new ? dt_next : dt;
+
+        // clamp of the step to the time range, and the new time
+        T g_tnew = a_t, g_dt = 0, g_dt_next = 0;
+        {
+            const T g_self = (dtn >= lo && dtn <= hi) ? a_dt : (T)0;
+            const T g_lo = (dtn < lo && lo < hi) ? a_dt : (T)0;
+            const T g_hi = (dtn > hi || hi < lo) ? a_dt : (T)0;
+            g_tnew -= g_lo + g_hi;
+            if (w.g_t_start || w.g_t_end) {
+                T g_ts_lo, g_te_lo, g_ts_hi, g_te_hi;
+                // tlo = minimum(t_start, t_end), thi = maximum(t_start, t_end) (problems.py:58-64)
+                max_backward<T>(-ts, -te, g_lo, g_ts_lo, g_te_lo);  // minimum(a, b) = -maximum(-a, -b): same split
+                max_backward<T>(ts, te, g_hi, g_ts_hi, g_te_hi);
+                if (w.g_t_start) w.g_t_start[g] += g_ts_lo + g_ts_hi;
+                if (w.g_t_end) w.g_t_end[g] += g_te_lo + g_te_hi;
+            }
+            if (running_new) g_dt_next = g_self;
+            else g_dt = g_self;
+        }
+        T g_t = g_tnew;
+        if (move) g_dt += g_tnew;
+
+        // controller history and step proposal
+        T g_ratio = 0, g_prev = 0, g_pprev = 0;
+        if (CTRL == 1) {
+            const bool keep = running_new && move;
+            g_ratio = keep ? a_prev : (T)0;
+            g_prev = keep ? a_pprev : a_prev;
+            g_pprev = keep ? (T)0 : a_pprev;
+        }
+        if (w.through_control) {
+            T g_raw = g_dt_next;
+            if (cp.has_dt_min || cp.has_dt_max) {
+                const T mag = abs_(raw);
+                const bool inside = (!cp.has_dt_min || mag >= w.dt_min) && (!cp.has_dt_max || mag <= w.dt_max);
+                g_raw = (inside && raw != (T)0) ? g_dt_next : (T)0;
+            }
+            g_dt += g_raw * factor;
+            const T g_factor = g_raw * dt;
+            const T g_F0 = (F0 >= cp.fmin && F0 <= cp.fmax) ? g_factor : (T)0;
+            g_ratio += g_F0 * F0 * (T)cp.e1 / ratio;
+            if (CTRL == 1) {
+                if (!cp.skip2) g_prev += g_F0 * F0 * (T)cp.e2 / prev;
+                if (!cp.skip3) g_pprev += g_F0 * F0 * (T)cp.e3 / pprev;
             }
         }
 
-        // ---- everything after the stages, reversed ----
-        // (The points of this iteration are counted in a loop that the whole wavefront runs together, with a clamped
-        // index in place of a guarded load: no lane leaves and rejoins here.  Written as each lane's own loop, this was a
-        // divergent region at whose end the compiler, for four instantiations on long float64 rows, copied registers of
-        // the parameter cotangents to accumulation registers ahead of the instruction that restores the execution mask;
-        // lanes that had no point left skipped the copy and went on with the values of an earlier iteration.)
-        int n_here = 0;
-        while (E > 0) {
-            const int at = cursor - n_here;
-            const bool more = at >= 0 && iterations_sorted[at < 0 ? 0 : at] == (int)i;
-            if (!__any(more)) break;
-            n_here += more ? 1 : 0;
+        // error ratio and error estimate; state update
+        const T tiny = (T)1e-38;
+        const T g_r = r > tiny ? g_ratio : (r == tiny ? g_ratio / (T)2 : (T)0);
+        T g_h = 0, g_k[7][F], g_y[F], g_y1[F];
+#pragma unroll
+        for (int f = 0; f < F; ++f) {
+            T gy = move ? (T)0 : a_y[f], gy1 = move ? a_y[f] : (T)0;
+            T gk[7] = {move ? (T)0 : a_k0[f], 0, 0, 0, 0, 0, move ? a_k0[f] : (T)0};
+            if (g_r != (T)0 && r > (T)0) {
+                T bk = 0;
+#pragma unroll
+                for (int s = 0; s < 7; ++s) bk = fma_((T)Tab::b_err[s], k[s][f], bk);
+                const T ay = abs_(y[f]), ay1 = abs_(y1[f]);
+                const T eb = fma_(cp.rtol, tmax(ay, ay1), cp.atol);
+                const T q = abs_(err[f]) / eb;
+                const T g_q = g_r * (q / sf) / r / sf;
+                const T g_err = g_q / eb * sign_(err[f]);
+                const T g_m = -g_q * q / eb * cp.rtol;
+                T ga, gb;
+                max_backward<T>(ay, ay1, g_m, ga, gb);
+                gy += ga * sign_(y[f]);
+                gy1 += gb * sign_(y1[f]);
+#pragma unroll
+                for (int s = 0; s < 7; ++s) gk[s] += g_err * (dt * (T)Tab::b_err[s]);
+                g_h += g_err * bk;
+            }
+            g_y[f] = gy, g_y1[f] = gy1;
+#pragma unroll
+            for (int s = 0; s < 7; ++s) g_k[s][f] = gk[s];
         }
-        cursor -= n_here;
-        finish_backward_sample<T, T, METHOD, CTRL, false, F>(q, 0, 0, 1, points_by_iteration + cursor + 1, n_here);
+
+        // dense output: the evaluation points this iteration wrote, one by one in their order (see finish_backward_sample)
+        T den = (t0 + dt) - t0;
+        const bool flat = !(abs_(den) > (T)0);
+        if (flat) den = (T)1;
+        T slope[F][4];  // the polynomial's coefficients, lowest power first, differentiated
+        auto build_slopes = [&]() {
+#pragma unroll
+            for (int f = 0; f < F; ++f) {
+                const T ks[7] = {k[0][f], k[1][f], k[2][f], k[3][f], k[4][f], k[5][f], k[6][f]};
+                T q[5][1];
+                quartic_elem<T, METHOD>(dt, y[f], y1[f], ks, true, q);
+                slope[f][0] = q[1][0], slope[f][1] = (T)2 * q[2][0], slope[f][2] = (T)3 * q[3][0], slope[f][3] = (T)4 * q[4][0];
+            }
+        };
+        auto add_point = [&](const T t, const T(&cotangent)[F], T *g_time) {
+            const T x = (t - t0) / den;
+            T g_x = 0;
+#pragma unroll
+            for (int f = 0; f < F; ++f) {
+                const T g0 = cotangent[f];
+                if (g0 == (T)0) continue;
+                const T ks[7] = {k[0][f], k[1][f], k[2][f], k[3][f], k[4][f], k[5][f], k[6][f]};
+                g_x += g0 * (slope[f][0] + x * (slope[f][1] + x * (slope[f][2] + x * slope[f][3])));
+                const T g1 = g0 * x, g2 = g1 * x, g3 = g2 * x, g4 = g3 * x;
+                if (METHOD == 1) {
+                    g_y[f] += g0;
+                    g_k[0][f] += g1 * dt;
+                    g_h += g1 * ks[0];
+#pragma unroll
+                    for (int s = 0; s < 7; ++s) {
+                        const T u = g2 * (T)Tsit5Tab::w[0][s] + g3 * (T)Tsit5Tab::w[1][s] + g4 * (T)Tsit5Tab::w[2][s];
+                        g_k[s][f] += u * dt;
+                        g_h += u * ks[s];
+                    }
+                } else {
+                    const T g_f0 = (T)-2 * g4 + (T)5 * g3 - (T)4 * g2 + g1, g_f1 = (T)2 * g4 - (T)3 * g3 + g2;
+                    const T g_mid = (T)16 * g4 - (T)32 * g3 + (T)16 * g2;
+                    g_y[f] += (T)-8 * g4 + (T)18 * g3 - (T)11 * g2 + g0 + g_mid;
+                    g_y1[f] += (T)-8 * g4 + (T)14 * g3 - (T)5 * g2;
+                    g_k[0][f] += g_f0 * dt;
+                    g_k[6][f] += g_f1 * dt;
+                    g_h += g_f0 * ks[0] + g_f1 * ks[6];
+#pragma unroll
+                    for (int s = 0; s < 7; ++s) {
+                        g_k[s][f] += g_mid * (dt * (T)Dopri5Tab::w[0][s]);
+                        g_h += g_mid * (T)Dopri5Tab::w[0][s] * ks[s];
+                    }
+                }
+            }
+            // x = (t - t0) / ((t0 + dt) - t0)
+            if (g_time) *g_time += g_x / den;
+            g_t -= g_x / den;
+            if (!flat) g_dt -= g_x * x / den;
+        };
+        lanes_t takes[AHEAD];
+        int n = 0;
+        if (E > 0) {
+            auto wrote = [&](int p, T time, int32_t by) {
+                return cursor - p >= lowest && (listed ? by == (int32_t)i : (i == 0 || dir * t0 < dir * time));
+            };
+#pragma unroll
+            for (int p = 0; p < AHEAD; ++p) {
+                const bool more = wrote(p, at[p], written_by[p]);
+                takes[p] = lanes_where(more), n += more ? 1 : 0;
+            }
+            if (takes[0]) build_slopes();
+            if (takes[AHEAD - 1]) {  // (some sample's step passed more points than are held)
+                for (bool more = n == AHEAD; lanes_where(more);) {
+                    const int e = max(cursor - n, 0);
+                    more = more && wrote(n, t_eval[listed ? pts[e] : e], listed ? its[e] : 0);
+                    n += more ? 1 : 0;
+                }
+                for (int p = n - 1; lanes_where(p >= AHEAD); --p) {
+                    if (p < AHEAD) continue;
+                    const int e = listed ? pts[cursor - p] : cursor - p;
+                    T cotangent[F];
+#pragma unroll
+                    for (int f = 0; f < F; ++f) cotangent[f] = grad_ys[(long long)e * F + f];
+                    add_point(t_eval[e], cotangent, w.g_t_eval ? w.g_t_eval + g * E + e : nullptr);
+                }
+            }
+        } else {
+            takes[0] = lanes_where(end_point);
+#pragma unroll
+            for (int p = 1; p < AHEAD; ++p) takes[p] = 0;
+            if (end_point) build_slopes();
+        }
+#pragma unroll
+        for (int p = AHEAD - 1; p >= 0; --p) {
+            if (!takes[p]) continue;
+            if (holds(takes[p])) {
+                T *g_time = E > 0 ? w.g_t_eval : w.g_t_end;
+                if (g_time) g_time += E == 0 ? g : g * E + (listed ? pts[cursor - p] : cursor - p);
+                add_point(at[p], g_at[p], g_time);
+            }
+        }
+        if (E > 0) {
+            cursor -= n;
+            load_ahead();
+        }
+        g_dt += g_h;
 
         // ---- the stages reversed ----
 #pragma unroll
         for (int s = 6; s >= 1; --s) {
-            T yi[F], gk[F], gy[F];
+            T gk[F], gy[F];
+#pragma unroll
+            for (int f = 0; f < F; ++f) gk[f] = g_k[s][f];
+            rhs.vjp(fma_((T)Tab::c[s], dt, t0), yi[s], gk, gy, gpar);
+            T g_step = 0;
 #pragma unroll
             for (int f = 0; f < F; ++f) {
+                const T g_in = s == 6 ? gy[f] + g_y1[f] : gy[f];
+                g_y[f] += g_in;
                 T sum = 0;
 #pragma unroll
-                for (int j = 0; j < s; ++j) sum = fma_((T)Tab::a[s][j], k[j][f], sum);
-                yi[f] = fma_(dt, sum, y[f]);
-                gk[f] = g_k[s][f];
+                for (int j = 0; j < s; ++j) {
+                    sum = fma_((T)Tab::a[s][j], k[j][f], sum);
+                    g_k[j][f] += (T)Tab::a[s][j] * dt * g_in;
+                }
+                g_step += g_in * sum;
             }
-            rhs.vjp(fma_((T)Tab::c[s], dt, t0), yi, gk, gy, gpar);
-#pragma unroll
-            for (int f = 0; f < F; ++f) g_ystage[f] = gy[f] + (s == 6 ? g_y1[f] : (T)0);
-            stage_backward_sample<T, T, METHOD, false, F>(q, 0, s, g_ystage, (const T *)nullptr, 0, 1);
+            g_dt += g_step;
         }
 
         // ---- the cotangents of the state before this iteration are those behind the one before it ----
@@ -274,7 +527,7 @@ __global__ void __launch_bounds__(64) whole_backward_kernel(const WholeBackward<
     }
     // (no iteration: nothing flows back through the loop, and the cotangents are still the zeros they started as)
     if (w.through_start)  // (`here` is the record's first entry now: t_start, y0, f(t_start, y0))
-        start_backward<T, CTRL, Term>(q.cp, rhs, q.through_control && !w.dt0_given, q.t_start[0], q.t_end[0], here.y, here.k0, a_y, a_k0, a_dt, gpar);
+        start_backward<T, CTRL, Term>(cp, rhs, w.through_control && !w.dt0_given, ts, te, here.y, here.k0, a_y, a_k0, a_dt, gpar);
 #pragma unroll
     for (int f = 0; f < F; ++f) w.a_y[g * F + f] = a_y[f], w.a_k0[g * F + f] = a_k0[f];
     w.a_t[g] = a_t, w.a_dt[g] = a_dt, w.a_prev[g] = a_prev, w.a_pprev[g] = a_pprev;
@@ -282,59 +535,15 @@ __global__ void __launch_bounds__(64) whole_backward_kernel(const WholeBackward<
     for (int j = 0; j < P; ++j) w.g_params[g * P + j] = gpar[j];
 }
 
-// Which iteration wrote which evaluation point (adjoints.py:215-234: the first whose new time has reached it; none for
-// a point at t_start, which the loop's set-up writes, and for one the solve never reached): one thread per point, a
-// binary search over the sample's recorded times.
-template <typename T> __global__ void __launch_bounds__(256) backward_hits_kernel(long long B, int E, long long L, const T *t_start, long long ts_stride, const T *t_end, long long te_stride,
-                                                                                  const T *t_eval, const T *rec_t, int32_t *iterations_sorted, int32_t *points_by_iteration) {
-    const long long at_point = (long long)blockIdx.x * 256 + threadIdx.x;
-    if (at_point >= B * E) return;
-    const long long b = at_point / E;
-    const int e = (int)(at_point - b * E);
-    const T ts = t_start[b * ts_stride], dir = t_end[b * te_stride] > ts ? (T)1 : (T)-1;
-    const T at = t_eval[at_point], v = dir * at;
-    long long lo = 0, hi = L;
-    while (lo < hi) {
-        const long long mid = (lo + hi) / 2;
-        if (dir * rec_t[(mid + 1) * B + b] < v) lo = mid + 1;
-        else hi = mid;
-    }
-    int32_t hit = lo < L ? (int32_t)lo : -1;
-    if (e == 0 && at == ts) hit = -1;
-    iterations_sorted[at_point] = hit, points_by_iteration[at_point] = e;
-}
-
-// Each sample's points ordered by the iteration that wrote them (stable: points of one iteration stay in their order).
-// One thread per sample.  Rows whose evaluation times run in the direction of the solve are in order already, which a
-// look along the row shows; the others are sorted by insertion.
-// (a template only so that each translation unit that instantiates the sweep has its own copy)
-template <typename T> __global__ void __launch_bounds__(256) backward_order_kernel(long long B, int E, int32_t *iterations_sorted, int32_t *points_by_iteration) {
-    const long long b = (long long)blockIdx.x * 256 + threadIdx.x;
-    if (b >= B) return;
-    int32_t *its = iterations_sorted + b * E, *pts = points_by_iteration + b * E;
-    bool ordered = true;
-    for (int e = 1; e < E; ++e) ordered = ordered && its[e - 1] <= its[e];
-    if (ordered) return;
-    for (int e = 1; e < E; ++e) {
-        const int32_t hit = its[e], point = pts[e];
-        int j = e - 1;
-        for (; j >= 0 && its[j] > hit; --j) its[j + 1] = its[j], pts[j + 1] = pts[j];
-        its[j + 1] = hit, pts[j + 1] = point;
-    }
-}
-
 template <typename T, int METHOD, int CTRL, typename Term>
 static int launch_backward(const tode_solve_args &a, const tode_controller &c, const tode_solve_adjoint &adj, hipStream_t stream) {
     const long long B = a.batch;
-    constexpr int F = Term::F;
     WholeBackward<T> w = {};
-    AdjointParams<T, T> &p = w.base;
-    p.batch = B, p.F = F, p.E = a.n_eval, p.through_control = adj.through_control;
-    p.t_start = (const T *)a.t_start, p.t_end = (const T *)a.t_end, p.t_eval = (const T *)a.t_eval, p.fixed_dt = nullptr;
-    p.grad_ys = (const T *)adj.grad_ys, p.hit_iteration = nullptr, p.running = nullptr;
-    p.g_t_start = (T *)adj.g_t_start, p.g_t_end = (T *)adj.g_t_end, p.g_t_eval = (T *)adj.g_t_eval, p.g_fixed_dt = nullptr;
-    p.cp = make_ctrl<T>(c);
-    p.dt_min = (T)c.dt_min, p.dt_max = (T)c.dt_max;
+    w.batch = B, w.E = a.n_eval, w.through_control = adj.through_control;
+    w.t_start = (const T *)a.t_start, w.t_end = (const T *)a.t_end, w.t_eval = (const T *)a.t_eval, w.grad_ys = (const T *)adj.grad_ys;
+    w.g_t_start = (T *)adj.g_t_start, w.g_t_end = (T *)adj.g_t_end, w.g_t_eval = (T *)adj.g_t_eval;
+    w.cp = make_ctrl<T>(c);
+    w.dt_min = (T)c.dt_min, w.dt_max = (T)c.dt_max;
     w.a_y = (T *)adj.a_y, w.a_k0 = (T *)adj.a_k0, w.a_t = (T *)adj.a_t, w.a_dt = (T *)adj.a_dt, w.a_prev = (T *)adj.a_prev, w.a_pprev = (T *)adj.a_pprev;
     const tode_solve_record &r = *a.record;
     w.iterations = adj.iterations;
@@ -344,13 +553,7 @@ static int launch_backward(const tode_solve_args &a, const tode_controller &c, c
     for (int i = 0; i < 4; ++i) w.scalars[i] = a.term_scalars[i];
     w.g_params = (T *)adj.g_params;
     w.points_by_iteration = adj.points_by_iteration, w.iterations_sorted = adj.iterations_sorted;
-    if (a.n_eval > 0 && !adj.points_by_iteration) {  // (not handed in: worked out here, into the caller's scratch)
-        int32_t *lists = (int32_t *)adj.scratch;
-        w.iterations_sorted = lists, w.points_by_iteration = lists + B * a.n_eval;
-        hipLaunchKernelGGL((backward_hits_kernel<T>), dim3((unsigned)((B * a.n_eval + 255) / 256)), dim3(256), 0, stream, B, a.n_eval, (long long)adj.iterations, (const T *)a.t_start,
-                           (long long)a.t_start_stride, (const T *)a.t_end, (long long)a.t_end_stride, (const T *)a.t_eval, (const T *)a.record->t, lists, lists + B * a.n_eval);
-        hipLaunchKernelGGL((backward_order_kernel<T>), dim3((unsigned)((B + 255) / 256)), dim3(256), 0, stream, B, a.n_eval, lists, lists + B * a.n_eval);
-    }
+    w.lists = (int32_t *)adj.scratch;
     w.through_start = adj.through_start, w.dt0_given = a.dt0 != nullptr;
     w.ts_stride = a.t_start_stride, w.te_stride = a.t_end_stride;
     hipLaunchKernelGGL((whole_backward_kernel<T, METHOD, CTRL, Term>), dim3((unsigned)((B + 63) / 64)), dim3(64), 0, stream, w);
@@ -426,7 +629,6 @@ int tode_solve_builtin_backward(const tode_solve_args *a, const tode_controller 
         !adj->a_k0 || !adj->a_t || !adj->a_dt || !adj->a_prev || !adj->a_pprev || !adj->g_params)
         return fail(TODE_E_INVALID, "null pointer");
     const bool own_lists = a->n_eval > 0 && !adj->points_by_iteration;
-    if (own_lists && (a->batch * (int64_t)a->n_eval + 255) / 256 > 2147483647) return fail(TODE_E_UNSUPPORTED, "too many evaluation points for the library to order them: hand the two lists in");
     if (own_lists && (!adj->scratch || adj->scratch_bytes < tode_solve_backward_scratch_bytes(a)))
         return fail(TODE_E_INVALID, "the scratch buffer holds %lld bytes, this sweep needs %lld (tode_solve_backward_scratch_bytes)", (long long)(adj->scratch ? adj->scratch_bytes : 0),
                     (long long)tode_solve_backward_scratch_bytes(a));
