@@ -1,6 +1,6 @@
 """The whole-solve kernels of the small systems, compiled for the host (tests/host_wavefront): with the address sanitizer and
-one lane per wavefront, what their loops do on inputs whose times leave the range of the type; and their short form of
-the division."""
+one lane per wavefront, what their loops do on inputs whose times leave the range of the type; their short form of
+the division; and their reverse sweep."""
 import os
 import re
 import shutil
@@ -28,7 +28,7 @@ def sources(tmp_path_factory):
         a, b = (re.sub(r"\|(%\d)\|", r"fabs(\1)", x).replace("%1", "a").replace("%2", "b") for x in m.group(2).split(", "))
         return f"r = {OPERATIONS[m.group(1)]}({a}, {b});"
 
-    for name in ("tode_math.h", "tode_solve.h", "tode_fast.hip", "tode_pair.hip"):
+    for name in ("tode_math.h", "tode_solve.h", "tode_fast.hip", "tode_pair.hip", "tode_backward.hip"):
         path = os.path.join(csrc, name)
         text = open(path).read()
         text = re.sub(r'asm\("(v_max|v_min)_f\d\d %0, ([^"]*)" : [^;]*;', operation, text)
@@ -83,6 +83,17 @@ def test_a_point_far_in_front_of_the_start(program, kernel, method, dtype, far):
     by the division (the product with the step's reciprocal made it an infinity less an infinity)."""
     flag, _, initialized, value = program(kernel, dtype, method, 1.0, 1.0, 1.0, far, 2.0)
     assert (flag, initialized) == (0, 1) and abs(value) == float("inf")
+
+
+def test_reverse_sweep_against_its_general_forms(sources):
+    """The one-kernel reverse sweep against the per-iteration reverse on random records: the same bits, whatever rule sends an
+    operand to a short form and a row of times to the walk or to the lists."""
+    build, compiler = sources
+    out = os.path.join(build, "sweep")
+    subprocess.run([*compiler, "-O1", "-march=native", "-fsanitize=address", os.path.join(HERE, "host_wavefront", "sweep.cpp"), "-o", out], check=True, timeout=600)
+    env = dict(os.environ, ASAN_OPTIONS="verify_asan_link_order=0")
+    r = subprocess.run([out, "0", "2000"], capture_output=True, text=True, timeout=300, env=env)
+    assert r.returncode == 0 and r.stdout.split() == ["4000", "0"], (r.stdout, r.stderr[-2000:])
 
 
 def test_quotients_next_to_a_rounding_boundary(sources):

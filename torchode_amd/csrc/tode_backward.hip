@@ -34,6 +34,7 @@ template <typename T> struct WholeBackward {
     long long ts_stride, te_stride;  // t_start / t_end: sample b at element b * stride
     int through_start;  // also carry the cotangents through the start of the loop (start_backward)
     int dt0_given;      // the first step was the caller's, not the start rule's
+    int plain;          // tolerances and exponents in the ranges of the short forms
 };
 
 template <typename T, int F> struct RecordEntry {
@@ -184,17 +185,38 @@ __device__ __forceinline__ void list_points(const WholeBackward<T> &w, const lon
     }
 }
 
+// Dividends of short-form quotients (quotient_with): zero, or from 2^-90 to 2^80 (float64: 2^-700 to 2^700), with divisors from
+// 2^-40 to 2^20, so that no quotient and no remainder is subnormal.  outside(): the lanes, of those that run, with one that is
+// not; those that are not numbers count among them.
+template <typename T> struct Dividends {
+    static constexpr int smallest = sizeof(T) == 4 ? -90 : -700, largest = sizeof(T) == 4 ? 80 : 700;
+    unsigned least = 0xffffffffu, most = 0;
+    __device__ __forceinline__ Dividends() {}
+    __device__ __forceinline__ Dividends(T a) { add(a); }
+    __device__ __forceinline__ Dividends(T a, T b) { add(a), add(b); }
+    __device__ __forceinline__ void add(T a) {
+        const unsigned bits = high_bits(abs_(a));
+        least = min(least, bits - 1u), most = max(most, bits);  // (zero wraps round to the largest)
+    }
+    __device__ __forceinline__ lanes_t outside() const {
+        return lanes_where(least < power_of_two_bits<T>(smallest) - 1u) | lanes_where(most >= power_of_two_bits<T>(largest));
+    }
+};
+
 // What bounds this kernel is one thread's chain: B = 65536 is one wavefront per SIMD, and the slowest sample's 107
 // iterations follow one another.  The evaluation points of an iteration are in registers before the iteration begins: AHEAD
 // of them, from the last one that no iteration has met yet downwards, are loaded as soon as the iteration before has taken
 // its own.  (Looked up in lists that two kernels in front of this one made, an iteration waited for memory two or three
 // times, first for the number of its points, then for each point's index, then for its time and cotangent: Van der Pol float32,
-// B = 65536, 50 points: 0.76 ms and 0.05 ms for the two kernels; 0.66 ms this way.)
+// B = 65536, 50 points: 0.76 ms and 0.05 ms for the two kernels; 0.66 ms this way.)  What remains is instructions: the
+// divisions, the square root and the two powers in the short forms of tode_math.h wherever the wavefront's operands allow
+// them, 0.66 -> 0.53 ms; float64, B = 20 000: 0.60 -> 0.56; decay with eight features, B = 20 000: 0.51 -> 0.43.
 template <typename T, int METHOD, int CTRL, typename Term>
 __global__ void __launch_bounds__(64) whole_backward_kernel(const WholeBackward<T> w) {
     using Tab = typename std::conditional<METHOD == 1, Tsit5Tab, Dopri5Tab>::type;
     constexpr int F = Term::F, P = Term::P;
-    constexpr int AHEAD = F <= 4 ? 4 : 2;  // points held: a step of these systems passes one to four
+    constexpr bool SHORT = F * sizeof(T) <= 32;  // the short forms (rows of eight doubles have no registers left for what they keep)
+    constexpr int AHEAD = F <= 4 ? 4 : (SHORT ? 2 : 1);  // points held: a step of these systems passes one to four
     const long long B = w.batch;
     const long long g = (long long)blockIdx.x * 64 + threadIdx.x;  // this thread's sample
     if (g >= B) return;
@@ -293,115 +315,192 @@ __global__ void __launch_bounds__(64) whole_backward_kernel(const WholeBackward<
         const T(&y1)[F] = yi[6];
 
         // ---- everything after the stages, reversed: the operations of finish_backward_sample, in its order ----
-        T acc = 0, err[F];
-#pragma unroll
-        for (int f = 0; f < F; ++f) {
-            err[f] = 0;
-#pragma unroll
-            for (int s = 0; s < 7; ++s) err[f] = fma_(dt * (T)Tab::b_err[s], k[s][f], err[f]);
-            const T m = tmax(abs_(y[f]), abs_(y1[f]));
-            const T x = (abs_(err[f]) / fma_(cp.rtol, m, cp.atol)) / sf;
-            acc = fma_(x, x, acc);
-        }
-        const T r = sqrt_(acc), ratio = tmax(r, (T)1e-38);
-        T F0 = cp.safety * rpow<T>(ratio, cp.e1);
-        if (CTRL == 1) {
-            F0 = F0 * (cp.skip2 ? (T)1 : rpow<T>(prev, cp.e2));
-            F0 = F0 * (cp.skip3 ? (T)1 : rpow<T>(pprev, cp.e3));
-        }
-        const T factor = tclamp(F0, cp.fmin, cp.fmax);
-        const T raw = dt * factor;
-        T dt_next = raw;
-        (void)limit_step<T, T>(cp, w.dt_min, w.dt_max, ratio, dt_next);
         const T t_new = move ? (t0 + dt) : t0;
         const T lo = tlo - t_new, hi = thi - t_new;
-        const T dtn = running_new ? dt_next : dt;
-
-        // clamp of the step to the time range, and the new time
-        T g_tnew = a_t, g_dt = 0, g_dt_next = 0;
+        T g_t, g_dt, g_prev = 0, g_pprev = 0, g_h, g_lo, g_hi, g_k[7][F], g_y[F], g_y1[F];
         {
+            using Div = DivSqrtFeatures<T, F>;
+            // error ratio and step factor, in the short forms where every lane's operands are in their ranges (control_common's,
+            // over a wider range of the errors: their squares may vanish in the sum, as they do in the general form).  A sample
+            // that sits through an iteration with a zero step has an error of zero; its controller's results reach nothing.
+            T acc = 0, err[F], eb[F], per_eb[F], q[F], x[F], r, ratio, F0;
+            lanes_t outside = 0, bounds_outside = 0;
+            unsigned smallest = 0xffffffffu;
+            T largest_eb = 0;
+#pragma unroll
+            for (int f = 0; f < F; ++f) {
+                err[f] = 0;
+#pragma unroll
+                for (int s = 0; s < 7; ++s) err[f] = fma_(dt * (T)Tab::b_err[s], k[s][f], err[f]);
+                if constexpr (SHORT) {
+                    eb[f] = fma_(cp.rtol, max_abs(y[f], y1[f]), cp.atol);
+                    per_eb[f] = reciprocal_estimate(eb[f]);
+                    q[f] = quotient_with(abs_(err[f]), eb[f], per_eb[f]);
+                    x[f] = Div::fast(q[f]);
+                    smallest = min(smallest, min(high_bits(abs_(err[f])) - 1u, high_bits(q[f]) - 1u));  // (zero wraps round to the largest)
+                    largest_eb = f == 0 ? eb[f] : max_ordered(largest_eb, eb[f]);
+                    acc = fma_(x[f], x[f], acc);
+                }
+            }
+            if constexpr (SHORT) {
+                constexpr unsigned from = power_of_two_bits<T>(-40), width = power_of_two_bits<T>(16) - from;
+                const bool idle = acc == (T)0 && !running_new;
+                acc = idle ? (T)1 : acc;
+                bounds_outside = lanes_where(!(largest_eb <= (T)0x1p+20));
+                outside = lanes_where(smallest < power_of_two_bits<T>(Dividends<T>::smallest) - 1u) | lanes_where(high_bits(acc) - from >= width) | bounds_outside;
+                r = ratio = sqrt_plain(acc);
+                F0 = cp.safety * expk<true>(dw_mul(logk<true>(ratio), (T)cp.e1));
+                if (CTRL == 1 && !cp.skip2) F0 = F0 * expk<true>(dw_mul(logk<true>(prev), (T)cp.e2));
+                if (CTRL == 1 && !cp.skip3) F0 = F0 * expk<true>(dw_mul(logk<true>(pprev), (T)cp.e3));
+                constexpr unsigned history = power_of_two_bits<T>(-20), history_width = power_of_two_bits<T>(20) - history;
+                lanes_t history_outside = 0;
+                if (CTRL == 1 && !cp.skip2) history_outside |= lanes_where(high_bits(prev) - history >= history_width);
+                if (CTRL == 1 && !cp.skip3) history_outside |= lanes_where(high_bits(pprev) - history >= history_width);
+                outside |= history_outside, bounds_outside |= history_outside;
+            }
+            if (!SHORT || !w.plain || outside) {
+                acc = 0;
+#pragma unroll
+                for (int f = 0; f < F; ++f) {
+                    eb[f] = fma_(cp.rtol, tmax(abs_(y[f]), abs_(y1[f])), cp.atol);
+                    q[f] = abs_(err[f]) / eb[f];
+                    x[f] = q[f] / sf;
+                    acc = fma_(x[f], x[f], acc);
+                }
+                r = sqrt_(acc), ratio = tmax(r, (T)1e-38);
+                F0 = cp.safety * rpow<T>(ratio, cp.e1);
+                if (CTRL == 1) {
+                    F0 = F0 * (cp.skip2 ? (T)1 : rpow<T>(prev, cp.e2));
+                    F0 = F0 * (cp.skip3 ? (T)1 : rpow<T>(pprev, cp.e3));
+                }
+            }
+            // Quotients of cotangents: the divisors' ranges are known, the dividends are looked at.  divisors_outside: lanes
+            // (of those that take part) whose divisor is outside.
+            const T per_ratio = reciprocal_estimate(ratio);
+            const lanes_t ratio_outside = lanes_where(!(ratio >= (T)0x1p-20)) | lanes_where(!(ratio <= (T)0x1p+20));
+            if (SHORT && !w.plain) bounds_outside = ~(lanes_t)0;
+
+            const T factor = tclamp(F0, cp.fmin, cp.fmax);
+            const T raw = dt * factor;
+            T dt_next = raw;
+            (void)limit_step<T, T>(cp, w.dt_min, w.dt_max, ratio, dt_next);
+            const T dtn = running_new ? dt_next : dt;
+
+            // clamp of the step to the time range, and the new time
             const T g_self = (dtn >= lo && dtn <= hi) ? a_dt : (T)0;
-            const T g_lo = (dtn < lo && lo < hi) ? a_dt : (T)0;
-            const T g_hi = (dtn > hi || hi < lo) ? a_dt : (T)0;
-            g_tnew -= g_lo + g_hi;
-            if (w.g_t_start || w.g_t_end) {
-                T g_ts_lo, g_te_lo, g_ts_hi, g_te_hi;
-                // tlo = minimum(t_start, t_end), thi = maximum(t_start, t_end) (problems.py:58-64)
-                max_backward<T>(-ts, -te, g_lo, g_ts_lo, g_te_lo);  // minimum(a, b) = -maximum(-a, -b): same split
-                max_backward<T>(ts, te, g_hi, g_ts_hi, g_te_hi);
-                if (w.g_t_start) w.g_t_start[g] += g_ts_lo + g_ts_hi;
-                if (w.g_t_end) w.g_t_end[g] += g_te_lo + g_te_hi;
-            }
-            if (running_new) g_dt_next = g_self;
-            else g_dt = g_self;
-        }
-        T g_t = g_tnew;
-        if (move) g_dt += g_tnew;
+            g_lo = (dtn < lo && lo < hi) ? a_dt : (T)0;
+            g_hi = (dtn > hi || hi < lo) ? a_dt : (T)0;
+            const T g_tnew = a_t - (g_lo + g_hi), g_dt_next = running_new ? g_self : (T)0;
+            g_dt = running_new ? (T)0 : g_self;
+            g_t = g_tnew;
+            if (move) g_dt += g_tnew;
 
-        // controller history and step proposal
-        T g_ratio = 0, g_prev = 0, g_pprev = 0;
-        if (CTRL == 1) {
-            const bool keep = running_new && move;
-            g_ratio = keep ? a_prev : (T)0;
-            g_prev = keep ? a_pprev : a_prev;
-            g_pprev = keep ? (T)0 : a_pprev;
-        }
-        if (w.through_control) {
-            T g_raw = g_dt_next;
-            if (cp.has_dt_min || cp.has_dt_max) {
-                const T mag = abs_(raw);
-                const bool inside = (!cp.has_dt_min || mag >= w.dt_min) && (!cp.has_dt_max || mag <= w.dt_max);
-                g_raw = (inside && raw != (T)0) ? g_dt_next : (T)0;
-            }
-            g_dt += g_raw * factor;
-            const T g_factor = g_raw * dt;
-            const T g_F0 = (F0 >= cp.fmin && F0 <= cp.fmax) ? g_factor : (T)0;
-            g_ratio += g_F0 * F0 * (T)cp.e1 / ratio;
+            // controller history and step proposal
+            T g_ratio = 0;
             if (CTRL == 1) {
-                if (!cp.skip2) g_prev += g_F0 * F0 * (T)cp.e2 / prev;
-                if (!cp.skip3) g_pprev += g_F0 * F0 * (T)cp.e3 / pprev;
+                const bool keep = running_new && move;
+                g_ratio = keep ? a_prev : (T)0;
+                g_prev = keep ? a_pprev : a_prev;
+                g_pprev = keep ? (T)0 : a_pprev;
+            }
+            if (w.through_control) {
+                T g_raw = g_dt_next;
+                if (cp.has_dt_min || cp.has_dt_max) {
+                    const T mag = abs_(raw);
+                    const bool inside = (!cp.has_dt_min || mag >= w.dt_min) && (!cp.has_dt_max || mag <= w.dt_max);
+                    g_raw = (inside && raw != (T)0) ? g_dt_next : (T)0;
+                }
+                g_dt += g_raw * factor;
+                const T g_factor = g_raw * dt;
+                const T g_F0 = (F0 >= cp.fmin && F0 <= cp.fmax) ? g_factor : (T)0;
+                const T g_powers = g_F0 * F0;
+                // (times an exponent of 2^-10 to 1/2: dividends a little below the smallest, of divisors between 2^-20 and 2^20)
+                const Dividends<T> d(g_powers);
+                if (SHORT && !(d.outside() | ratio_outside | bounds_outside)) {
+                    g_ratio += quotient_with(g_powers * (T)cp.e1, ratio, per_ratio);
+                    if (CTRL == 1) {
+                        if (!cp.skip2) g_prev += quotient_plain(g_powers * (T)cp.e2, prev);
+                        if (!cp.skip3) g_pprev += quotient_plain(g_powers * (T)cp.e3, pprev);
+                    }
+                } else {
+                    g_ratio += g_powers * (T)cp.e1 / ratio;
+                    if (CTRL == 1) {
+                        if (!cp.skip2) g_prev += g_powers * (T)cp.e2 / prev;
+                        if (!cp.skip3) g_pprev += g_powers * (T)cp.e3 / pprev;
+                    }
+                }
+            }
+
+            // error ratio and error estimate; state update
+            const T tiny = (T)1e-38;
+            const T g_r = r > tiny ? g_ratio : (r == tiny ? g_ratio / (T)2 : (T)0);
+            g_h = 0;
+#pragma unroll
+            for (int f = 0; f < F; ++f) {
+                g_y[f] = move ? (T)0 : a_y[f], g_y1[f] = move ? a_y[f] : (T)0;
+#pragma unroll
+                for (int s = 0; s < 7; ++s) g_k[s][f] = 0;
+                g_k[0][f] = move ? (T)0 : a_k0[f], g_k[6][f] = move ? a_k0[f] : (T)0;
+            }
+            if (g_r != (T)0 && r > (T)0) {
+                T g_q[F], g_err[F], g_m[F];
+                lanes_t general = ~(lanes_t)0;
+                if constexpr (SHORT) {  // (r is the ratio where it is in range)
+                    Dividends<T> d;
+#pragma unroll
+                    for (int f = 0; f < F; ++f) {
+                        const T g_x = g_r * x[f], over_r = quotient_with(g_x, r, per_ratio);
+                        g_q[f] = Div::fast(over_r);
+                        const T g_eb = -g_q[f] * q[f];
+                        g_err[f] = quotient_with(g_q[f], eb[f], per_eb[f]);
+                        g_m[f] = quotient_with(g_eb, eb[f], per_eb[f]);
+                        d.add(g_x), d.add(over_r), d.add(g_q[f]), d.add(g_eb);
+                    }
+                    general = d.outside() | ((ratio_outside | bounds_outside) & lanes_where(true));
+                }
+                if (general) {
+#pragma unroll
+                    for (int f = 0; f < F; ++f) {
+                        g_q[f] = g_r * x[f] / r / sf;
+                        g_err[f] = g_q[f] / eb[f];
+                        g_m[f] = -g_q[f] * q[f] / eb[f];
+                    }
+                }
+#pragma unroll
+                for (int f = 0; f < F; ++f) {
+                    T bk = 0;
+#pragma unroll
+                    for (int s = 0; s < 7; ++s) bk = fma_((T)Tab::b_err[s], k[s][f], bk);
+                    const T g_e = g_err[f] * sign_(err[f]);
+                    T ga, gb;
+                    max_backward<T>(abs_(y[f]), abs_(y1[f]), g_m[f] * cp.rtol, ga, gb);
+                    g_y[f] += ga * sign_(y[f]);
+                    g_y1[f] += gb * sign_(y1[f]);
+#pragma unroll
+                    for (int s = 0; s < 7; ++s) g_k[s][f] += g_e * (dt * (T)Tab::b_err[s]);
+                    g_h += g_e * bk;
+                }
             }
         }
-
-        // error ratio and error estimate; state update
-        const T tiny = (T)1e-38;
-        const T g_r = r > tiny ? g_ratio : (r == tiny ? g_ratio / (T)2 : (T)0);
-        T g_h = 0, g_k[7][F], g_y[F], g_y1[F];
-#pragma unroll
-        for (int f = 0; f < F; ++f) {
-            T gy = move ? (T)0 : a_y[f], gy1 = move ? a_y[f] : (T)0;
-            T gk[7] = {move ? (T)0 : a_k0[f], 0, 0, 0, 0, 0, move ? a_k0[f] : (T)0};
-            if (g_r != (T)0 && r > (T)0) {
-                T bk = 0;
-#pragma unroll
-                for (int s = 0; s < 7; ++s) bk = fma_((T)Tab::b_err[s], k[s][f], bk);
-                const T ay = abs_(y[f]), ay1 = abs_(y1[f]);
-                const T eb = fma_(cp.rtol, tmax(ay, ay1), cp.atol);
-                const T q = abs_(err[f]) / eb;
-                const T g_q = g_r * (q / sf) / r / sf;
-                const T g_err = g_q / eb * sign_(err[f]);
-                const T g_m = -g_q * q / eb * cp.rtol;
-                T ga, gb;
-                max_backward<T>(ay, ay1, g_m, ga, gb);
-                gy += ga * sign_(y[f]);
-                gy1 += gb * sign_(y1[f]);
-#pragma unroll
-                for (int s = 0; s < 7; ++s) gk[s] += g_err * (dt * (T)Tab::b_err[s]);
-                g_h += g_err * bk;
-            }
-            g_y[f] = gy, g_y1[f] = gy1;
-#pragma unroll
-            for (int s = 0; s < 7; ++s) g_k[s][f] = gk[s];
+        if (w.g_t_start || w.g_t_end) {
+            T g_ts_lo, g_te_lo, g_ts_hi, g_te_hi;
+            // tlo = minimum(t_start, t_end), thi = maximum(t_start, t_end) (problems.py:58-64)
+            max_backward<T>(-ts, -te, g_lo, g_ts_lo, g_te_lo);  // minimum(a, b) = -maximum(-a, -b): same split
+            max_backward<T>(ts, te, g_hi, g_ts_hi, g_te_hi);
+            if (w.g_t_start) w.g_t_start[g] += g_ts_lo + g_ts_hi;
+            if (w.g_t_end) w.g_t_end[g] += g_te_lo + g_te_hi;
         }
 
         // dense output: the evaluation points this iteration wrote, one by one in their order (see finish_backward_sample)
         T den = (t0 + dt) - t0;
         const bool flat = !(abs_(den) > (T)0);
         if (flat) den = (T)1;
+        const T per_den = reciprocal_estimate(den);
+        const lanes_t den_outside = SHORT ? lanes_where(!(abs_(den) >= (T)0x1p-20)) | lanes_where(!(abs_(den) <= (T)0x1p+20)) : ~(lanes_t)0;
         T slope[F][4];  // the polynomial's coefficients, lowest power first, differentiated
-        auto build_slopes = [&]() {
+        auto build_slopes = [&](int first, int last) {
 #pragma unroll
-            for (int f = 0; f < F; ++f) {
+            for (int f = first; f < last; ++f) {
                 const T ks[7] = {k[0][f], k[1][f], k[2][f], k[3][f], k[4][f], k[5][f], k[6][f]};
                 T q[5][1];
                 quartic_elem<T, METHOD>(dt, y[f], y1[f], ks, true, q);
@@ -409,12 +508,15 @@ __global__ void __launch_bounds__(64) whole_backward_kernel(const WholeBackward<
             }
         };
         auto add_point = [&](const T t, const T(&cotangent)[F], T *g_time) {
-            const T x = (t - t0) / den;
+            const T from_t0 = t - t0;
+            T x = quotient_with(from_t0, den, per_den);
+            if (Dividends<T>(from_t0).outside() | (den_outside & lanes_where(true))) x = from_t0 / den;
             T g_x = 0;
 #pragma unroll
             for (int f = 0; f < F; ++f) {
                 const T g0 = cotangent[f];
                 if (g0 == (T)0) continue;
+                if (!SHORT) build_slopes(f, f + 1);
                 const T ks[7] = {k[0][f], k[1][f], k[2][f], k[3][f], k[4][f], k[5][f], k[6][f]};
                 g_x += g0 * (slope[f][0] + x * (slope[f][1] + x * (slope[f][2] + x * slope[f][3])));
                 const T g1 = g0 * x, g2 = g1 * x, g3 = g2 * x, g4 = g3 * x;
@@ -444,9 +546,12 @@ __global__ void __launch_bounds__(64) whole_backward_kernel(const WholeBackward<
                 }
             }
             // x = (t - t0) / ((t0 + dt) - t0)
-            if (g_time) *g_time += g_x / den;
-            g_t -= g_x / den;
-            if (!flat) g_dt -= g_x * x / den;
+            const T g_xx = g_x * x;
+            T g_at = quotient_with(g_x, den, per_den), g_den = quotient_with(g_xx, den, per_den);
+            if (Dividends<T>(g_x, g_xx).outside() | (den_outside & lanes_where(true))) g_at = g_x / den, g_den = g_xx / den;
+            if (g_time) *g_time += g_at;
+            g_t -= g_at;
+            if (!flat) g_dt -= g_den;
         };
         lanes_t takes[AHEAD];
         int n = 0;
@@ -459,7 +564,7 @@ __global__ void __launch_bounds__(64) whole_backward_kernel(const WholeBackward<
                 const bool more = wrote(p, at[p], written_by[p]);
                 takes[p] = lanes_where(more), n += more ? 1 : 0;
             }
-            if (takes[0]) build_slopes();
+            if (SHORT && takes[0]) build_slopes(0, F);
             if (takes[AHEAD - 1]) {  // (some sample's step passed more points than are held)
                 for (bool more = n == AHEAD; lanes_where(more);) {
                     const int e = max(cursor - n, 0);
@@ -479,7 +584,7 @@ __global__ void __launch_bounds__(64) whole_backward_kernel(const WholeBackward<
             takes[0] = lanes_where(end_point);
 #pragma unroll
             for (int p = 1; p < AHEAD; ++p) takes[p] = 0;
-            if (end_point) build_slopes();
+            if (SHORT && end_point) build_slopes(0, F);
         }
 #pragma unroll
         for (int p = AHEAD - 1; p >= 0; --p) {
@@ -544,6 +649,8 @@ static int launch_backward(const tode_solve_args &a, const tode_controller &c, c
     w.g_t_start = (T *)adj.g_t_start, w.g_t_end = (T *)adj.g_t_end, w.g_t_eval = (T *)adj.g_t_eval;
     w.cp = make_ctrl<T>(c);
     w.dt_min = (T)c.dt_min, w.dt_max = (T)c.dt_max;
+    const auto counts = [](double e) { return e >= 0x1p-10 || e <= -0x1p-10; };  // (a cotangent times an exponent)
+    w.plain = w.cp.plain && !w.cp.shortcut_exponent() && counts(w.cp.e1) && (w.cp.skip2 || counts(w.cp.e2)) && (w.cp.skip3 || counts(w.cp.e3));
     w.a_y = (T *)adj.a_y, w.a_k0 = (T *)adj.a_k0, w.a_t = (T *)adj.a_t, w.a_dt = (T *)adj.a_dt, w.a_prev = (T *)adj.a_prev, w.a_pprev = (T *)adj.a_pprev;
     const tode_solve_record &r = *a.record;
     w.iterations = adj.iterations;
