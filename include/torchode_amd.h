@@ -24,7 +24,7 @@
 extern "C" {
 #endif
 
-#define TODE_ABI_VERSION 23
+#define TODE_ABI_VERSION 24
 
 /* floating point type of data (y) and time (t) arrays */
 enum { TODE_F32 = 0, TODE_F64 = 1 };
@@ -433,13 +433,24 @@ int tode_mlp_outer_products(const tode_mlp_reverse *p, int64_t rows, int32_t acc
 /*
  * The start of the loop reversed (y = y0, k0 = f(t_start, y0), the start rule's first step clamped to the time range; the times
  * are constants): p->t, y, k0 are the record's first entry, p->g_y receives the cotangent of y0; its two evaluations of the
- * network (one without through_rule) take 2 B (B) rows of the stage buffers.
+ * network (one without through_rule) take 2 B (B) rows of the stage buffers.  With grad_ys the cotangent of a first evaluation
+ * point at t_start, a copy of y0 that no iteration wrote, is added to that of y0.
+ *
+ * tode_mlp_sweep_begin: what the sweep needs to know of a record (tode_solve_record, L iterations) ahead of its iterations, in one
+ * launch: which iteration wrote which evaluation point (hit_iteration [B,E]; -1: none, or a first point at t_start;
+ * adjoints.py:215-234, for times that run in the solve's direction), which samples moved in which iteration (moved [L,B]), and
+ * t_start and t_end as dense arrays.
  */
+int tode_mlp_sweep_begin(int64_t batch, int32_t n_eval, int64_t iterations, const void *t_start, int64_t t_start_stride, const void *t_end, int64_t t_end_stride,
+                         const void *t_eval, const void *rec_t, const int32_t *rec_n_accepted, int32_t *hit_iteration, int32_t *moved, void *t_start_out, void *t_end_out,
+                         void *stream);
 typedef struct tode_mlp_start {
     const void *t_end;                /* [B] */
     const void *a_y, *a_k0, *a_dt;    /* [B,F], [B,F], [B] cotangents of that first loop state */
     int32_t through_rule;             /* the first step is a function of y0 and the weights (no step of the user's, gradients
                                          through the step sizes) */
+    int32_t n_eval;
+    const void *grad_ys, *t_eval;     /* [B,E,F], [B,E]; both NULL: not wanted */
 } tode_mlp_start;
 int tode_mlp_start_backward(const tode_mlp_reverse *p, const tode_mlp_start *start, const tode_controller *c, void *stream);
 int tode_mlp_weight_gradients(const tode_mlp_reverse *p, void *out, void *stream);
@@ -679,7 +690,9 @@ typedef struct tode_solve_adjoint {
                                       the time range): a_y is then the cotangent of y0 and g_params includes the
                                       start's share.  The times count as constants in that part, so a caller that
                                       wants g_t_start / g_t_end passes 0 and does the start itself.  args->dt0 is not
-                                      read, only looked at: non-NULL says that the first step was the caller's */
+                                      read, only looked at: non-NULL says that the first step was the caller's.
+                                      2: as 1, and the cotangent of a first evaluation point at t_start, which is a copy of
+                                      y0 that no iteration wrote (adjoints.py:95-98), is added to a_y */
     void *scratch;                 /* tode_solve_backward_scratch_bytes(args) bytes (two int32 lists of [B,E]); looked at
                                       only when the two lists above are NULL and E > 0 */
     int64_t scratch_bytes;

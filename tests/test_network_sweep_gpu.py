@@ -8,6 +8,7 @@ import pytest
 import torch
 
 import torchode_amd as to
+from torchode_amd import _lib
 
 pytestmark = pytest.mark.gpu
 
@@ -236,3 +237,35 @@ def test_rows_that_do_not_fit_into_memory(monkeypatch):
     assert len(refused) == 1 and torch.equal(got[0], want[0])
     for a, b in zip(got, want):
         assert float((a.double() - b.double()).norm()) <= 2e-5 * float(b.double().norm())
+
+
+@pytest.mark.parametrize("batch, points, iterations, sign", [(1, 1, 1, 1.0), (300, 7, 5, 1.0), (300, 7, 5, -1.0), (5, 3, 200, 1.0), (257, 64, 0, -1.0)])
+def test_what_a_sweep_needs_of_its_record(batch, points, iterations, sign):
+    """tode_mlp_sweep_begin against torch operations: points on recorded times, in front of the start and beyond the end, a first
+    point at t_start, rejected steps (times that repeat), columns of a wider array as start and end, more points than
+    iterations and the other way round."""
+    g = torch.Generator().manual_seed(batch + points)
+    steps = torch.rand(iterations, batch, generator=g) * (torch.rand(iterations, batch, generator=g) < 0.7)
+    t = torch.cat([torch.randn(1, batch, generator=g), steps]).cumsum(0) if iterations else torch.randn(1, batch, generator=g)
+    at = torch.rand(batch, points, generator=g) * (t[-1] - t[0])[:, None] * 1.4 + t[0][:, None] - 0.1
+    on = torch.randint(0, iterations + 1, (batch, points), generator=g)
+    at = torch.where(torch.rand(batch, points, generator=g) < 0.4, torch.gather(t.T, 1, on), at).sort(dim=1).values
+    at[::2, 0] = torch.minimum(t[0], at[:, 0])[::2] if points > 1 else t[0][::2]
+    t, at = sign * t, sign * at
+    ends = torch.stack([t[0], t[0] + sign, t[0]], dim=1).contiguous().cuda()
+    accepted = torch.cat([torch.zeros(1, batch, dtype=torch.int32), (steps > 0).to(torch.int32).cumsum(0).to(torch.int32)])
+    later = sign * t[1:].T
+    hit = torch.searchsorted(later.contiguous(), (sign * at).contiguous(), out_int32=True) if iterations else torch.zeros(batch, points, dtype=torch.int32)
+    hit = torch.where(hit < iterations, hit, -1)
+    hit[:, 0] = torch.where(at[:, 0] == t[0], -1, hit[:, 0])
+    t_dev, at_dev, accepted_dev = t.contiguous().cuda(), at.contiguous().cuda(), accepted.cuda()
+    new = lambda *shape, dtype=torch.int32: torch.full(shape, 7, dtype=dtype, device="cuda")
+    hits, moved, t_start, t_end = new(batch, points), new(max(iterations, 1), batch), new(batch, dtype=torch.float32), new(batch, dtype=torch.float32)
+    rc = _lib.load().tode_mlp_sweep_begin(
+        batch, points, iterations, ends.data_ptr(), 3, ends.data_ptr() + 4, 3, at_dev.data_ptr(), t_dev.data_ptr(), accepted_dev.data_ptr(), hits.data_ptr(), moved.data_ptr(),
+        t_start.data_ptr(), t_end.data_ptr(), _lib.stream_of(ends),
+    )  # fmt: skip
+    assert rc == 0
+    assert torch.equal(hits.cpu(), hit) and torch.equal(t_start, ends[:, 0]) and torch.equal(t_end, ends[:, 1])
+    if iterations:
+        assert torch.equal(moved.cpu(), (accepted[1:] > accepted[:-1]).to(torch.int32))

@@ -13,7 +13,7 @@ import torch
 _HERE = os.path.dirname(os.path.abspath(__file__))
 LIB_PATH = os.path.join(_HERE, "libtorchode_amd.so")
 
-ABI_VERSION = 23
+ABI_VERSION = 24
 END_ONLY_MAX_BATCH = 2048 * 64  # TODE_END_ONLY_MAX_BATCH
 MLP_PACKED_SIZE = {"float32": 152 * 256, "bfloat16": 92 * 256}
 MLP_SUMS_SIZE, MLP_REVERSE_PACKED_SIZE = 64 * 256 + 256 + 256 + 64 * 256 + 64, 144 * 256  # TODE_MLP_*_SIZE
@@ -49,6 +49,7 @@ EXPORTS = (
     "tode_mlp_pack_weights_reverse",
     "tode_mlp_stages",
     "tode_mlp_stages_backward",
+    "tode_mlp_sweep_begin",
     "tode_mlp_start_backward",
     "tode_mlp_outer_products",
     "tode_mlp_weight_gradients",
@@ -220,7 +221,7 @@ class MlpReverse(C.Structure):
 class MlpStart(C.Structure):
     """struct tode_mlp_start"""
 
-    _fields_ = [(name, C.c_void_p) for name in ("t_end", "a_y", "a_k0", "a_dt")] + [("through_rule", C.c_int32)]
+    _fields_ = [(name, C.c_void_p) for name in ("t_end", "a_y", "a_k0", "a_dt")] + [("through_rule", C.c_int32), ("n_eval", C.c_int32), ("grad_ys", C.c_void_p), ("t_eval", C.c_void_p)]
 
 
 class StepAdjoint(C.Structure):
@@ -365,6 +366,8 @@ def load():
         lib.tode_mlp_stages_backward.argtypes = [C.POINTER(MlpReverse), C.c_void_p]
         lib.tode_mlp_outer_products.restype = C.c_int
         lib.tode_mlp_outer_products.argtypes = [C.POINTER(MlpReverse), C.c_int64, C.c_int32, C.c_void_p]
+        lib.tode_mlp_sweep_begin.restype = C.c_int
+        lib.tode_mlp_sweep_begin.argtypes = [C.c_int64, C.c_int32, C.c_int64, C.c_void_p, C.c_int64, C.c_void_p, C.c_int64] + [C.c_void_p] * 8
         lib.tode_mlp_start_backward.restype = C.c_int
         lib.tode_mlp_start_backward.argtypes = [C.POINTER(MlpReverse), C.POINTER(MlpStart), C.POINTER(Controller), C.c_void_p]
         lib.tode_mlp_weight_gradients.restype = C.c_int

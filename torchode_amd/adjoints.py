@@ -650,7 +650,8 @@ class AutoDiffAdjoint(nn.Module):
             # record in one kernel, with a record of a few entries more.  A batch that leaves that kernel's case, or
             # takes more iterations than the record holds, goes the long way below.
             solution = self._solve_recording_in_one_kernel(lib, a, ctrl, out, stream, record, dict(
-                B=B, E=E, F=F, dtype=dtype, ttype=ttype, dev=dev, ts=ts, ys=ys, has_dt0=dt0 is not None, with_stats=term.with_stats))  # fmt: skip
+                B=B, E=E, F=F, dtype=dtype, ttype=ttype, dev=dev, ts=ts, ys=ys, has_dt0=dt0 is not None, with_stats=term.with_stats,
+                ends_at_last_point=E > 1 and B > 0 and (t_end_ptr, t_end_stride) == (t_eval_ptr + (E - 1) * t_eval.element_size(), E)))  # fmt: skip
             if solution is not None or mlp:
                 return solution
         workspace = torch.empty(held["workspace_bytes"], dtype=torch.uint8, device=dev)
@@ -734,6 +735,8 @@ class AutoDiffAdjoint(nn.Module):
             return None
         L = fl[_lib.FLAG_MAX_ITERATIONS]
         record.iterations, record.arrays = L, fields
+        # (every sample has reached its t_end, where that is the last column of t_eval: its last point has been written)
+        record.wrote_points = q["ends_at_last_point"]
         self._remember_record_entries(shape, L + 1 + 4)
         stats: Dict[str, Any] = {}
         if q["with_stats"]:

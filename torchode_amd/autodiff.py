@@ -126,6 +126,7 @@ class LoopRecord:
         self.states: List[tuple] = []
         self.iterations = 0  # set by the forward pass when the loop has stopped
         self.arrays = None  # the same record as entry-major arrays, where the whole-solve kernel wrote it
+        self.wrote_points = False  # known without a look at the device: some iteration wrote an evaluation point
         self.flags = None  # that kernel's flag words, still on the device
 
     def snapshot(self, t, dt, y, k0, hist, ints):
@@ -161,6 +162,23 @@ class Replay:
     """One loop iteration (and the start of the loop) as differentiable torch operations."""
 
     def __init__(self, method, controller, term, args, problem: InitialValueProblem, through_control: bool, dt0=None):
+        self.method, self.controller = method, controller
+        self.dt0 = dt0
+        self.term, self.args = term, args
+        self.through_control = through_control
+        self.t_start, self.t_end, self.t_eval = problem.t_start, problem.t_end, problem.t_eval
+        self._direction = None
+
+    def __getattr__(self, name):
+        # the method's coefficients and the controller's settings are read when a sweep in torch operations (or the start of
+        # the loop in them) asks for the first of them: the kernels' sweeps have their own
+        if name.startswith("__") or "a" in self.__dict__:
+            raise AttributeError(name)
+        self._read_coefficients()
+        return getattr(self, name)
+
+    def _read_coefficients(self):
+        method, controller = self.method, self.controller
         if isinstance(method, Euler):  # (reference euler.py:29-56: one slope, no error estimate, linear dense output)
             self.a, self.c, self.b, self.b_err = [[]], [0.0], [1.0], None
             self.fsal = self.ssal = False
@@ -182,7 +200,7 @@ class Replay:
         c = controller.c_struct()
         self.pid = c.kind == _lib.CTRL_PID
         # fixed steps (reference step_size_controllers.py:116-167): every step accepted, the next step is dt0 again
-        self.fixed, self.dt0 = c.kind == _lib.CTRL_FIXED, dt0
+        self.fixed = c.kind == _lib.CTRL_FIXED
         self.atol, self.rtol = float(c.atol), float(c.rtol)
         self.safety, self.fmin, self.fmax = float(c.safety), float(c.factor_min), float(c.factor_max)
         self.dt_min = float(c.dt_min) if c.has_dt_min else None
@@ -192,10 +210,6 @@ class Replay:
             self.e1, self.e2, self.e3 = -(k_i + k_p + k_d), k_p + 2 * k_d, -k_d
         else:
             self.e1, self.e2, self.e3 = -1.0 / self.order, 0.0, 0.0
-        self.term, self.args = term, args
-        self.through_control = through_control
-        self.t_start, self.t_end, self.t_eval = problem.t_start, problem.t_end, problem.t_eval
-        self._direction = None
 
     @property
     def direction(self):
@@ -462,7 +476,7 @@ def reverse_sweep_whole(adjoint, replay: Replay, term, problem, dt0, record, gra
     # the start of the loop in the kernel too, unless a time wants a gradient (the kernel takes the times of that part
     # as constants): what comes back is then the cotangent of y0 itself
     through_start = getattr(adjoint, "backward_start_in_kernel", True) and not any(wants(x) for x in (replay.t_start, replay.t_end, replay.t_eval, dt0))
-    ad.through_start = int(through_start)
+    ad.through_start = 2 if through_start else 0
     if dt0 is not None:
         a.dt0 = dt0.data_ptr()  # (not read: it says that the first step was given)
     ad.scratch, ad.scratch_bytes = scratch.data_ptr(), scratch.numel()
@@ -573,9 +587,9 @@ class NetworkSweep:
         return splits
 
     def _at(self, state, evaluations):
-        """The state an iteration starts from, and room for that many evaluations' rows."""
+        """The state an iteration starts from (addresses of its arrays), and room for that many evaluations' rows."""
         a = self.args
-        a.t, a.dt, a.y, a.k0 = (state[k].data_ptr() for k in ("t", "dt", "y", "k0"))
+        a.t, a.dt, a.y, a.k0 = state["t"], state["dt"], state["y"], state["k0"]
         if self.sums is None:
             self.held = 0
         elif self.held + evaluations > self.room:
@@ -600,18 +614,19 @@ class NetworkSweep:
     def stages(self, state):
         y1 = self._at(state, 6)
         _lib.check(self.lib.tode_mlp_stages(self.ref, self.stream), "tode_mlp_stages")
-        return [state["k0"], *self.k.unbind(0)], y1
+        return y1
 
     def stages_backward(self, g_k, g_y, g_t, g_dt):
         a = self.args
         a.g_k, a.g_y, a.g_t, a.g_dt = g_k.data_ptr(), g_y.data_ptr(), g_t.data_ptr(), g_dt.data_ptr()
         _lib.check(self.lib.tode_mlp_stages_backward(self.ref, self.stream), "tode_mlp_stages_backward")
 
-    def start_backward(self, controller, state, t_end, a_y, a_k0, a_dt, g_y, through_rule):
-        """The start of the loop reversed; ``g_y`` becomes the cotangent of ``y0``."""
+    def start_backward(self, controller, state, t_end, a_y, a_k0, a_dt, g_y, through_rule, grad_ys, t_eval):
+        """The start of the loop reversed; ``g_y`` becomes the cotangent of ``y0``, that of a point at ``t_start`` included."""
         self._at(state, 2 if through_rule else 1)
         self.args.g_y = g_y.data_ptr()
-        start = _lib.MlpStart(t_end.data_ptr(), a_y.data_ptr(), a_k0.data_ptr(), a_dt.data_ptr(), int(bool(through_rule)))
+        start = _lib.MlpStart(t_end.data_ptr(), a_y.data_ptr(), a_k0.data_ptr(), a_dt.data_ptr(), int(bool(through_rule)),
+                              t_eval.shape[1], grad_ys.data_ptr(), t_eval.data_ptr())  # fmt: skip
         _lib.check(self.lib.tode_mlp_start_backward(self.ref, _lib.C.byref(start), controller, self.stream), "tode_mlp_start_backward")
 
     def weight_gradients(self, params):
@@ -629,7 +644,7 @@ class NetworkSweep:
         return list(torch.autograd.grad([x for x, _ in pairs], params, [g for _, g in pairs], allow_unused=True, retain_graph=True))
 
 
-def reverse_sweep_kernels(adjoint, replay: Replay, term, args, problem, dt0_given, dt0, states, hits, grad_ys, params, params_given, arrays=None):
+def reverse_sweep_kernels(adjoint, replay: Replay, term, args, problem, dt0_given, dt0, states, hits, grad_ys, params, params_given, arrays=None, iterations=0):
     """The iterations in reverse through the library's reverse kernels (tode_step_finish_backward,
     tode_step_stage_backward): per iteration the stage values are recomputed by the forward stage kernel and ``f``
     (six evaluations under grad mode, each a small graph of its own), the finish kernel is reversed in one launch,
@@ -647,20 +662,25 @@ def reverse_sweep_kernels(adjoint, replay: Replay, term, args, problem, dt0_give
     new = lambda *shape, dt=dtype: torch.empty(shape, dtype=dt, device=dev)
     zeros = lambda *shape, dt=dtype: torch.zeros(shape, dtype=dt, device=dev)
     contiguous = lambda x, dt: x.detach().to(dt).contiguous()
-    t_start, t_end = contiguous(replay.t_start, ttype), contiguous(replay.t_end, ttype)
     t_eval = None if replay.t_eval is None else contiguous(replay.t_eval, ttype)
+    if arrays is None:
+        t_start, t_end = contiguous(replay.t_start, ttype), contiguous(replay.t_end, ttype)
     fixed = ctrl.kind == _lib.CTRL_FIXED
     fixed_dt = contiguous(dt0, ttype) if fixed else None
-    n_iterations = len(states) - 1
+    n_iterations = len(states) - 1 if arrays is None else iterations
 
     # which iteration wrote which evaluation point
     hit_iteration = None
     if hits is None:  # (a record in arrays, of a batch in the whole-solve kernel's case: times that run in the solve's direction)
-        direction = replay.direction.detach().to(ttype)
-        new_times = (direction[None, :] * arrays["t"][1 : n_iterations + 1]).t().contiguous()  # [B, iterations], ascending
-        hit_iteration = torch.searchsorted(new_times, direction[:, None] * t_eval, out_int32=True)
-        hit_iteration = torch.where(hit_iteration < n_iterations, hit_iteration, -1)
-        hit_iteration[:, 0] = torch.where(t_eval[:, 0] == t_start, -1, hit_iteration[:, 0])
+        # (and the decisions of all iterations, and dense times: one launch)
+        given = [x.detach() if x.stride(0) >= 1 else x.detach().contiguous() for x in (replay.t_start, replay.t_end)]
+        t_start, t_end = new(B, dt=ttype), new(B, dt=ttype)
+        hit_iteration, moved_all = new(B, E, dt=torch.int32), new(max(n_iterations, 1), B, dt=torch.int32)
+        rc = lib.tode_mlp_sweep_begin(
+            B, E, n_iterations, given[0].data_ptr(), given[0].stride(0), given[1].data_ptr(), given[1].stride(0), t_eval.data_ptr(), arrays["t"].data_ptr(),
+            arrays["n_accepted"].data_ptr(), hit_iteration.data_ptr(), moved_all.data_ptr(), t_start.data_ptr(), t_end.data_ptr(), stream,
+        )  # fmt: skip
+        _lib.check(rc, "tode_mlp_sweep_begin")
     elif E > 0:
         hit_iteration = torch.full((B, E), -1, dtype=torch.int32, device=dev)
         for n, h in enumerate(hits):
@@ -675,17 +695,19 @@ def reverse_sweep_kernels(adjoint, replay: Replay, term, args, problem, dt0_give
     g_t_eval = zeros(B, E, dt=ttype) if (E > 0 and wants(replay.t_eval)) else None
     g_fixed_dt = zeros(B, dt=ttype) if (fixed and wants(dt0) and replay.through_control) else None
 
-    # a scratch state for the forward stage kernel (it reads t, dt, y and the k's, and writes ystage / tnode)
+    # a scratch state for the forward stage kernel (it reads t, dt, y and the k's, and writes ystage / tnode), which the
+    # network's sweep of a record in arrays does without
     st = _lib.StepState()
     st.dtype, st.time_dtype, st.method, st.n_features, st.n_eval = _lib.DTYPES[dtype], _lib.DTYPES[ttype], method.method_id, F, 0
     st.batch, st.max_steps = B, -1
-    clear = zeros(_lib.STEP_FLAG_WORDS, dt=torch.int32)
-    idle = zeros(B, dt=torch.int32)
-    st.flags = clear.data_ptr()
-    st.fixed_dt = _lib.ptr(fixed_dt)
-    st.t_start, st.t_end = t_start.data_ptr(), t_end.data_ptr()
-    for name in ("running", "cursor", "n_steps", "n_accepted", "status", "monotone"):
-        setattr(st, name, idle.data_ptr())
+    if arrays is None:
+        clear = zeros(_lib.STEP_FLAG_WORDS, dt=torch.int32)
+        idle = zeros(B, dt=torch.int32)
+        st.flags = clear.data_ptr()
+        st.fixed_dt = _lib.ptr(fixed_dt)
+        st.t_start, st.t_end = t_start.data_ptr(), t_end.data_ptr()
+        for name in ("running", "cursor", "n_steps", "n_accepted", "status", "monotone"):
+            setattr(st, name, idle.data_ptr())
     sref = _lib.C.byref(st)
 
     ad = _lib.StepAdjoint()
@@ -719,25 +741,25 @@ def reverse_sweep_kernels(adjoint, replay: Replay, term, args, problem, dt0_give
     grad_params = [None] * len(params)
     last = n_iterations - 1
     if arrays is not None:
-        # (the decisions of all iterations in two launches, and two sets of cotangents that take turns instead of copies)
-        moved_all = (arrays["n_accepted"][1:] > arrays["n_accepted"][:-1]).to(torch.int32)
-        running_all = (arrays["running"][1:] != 0).to(torch.int32)
+        # (two sets of cotangents that take turns instead of copies; entries of the record by their addresses)
         spare = (new(7, B, F), new(B, F), new(B, dt=ttype), new(B, dt=ttype), new(2, B))
         sets = [(g_k, g_y, g_t, g_dt, g_hist), spare]
+        slopes = [x.data_ptr() for x in network.k.unbind(0)]
+        places = [(k, x.data_ptr(), x.stride(0) * x.element_size()) for k, x in arrays.items()]
+        entry = lambda n: {k: at + n * size for k, at, size in places}
     for n in range(last, -1, -1):
         if arrays is not None:
-            now = states[n]
+            now, then = entry(n), entry(n + 1)
             g_k, g_y, g_t, g_dt, g_hist = sets[n % 2]
             for i in range(7):
                 ad.g_k[i] = g_k[i].data_ptr()
             ad.g_y, ad.g_t, ad.g_dt, ad.g_prev, ad.g_pprev = (x.data_ptr() for x in (g_y, g_t, g_dt, g_hist[0], g_hist[1]))
-            ks, y1 = network.stages(now)
+            y1 = network.stages(now)
             ad.iteration, ad.end_point = n, 0
-            ad.t, ad.dt, ad.y = (now[k].data_ptr() for k in ("t", "dt", "y"))
-            ad.ratio_prev, ad.ratio_pprev = now["prev"].data_ptr(), now["pprev"].data_ptr()
-            ad.moved, ad.running_next = moved_all[n].data_ptr(), running_all[n].data_ptr()
-            for i in range(7):
-                ad.k[i] = ks[i].data_ptr()
+            ad.t, ad.dt, ad.y, ad.ratio_prev, ad.ratio_pprev = now["t"], now["dt"], now["y"], now["prev"], now["pprev"]
+            ad.moved, ad.running_next = moved_all.data_ptr() + 4 * B * n, then["running"]
+            for i, at in enumerate([now["k0"], *slopes]):
+                ad.k[i] = at
             ad.y1 = y1.data_ptr()
             for name, value in zip(("a_y", "a_k0", "a_t", "a_dt", "a_prev", "a_pprev"), adj or [None] * 6):
                 setattr(ad, name, _lib.ptr(value))
@@ -758,7 +780,8 @@ def reverse_sweep_kernels(adjoint, replay: Replay, term, args, problem, dt0_give
         st.k[0] = now["k0"].data_ptr()
         ks, inputs = [now["k0"]], [None]
         if network is not None:
-            ks, y1 = network.stages(now)
+            y1 = network.stages({k: now[k].data_ptr() for k in ("t", "dt", "y", "k0")})
+            ks = [now["k0"], *network.k.unbind(0)]
         for i in range(1, 7 if network is None else 1):
             yi, ti = new(B, F), new(B, dt=ttype)
             st.ystage[i], st.tnode = yi.data_ptr(), ti.data_ptr()
@@ -807,7 +830,7 @@ def reverse_sweep_kernels(adjoint, replay: Replay, term, args, problem, dt0_give
         # the start of the loop in kernels as well (they take its times as constants): what comes back is the cotangent of y0
         a_y, a_k0, _, a_dt = adj[:4]
         g_y = sets[1][1]
-        network.start_backward(cref, states[0], t_end, a_y, a_k0, a_dt, g_y, dt0_given is None and replay.through_control)
+        network.start_backward(cref, entry(0), t_end, a_y, a_k0, a_dt, g_y, dt0_given is None and replay.through_control, grad_ys, t_eval)
         adj, through_start = (g_y, *adj[1:]), True
     if network is not None:
         grad_params = network.weight_gradients(params)
@@ -855,6 +878,7 @@ class SolveThroughLoop(torch.autograd.Function):
         ctx.times = InitialValueProblem(plain.y0, problem.t_start, problem.t_end, problem.t_eval)
         ctx.record, ctx.params = record, params
         ctx.n_initialized = solution.stats["n_initialized"]
+        ctx.set_materialize_grads(False)  # (no zeros made for the outputs that are whole numbers)
         stats = solution.stats
         n_f_evals = stats["n_f_evals"] if "n_f_evals" in stats else torch.empty(0, dtype=torch.long)
         outs = (solution.ys, solution.status, stats["n_steps"], stats["n_accepted"], stats["n_initialized"], n_f_evals)
@@ -864,10 +888,12 @@ class SolveThroughLoop(torch.autograd.Function):
     @staticmethod
     def backward(ctx, grad_ys, *unused):
         adjoint, problem, term, params = ctx.adjoint, ctx.problem, ctx.term, list(ctx.params)
+        if grad_ys is None:
+            grad_ys = torch.zeros((problem.batch_size, max(problem.n_evaluation_points, 1), problem.n_features), dtype=problem.data_dtype, device=problem.device)
         if ctx.record.flags is not None and ctx.record.flags.tolist()[_lib.FLAG_NEEDS_GENERAL]:
             raise RuntimeError("the record of the loop state was too short for the solve it was sized from")
         # (a second initialized point of some sample was written by an iteration: the usual case, told by one reduction)
-        some_iteration_wrote = problem.n_evaluation_points > 1 and int(ctx.n_initialized.max()) > 1
+        some_iteration_wrote = problem.n_evaluation_points > 1 and (ctx.record.wrote_points or int(ctx.n_initialized.max()) > 1)
         if problem.n_evaluation_points > 0 and not some_iteration_wrote and not ctx.record.any_point_written(problem):
             # No iteration wrote an evaluation point (every sample's points lie at t_start, or the batch stopped before
             # one was reached): ys is a copy of y0 where t_eval[:, 0] == t_start and nothing else, so in the reference's
@@ -914,22 +940,21 @@ class SolveThroughLoop(torch.autograd.Function):
             adj, grad_params = swept
         else:
             LAST_SWEEP = "kernels" if use_kernels else "torch"
-            states = ctx.record.trimmed(ctx.record.iterations)
             # (a record in arrays that no sweep of one kernel takes is the network's: the other long-row term leaves none)
             arrays = ctx.record.arrays if use_kernels and E > 0 and NetworkSweep.takes(adjoint, term, y0, problem.t_start) else None
+            states = ctx.record.trimmed(ctx.record.iterations) if arrays is None else None
             hits = simulate_hits(replay, states, E) if arrays is None else None
             if use_kernels:
                 adj, grad_params = reverse_sweep_kernels(
-                    adjoint, replay, term, args, problem, ctx.dt0, dt0, states, hits, grad_ys, params, list(ctx.params), arrays
+                    adjoint, replay, term, args, problem, ctx.dt0, dt0, states, hits, grad_ys, params, list(ctx.params), arrays, ctx.record.iterations
                 )
             else:
                 adj, grad_params = reverse_sweep_torch(replay, states, hits, grad_ys, params)
 
         # ---- the start of the loop: y = y0, k0 = f(t_start, y0), dt from the start step rule or dt0 ----
-        if adj.get("through_start"):  # (the whole-sweep kernel went through it as well)
-            grad_y0 = adj["y"]
-        else:
-            grad_y0 = SolveThroughLoop.start_backward(ctx, replay, adj, y0, dt0, params, grad_params)
+        if adj.get("through_start"):  # (the sweep's kernels went through it as well, and added the cotangent of a point at t_start)
+            return (None, None, None, None, None, adj["y"], *grad_params)
+        grad_y0 = SolveThroughLoop.start_backward(ctx, replay, adj, y0, dt0, params, grad_params)
         if E > 0:
             at_start = problem.t_eval[:, 0] == problem.t_start
             first = torch.where(at_start[:, None], grad_ys[:, 0], torch.zeros_like(grad_ys[:, 0]))

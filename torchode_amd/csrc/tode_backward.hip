@@ -32,7 +32,7 @@ template <typename T> struct WholeBackward {
     const int32_t *points_by_iteration, *iterations_sorted;
     int32_t *lists;  // room for both, for wavefronts with a row of times in no order (list_points)
     long long ts_stride, te_stride;  // t_start / t_end: sample b at element b * stride
-    int through_start;  // also carry the cotangents through the start of the loop (start_backward)
+    int through_start;  // also carry the cotangents through the start of the loop (start_backward); 2: and a point at t_start's
     int dt0_given;      // the first step was the caller's, not the start rule's
     int plain;          // tolerances and exponents in the ranges of the short forms
 };
@@ -633,6 +633,10 @@ __global__ void __launch_bounds__(64) whole_backward_kernel(const WholeBackward<
     // (no iteration: nothing flows back through the loop, and the cotangents are still the zeros they started as)
     if (w.through_start)  // (`here` is the record's first entry now: t_start, y0, f(t_start, y0))
         start_backward<T, CTRL, Term>(cp, rhs, w.through_control && !w.dt0_given, ts, te, here.y, here.k0, a_y, a_k0, a_dt, gpar);
+    if (w.through_start == 2 && E > 0 && t_eval[0] == ts) {
+#pragma unroll
+        for (int f = 0; f < F; ++f) a_y[f] += grad_ys[f];
+    }
 #pragma unroll
     for (int f = 0; f < F; ++f) w.a_y[g * F + f] = a_y[f], w.a_k0[g * F + f] = a_k0[f];
     w.a_t[g] = a_t, w.a_dt[g] = a_dt, w.a_prev[g] = a_prev, w.a_pprev[g] = a_pprev;

@@ -417,8 +417,34 @@ __global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(1, 1))
         product(0, g_k0);
 #pragma unroll
         for (int r = 0; r < 4; ++r) g_y0[r] += gi[r];
+        if (st.grad_ys && ((const float *)st.t_eval)[b * st.n_eval] == ((const float *)p.t)[b]) {
+            const float *first = (const float *)st.grad_ys + b * st.n_eval * FR;
+#pragma unroll
+            for (int r = 0; r < 4; ++r) g_y0[r] += f0 + r < FR ? first[f0 + r] : 0.0f;
+        }
         if (live) mlp_put((float *)p.g_y + b * FR, f0, FR, g_y0);
     }
+}
+
+// Ahead of a sweep (tode_mlp_sweep_begin): a point's iteration by binary search over its sample's recorded times, one thread per
+// point; a sample's move and its dense times by further uses of the same threads.  A few microseconds, where the same in torch
+// operations took fifteen launches.
+__global__ void __launch_bounds__(256) mlp_sweep_begin_kernel(long long B, int E, long long L, const float *t_start, long long ts_stride, const float *t_end, long long te_stride,
+                                                              const float *t_eval, const float *rec_t, const int32_t *rec_n_accepted, int32_t *hit_iteration, int32_t *moved,
+                                                              float *t_start_out, float *t_end_out) {
+    const long long i = (long long)blockIdx.x * 256 + threadIdx.x;
+    if (i < B) t_start_out[i] = t_start[i * ts_stride], t_end_out[i] = t_end[i * te_stride];
+    if (i < L * B) moved[i] = rec_n_accepted[i + B] > rec_n_accepted[i] ? 1 : 0;
+    if (i >= B * E) return;
+    const long long b = i / E;
+    const float ts = t_start[b * ts_stride], dir = t_end[b * te_stride] > ts ? 1.0f : -1.0f, at = t_eval[i], v = dir * at;
+    long long lo = 0, hi = L;
+    while (lo < hi) {
+        const long long mid = (lo + hi) / 2;
+        if (dir * rec_t[(mid + 1) * B + b] >= v) hi = mid;
+        else lo = mid + 1;
+    }
+    hit_iteration[i] = lo < L && !(i == b * E && at == ts) ? (int32_t)lo : -1;
 }
 
 // The operands of four rows (k of the matrix instructions) for one wavefront: lane (q, c) holds row 4 step + q.  Rows past
@@ -598,6 +624,7 @@ int tode_mlp_start_backward(const tode_mlp_reverse *p, const tode_mlp_start *sta
     const int rc = check_mlp_reverse(p);
     if (rc || p->batch == 0) return rc;
     if (!start || !c || !start->t_end || !start->a_y || !start->a_k0 || !start->a_dt) return fail(TODE_E_INVALID, "null pointer");
+    if (start->grad_ys && (!start->t_eval || start->n_eval < 1)) return fail(TODE_E_INVALID, "grad_ys without evaluation points");
     if (c->kind != TODE_CTRL_INTEGRAL && c->kind != TODE_CTRL_PID) return fail(TODE_E_INVALID, "unknown controller kind %d", c->kind);
     const CtrlParams<float> cp = make_ctrl<float>(*c);
     const bool integral = c->kind == TODE_CTRL_INTEGRAL;
@@ -611,6 +638,21 @@ int tode_mlp_start_backward(const tode_mlp_reverse *p, const tode_mlp_start *sta
         hipLaunchKernelGGL((mlp_start_backward_kernel<false>), grid_back, dim3(256), 0, s, *p, *start, cp, integral);
     }
     return check_hip(hipGetLastError(), "tode_mlp_start_backward");
+}
+
+int tode_mlp_sweep_begin(int64_t batch, int32_t n_eval, int64_t iterations, const void *t_start, int64_t t_start_stride, const void *t_end, int64_t t_end_stride,
+                         const void *t_eval, const void *rec_t, const int32_t *rec_n_accepted, int32_t *hit_iteration, int32_t *moved, void *t_start_out, void *t_end_out,
+                         void *stream) {
+    using namespace tode;
+    if (batch < 0 || n_eval < 1 || iterations < 0 || t_start_stride < 1 || t_end_stride < 1) return fail(TODE_E_INVALID, "bad sizes");
+    if (batch == 0) return TODE_OK;
+    if (!t_start || !t_end || !t_eval || !rec_t || !rec_n_accepted || !hit_iteration || (iterations > 0 && !moved) || !t_start_out || !t_end_out) return fail(TODE_E_INVALID, "null pointer");
+    const long long threads = batch * (n_eval > iterations ? n_eval : iterations);
+    if ((threads + 255) / 256 > 2147483647) return fail(TODE_E_UNSUPPORTED, "batch too large");
+    hipLaunchKernelGGL(mlp_sweep_begin_kernel, dim3((unsigned)((threads + 255) / 256)), dim3(256), 0, (hipStream_t)stream, (long long)batch, n_eval, (long long)iterations,
+                       (const float *)t_start, (long long)t_start_stride, (const float *)t_end, (long long)t_end_stride, (const float *)t_eval, (const float *)rec_t, rec_n_accepted,
+                       hit_iteration, moved, (float *)t_start_out, (float *)t_end_out);
+    return check_hip(hipGetLastError(), "tode_mlp_sweep_begin");
 }
 
 int tode_mlp_outer_products(const tode_mlp_reverse *p, int64_t rows, int32_t accumulate, void *stream) {
