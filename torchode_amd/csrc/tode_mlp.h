@@ -130,14 +130,48 @@ __device__ __forceinline__ int block_or(MlpShared &sh, int &vslot, int bits) {
 // and underflows to 0 exactly where tanh saturates, so no range checks are needed.
 __device__ __forceinline__ float mlp_tanh(float x) {
     const float e = __builtin_amdgcn_exp2f(x * 2.8853900817779268f);  // 2 / ln 2
-    return 1.0f - 2.0f * __builtin_amdgcn_rcpf(e + 1.0f);
+    return fma_(-2.0f, __builtin_amdgcn_rcpf(e + 1.0f), 1.0f);  // (2 r is exact)
+}
+
+// tanh(x) to an ulp and a half: up to 1 an odd polynomial of degree 15 (fitted to the smallest relative error, 5e-9), beyond it
+// the form above; 0.31 ulp in the mean over normal arguments.  No branch, so that the compiler can place it between matrix
+// instructions: the math library's tanhf branches on |x|, and each of its sixteen values of an evaluation stood by itself between
+// the two products.
+__device__ __forceinline__ float mlp_tanh_accurate(float x) {
+    const float e = __builtin_amdgcn_exp2f(__builtin_fabsf(x) * 2.8853900817779268f);
+    const float far = __builtin_copysignf(fma_(-2.0f, __builtin_amdgcn_rcpf(e + 1.0f), 1.0f), x);
+    const float z = x * x;
+    float p = -0x1.77dcb2p-12f;
+    p = fma_(p, z, 0x1.2da4c0p-9f);
+    p = fma_(p, z, -0x1.0460b0p-7f);
+    p = fma_(p, z, 0x1.60098cp-6f);
+    p = fma_(p, z, -0x1.b96222p-5f);
+    p = fma_(p, z, 0x1.110be2p-3f);
+    p = fma_(p, z, -0x1.55553cp-2f);
+    const float near = fma_(x * z, p, x);
+    return __builtin_fabsf(x) < 1.0f ? near : far;  // (not a number: e is, and far with it)
+}
+
+// One of sixteen groups of four matrix instructions with the VALUES instructions of a tanh spread between them: a wavefront
+// issues in order, and a group's worth of tanh behind the fourth instruction leaves the matrix cores idle for most of it.
+template <int VALUES> __device__ __forceinline__ void mlp_interleave() {
+#pragma unroll
+    for (int n = 0; n < 4; ++n) {
+        __builtin_amdgcn_sched_group_barrier(0x8, 1, 0);  // matrix instruction
+        __builtin_amdgcn_sched_group_barrier(0x2 | 0x400, (VALUES + 3) / 4, 0);  // vector instructions
+    }
+    __builtin_amdgcn_sched_barrier(0);
 }
 
 // out[r] = f(tn, yi)[16w + 4q + r] for the lane's sample.
-// LIBRARY_TANH: the math library's tanh (within an ulp or two; the gradient's kernels, whose f stands where torch's was)
-// instead of mlp_tanh.  hidden: where not null, the sample's row of 256 hidden activations in memory.
-template <bool LIBRARY_TANH = false>
+// ACCURATE_TANH: for the gradient's kernels, whose f stands where torch's was.  hidden: where not null, the sample's row of 256
+// hidden activations in memory.
+// The order of the matrix instructions hides tanh behind them: layer 1 for two of the four tiles of hidden units, then for the
+// other two while the first two go through tanh, then layer 2 over the first two while the other two do (each sum in the
+// order of its inputs all the same).  MEASURED_B
+template <bool ACCURATE_TANH = false>
 __device__ __forceinline__ void mlp_rhs(MlpShared &sh, const MlpWeights &W, float tn, const float (&yi)[4], float (&out)[4], float *hidden = nullptr) {
+    constexpr int TANH = ACCURATE_TANH ? 17 : 6;
     const int lane = threadIdx.x & 63, w = threadIdx.x >> 6, q = lane >> 4, c = lane & 15;
     *reinterpret_cast<float4 *>(sh.x + c * MLP_XS + 16 * w + 4 * q) = make_float4(yi[0], yi[1], yi[2], yi[3]);
     if (w == 0 && q == 0) sh.x[c * MLP_XS + MLP_F] = tn;
@@ -154,32 +188,45 @@ __device__ __forceinline__ void mlp_rhs(MlpShared &sh, const MlpWeights &W, floa
         a1[16] = sh.x[c * MLP_XS + MLP_F + q];
     }
     asm volatile("" ::: "memory");
-    mfma_acc h[4];
+    const auto hidden_unit = [](float x) { return ACCURATE_TANH ? mlp_tanh_accurate(x) : mlp_tanh(x); };
+    mfma_acc h[4], acc[4];
 #pragma unroll
-    for (int tile = 0; tile < 4; ++tile) h[tile] = {W.b1[tile][0], W.b1[tile][1], W.b1[tile][2], W.b1[tile][3]};
+    for (int tile = 0; tile < 4; ++tile) h[tile] = {W.b1[tile][0], W.b1[tile][1], W.b1[tile][2], W.b1[tile][3]}, acc[tile] = {0.0f, 0.0f, 0.0f, 0.0f};
 #pragma unroll
     for (int kk = 0; kk < 17; ++kk) {
 #pragma unroll
-        for (int tile = 0; tile < 4; ++tile) h[tile] = __builtin_amdgcn_mfma_f32_16x16x4f32(W.w1[kk][tile], a1[kk], h[tile], 0, 0, 0);
+        for (int tile = 0; tile < 2; ++tile) h[tile] = __builtin_amdgcn_mfma_f32_16x16x4f32(W.w1[kk][tile], a1[kk], h[tile], 0, 0, 0);
     }
 #pragma unroll
-    for (int tile = 0; tile < 4; ++tile)
+    for (int tile = 2; tile < 4; ++tile) h[tile] = __builtin_amdgcn_mfma_f32_16x16x4f32(W.w1[0][tile], a1[0], h[tile], 0, 0, 0);
+    __builtin_amdgcn_sched_barrier(0);
 #pragma unroll
-        for (int r = 0; r < 4; ++r) h[tile][r] = LIBRARY_TANH ? tanhf(h[tile][r]) : mlp_tanh(h[tile][r]);
+    for (int n = 0; n < 8; ++n) {
+#pragma unroll
+        for (int kk = 1 + 2 * n; kk < 3 + 2 * n; ++kk)
+#pragma unroll
+            for (int tile = 2; tile < 4; ++tile) h[tile] = __builtin_amdgcn_mfma_f32_16x16x4f32(W.w1[kk][tile], a1[kk], h[tile], 0, 0, 0);
+        float unit = hidden_unit(h[n / 4][n % 4]);
+        if (n < 7) asm volatile("" : "+v"(unit), "+v"(a1[3 + 2 * n]), "+v"(a1[4 + 2 * n]));  // (the next group behind this value)
+        h[n / 4][n % 4] = unit;
+        mlp_interleave<TANH>();
+    }
+#pragma unroll
+    for (int n = 0; n < 8; ++n) {
+#pragma unroll
+        for (int ft = 0; ft < 4; ++ft) acc[ft] = __builtin_amdgcn_mfma_f32_16x16x4f32(W.w2[ft][n / 4][n % 4], h[n / 4][n % 4], acc[ft], 0, 0, 0);
+        h[2 + n / 4][n % 4] = hidden_unit(h[2 + n / 4][n % 4]);
+        mlp_interleave<TANH>();
+    }
     if (hidden) {
 #pragma unroll
         for (int tile = 0; tile < 4; ++tile)
             *reinterpret_cast<float4 *>(hidden + 64 * w + 16 * tile + 4 * q) = make_float4(h[tile][0], h[tile][1], h[tile][2], h[tile][3]);
     }
-    mfma_acc acc[4];
 #pragma unroll
-    for (int ft = 0; ft < 4; ++ft) acc[ft] = {0.0f, 0.0f, 0.0f, 0.0f};
+    for (int n = 8; n < 16; ++n)
 #pragma unroll
-    for (int tile = 0; tile < 4; ++tile)
-#pragma unroll
-        for (int r = 0; r < 4; ++r)
-#pragma unroll
-            for (int ft = 0; ft < 4; ++ft) acc[ft] = __builtin_amdgcn_mfma_f32_16x16x4f32(W.w2[ft][tile][r], h[tile][r], acc[ft], 0, 0, 0);
+        for (int ft = 0; ft < 4; ++ft) acc[ft] = __builtin_amdgcn_mfma_f32_16x16x4f32(W.w2[ft][n / 4][n % 4], h[n / 4][n % 4], acc[ft], 0, 0, 0);
 #pragma unroll
     for (int ft = 0; ft < 4; ++ft) *reinterpret_cast<float4 *>(sh.part[ft][w][lane]) = make_float4(acc[ft][0], acc[ft][1], acc[ft][2], acc[ft][3]);
     lds_barrier();

@@ -157,33 +157,50 @@ __device__ __forceinline__ void mlp_vjp(MlpReverseShared &sh, const MlpReverseWe
             g[4 * j] = v.x, g[4 * j + 1] = v.y, g[4 * j + 2] = v.z, g[4 * j + 3] = v.w;
         }
     }
-    mfma_acc d[4];
+    mfma_acc d[4], acc[4];
 #pragma unroll
-    for (int u = 0; u < 4; ++u) d[u] = {0.0f, 0.0f, 0.0f, 0.0f};
+    for (int u = 0; u < 4; ++u) d[u] = {0.0f, 0.0f, 0.0f, 0.0f}, acc[u] = {0.0f, 0.0f, 0.0f, 0.0f};
+    gt = 0;
+    const auto in_front_of_tanh = [&](int n) {
+        const int u = n / 4, r = n % 4;
+        const float hv = r == 0 ? h[u].x : r == 1 ? h[u].y : r == 2 ? h[u].z : h[u].w;
+        const float v = d[u][r] * fma_(-hv, hv, 1.0f);
+        gt = fma_(W.wt[n], v, gt);
+        return v;
+    };
+    // (in the order of mlp_rhs: two tiles of hidden units at a time, the first two's way through tanh's derivative behind the
+    // other two's products and theirs behind the first two's part of the second product)
 #pragma unroll
     for (int kk = 0; kk < 16; ++kk)
 #pragma unroll
-        for (int u = 0; u < 4; ++u) d[u] = __builtin_amdgcn_mfma_f32_16x16x4f32(W.w2t[kk][u], g[kk], d[u], 0, 0, 0);
-    gt = 0;
+        for (int u = 0; u < 2; ++u) d[u] = __builtin_amdgcn_mfma_f32_16x16x4f32(W.w2t[kk][u], g[kk], d[u], 0, 0, 0);
+    __builtin_amdgcn_sched_barrier(0);
 #pragma unroll
-    for (int u = 0; u < 4; ++u) {
-        const float hv[4] = {h[u].x, h[u].y, h[u].z, h[u].w};
+    for (int n = 0; n < 8; ++n) {
 #pragma unroll
-        for (int r = 0; r < 4; ++r) {
-            d[u][r] = d[u][r] * fma_(-hv[r], hv[r], 1.0f);
-            gt = fma_(W.wt[4 * u + r], d[u][r], gt);
-        }
-        if (cotangents) *reinterpret_cast<float4 *>(cotangents + 64 * w + 16 * u + 4 * q) = make_float4(d[u][0], d[u][1], d[u][2], d[u][3]);
+        for (int kk = 2 * n; kk < 2 * n + 2; ++kk)
+#pragma unroll
+            for (int u = 2; u < 4; ++u) d[u] = __builtin_amdgcn_mfma_f32_16x16x4f32(W.w2t[kk][u], g[kk], d[u], 0, 0, 0);
+        float v = in_front_of_tanh(n);
+        if (n < 7) asm volatile("" : "+v"(v), "+v"(g[2 * n + 2]), "+v"(g[2 * n + 3]));  // (the next group behind this value)
+        d[n / 4][n % 4] = v;
+        mlp_interleave<3>();
     }
-    mfma_acc acc[4];
 #pragma unroll
-    for (int it = 0; it < 4; ++it) acc[it] = {0.0f, 0.0f, 0.0f, 0.0f};
+    for (int n = 0; n < 8; ++n) {
 #pragma unroll
-    for (int u = 0; u < 4; ++u)
+        for (int it = 0; it < 4; ++it) acc[it] = __builtin_amdgcn_mfma_f32_16x16x4f32(W.w1t[it][n], d[n / 4][n % 4], acc[it], 0, 0, 0);
+        d[2 + n / 4][n % 4] = in_front_of_tanh(8 + n);
+        mlp_interleave<3>();
+    }
+    if (cotangents) {
 #pragma unroll
-        for (int r = 0; r < 4; ++r)
+        for (int u = 0; u < 4; ++u) *reinterpret_cast<float4 *>(cotangents + 64 * w + 16 * u + 4 * q) = make_float4(d[u][0], d[u][1], d[u][2], d[u][3]);
+    }
 #pragma unroll
-            for (int it = 0; it < 4; ++it) acc[it] = __builtin_amdgcn_mfma_f32_16x16x4f32(W.w1t[it][4 * u + r], d[u][r], acc[it], 0, 0, 0);
+    for (int n = 8; n < 16; ++n)
+#pragma unroll
+        for (int it = 0; it < 4; ++it) acc[it] = __builtin_amdgcn_mfma_f32_16x16x4f32(W.w1t[it][n], d[n / 4][n % 4], acc[it], 0, 0, 0);
 #pragma unroll
     for (int it = 0; it < 4; ++it) *reinterpret_cast<float4 *>(sh.part[it][w][lane]) = make_float4(acc[it][0], acc[it][1], acc[it][2], acc[it][3]);
     lds_barrier();
