@@ -25,6 +25,7 @@ struct __align__(16) MlpShared {
     float part[4][4][64][4];        // [output tile][wavefront it comes from][lane][4 features]
     float red[2][4][MLP_TILE][2];   // per-wavefront partial sums of up to two per-sample reductions
     int vote[2][4];                 // per-wavefront bits of the workgroup-wide "or"
+    float b1[MLP_H], b2[MLP_F];     // (bfloat16 variant) the biases
 };
 
 struct MlpWeights {
@@ -39,11 +40,16 @@ struct MlpWeights {
 typedef __bf16 mlp_bf16x4 __attribute__((ext_vector_type(4)));
 typedef unsigned mlp_u32x2 __attribute__((ext_vector_type(2)));
 
+// Four values rounded to nearest even, two by one instruction.  Put together as words: a vector of four bfloat16 that goes to a
+// matrix instruction the compiler makes of four conversions and two permutations.
+typedef __bf16 mlp_bf16x2 __attribute__((ext_vector_type(2)));
+typedef float mlp_f32x2 __attribute__((ext_vector_type(2)));
+__device__ __forceinline__ unsigned mlp_round(float a, float b) { return __builtin_bit_cast(unsigned, __builtin_convertvector(mlp_f32x2{a, b}, mlp_bf16x2)); }
+__device__ __forceinline__ mlp_bf16x4 mlp_round(float a, float b, float c, float d) { return __builtin_bit_cast(mlp_bf16x4, mlp_u32x2{mlp_round(a, b), mlp_round(c, d)}); }
+
 struct MlpWeightsBf16 {
     mlp_bf16x4 w1[5][4];  // W1[64w + 16 tile + c][16 ks + 4q + j], inputs 65..79 are zero
-    float b1[4][4];
     mlp_bf16x4 w2[4][4];  // [ft][tile]: W2[16 ft + c][64w + 16 tile + 4q + j]
-    float b2[4];
 };
 
 // Which input column lane group q feeds at k-step kk of the first layer: 16 features each for
@@ -168,7 +174,7 @@ template <int VALUES> __device__ __forceinline__ void mlp_interleave() {
 // hidden activations in memory.
 // The order of the matrix instructions hides tanh behind them: layer 1 for two of the four tiles of hidden units, then for the
 // other two while the first two go through tanh, then layer 2 over the first two while the other two do (each sum in the
-// order of its inputs all the same).  MEASURED_B
+// order of its inputs all the same).
 template <bool ACCURATE_TANH = false>
 __device__ __forceinline__ void mlp_rhs(MlpShared &sh, const MlpWeights &W, float tn, const float (&yi)[4], float (&out)[4], float *hidden = nullptr) {
     constexpr int TANH = ACCURATE_TANH ? 17 : 6;
@@ -250,13 +256,13 @@ __device__ __forceinline__ void mlp_rhs(MlpShared &sh, const MlpWeightsBf16 &W, 
 #pragma unroll
         for (int ks = 0; ks < 5; ++ks) {
             const float4 v = *reinterpret_cast<const float4 *>(row + 16 * ks);
-            a1[ks] = {(__bf16)v.x, (__bf16)v.y, (__bf16)v.z, (__bf16)v.w};
+            a1[ks] = mlp_round(v.x, v.y, v.z, v.w);
         }
     }
-    asm volatile("" ::: "memory");
     mfma_acc h[4];
 #pragma unroll
-    for (int tile = 0; tile < 4; ++tile) h[tile] = {W.b1[tile][0], W.b1[tile][1], W.b1[tile][2], W.b1[tile][3]};
+    for (int tile = 0; tile < 4; ++tile) h[tile] = *reinterpret_cast<const mfma_acc *>(sh.b1 + 64 * w + 16 * tile + 4 * q);
+    asm volatile("" ::: "memory");
 #pragma unroll
     for (int ks = 0; ks < 5; ++ks) {
 #pragma unroll
@@ -265,7 +271,7 @@ __device__ __forceinline__ void mlp_rhs(MlpShared &sh, const MlpWeightsBf16 &W, 
     mlp_bf16x4 hb[4];
 #pragma unroll
     for (int tile = 0; tile < 4; ++tile)
-        hb[tile] = {(__bf16)mlp_tanh(h[tile][0]), (__bf16)mlp_tanh(h[tile][1]), (__bf16)mlp_tanh(h[tile][2]), (__bf16)mlp_tanh(h[tile][3])};
+        hb[tile] = mlp_round(mlp_tanh(h[tile][0]), mlp_tanh(h[tile][1]), mlp_tanh(h[tile][2]), mlp_tanh(h[tile][3]));
     mfma_acc acc[4];
 #pragma unroll
     for (int ft = 0; ft < 4; ++ft) acc[ft] = {0.0f, 0.0f, 0.0f, 0.0f};
@@ -279,10 +285,11 @@ __device__ __forceinline__ void mlp_rhs(MlpShared &sh, const MlpWeightsBf16 &W, 
     float4 s[4];
 #pragma unroll
     for (int from = 0; from < 4; ++from) s[from] = *reinterpret_cast<const float4 *>(sh.part[w][from][lane]);
-    out[0] = ((s[0].x + s[1].x) + (s[2].x + s[3].x)) + W.b2[0];
-    out[1] = ((s[0].y + s[1].y) + (s[2].y + s[3].y)) + W.b2[1];
-    out[2] = ((s[0].z + s[1].z) + (s[2].z + s[3].z)) + W.b2[2];
-    out[3] = ((s[0].w + s[1].w) + (s[2].w + s[3].w)) + W.b2[3];
+    const float4 b2 = *reinterpret_cast<const float4 *>(sh.b2 + 16 * w + 4 * q);
+    out[0] = ((s[0].x + s[1].x) + (s[2].x + s[3].x)) + b2.x;
+    out[1] = ((s[0].y + s[1].y) + (s[2].y + s[3].y)) + b2.y;
+    out[2] = ((s[0].z + s[1].z) + (s[2].z + s[3].z)) + b2.z;
+    out[3] = ((s[0].w + s[1].w) + (s[2].w + s[3].w)) + b2.w;
 }
 
 // Packed weights (tode_mlp_pack_weights) into the registers of thread tid.
@@ -306,20 +313,28 @@ __device__ __forceinline__ void mlp_load(MlpWeights &W, const float *packed, int
 
 __device__ __forceinline__ void mlp_load(MlpWeightsBf16 &W, const float *packed, int tid) {
     const uint4 *src = reinterpret_cast<const uint4 *>(packed) + tid;
-    unsigned v[MLP_REGS_BF16];
 #pragma unroll
-    for (int i = 0; i < MLP_REGS_BF16 / 4; ++i) {
+    for (int i = 0; i < 10; ++i) {
         const uint4 u = src[i * 256];
-        v[4 * i] = u.x, v[4 * i + 1] = u.y, v[4 * i + 2] = u.z, v[4 * i + 3] = u.w;
+        W.w1[i / 2][2 * (i % 2)] = __builtin_bit_cast(mlp_bf16x4, (mlp_u32x2){u.x, u.y});
+        W.w1[i / 2][2 * (i % 2) + 1] = __builtin_bit_cast(mlp_bf16x4, (mlp_u32x2){u.z, u.w});
     }
 #pragma unroll
-    for (int j = 0; j < 20; ++j) W.w1[j / 4][j % 4] = __builtin_bit_cast(mlp_bf16x4, (mlp_u32x2){v[2 * j], v[2 * j + 1]});
+    for (int i = 0; i < 8; ++i) {
+        const uint4 u = src[(14 + i) * 256];
+        W.w2[i / 2][2 * (i % 2)] = __builtin_bit_cast(mlp_bf16x4, (mlp_u32x2){u.x, u.y});
+        W.w2[i / 2][2 * (i % 2) + 1] = __builtin_bit_cast(mlp_bf16x4, (mlp_u32x2){u.z, u.w});
+    }
+}
+
+// The bfloat16 variant's biases to LDS: b1[64w + 16 tile + 4q ..] from one lane of the sixteen that hold it, b2[16w + 4q ..] likewise.
+__device__ __forceinline__ void mlp_load_biases(MlpShared &sh, const float *packed, int tid) {
+    const int lane = tid & 63, w = tid >> 6, q = lane >> 4;
+    if ((lane & 15) != 0) return;
+    const float4 *src = reinterpret_cast<const float4 *>(packed) + tid;
 #pragma unroll
-    for (int j = 0; j < 16; ++j) W.b1[j / 4][j % 4] = __uint_as_float(v[40 + j]);
-#pragma unroll
-    for (int j = 0; j < 16; ++j) W.w2[j / 4][j % 4] = __builtin_bit_cast(mlp_bf16x4, (mlp_u32x2){v[56 + 2 * j], v[56 + 2 * j + 1]});
-#pragma unroll
-    for (int j = 0; j < 4; ++j) W.b2[j] = __uint_as_float(v[88 + j]);
+    for (int tile = 0; tile < 4; ++tile) *reinterpret_cast<float4 *>(sh.b1 + 64 * w + 16 * tile + 4 * q) = src[(10 + tile) * 256];
+    *reinterpret_cast<float4 *>(sh.b2 + 16 * w + 4 * q) = src[22 * 256];
 }
 
 // Per-sample sums over the 64 features of two quantities at once: the lane's four features, the

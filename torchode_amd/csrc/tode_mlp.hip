@@ -61,8 +61,10 @@ static __global__ void mlp_pack_kernel(const float *raw, float *packed, int H, i
 // short raises TODE_FLAG_NEEDS_GENERAL (TODE_FLAG_MAX_ITERATIONS says how long it has to be).  For gradients: f there takes the
 // math library's tanh, since it stands where torch's evaluations of the network stood.  Network of 64 and 256 at B = 4096:
 // solve and record in 0.105 ms, where the per-step kernels around torch's products took 2.6 ms.
+template <typename Weights> constexpr int mlp_wavefronts = std::is_same<Weights, MlpWeightsBf16>::value ? 3 : 2;  // per SIMD
+
 template <int METHOD, int CTRL, typename Weights, bool FULL, bool RECORD>
-__global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2, 2))) solve_mlp_kernel(const SolveParams<float> p, const float *packed, const MlpOut o) {
+__global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(mlp_wavefronts<Weights>, mlp_wavefronts<Weights>))) solve_mlp_kernel(const SolveParams<float> p, const float *packed, const MlpOut o) {
     using T = float;
     using Tab = typename std::conditional<METHOD == 1, Tsit5Tab, Dopri5Tab>::type;
     constexpr int F = MLP_F;
@@ -113,6 +115,7 @@ __global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2, 2))
     // ---- weights into registers ----
     Weights W;
     mlp_load(W, packed, tid);
+    if constexpr (std::is_same<Weights, MlpWeightsBf16>::value) mlp_load_biases(sh, packed, tid);
     for (int i = tid; i < MLP_TILE * MLP_XS; i += 256) sh.x[i] = 0.0f;  // also the zero columns from 65 on
     for (int i = tid; i < rows * E; i += 256) te_s[i] = end_only ? p.t_end[(b0 + i) * p.te_stride] : p.t_eval[b0 * E + i];
     __syncthreads();
