@@ -12,10 +12,10 @@
 //   mlp_weight_gradient_sum_kernel  the splits' sums added in order, once per sweep.
 //
 // What bounds them, network of 64 and 256 at B = 4096 (one workgroup per compute unit, one wavefront per SIMD): six
-// evaluations forward 32 us, back 30 us, of which the matrix cores are busy 10.6 and 10.2 us -- the rest are the round trips
-// through LDS between two products, tanh, the stage sums and 150 KB of weights loaded per workgroup; the outer products of 20
-// evaluations 91 us (35 us of matrix instructions, 200 MB of rows at 2.2 TB/s; four calls of an iteration each with one step
-// of loads ahead took 215 us).  A solve and its backward pass: 9.75 ms through autograd, 1.27 ms.
+// evaluations forward 28 us, back 29 us, of which the matrix cores are busy 10.6 and 10.2 us -- the rest are the round trips
+// through LDS between two products, the stage sums and 150 KB of weights loaded per workgroup; the outer products of 20
+// evaluations 69 us (39 us of matrix instructions, 200 MB of rows at 2.9 TB/s).  A solve and its backward pass: 9.75 ms through
+// autograd, 0.80 ms.
 //
 // All products are on v_mfma_f32_16x16x4_f32.  For the vector-Jacobian product the weights are packed a second time,
 // transposed (tode_mlp_pack_weights_reverse), so that the same two facts hold as in the forward kernel: every lane keeps its
@@ -464,38 +464,48 @@ __global__ void __launch_bounds__(256) mlp_sweep_begin_kernel(long long B, int E
     hit_iteration[i] = lo < L && !(i == b * E && at == ts) ? (int32_t)lo : -1;
 }
 
-// The operands of four rows (k of the matrix instructions) for one wavefront: lane (q, c) holds row 4 step + q.  Rows past
-// the end repeat the last one with cotangents of zero.
-constexpr int MLP_OUTER_AHEAD = 3;
+// The operands of four rows (k of the matrix instructions) for one wavefront: lane (q, c) holds row 4 step + q, and of it the
+// hidden units 64w + 4c + u and the features 4c + i (which of them is which row or column of a tile is free, and four
+// neighbours are one load).  Rows past the end repeat the last one with cotangents of zero.
+constexpr int MLP_OUTER_AHEAD = 4;
 struct MlpOuterRows {
     float h[4], d[4], g[4], x[4], t;
 };
 
-__device__ __forceinline__ MlpOuterRows mlp_outer_rows(const tode_mlp_reverse &p, long long row, long long end, int w, int c) {
-    const bool in = row < end;
-    const long long at = in ? row : end - 1;
-    const int FR = p.n_features;
-    MlpOuterRows v;
+// The lane's four features of a row, without a branch; those past the problem's repeat the first ones (their sums go nowhere).
+// QUADS: rows are whole groups of four.
+template <bool QUADS> __device__ __forceinline__ void mlp_outer_get(const float *row, int f0, int FR, float (&v)[4]) {
+    if (QUADS) {
+        const float4 u = *reinterpret_cast<const float4 *>(row + (f0 < FR ? f0 : 0));
+        v[0] = u.x, v[1] = u.y, v[2] = u.z, v[3] = u.w;
+    } else {
 #pragma unroll
-    for (int u = 0; u < 4; ++u) {
-        v.h[u] = ((const float *)p.hidden)[at * MLP_H + 64 * w + 16 * u + c];
-        v.d[u] = ((const float *)p.hidden_cotangents)[at * MLP_H + 64 * w + 16 * u + c];
-        const int f = 16 * u + c;
-        v.g[u] = f < FR ? ((const float *)p.stage_cotangents)[at * FR + f] : 0.0f;
-        v.x[u] = f < FR ? ((const float *)p.stage_inputs)[at * FR + f] : 0.0f;
-        v.d[u] = in ? v.d[u] : 0.0f;
-        v.g[u] = in ? v.g[u] : 0.0f;
+        for (int r = 0; r < 4; ++r) v[r] = row[f0 + r < FR ? f0 + r : 0];
     }
-    v.t = ((const float *)p.stage_times)[at];
-    return v;
+}
+
+// The rows row .. row + 3 (the same for the whole wavefront) of a share that ends at `end`; those past it repeat the last one.
+// (Nothing is done to the values here: that would be the place where their loads are waited for.)
+template <bool QUADS> __device__ __forceinline__ void mlp_outer_rows(const tode_mlp_reverse &p, long long row, long long end, int w, int q, int c, MlpOuterRows &v) {
+    const long long from = min(row, end - 1);
+    const int at = min(q, (int)min(end - 1 - from, 3ll)), FR = p.n_features;
+    const float4 h = *reinterpret_cast<const float4 *>((const float *)p.hidden + from * MLP_H + (at * MLP_H + 64 * w + 4 * c));
+    const float4 d = *reinterpret_cast<const float4 *>((const float *)p.hidden_cotangents + from * MLP_H + (at * MLP_H + 64 * w + 4 * c));
+    v.h[0] = h.x, v.h[1] = h.y, v.h[2] = h.z, v.h[3] = h.w;
+    v.d[0] = d.x, v.d[1] = d.y, v.d[2] = d.z, v.d[3] = d.w;
+    mlp_outer_get<QUADS>((const float *)p.stage_cotangents + from * FR + at * FR, 4 * c, FR, v.g);
+    mlp_outer_get<QUADS>((const float *)p.stage_inputs + from * FR + at * FR, 4 * c, FR, v.x);
+    v.t = ((const float *)p.stage_times + from)[at];
 }
 
 // dW2[f][u] = sum over rows g[f] h[u],  dW1[u][i] = sum over rows d[u] x[i],  and the biases' and the time column's sums:
 // every workgroup takes a share of the rows and holds all sums of it in registers (wavefront w: units 64w .. 64w + 63, 128
-// accumulators), 32 matrix instructions (0.45 us) per four rows with the operands of the next three such steps on their way:
-// one wavefront per SIMD has nothing else to cover the memory's latency with.  The sums of a share go to the workgroup's
+// accumulators), 32 matrix instructions (0.45 us) per four rows with the operands of the next four such steps on their way:
+// one wavefront per SIMD has nothing else to cover the memory's latency with.  82 000 rows: 69 us, of which the matrix
+// instructions are 39; 92 with a load per value, half of whose instructions were addresses.  The sums of a share go to the workgroup's
 // own slot, added to those of earlier calls (`accumulate`).
-__global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(1, 2))) mlp_weight_gradient_kernel(const tode_mlp_reverse p, long long rows, long long rows_per_split, int accumulate) {
+template <bool QUADS>
+__global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(1, 1))) mlp_weight_gradient_kernel(const tode_mlp_reverse p, long long rows, long long rows_per_split, int accumulate) {
     const int tid = threadIdx.x, lane = tid & 63, w = tid >> 6, q = lane >> 4, c = lane & 15;
     const long long first = (long long)blockIdx.x * rows_per_split, end = min(rows, first + rows_per_split);
     mfma_acc a2[4][4], a1[4][4];
@@ -509,12 +519,17 @@ __global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(1, 2))
     if (first < end) {
         MlpOuterRows ring[MLP_OUTER_AHEAD];
 #pragma unroll
-        for (int n = 0; n < MLP_OUTER_AHEAD; ++n) ring[n] = mlp_outer_rows(p, first + 4 * n + q, end, w, c);
+        for (int n = 0; n < MLP_OUTER_AHEAD; ++n) mlp_outer_rows<QUADS>(p, first + 4 * n, end, w, q, c, ring[n]);
         for (long long row = first; row < end; row += 4 * MLP_OUTER_AHEAD) {
 #pragma unroll
             for (int n = 0; n < MLP_OUTER_AHEAD; ++n) {
-                const MlpOuterRows here = ring[n];
-                ring[n] = mlp_outer_rows(p, row + 4 * (MLP_OUTER_AHEAD + n) + q, end, w, c);
+                MlpOuterRows here = ring[n];
+                if (row + 4 * n + 4 > end) {  // (the share's last rows: cotangents of zero for those past its end)
+                    const bool in = row + 4 * n + q < end;
+#pragma unroll
+                    for (int u = 0; u < 4; ++u) here.d[u] = in ? here.d[u] : 0.0f, here.g[u] = in ? here.g[u] : 0.0f;
+                }
+                mlp_outer_rows<QUADS>(p, row + 4 * (MLP_OUTER_AHEAD + n), end, w, q, c, ring[n]);
 #pragma unroll
                 for (int u = 0; u < 4; ++u) {
 #pragma unroll
@@ -531,28 +546,38 @@ __global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(1, 2))
     }
     float *out = (float *)p.sums + (long long)blockIdx.x * MLP_SUMS;
     auto put = [&](int i, float v) { out[i] = accumulate ? out[i] + v : v; };
+    auto put_four = [&](int i, float a, float b, float c, float d) {
+        float4 *to = reinterpret_cast<float4 *>(out + i);
+        float4 v = make_float4(a, b, c, d);
+        if (accumulate) {
+            const float4 before = *to;
+            v = make_float4(before.x + a, before.y + b, before.z + c, before.w + d);
+        }
+        *to = v;
+    };
+#pragma unroll
+    for (int i = 0; i < 4; ++i)
+#pragma unroll
+        for (int r = 0; r < 4; ++r) {
+            const int feature = 4 * (4 * q + r) + i;
+            put_four(feature * MLP_H + 64 * w + 4 * c, a1[i][0][r], a1[i][1][r], a1[i][2][r], a1[i][3][r]);
+            put_four(MLP_SUM_W2 + feature * MLP_H + 64 * w + 4 * c, a2[i][0][r], a2[i][1][r], a2[i][2][r], a2[i][3][r]);
+        }
 #pragma unroll
     for (int u = 0; u < 4; ++u) {
-        const int unit = 64 * w + 16 * u + c;
-#pragma unroll
-        for (int i = 0; i < 4; ++i)
-#pragma unroll
-            for (int r = 0; r < 4; ++r) {
-                put((16 * i + 4 * q + r) * MLP_H + unit, a1[i][u][r]);
-                put(MLP_SUM_W2 + (16 * i + 4 * q + r) * MLP_H + unit, a2[i][u][r]);
-            }
+        const int unit = 64 * w + 4 * c + u;
 #pragma unroll
         for (int off = 16; off < 64; off <<= 1) at[u] += __shfl_xor(at[u], off), ab[u] += __shfl_xor(ab[u], off), ag[u] += __shfl_xor(ag[u], off);
         if (q == 0) {
             put(MLP_SUM_W1T + unit, at[u]);
             put(MLP_SUM_B1 + unit, ab[u]);
-            if (w == 0) put(MLP_SUM_B2 + 16 * u + c, ag[u]);
+            if (w == 0) put(MLP_SUM_B2 + 4 * c + u, ag[u]);
         }
     }
 }
 
-// The splits of 64 sums per workgroup, a quarter of the splits per wavefront with eight loads in flight (one thread per sum
-// over all splits waited for memory 64 times in a row: 68 us for 34 MB); always in the same order.  out in the order of
+// The splits of 64 sums per workgroup, a quarter of the splits per wavefront with 32 loads in flight (one thread per sum over
+// all splits waited for memory 64 times in a row: 68 us for 34 MB; eight loads in flight: 20 us); always in the same order.  out in the order of
 // the weights: W1 [H x (F + 1)] | b1 | W2 [F x H] | b2.
 static __global__ void __launch_bounds__(256) mlp_weight_gradient_sum_kernel(const float *sums, int splits, int H, int FR, float *out) {
     __shared__ float part[4][64];
@@ -560,10 +585,13 @@ static __global__ void __launch_bounds__(256) mlp_weight_gradient_sum_kernel(con
     const int share = (splits + 3) / 4, first = w * share, end = min(splits, first + share);
     float s[8] = {0, 0, 0, 0, 0, 0, 0, 0};
     if (i < MLP_SUMS) {
-        for (int k = first; k < end; k += 8)
+        for (int k = first; k < end; k += 32) {
+            float v[32];
 #pragma unroll
-            for (int j = 0; j < 8; ++j)
-                if (k + j < end) s[j] += sums[(long long)(k + j) * MLP_SUMS + i];
+            for (int j = 0; j < 32; ++j) v[j] = k + j < end ? sums[(long long)(k + j) * MLP_SUMS + i] : 0.0f;
+#pragma unroll
+            for (int j = 0; j < 32; ++j) s[j % 8] += v[j];
+        }
     }
     part[w][lane] = ((s[0] + s[1]) + (s[2] + s[3])) + ((s[4] + s[5]) + (s[6] + s[7]));
     __syncthreads();
@@ -679,7 +707,9 @@ int tode_mlp_outer_products(const tode_mlp_reverse *p, int64_t rows, int32_t acc
     if (!p->sums) return fail(TODE_E_INVALID, "null pointer");
     if (rows < 0) return fail(TODE_E_INVALID, "rows %lld", (long long)rows);
     const long long per_split = ((rows + p->splits - 1) / p->splits + 3) / 4 * 4;
-    hipLaunchKernelGGL(mlp_weight_gradient_kernel, dim3(p->splits), dim3(256), 0, (hipStream_t)stream, *p, (long long)rows, per_split, accumulate);
+    // (rows of the features as 16-byte values, as everywhere in these kernels, where they are whole groups of four)
+    if ((p->n_features & 3) == 0) hipLaunchKernelGGL((mlp_weight_gradient_kernel<true>), dim3(p->splits), dim3(256), 0, (hipStream_t)stream, *p, (long long)rows, per_split, accumulate);
+    else hipLaunchKernelGGL((mlp_weight_gradient_kernel<false>), dim3(p->splits), dim3(256), 0, (hipStream_t)stream, *p, (long long)rows, per_split, accumulate);
     return check_hip(hipGetLastError(), "tode_mlp_outer_products");
 }
 
