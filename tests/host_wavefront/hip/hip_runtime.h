@@ -104,6 +104,7 @@ inline double __hiloint2double(int hi, int lo) { return host::bits<double>(((uns
 #define __builtin_amdgcn_fence(...)
 #define __builtin_amdgcn_s_barrier() __syncthreads()
 #define __builtin_amdgcn_mov_dpp(v, ...) (v)
+#define __builtin_amdgcn_readlane(v, lane) (v)
 #define __builtin_amdgcn_ballot_w64(c) ((c) ? 1ull : 0ull)
 #define __builtin_amdgcn_inverse_ballot_w64(l) (((l) & 1ull) != 0)
 #define __builtin_amdgcn_rcpf(x) (1.0f / (x))

@@ -39,6 +39,13 @@ template <typename TT, typename T> struct AdjointParams {
     TT dt_min, dt_max;
 };
 
+// The value that lane `src` (the same for the whole wavefront) holds.
+__device__ __forceinline__ float wave_read(float v, int src) { return __int_as_float(__builtin_amdgcn_readlane(__float_as_int(v), src)); }
+__device__ __forceinline__ double wave_read(double v, int src) {
+    const int lo = __builtin_amdgcn_readlane(__double2loint(v), src), hi = __builtin_amdgcn_readlane(__double2hiint(v), src);
+    return __hiloint2double(hi, lo);
+}
+
 template <typename T> __device__ __forceinline__ T sign_(T x) { return x > (T)0 ? (T)1 : (x < (T)0 ? (T)-1 : (T)0); }
 
 // cotangents of the operands of maximum(a, b) given the cotangent g of the result
@@ -262,22 +269,38 @@ __device__ __forceinline__ void finish_backward_sample(const AdjointParams<TT, T
                 quartic_elem<T, METHOD>(h, y[f], y1[f], ks, true, q);
             }
             for (int base = 0; base < n_points; base += 64) {
+                // (a lane works out the position of its own point; the cotangents of four points are on their way together: one by
+                // one, each waited for its time, a division and its cotangent, 24 instead of 19 us of finish_backward_kernel at
+                // B = 4096 and ten points)
                 const int mine = base + f_first;
+                const TT at = E == 0 ? te : p.t_eval[b * E + (mine < n_points ? mine : 0)];
+                const T x_mine = (T)((at - t0) / den);
                 unsigned long long marks = __ballot(mine < n_points && (E == 0 || p.hit_iteration[b * E + mine] == p.iteration));
                 while (marks) {
-                    const int e = base + __builtin_ctzll(marks);
-                    marks &= marks - 1;
-                    if (f >= F) continue;
-                    const T x = (T)(((E > 0 ? p.t_eval[b * E + e] : te) - t0) / den);
-                    T g = p.grad_ys[(b * (long long)(E > 0 ? E : 1) + e) * F + f];
-                    if (g == (T)0) continue;  // (adds nothing, wherever the point lies: its position may be an infinity)
-                    any = true;
-                    if (POINTWISE) {
-                        const Wide g_x = (Wide)(g * (q[1][0] + x * ((T)2 * q[2][0] + x * ((T)3 * q[3][0] + x * (T)4 * q[4][0]))));
-                        g_points += g_x, g_points_x += g_x * (Wide)x;
+                    int at_lane[4];
+                    T cotangent[4];
+                    int n_taken = 0;
+#pragma unroll
+                    for (int j = 0; j < 4; ++j) {
+                        at_lane[j] = marks ? __builtin_ctzll(marks) : at_lane[j > 0 ? j - 1 : 0];
+                        n_taken += marks ? 1 : 0;
+                        marks &= marks - 1;
+                        cotangent[j] = p.grad_ys[(b * (long long)(E > 0 ? E : 1) + base + at_lane[j]) * F + (f < F ? f : 0)];
                     }
 #pragma unroll
-                    for (int n = 0; n < 5; ++n) G[n] += g, g = g * x;
+                    for (int j = 0; j < 4; ++j) {
+                        if (j >= n_taken) break;
+                        const T x = wave_read(x_mine, at_lane[j]);
+                        T g = cotangent[j];
+                        if (f >= F || g == (T)0) continue;  // (adds nothing, wherever the point lies: its position may be an infinity)
+                        any = true;
+                        if (POINTWISE) {
+                            const Wide g_x = (Wide)(g * (q[1][0] + x * ((T)2 * q[2][0] + x * ((T)3 * q[3][0] + x * (T)4 * q[4][0]))));
+                            g_points += g_x, g_points_x += g_x * (Wide)x;
+                        }
+#pragma unroll
+                        for (int n = 0; n < 5; ++n) G[n] += g, g = g * x;
+                    }
                 }
             }
             if (f < F) spread(f, G, any);

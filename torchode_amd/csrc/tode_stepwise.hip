@@ -196,13 +196,6 @@ __global__ void __launch_bounds__(256) init_b_kernel(const StepParams<TT, T> p, 
 
 // Quartic of the attempted step for one feature, evaluated at time te (tsit5.py:123-139,
 // dopri5.py:53-60, interpolation.py:25-40, 138-175).  ks[s] = k_s[b,f].
-// The value that lane `src` of the wavefront holds; `src` is the same for all lanes.
-__device__ __forceinline__ float wave_read(float v, int src) { return __int_as_float(__builtin_amdgcn_readlane(__float_as_int(v), src)); }
-__device__ __forceinline__ double wave_read(double v, int src) {
-    const int lo = __builtin_amdgcn_readlane(__double2loint(v), src), hi = __builtin_amdgcn_readlane(__double2hiint(v), src);
-    return __hiloint2double(hi, lo);
-}
-
 template <typename T> __device__ __forceinline__ T quartic_at(const T (&q)[5][1], T x) {
     T y = q[4][0];
     y = fma_(y, x, q[3][0]);
