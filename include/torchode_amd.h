@@ -345,6 +345,25 @@ int tode_solve_builtin_fast_static(const tode_solve_args *args, const tode_contr
  * the loop through the per-step or the operator entry points instead.
  */
 int64_t tode_solve_workspace_bytes(const tode_solve_args *args);
+
+/*
+ * The first part of tode_solve_builtin_auto, its one kernel in the common case, in two calls, so that the host has the
+ * kernel's time for work of its own: begin decides and launches, end waits for the flag words (tode_solve_builtin_fast_sync).
+ * No workspace is needed; with n_eval == 0 args->y_idle is read, [B,F] that live until end has returned.  After a begin that
+ * returned TODE_OK, end is called with the same args (only where they point matters) and stream, once, and gives
+ * flags_out[TODE_FLAG_WORDS]: with TODE_FLAG_NEEDS_GENERAL set the caller goes on to tode_solve_builtin_auto with
+ * allow_one_kernel 0 (a small system) or treats the problem as tode_solve_builtin_auto's TODE_E_UNSUPPORTED (the other
+ * terms); else the solve is complete in stream order and took flags_out[TODE_FLAG_MAX_ITERATIONS] iterations.  begin returns
+ * the errors of tode_solve_builtin_auto.  A ticket holds one of 64 slots of its device until its end.
+ */
+typedef struct tode_solve_ticket {
+    void *pool;
+    int32_t slot, sequence;
+    int32_t flags[TODE_FLAG_WORDS];
+} tode_solve_ticket;
+int tode_solve_builtin_begin(const tode_solve_args *args, const tode_controller *controller, int64_t *out_n_steps, int64_t *out_n_accepted, int64_t *out_n_initialized,
+                             int64_t *out_status, int32_t allow_one_kernel, void *stream, tode_solve_ticket *ticket);
+int tode_solve_builtin_end(tode_solve_ticket *ticket, const tode_solve_args *args, const int64_t *n_steps, void *stream, int32_t *flags_out);
 int tode_solve_builtin_auto(const tode_solve_args *args, const tode_controller *controller, int64_t *out_n_steps,
                             int64_t *out_n_accepted, int64_t *out_n_initialized, int64_t *out_status, void *workspace,
                             int64_t workspace_bytes, int32_t allow_one_kernel, void *stream, int64_t *iterations);

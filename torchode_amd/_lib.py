@@ -41,6 +41,8 @@ EXPORTS = (
     "tode_solve_builtin_fast_sync",
     "tode_solve_builtin_fast_static",
     "tode_solve_builtin_auto",
+    "tode_solve_builtin_begin",
+    "tode_solve_builtin_end",
     "tode_solve_builtin_backward",
     "tode_solve_backward_scratch_bytes",
     "tode_solve_workspace_bytes",
@@ -156,6 +158,12 @@ class SolveRecord(C.Structure):
     """struct tode_solve_record"""
 
     _fields_ = [("capacity", C.c_int64)] + [(n, C.c_void_p) for n in ("t", "dt", "y", "k0", "prev", "pprev", "running", "n_accepted")]
+
+
+class SolveTicket(C.Structure):
+    """struct tode_solve_ticket"""
+
+    _fields_ = [("pool", C.c_void_p), ("slot", C.c_int32), ("sequence", C.c_int32), ("flags", C.c_int32 * FLAG_WORDS)]
 
 
 class SolveAdjoint(C.Structure):
@@ -380,6 +388,10 @@ def load():
         lib.tode_solve_workspace_bytes.argtypes = [C.POINTER(SolveArgs)]
         lib.tode_solve_builtin_auto.restype = C.c_int
         lib.tode_solve_builtin_auto.argtypes = [C.POINTER(SolveArgs), C.POINTER(Controller)] + [C.c_void_p] * 5 + [C.c_int64, C.c_int32, C.c_void_p, C.POINTER(C.c_int64)]
+        lib.tode_solve_builtin_begin.restype = C.c_int
+        lib.tode_solve_builtin_begin.argtypes = [C.POINTER(SolveArgs), C.POINTER(Controller)] + [C.c_void_p] * 4 + [C.c_int32, C.c_void_p, C.POINTER(SolveTicket)]
+        lib.tode_solve_builtin_end.restype = C.c_int
+        lib.tode_solve_builtin_end.argtypes = [C.POINTER(SolveTicket), C.POINTER(SolveArgs), C.c_void_p, C.c_void_p, C.POINTER(C.c_int32)]
         lib.tode_solve_backward_scratch_bytes.restype = C.c_int64
         lib.tode_solve_backward_scratch_bytes.argtypes = [C.POINTER(SolveArgs)]
         lib.tode_solve_builtin_backward.restype = C.c_int

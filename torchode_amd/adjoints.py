@@ -20,6 +20,7 @@ _PROTOCOL_NAMES = (
 )  # fmt: skip
 
 
+_FlagArray = _lib.C.c_int32 * _lib.FLAG_WORDS
 _F_EVAL_VALUES: Dict[int, torch.Tensor] = {}  # count -> 0-dim int64 tensor (never written to)
 
 
@@ -632,8 +633,7 @@ class AutoDiffAdjoint(nn.Module):
                 params.data_ptr() if params.numel() else None,
                 None if shared is None else shared.data_ptr(), 0 if shared is None else shared.numel(),
             )  # fmt: skip  (what the general kernel needs besides lives in the workspace)
-            held.update(key=key, args=a, workspace_bytes=lib.tode_solve_workspace_bytes(_lib.C.byref(a)), scalars=tuple(scal[:4]),
-                        keep=(params, dt0_, shared))  # fmt: skip
+            held.update(key=key, args=a, scalars=tuple(scal[:4]), keep=(params, dt0_, shared))
         elif held["scalars"] != tuple((list(getattr(f, "builtin_scalars", lambda: ())()) + [0.0] * 4)[:4]):
             held.clear()  # (a scalar of the term was reassigned: describe the call anew)
             return self._solve_persistent(problem, term, dt0, record=record)
@@ -641,8 +641,8 @@ class AutoDiffAdjoint(nn.Module):
         a.ys = ys.data_ptr()
         a_ref = _lib.C.byref(a)
 
-        # One call: the one-kernel path where the batch is in its shape, the general kernel where it is not or where
-        # the first reported that the batch leaves the common case, the int64 stats as the reference returns them.
+        # The one-kernel path where the batch is in its shape; the general kernel where it is not or where the first
+        # reported that the batch leaves the common case; the int64 stats as the reference returns them.
         out = torch.empty((4, B), dtype=torch.int64, device=dev)
         o0, row = out.data_ptr(), 8 * B
         if record is not None:
@@ -654,24 +654,41 @@ class AutoDiffAdjoint(nn.Module):
                 ends_at_last_point=E > 1 and B > 0 and (t_end_ptr, t_end_stride) == (t_eval_ptr + (E - 1) * t_eval.element_size(), E)))  # fmt: skip
             if solution is not None or mlp:
                 return solution
-        workspace = torch.empty(held["workspace_bytes"], dtype=torch.uint8, device=dev)
-        iterations = _lib.C.c_int64(0)
-        rc = lib.tode_solve_builtin_auto(
-            a_ref, _lib.C.byref(ctrl), o0, o0 + row, o0 + 2 * row, o0 + 3 * row, workspace.data_ptr(), held["workspace_bytes"],
-            1 if self.use_fast_path else 0, stream, _lib.C.byref(iterations),
-        )  # fmt: skip  (returns after the solve's one host synchronisation)
+        ctrl_ref = _lib.C.byref(ctrl)
+        if E == 0:
+            y_idle = torch.empty((B, F), dtype=dtype, device=dev)
+            a.y_idle = y_idle.data_ptr()
+        ticket, flags = _lib.SolveTicket(), _FlagArray()
+        rc = lib.tode_solve_builtin_begin(a_ref, ctrl_ref, o0, o0 + row, o0 + 2 * row, o0 + 3 * row, 1 if self.use_fast_path else 0, stream, _lib.C.byref(ticket))
         if rc == _lib.E_UNSUPPORTED:
             return None  # no whole-solve kernel for this case: the caller takes the per-step or the operator path
         if rc:
-            _lib.check(rc, "tode_solve_builtin_auto")
-        stats: Dict[str, Any] = {}
+            _lib.check(rc, "tode_solve_builtin_begin")
+        try:  # (while the kernel runs)
+            stats: Dict[str, Any] = {"n_f_evals": None} if term.with_stats else {}
+            stats["n_steps"], stats["n_accepted"], stats["n_initialized"], status = out.unbind(0)
+        finally:
+            rc = lib.tode_solve_builtin_end(_lib.C.byref(ticket), a_ref, o0, stream, flags)  # (the solve's one host synchronisation)
+        if rc:
+            _lib.check(rc, "tode_solve_builtin_end")
+        iterations = flags[_lib.FLAG_MAX_ITERATIONS]
+        if flags[_lib.FLAG_NEEDS_GENERAL]:
+            if f.builtin_kind not in _lib.GENERAL_TERMS:
+                return None
+            workspace_bytes, count = lib.tode_solve_workspace_bytes(a_ref), _lib.C.c_int64(0)
+            workspace = torch.empty(workspace_bytes, dtype=torch.uint8, device=dev)
+            rc = lib.tode_solve_builtin_auto(
+                a_ref, ctrl_ref, o0, o0 + row, o0 + 2 * row, o0 + 3 * row, workspace.data_ptr(), workspace_bytes, 0, stream, _lib.C.byref(count),
+            )  # fmt: skip
+            if rc:
+                _lib.check(rc, "tode_solve_builtin_auto")
+            iterations = count.value
         if term.with_stats:
-            stats["n_f_evals"] = _f_evals((2 if dt0 is None else 1) + 6 * iterations.value, B)
-        stats["n_steps"], stats["n_accepted"], stats["n_initialized"], status = out.unbind(0)
+            stats["n_f_evals"] = _f_evals((2 if dt0 is None else 1) + 6 * iterations, B)
         if record is not None:
             # The same solve through the general kernel again, stopped where the first pass stopped, writing the
             # state before every iteration: entry i of every array is what the per-step kernels' loop holds there.
-            L, n = iterations.value, iterations.value + 1
+            L, n = iterations, iterations + 1
             new = lambda *shape, dt=dtype: torch.empty(shape, dtype=dt, device=dev)
             fields, rec = self._record_arrays(n, B, F, dtype, ttype, dev)
             again = _lib.SolveArgs.from_buffer_copy(a)

@@ -346,12 +346,12 @@ int tode_mlp_pack_weights_for(const void *raw, int64_t n_raw, int32_t n_features
     return tode::mlp_pack_weights((const float *)raw, (long long)n_raw, n_features, matrix_inputs, (float *)packed, (hipStream_t)stream);
 }
 
-int tode_solve_builtin_fast_sync(const tode_solve_args *a, const tode_controller *c, int64_t *ns, int64_t *na, int64_t *ni,
-                                 int64_t *st, void *stream, int32_t *flags_out) {
+// The launch of tode_solve_builtin_fast_sync, and its wait.  A ticket without a slot (-1) has nothing to wait for: its flags are set.
+static int fast_begin(const tode_solve_args *a, const tode_controller *c, int64_t *ns, int64_t *na, int64_t *ni, int64_t *st, void *stream, tode_solve_ticket *ticket) {
     using namespace tode;
-    if (!a || !c || !flags_out) return fail(TODE_E_INVALID, "null argument");
     hipStream_t s = (hipStream_t)stream;
     FlagPool *pool = nullptr;
+    ticket->slot = -1;
     int rc = flag_pool(s, &pool);
     if (rc) return rc;
     int slot = -1;
@@ -370,32 +370,51 @@ int tode_solve_builtin_fast_sync(const tode_solve_args *a, const tode_controller
     g_flag_target = &target;
     rc = tode_solve_builtin_fast(&b, c, ns, na, ni, st, stream);
     g_flag_target = nullptr;
+    ticket->flags[TODE_FLAG_MAX_ITERATIONS] = ticket->flags[TODE_FLAG_NON_MONOTONE] = ticket->flags[TODE_FLAG_NEEDS_GENERAL] = 0;
+    ticket->flags[TODE_FLAG_FIRST_FAILURE] = INT_MAX;
     if (rc == TODE_E_UNSUPPORTED && (a->n_eval > 0 || a->y_idle) && !c->has_dt_min && !c->has_dt_max &&
         a->term != TODE_TERM_REACTION_DIFFUSION && a->term != TODE_TERM_MLP) {
         // a small system in a shape the fast kernels do not take (no evaluation points, or very many of them, in a
         // batch too large for the two-wavefront kernel) or with a controller exponent that is not computed through pow:
         // no solve kernel was launched, and the caller is sent to the general kernel like any batch that leaves the
         // common case
-        flags_out[TODE_FLAG_MAX_ITERATIONS] = 0;
-        flags_out[TODE_FLAG_FIRST_FAILURE] = INT_MAX;
-        flags_out[TODE_FLAG_NON_MONOTONE] = 0;
-        flags_out[TODE_FLAG_NEEDS_GENERAL] = 1;
+        ticket->flags[TODE_FLAG_NEEDS_GENERAL] = 1;
         rc = TODE_OK;
-    } else if (rc == TODE_OK && a->batch == 0) {  // nothing was launched
-        flags_out[TODE_FLAG_MAX_ITERATIONS] = 0;
-        flags_out[TODE_FLAG_FIRST_FAILURE] = INT_MAX;
-        flags_out[TODE_FLAG_NON_MONOTONE] = flags_out[TODE_FLAG_NEEDS_GENERAL] = 0;
-    } else if (rc == TODE_OK) {
-        const int32_t *host = pool->host + slot * FLAG_SLOT_WORDS;
-        rc = wait_for_flags(host, sequence, s);
-        if (rc == TODE_OK)
-            for (int i = 0; i < TODE_FLAG_WORDS; ++i) flags_out[i] = host[i];
-        if (rc == TODE_OK && a->n_eval == 0 && !flags_out[TODE_FLAG_NEEDS_GENERAL])
-            rc = tode_select_end_point(a->batch, a->n_features, a->dtype, flags_out[TODE_FLAG_MAX_ITERATIONS], ns, a->ys, a->y_idle, stream);
-    }
-    // (after a failed wait the slot's words may be anything: the slot stays out of use)
+    } else if (rc == TODE_OK && a->batch > 0) {
+        ticket->pool = pool, ticket->slot = slot, ticket->sequence = sequence;
+        return TODE_OK;
+    }  // (an empty batch: nothing was launched)
     if (rc == TODE_OK || rc == TODE_E_INVALID || rc == TODE_E_UNSUPPORTED) pool->busy[slot].store(0, std::memory_order_release);
     return rc;
+}
+
+static int fast_end(tode_solve_ticket *ticket, const tode_solve_args *a, const int64_t *ns, void *stream, int32_t *flags_out) {
+    using namespace tode;
+    hipStream_t s = (hipStream_t)stream;
+    int rc = TODE_OK;
+    const int slot = ticket->slot;
+    if (slot >= 0) {
+        FlagPool *pool = (FlagPool *)ticket->pool;
+        const int32_t *host = pool->host + slot * FLAG_SLOT_WORDS;
+        rc = wait_for_flags(host, ticket->sequence, s);
+        ticket->slot = -1;
+        if (rc) return rc;  // (after a failed wait the slot's words may be anything: the slot stays out of use)
+        for (int i = 0; i < TODE_FLAG_WORDS; ++i) ticket->flags[i] = host[i];
+        pool->busy[slot].store(0, std::memory_order_release);
+        if (a->n_eval == 0 && !ticket->flags[TODE_FLAG_NEEDS_GENERAL])
+            rc = tode_select_end_point(a->batch, a->n_features, a->dtype, ticket->flags[TODE_FLAG_MAX_ITERATIONS], ns, a->ys, a->y_idle, stream);
+    }
+    for (int i = 0; i < TODE_FLAG_WORDS; ++i) flags_out[i] = ticket->flags[i];
+    return rc;
+}
+
+int tode_solve_builtin_fast_sync(const tode_solve_args *a, const tode_controller *c, int64_t *ns, int64_t *na, int64_t *ni,
+                                 int64_t *st, void *stream, int32_t *flags_out) {
+    using namespace tode;
+    if (!a || !c || !flags_out) return fail(TODE_E_INVALID, "null argument");
+    tode_solve_ticket ticket;
+    const int rc = fast_begin(a, c, ns, na, ni, st, stream, &ticket);
+    return rc ? rc : fast_end(&ticket, a, ns, stream, flags_out);
 }
 
 int tode_solve_builtin_fast_static(const tode_solve_args *a, const tode_controller *c, int64_t *ns, int64_t *na, int64_t *ni,
@@ -533,33 +552,18 @@ int64_t tode_solve_workspace_bytes(const tode_solve_args *a) {
     return tode::workspace_layout(*a).bytes;
 }
 
-int tode_solve_builtin_auto(const tode_solve_args *a, const tode_controller *c, int64_t *ns, int64_t *na, int64_t *ni, int64_t *st,
-                            void *workspace, int64_t workspace_bytes, int32_t allow_one_kernel, void *stream, int64_t *iterations) {
+int tode_solve_builtin_begin(const tode_solve_args *a, const tode_controller *c, int64_t *ns, int64_t *na, int64_t *ni, int64_t *st, int32_t allow_one_kernel, void *stream,
+                             tode_solve_ticket *ticket) {
     using namespace tode;
-    if (!a || !c || !iterations) return fail(TODE_E_INVALID, "null argument");
+    if (!a || !c || !ticket) return fail(TODE_E_INVALID, "null argument");
     if (a->batch < 0 || a->n_features <= 0 || a->n_eval < 0 || a->n_params < 0)
         return fail(TODE_E_INVALID, "bad sizes: batch=%lld F=%d E=%d P=%d", (long long)a->batch, a->n_features, a->n_eval, a->n_params);
     if (!known_dtype(a->dtype)) return fail(TODE_E_INVALID, "unknown dtype %d", a->dtype);
-    const bool one_dtype = !(a->dtype & TODE_DTYPE_PAIR);  // (time and data in different types: the general kernel)
-    const Workspace w = workspace_layout(*a);
-    if (!workspace || workspace_bytes < w.bytes)
-        return fail(TODE_E_INVALID, "the workspace holds %lld bytes, this problem needs %lld (tode_solve_workspace_bytes)", (long long)workspace_bytes, (long long)w.bytes);
     if (a->batch > 0 && (!ns || !na || !ni || !st)) return fail(TODE_E_INVALID, "null output pointer");
-    hipStream_t s = (hipStream_t)stream;
-    unsigned char *ws = (unsigned char *)workspace;
+    const bool one_dtype = !(a->dtype & TODE_DTYPE_PAIR);  // (time and data in different types: the general kernel)
     const int64_t B = a->batch, E = a->n_eval, elem = data_type(a->dtype) == TODE_F64 ? 8 : 4;
-    const bool small_system = a->term == TODE_TERM_LINEAR_DECAY || a->term == TODE_TERM_VAN_DER_POL || a->term == TODE_TERM_LORENZ63;
-
-    tode_solve_args b = *a;
-    b.iteration_cap = -1;
-    b.pending = nullptr;
-    b.record = nullptr;
-    b.y_idle = E == 0 ? ws + w.y_idle : nullptr;
-
-    // The common case first: one kernel that writes what the reference returns.  It reports through its flag words when the
-    // batch needs the general kernel (rows of evaluation points that are not monotone, a non-success status, non-finite values).
     bool one_kernel = one_dtype && !c->has_dt_min && !c->has_dt_max;
-    if (small_system) {
+    if (a->term == TODE_TERM_LINEAR_DECAY || a->term == TODE_TERM_VAN_DER_POL || a->term == TODE_TERM_LORENZ63) {
         // (no evaluation points, or more than fit on chip: built for batches that leave SIMDs to spare)
         one_kernel = one_kernel && allow_one_kernel && ((E > 0 && E * elem <= 1024) || (B > 0 && B <= TODE_END_ONLY_MAX_BATCH));
     } else {
@@ -572,9 +576,50 @@ int tode_solve_builtin_auto(const tode_solve_args *a, const tode_controller *c, 
             return fail(TODE_E_INVALID, "unknown term %d", a->term);
         if (!one_kernel) return fail(TODE_E_UNSUPPORTED, "no whole-solve kernel for this term in this shape, dtype or controller setting");
     }
-    if (one_kernel) {
+    tode_solve_args b = *a;
+    b.iteration_cap = -1, b.pending = nullptr, b.record = nullptr;
+    if (one_kernel) return fast_begin(&b, c, ns, na, ni, st, stream, ticket);
+    ticket->slot = -1;
+    ticket->flags[TODE_FLAG_MAX_ITERATIONS] = ticket->flags[TODE_FLAG_NON_MONOTONE] = 0;
+    ticket->flags[TODE_FLAG_FIRST_FAILURE] = INT_MAX, ticket->flags[TODE_FLAG_NEEDS_GENERAL] = 1;
+    return TODE_OK;
+}
+
+int tode_solve_builtin_end(tode_solve_ticket *ticket, const tode_solve_args *a, const int64_t *ns, void *stream, int32_t *flags_out) {
+    using namespace tode;
+    if (!ticket || !a || !flags_out) return fail(TODE_E_INVALID, "null argument");
+    return fast_end(ticket, a, ns, stream, flags_out);
+}
+
+int tode_solve_builtin_auto(const tode_solve_args *a, const tode_controller *c, int64_t *ns, int64_t *na, int64_t *ni, int64_t *st,
+                            void *workspace, int64_t workspace_bytes, int32_t allow_one_kernel, void *stream, int64_t *iterations) {
+    using namespace tode;
+    if (!a || !c || !iterations) return fail(TODE_E_INVALID, "null argument");
+    if (a->batch < 0 || a->n_features <= 0 || a->n_eval < 0 || a->n_params < 0)
+        return fail(TODE_E_INVALID, "bad sizes: batch=%lld F=%d E=%d P=%d", (long long)a->batch, a->n_features, a->n_eval, a->n_params);
+    if (!known_dtype(a->dtype)) return fail(TODE_E_INVALID, "unknown dtype %d", a->dtype);
+    const Workspace w = workspace_layout(*a);
+    if (!workspace || workspace_bytes < w.bytes)
+        return fail(TODE_E_INVALID, "the workspace holds %lld bytes, this problem needs %lld (tode_solve_workspace_bytes)", (long long)workspace_bytes, (long long)w.bytes);
+    if (a->batch > 0 && (!ns || !na || !ni || !st)) return fail(TODE_E_INVALID, "null output pointer");
+    hipStream_t s = (hipStream_t)stream;
+    unsigned char *ws = (unsigned char *)workspace;
+    const int64_t B = a->batch, E = a->n_eval;
+    const bool small_system = a->term == TODE_TERM_LINEAR_DECAY || a->term == TODE_TERM_VAN_DER_POL || a->term == TODE_TERM_LORENZ63;
+
+    tode_solve_args b = *a;
+    b.iteration_cap = -1;
+    b.pending = nullptr;
+    b.record = nullptr;
+    b.y_idle = E == 0 ? ws + w.y_idle : nullptr;
+
+    // The common case first: one kernel that writes what the reference returns.  It reports through its flag words when the
+    // batch needs the general kernel (rows of evaluation points that are not monotone, a non-success status, non-finite values).
+    {
+        tode_solve_ticket ticket;
         int32_t fl[TODE_FLAG_WORDS];
-        int rc = tode_solve_builtin_fast_sync(&b, c, ns, na, ni, st, stream, fl);
+        int rc = tode_solve_builtin_begin(&b, c, ns, na, ni, st, allow_one_kernel, stream, &ticket);
+        if (rc == TODE_OK) rc = fast_end(&ticket, &b, ns, stream, fl);
         if (rc) return rc;
         if (!fl[TODE_FLAG_NEEDS_GENERAL]) {
             *iterations = fl[TODE_FLAG_MAX_ITERATIONS];
