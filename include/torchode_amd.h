@@ -444,6 +444,9 @@ typedef struct tode_mlp_reverse {
     void *g_y, *g_y1;            /* [B,F] in (and out: g_y) */
     void *g_t, *g_dt;            /* [B] in and out */
     void *sums;                  /* [splits, TODE_MLP_SUMS_SIZE], null where no weight wants a gradient */
+    int64_t stage_rows;          /* tode_mlp_stages_backward: rows from one stage's part of k, hidden and the three buffers after
+                                    it to the next one's, where one call of tode_mlp_stages took several iterations (batch =
+                                    iterations x samples, and k and the buffers point at the iteration's rows here); 0: batch */
 } tode_mlp_reverse;
 int tode_mlp_pack_weights_reverse(const void *raw, int64_t n_raw, int32_t n_features, void *packed, void *stream);
 int tode_mlp_stages(const tode_mlp_reverse *p, void *stream);

@@ -223,7 +223,7 @@ class MlpReverse(C.Structure):
         (name, C.c_void_p)
         for name in ("packed", "packed_reverse", "t", "dt", "y", "k0", "k", "stage_inputs", "stage_times", "hidden", "hidden_cotangents", "stage_cotangents",
                      "g_k", "g_y", "g_y1", "g_t", "g_dt", "sums")
-    ]  # fmt: skip
+    ] + [("stage_rows", C.c_int64)]  # fmt: skip
 
 
 class MlpStart(C.Structure):

@@ -544,7 +544,7 @@ class NetworkSweep:
             and y0.shape[0] > 0
         )
 
-    def __init__(self, lib, method_id, f, B, F, iterations, g_k, g_y, g_y1, g_t, g_dt, stream):
+    def __init__(self, lib, method_id, f, B, F, iterations, g_k, g_y, g_y1, g_t, g_dt, stream, in_arrays):
         dev, H = g_k.device, f.W2.shape[1]
         new = lambda *shape: torch.empty(shape, dtype=torch.float32, device=dev)
         self.lib, self.stream, self.f, self.started = lib, stream, f, False
@@ -557,14 +557,19 @@ class NetworkSweep:
         # The weights' gradients are sums over the rows of all evaluations.  A call for them ends with 133 KB of sums per
         # share of the rows (one per compute unit, at least 64 rows each), so the evaluations of several iterations are
         # kept for one call, as far as they fit into ROOM.
-        per_evaluation = 4 * B * (2 * 256 + 2 * F + 1)
+        # Where all of them fit and the record is in arrays, one launch forms the stages of every iteration: they depend on
+        # the record alone, and two workgroups to a compute unit then hide each other's waits (B = 4096, three iterations: three
+        # launches of 28 us, one of 63).
+        per_evaluation = 4 * B * (2 * 256 + 3 * F + 1)
         room = max(6, min(6 * iterations + 2, self.ROOM // per_evaluation)) if wanted else 6
-        self.held, self.B, self.k = 0, B, new(6, B, F)
+        self.held, self.B, self.F = 0, B, F
+        self.iterations = iterations if in_arrays and wanted and iterations > 1 and room == 6 * iterations + 2 else 0  # (0: one at a time)
         try:
             splits = self._allocate(room, new, F, wanted)
         except torch.cuda.OutOfMemoryError:  # (what one iteration takes has to be there)
             if room == 6:
                 raise
+            self.iterations = 0
             splits = self._allocate(6, new, F, wanted)
         self.keep = (raw, packed, packed_reverse, g_y1)
         self.args = _lib.MlpReverse(method_id, F, H, splits, B)
@@ -579,7 +584,8 @@ class NetworkSweep:
     def _allocate(self, room, new, F, wanted) -> int:
         """The rows of ``room`` evaluations and the shares' sums; returns the number of shares."""
         self.room, splits = room, max(1, min(256, (room * self.B) // 64))
-        self.inputs = self.times = self.hidden = self.cotangents = self.derivatives = self.sums = None
+        self.k = self.inputs = self.times = self.hidden = self.cotangents = self.derivatives = self.sums = None
+        self.k = new(6, max(self.iterations, 1) * self.B, F)
         rows = lambda *last: new(room, self.B, *last)
         self.inputs, self.times, self.hidden = rows(F), rows(), rows(256)
         if wanted:
@@ -616,6 +622,23 @@ class NetworkSweep:
         _lib.check(self.lib.tode_mlp_stages(self.ref, self.stream), "tode_mlp_stages")
         return y1
 
+    def iteration(self, n, entry):
+        """The stages of iteration ``n`` of a record in arrays: the addresses of their six derivatives and of the last one's input."""
+        row, slopes = 4 * self.F, self.k.data_ptr()
+        if self.iterations == 0:
+            y1 = self.stages(entry(n))
+            return [slopes + i * self.B * row for i in range(6)], y1.data_ptr()
+        a, L, B = self.args, self.iterations, self.B
+        if self.held == 0:
+            self._at(entry(0), 6 * L)
+            a.batch = L * B
+            _lib.check(self.lib.tode_mlp_stages(self.ref, self.stream), "tode_mlp_stages")
+            a.batch, a.stage_rows = B, L * B
+        now, first = entry(n), n * B
+        a.t, a.dt, a.y, a.k0, a.k = now["t"], now["dt"], now["y"], now["k0"], slopes + first * row
+        a.hidden, a.hidden_cotangents, a.stage_cotangents = (x.data_ptr() + first * 4 * x.shape[-1] for x in (self.hidden, self.cotangents, self.derivatives))
+        return [slopes + (i * L * B + first) * row for i in range(6)], self.inputs.data_ptr() + (5 * L * B + first) * row
+
     def stages_backward(self, g_k, g_y, g_t, g_dt):
         a = self.args
         a.g_k, a.g_y, a.g_t, a.g_dt = g_k.data_ptr(), g_y.data_ptr(), g_t.data_ptr(), g_dt.data_ptr()
@@ -624,7 +647,7 @@ class NetworkSweep:
     def start_backward(self, controller, state, t_end, a_y, a_k0, a_dt, g_y, through_rule, grad_ys, t_eval):
         """The start of the loop reversed; ``g_y`` becomes the cotangent of ``y0``, that of a point at ``t_start`` included."""
         self._at(state, 2 if through_rule else 1)
-        self.args.g_y = g_y.data_ptr()
+        self.args.g_y, self.args.k, self.args.stage_rows = g_y.data_ptr(), self.k.data_ptr(), 0
         start = _lib.MlpStart(t_end.data_ptr(), a_y.data_ptr(), a_k0.data_ptr(), a_dt.data_ptr(), int(bool(through_rule)),
                               t_eval.shape[1], grad_ys.data_ptr(), t_eval.data_ptr())  # fmt: skip
         _lib.check(self.lib.tode_mlp_start_backward(self.ref, _lib.C.byref(start), controller, self.stream), "tode_mlp_start_backward")
@@ -729,7 +752,7 @@ def reverse_sweep_kernels(adjoint, replay: Replay, term, args, problem, dt0_give
     f, with_args = term.f, term.with_args
     network = None
     if NetworkSweep.takes(adjoint, term, y0, t_start):  # (always so where `arrays` are given)
-        network = NetworkSweep(lib, method.method_id, f, B, F, n_iterations, g_k, g_y, g_y1, g_t, g_dt, stream)
+        network = NetworkSweep(lib, method.method_id, f, B, F, n_iterations, g_k, g_y, g_y1, g_t, g_dt, stream, arrays is not None)
 
     def rhs(tt, yy):
         out = f(tt, yy, args) if with_args else f(tt, yy)
@@ -744,7 +767,6 @@ def reverse_sweep_kernels(adjoint, replay: Replay, term, args, problem, dt0_give
         # (two sets of cotangents that take turns instead of copies; entries of the record by their addresses)
         spare = (new(7, B, F), new(B, F), new(B, dt=ttype), new(B, dt=ttype), new(2, B))
         sets = [(g_k, g_y, g_t, g_dt, g_hist), spare]
-        slopes = [x.data_ptr() for x in network.k.unbind(0)]
         places = [(k, x.data_ptr(), x.stride(0) * x.element_size()) for k, x in arrays.items()]
         entry = lambda n: {k: at + n * size for k, at, size in places}
     for n in range(last, -1, -1):
@@ -754,13 +776,13 @@ def reverse_sweep_kernels(adjoint, replay: Replay, term, args, problem, dt0_give
             for i in range(7):
                 ad.g_k[i] = g_k[i].data_ptr()
             ad.g_y, ad.g_t, ad.g_dt, ad.g_prev, ad.g_pprev = (x.data_ptr() for x in (g_y, g_t, g_dt, g_hist[0], g_hist[1]))
-            y1 = network.stages(now)
+            slopes, y1 = network.iteration(n, entry)
             ad.iteration, ad.end_point = n, 0
             ad.t, ad.dt, ad.y, ad.ratio_prev, ad.ratio_pprev = now["t"], now["dt"], now["y"], now["prev"], now["pprev"]
             ad.moved, ad.running_next = moved_all.data_ptr() + 4 * B * n, then["running"]
             for i, at in enumerate([now["k0"], *slopes]):
                 ad.k[i] = at
-            ad.y1 = y1.data_ptr()
+            ad.y1 = y1
             for name, value in zip(("a_y", "a_k0", "a_t", "a_dt", "a_prev", "a_pprev"), adj or [None] * 6):
                 setattr(ad, name, _lib.ptr(value))
             _lib.check(lib.tode_step_finish_backward(aref, cref, stream), "tode_step_finish_backward")

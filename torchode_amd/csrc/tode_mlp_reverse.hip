@@ -219,7 +219,7 @@ template <int METHOD> __global__ void __launch_bounds__(256) __attribute__((amdg
     using Tab = typename std::conditional<METHOD == 1, Tsit5Tab, Dopri5Tab>::type;
     __shared__ MlpReverseShared sh;
     const int tid = threadIdx.x, lane = tid & 63, w = tid >> 6, q = lane >> 4, c = lane & 15, FR = p.n_features, f0 = 16 * w + 4 * q;
-    const long long B = p.batch, tiles = (B + MLP_TILE - 1) / MLP_TILE;
+    const long long B = p.batch, R = p.stage_rows > 0 ? p.stage_rows : B, tiles = (B + MLP_TILE - 1) / MLP_TILE;
     MlpReverseWeights W;
     mlp_load(W, (const float *)p.packed_reverse, tid);
     int slot = 0;
@@ -230,14 +230,14 @@ template <int METHOD> __global__ void __launch_bounds__(256) __attribute__((amdg
         float k[6][4], gk[7][4], gy[4], gy1[4], g_t = 0, g_dt = 0;
         mlp_get((const float *)p.k0 + b * FR, f0, FR, k[0]);
 #pragma unroll
-        for (int s = 1; s < 6; ++s) mlp_get((const float *)p.k + ((s - 1) * B + b) * FR, f0, FR, k[s]);
+        for (int s = 1; s < 6; ++s) mlp_get((const float *)p.k + ((s - 1) * R + b) * FR, f0, FR, k[s]);
 #pragma unroll
         for (int s = 0; s < 7; ++s) mlp_get((const float *)p.g_k + (s * B + b) * FR, f0, FR, gk[s]);
         mlp_get((const float *)p.g_y + b * FR, f0, FR, gy);
         mlp_get((const float *)p.g_y1 + b * FR, f0, FR, gy1);
 #pragma unroll
         for (int s = 6; s >= 1; --s) {
-            const long long row = (s - 1) * B + b;
+            const long long row = (s - 1) * R + b;
             if (live && p.stage_cotangents) mlp_put((float *)p.stage_cotangents + row * FR, f0, FR, gk[s]);  // (final: the weights' gradients read it)
             float gi[4], gt;
             mlp_vjp(sh, W, gk[s], (const float *)p.hidden + row * MLP_H, live && p.hidden_cotangents ? (float *)p.hidden_cotangents + row * MLP_H : nullptr, gi, gt);
@@ -613,6 +613,7 @@ static int check_mlp_reverse(const tode_mlp_reverse *p) {
     if (p->n_features < 1 || p->n_features > MLP_F || p->n_hidden < 1 || p->n_hidden > MLP_H)
         return fail(TODE_E_UNSUPPORTED, "the network's kernels take 1 to %d features and 1 to %d hidden units, got %d and %d", MLP_F, MLP_H, p->n_features, p->n_hidden);
     if (p->batch < 0 || p->batch > (1ll << 40)) return fail(TODE_E_INVALID, "batch %lld", (long long)p->batch);
+    if (p->stage_rows != 0 && p->stage_rows < p->batch) return fail(TODE_E_INVALID, "stage_rows %lld for a batch of %lld", (long long)p->stage_rows, (long long)p->batch);
     if (p->splits < 1 || p->splits > TODE_MLP_MAX_SPLITS) return fail(TODE_E_INVALID, "splits %d", p->splits);
     if (p->batch > 0 && (!p->packed || !p->packed_reverse || !p->t || !p->dt || !p->y || !p->k0 || !p->k || !p->stage_inputs || !p->stage_times || !p->hidden ||
                          !p->g_k || !p->g_y || !p->g_y1 || !p->g_t || !p->g_dt))
