@@ -558,8 +558,8 @@ class NetworkSweep:
         # share of the rows (one per compute unit, at least 64 rows each), so the evaluations of several iterations are
         # kept for one call, as far as they fit into ROOM.
         # Where all of them fit and the record is in arrays, one launch forms the stages of every iteration: they depend on
-        # the record alone, and two workgroups to a compute unit then hide each other's waits (B = 4096, three iterations: three
-        # launches of 28 us, one of 63).
+        # the record alone, and two workgroups to a compute unit then hide each other's waits (B = 4096, three iterations: 90 us
+        # in three launches, 63 in one).
         per_evaluation = 4 * B * (2 * 256 + 3 * F + 1)
         room = max(6, min(6 * iterations + 2, self.ROOM // per_evaluation)) if wanted else 6
         self.held, self.B, self.F = 0, B, F

@@ -59,8 +59,9 @@ static __global__ void mlp_pack_kernel(const float *raw, float *packed, int H, i
 // RECORD: the loop state before every iteration of the workgroup goes to p.rec_* (tode_solve_record), and the state its samples
 // are left in fills the record up to its capacity with `running` 0, as in the small systems' kernels; a record that is too
 // short raises TODE_FLAG_NEEDS_GENERAL (TODE_FLAG_MAX_ITERATIONS says how long it has to be).  For gradients: f there takes the
-// math library's tanh, since it stands where torch's evaluations of the network stood.  Network of 64 and 256 at B = 4096:
-// solve and record in 0.105 ms, where the per-step kernels around torch's products took 2.6 ms.
+// accurate tanh (mlp_tanh_accurate), since it stands where torch's evaluations of the network stood.  Network of 64 and 256 at
+// B = 4096: solve and record in 0.096 ms (0.106 with the math library's tanh and its branches, 2.6 through the per-step kernels
+// around torch's products).
 template <typename Weights> constexpr int mlp_wavefronts = std::is_same<Weights, MlpWeightsBf16>::value ? 3 : 2;  // per SIMD
 
 template <int METHOD, int CTRL, typename Weights, bool FULL, bool RECORD>

@@ -3,8 +3,9 @@
 // weights.  The reference leaves all of it to autograd over its loop (adjoints.py:135-260); through autograd it is, per
 // iteration, six evaluations of the network and six vector-Jacobian products of some fifteen launches each.  Here:
 //
-//   mlp_stages_kernel           all six stages of the iteration again (a tile of 16 samples per workgroup, laid out as in
-//                               the whole-solve kernel), keeping stage inputs, derivatives and hidden activations;
+//   mlp_stages_kernel           all six stages of an iteration again (a tile of 16 samples per workgroup, laid out as in
+//                               the whole-solve kernel), keeping stage inputs, derivatives and hidden activations; of all
+//                               iterations in one launch where their rows fit, since they depend on the record alone;
 //   mlp_stages_backward_kernel  the six stages in reverse: the network's vector-Jacobian product and the stage sums' reverse,
 //                               the cotangents of all stage derivatives in registers between them;
 //   mlp_weight_gradient_kernel  the two outer products over the rows of all evaluations of several iterations, split over
@@ -12,9 +13,10 @@
 //   mlp_weight_gradient_sum_kernel  the splits' sums added in order, once per sweep.
 //
 // What bounds them, network of 64 and 256 at B = 4096 (one workgroup per compute unit, one wavefront per SIMD): six
-// evaluations forward 28 us, back 29 us, of which the matrix cores are busy 10.6 and 10.2 us -- the rest are the round trips
-// through LDS between two products, the stage sums and 150 KB of weights loaded per workgroup; the outer products of 20
-// evaluations 69 us (39 us of matrix instructions, 200 MB of rows at 2.9 TB/s).  A solve and its backward pass: 9.75 ms through
+// evaluations forward 28 us (three iterations in one launch 63 us, two workgroups to a compute unit), back 29 us, of which the
+// matrix cores are busy 10.6 and 10.2 us -- the rest are the round trips through LDS between two products, the stage sums and
+// 150 KB of weights loaded per workgroup; the outer products of 20 evaluations 69 us (39 us of matrix instructions, 200 MB of
+// rows at 2.9 TB/s).  A solve and its backward pass: 9.75 ms through
 // autograd, 0.80 ms.
 //
 // All products are on v_mfma_f32_16x16x4_f32.  For the vector-Jacobian product the weights are packed a second time,
