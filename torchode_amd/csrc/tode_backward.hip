@@ -52,6 +52,16 @@ template <typename T, int F> __device__ __forceinline__ RecordEntry<T, F> load_e
     return r;
 }
 
+// A loaded entry waited for here and not where its values are copied at the end of the iteration: there the wait is behind the
+// loads of the next evaluation points, and would be for those too.
+template <typename T, int F> __device__ __forceinline__ void entry_is_here(RecordEntry<T, F> &r) {
+#if defined(__HIP_DEVICE_COMPILE__)
+    asm volatile("" : "+v"(r.t), "+v"(r.dt), "+v"(r.prev), "+v"(r.pprev), "+v"(r.running), "+v"(r.n_accepted));
+#pragma unroll
+    for (int f = 0; f < F; ++f) asm volatile("" : "+v"(r.y[f]), "+v"(r.k0[f]));
+#endif
+}
+
 // cotangent shares of minimum(a, b) (or maximum with the comparison turned round) for operand a: all of it where a
 // is the one taken, half on a tie (torch.minimum / torch.maximum)
 template <typename T> __device__ __forceinline__ T share_of_min(T a, T b) { return a < b ? (T)1 : (a == b ? (T)0.5 : (T)0); }
@@ -210,7 +220,8 @@ template <typename T> struct Dividends {
 // times, first for the number of its points, then for each point's index, then for its time and cotangent: Van der Pol float32,
 // B = 65536, 50 points: 0.76 ms and 0.05 ms for the two kernels; 0.66 ms this way.)  What remains is instructions: the
 // divisions, the square root and the two powers in the short forms of tode_math.h wherever the wavefront's operands allow
-// them, 0.66 -> 0.53 ms; float64, B = 20 000: 0.60 -> 0.56; decay with eight features, B = 20 000: 0.51 -> 0.43.
+// them, 0.66 -> 0.53 ms; and the waits for what was loaded ahead only where it is used (they stood behind each point's index,
+// and at the end of the iteration behind the copies of the record's entry): 0.53 -> 0.46, float64, B = 20 000, 0.56 -> 0.49.
 template <typename T, int METHOD, int CTRL, typename Term>
 __global__ void __launch_bounds__(64) whole_backward_kernel(const WholeBackward<T> w) {
     using Tab = typename std::conditional<METHOD == 1, Tsit5Tab, Dopri5Tab>::type;
@@ -247,10 +258,22 @@ __global__ void __launch_bounds__(64) whole_backward_kernel(const WholeBackward<
     const T dir = te > ts ? (T)1 : (T)-1;
     const int32_t *its = nullptr, *pts = nullptr;
     int lowest = 0, cursor = E - 1;
+    bool listed = false;  // (a mask's truth, the same in all lanes: a scalar branch)
     if (E > 0) {
         bool in_order = w.points_by_iteration == nullptr;
-        for (int e = 1; in_order && e < E; ++e) in_order = dir * t_eval[e - 1] <= dir * t_eval[e];  // (false for a time that is not a number)
-        if (lanes_where(!in_order)) {
+        T last = t_eval[0];
+        for (int e = 1; in_order && e < E; e += 8) {  // (eight loads on the way at a time: one by one they were fifty trips to memory)
+            T next[8];
+#pragma unroll
+            for (int j = 0; j < 8; ++j) next[j] = t_eval[min(e + j, E - 1)];
+#pragma unroll
+            for (int j = 0; j < 8; ++j) {  // (false for a time that is not a number)
+                in_order = in_order && dir * last <= dir * next[j];
+                last = next[j];
+            }
+        }
+        listed = lanes_where(!in_order) != 0;
+        if (listed) {
             its = w.iterations_sorted + g * E, pts = w.points_by_iteration + g * E;
             if (w.points_by_iteration == nullptr) {
                 int32_t *const own = w.lists + g * E, *const own_points = own + B * E;
@@ -262,18 +285,23 @@ __global__ void __launch_bounds__(64) whole_backward_kernel(const WholeBackward<
             while (cursor >= lowest && dir * after.t < dir * t_eval[cursor]) --cursor;  // (never reached)
         }
     }
-    const bool listed = its != nullptr;
     T at[AHEAD], g_at[AHEAD][F];
     int32_t written_by[AHEAD];
+    // (All indices before all values: an index taken from the lists, or the bare chance of one, is waited for where it is used, and
+    // one at a time those waits stood behind the values of the point before.)
     auto load_ahead = [&]() {
+        int e[AHEAD];
+#pragma unroll
+        for (int p = 0; p < AHEAD; ++p) e[p] = max(cursor - p, 0), written_by[p] = 0;
+        if (listed) {
+#pragma unroll
+            for (int p = 0; p < AHEAD; ++p) written_by[p] = its[e[p]], e[p] = pts[e[p]];
+        }
 #pragma unroll
         for (int p = 0; p < AHEAD; ++p) {
-            int e = max(cursor - p, 0);
-            written_by[p] = 0;
-            if (listed) written_by[p] = its[e], e = pts[e];
-            at[p] = t_eval[e];
+            at[p] = t_eval[e[p]];
 #pragma unroll
-            for (int f = 0; f < F; ++f) g_at[p][f] = grad_ys[(long long)e * F + f];
+            for (int f = 0; f < F; ++f) g_at[p][f] = grad_ys[(long long)e[p] * F + f];
         }
     };
     if (E > 0) {
@@ -285,12 +313,13 @@ __global__ void __launch_bounds__(64) whole_backward_kernel(const WholeBackward<
     }
 
     for (long long i = L - 1; i >= 0; --i) {
-        const RecordEntry<T, F> before = load_entry<T, F>(w, i > 0 ? i - 1 : 0, g);  // (used by the next pass of this loop)
+        RecordEntry<T, F> before = load_entry<T, F>(w, i > 0 ? i - 1 : 0, g);  // (used by the next pass of this loop)
         const bool end_point = E == 0 && i == L - 1;
         // An iteration that none of the wavefront's samples took part in (all had finished before it) changes nothing for
         // them -- no move, no point written, the step and the history kept -- so its reverse hands every cotangent on as
         // it is.  (Without evaluation points the batch's last iteration is the one whose interpolant gives the result.)
         if (!end_point && !lanes_where(here.running != 0)) {
+            if constexpr (SHORT) entry_is_here(before);
             after = here, here = before;
             continue;
         }
@@ -595,6 +624,7 @@ __global__ void __launch_bounds__(64) whole_backward_kernel(const WholeBackward<
                 add_point(at[p], g_at[p], g_time);
             }
         }
+        if constexpr (SHORT) entry_is_here(before);  // (eight doubles a row: no registers for it)
         if (E > 0) {
             cursor -= n;
             load_ahead();
