@@ -799,6 +799,29 @@ def test_points_of_the_whole_sweep_against_lists_handed_in(rows, features, dtype
 
 
 @pytest.mark.gpu
+@pytest.mark.parametrize("E,swapped", [(2, None), (3, 1), (8, None), (9, 7), (10, 8), (12, 8), (12, 9), (12, 10), (17, 15), (18, 16)])
+def test_order_of_a_row_is_checked_to_its_last_point(E, swapped):
+    """The whole sweep looks at eight times of a row at once for their order: one pair of neighbours out of order, `swapped` and
+    the next, on either side of eight's edges and at the row's end, against lists made by torch operations: the same bits."""
+    B = 5
+    g = torch.Generator().manual_seed(E)
+    k, y0 = (0.1 + 3 * torch.rand(B, 2, generator=g)).cuda(), (torch.rand(B, 2, generator=g) * 2 - 1).cuda()
+    t_eval = torch.linspace(0.1, 2, E)[None, :].repeat(B, 1)
+    if swapped is not None:
+        t_eval[3, [swapped, swapped + 1]] = t_eval[3, [swapped + 1, swapped]]
+    cotangent = torch.randn(B, E, 2, generator=g).cuda()
+    results = []
+    for lists in (False, True):
+        leaf, y = k.clone().requires_grad_(), y0.clone().requires_grad_()
+        solver = to.AutoDiffAdjoint(to.Tsit5(), to.PIDController(1e-6, 1e-3, 0.2, 0.5, 0.0))
+        solver.backward_points_in_torch = lists
+        problem = to.InitialValueProblem(y, torch.zeros(B).cuda(), torch.full((B,), 2.0).cuda(), t_eval.cuda())
+        results.append(torch.autograd.grad(solver.solve(problem, to.ODETerm(to.LinearDecay(leaf))).ys, [y, leaf], cotangent))
+    for a, b in zip(*results):
+        assert bool(a.isfinite().all()) and bool((a != 0).any()) and torch.equal(a, b)
+
+
+@pytest.mark.gpu
 @pytest.mark.parametrize("features", [3, 4, 8])
 @pytest.mark.parametrize("method,kind", [(to.Dopri5, "integral"), (to.Dopri5, "pid"), (to.Tsit5, "integral"), (to.Tsit5, "pid")])
 def test_whole_sweep_kernel_when_every_sample_has_used_up_its_points(method, kind, features):
