@@ -24,7 +24,7 @@
 extern "C" {
 #endif
 
-#define TODE_ABI_VERSION 24
+#define TODE_ABI_VERSION 25
 
 /* floating point type of data (y) and time (t) arrays */
 enum { TODE_F32 = 0, TODE_F64 = 1 };
@@ -702,7 +702,7 @@ typedef struct tode_solve_adjoint {
     const int32_t *iterations_sorted;   /* [B,E]: those iterations in the same order, ascending; -1 (first) for a point that
                                            no iteration wrote.  Both NULL when E == 0 -- or to have the sweep tell by
                                            the record's times (it needs lists only for rows of times in no order, and
-                                           makes them in `scratch`) */
+                                           makes them in `scratch`; tode_solve_backward_lists is quicker) */
     int64_t iterations;            /* L: iterations of the loop; the record's entries 0..L are read */
     int32_t through_control;       /* as in tode_step_adjoint */
     int32_t through_start;         /* 0: the results are the cotangents of the loop's first state.  1: the kernel also
@@ -727,6 +727,16 @@ typedef struct tode_solve_adjoint {
     void *g_t_eval;                /* [B,E], added to; NULL: not wanted */
 } tode_solve_adjoint;
 int64_t tode_solve_backward_scratch_bytes(const tode_solve_args *args);
+/*
+ * Rows of t_eval that do not run in the direction of their solve, long ones: the sweep makes its lists for such a row with one thread,
+ * and many times the threads are quicker.  tode_mark_unordered_rows sets args->flags[TODE_FLAG_NON_MONOTONE] where there is one
+ * (launched behind a solve with a pending mask, which leaves the word at 0); tode_solve_backward_lists makes the two lists of
+ * tode_solve_adjoint from the record's times into adjoint->scratch, iterations_sorted first and points_by_iteration behind it
+ * ([B,E] each), for the caller to hand in.  Of *args the times with their strides, the sizes and (lists) the record are read, of
+ * *adjoint the iterations and the scratch.  TODE_E_UNSUPPORTED (more points than one launch takes): leave the lists to the sweep.
+ */
+int tode_mark_unordered_rows(const tode_solve_args *args, void *stream);
+int tode_solve_backward_lists(const tode_solve_args *args, const tode_solve_adjoint *adjoint, void *stream);
 int tode_solve_builtin_backward(const tode_solve_args *args, const tode_controller *controller, const tode_solve_adjoint *adjoint, void *stream);
 
 /* ------------------------------------------------------------------------------------------

@@ -11,7 +11,7 @@ import torch.nn as nn
 
 import torchode_amd as to
 from oracle import torch_loop
-from torchode_amd import autodiff
+from torchode_amd import _lib, autodiff
 from torchode_amd.autodiff import Replay, simulate_hits
 
 gpu = pytest.mark.gpu
@@ -768,12 +768,13 @@ def test_whole_sweep_kernel_agrees_with_the_per_iteration_kernels_and_the_torch_
 @pytest.mark.gpu
 @pytest.mark.parametrize("features,dtype", [(2, torch.float32), (2, torch.float64), (4, torch.float32), (8, torch.float32), (8, torch.float64)])
 @pytest.mark.parametrize("rows", ["ordered", "some-shuffled", "repeated", "beyond-the-end"])
-def test_points_of_the_whole_sweep_against_lists_handed_in(rows, features, dtype):
+@pytest.mark.parametrize("E", [61, 83])
+def test_points_of_the_whole_sweep_against_lists_handed_in(E, rows, features, dtype):
     """Which points an iteration wrote, found by walking rows of times (the points held in registers ahead and further ones), or
     by lists where a wavefront has a row in no order, against lists made by torch operations: the same bits.  150 samples are
     three wavefronts, of which the middle one alone has shuffled rows; 61 points in a dozen steps are many more than are held;
     repeated points lie at t_start and on the ends of steps (a point of another row's); points beyond t_end are never reached."""
-    B, E = 150, 61
+    B = 150
     g = torch.Generator().manual_seed(11)
     k = (0.1 + 3 * torch.rand(B, features, generator=g, dtype=torch.float64)).to(dtype).cuda()
     y0 = (torch.rand(B, features, generator=g, dtype=torch.float64) * 2 - 1).to(dtype).cuda()
@@ -787,15 +788,70 @@ def test_points_of_the_whole_sweep_against_lists_handed_in(rows, features, dtype
         t_end = t_eval[:, 40].clone()
     cotangent = torch.randn(B, E, features, generator=g, dtype=torch.float64).to(dtype).cuda()
     results = []
-    for lists in (False, True):
+    for lists in ("torch", "ahead", "sweep"):  # (made by torch operations; by kernels in front, where a row is in no order; by the sweep)
         leaf, y = k.clone().requires_grad_(), y0.clone().requires_grad_()
         solver = to.AutoDiffAdjoint(to.Tsit5(), to.PIDController(1e-6, 1e-3, 0.2, 0.5, 0.0))
-        solver.backward_points_in_torch = lists
+        solver.backward_points_in_torch, solver.backward_lists_ahead = lists == "torch", lists == "ahead"
         sol = solver.solve(to.InitialValueProblem(y, t_start.cuda(), t_end.cuda(), t_eval.cuda()), to.ODETerm(to.LinearDecay(leaf)))
         ys = torch.where(sol.ys.detach().isfinite(), sol.ys, torch.zeros_like(sol.ys))
         results.append(torch.autograd.grad(ys, [y, leaf], cotangent if rows != "beyond-the-end" else cotangent * (torch.arange(E, device="cuda") < 40)[None, :, None]))
-    for a, b in zip(*results):
-        assert bool(a.isfinite().all()) and bool((a != 0).any()) and torch.equal(a, b)
+    for a, b, c in zip(*results):
+        assert bool(a.isfinite().all()) and bool((a != 0).any()) and torch.equal(a, b) and torch.equal(a, c)
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("dtype", [torch.float32, torch.float64])
+@pytest.mark.parametrize("B,E,L", [(1, 1, 0), (1, 1, 1), (3, 2, 5), (65, 300, 1), (257, 33, 40)])
+def test_lists_of_a_batch_with_rows_in_no_order(B, E, L, dtype):
+    """tode_solve_backward_lists against plain Python: both directions, points on recorded times, in front of the start and behind
+    the end, a first point at t_start, one that is not a number, rejected steps (times that repeat), and the columns of a wider array
+    as start and end."""
+    g = torch.Generator().manual_seed(B + E + L)
+    sign = torch.where(torch.rand(B, generator=g) < 0.5, -1.0, 1.0).to(dtype)
+    t = torch.cat([torch.randn(1, B, generator=g), torch.rand(L, B, generator=g) * (torch.rand(L, B, generator=g) < 0.7)]).cumsum(0).to(dtype)
+    at = (torch.rand(B, E, generator=g).to(dtype) * 1.4 - 0.2) * (t[-1] - t[0])[:, None] + t[0][:, None]
+    on = torch.gather(t.T, 1, torch.randint(0, L + 1, (B, E), generator=g))
+    at = torch.where(torch.rand(B, E, generator=g) < 0.4, on, at)
+    at[::2, 0], at[-1, -1] = t[0, ::2], (float("nan") if E > 1 else at[-1, -1])
+    t, at = sign * t, sign[:, None] * at
+    ends = torch.stack([t[0], t[0] + sign], dim=1).contiguous().cuda()
+    dev_t, dev_at = t.contiguous().cuda(), at.contiguous().cuda()
+    lists = torch.full((2, B, E), 77, dtype=torch.int32, device="cuda")
+    rec = _lib.SolveRecord(L + 1, dev_t.data_ptr())
+    a, ad = _lib.SolveArgs(), _lib.SolveAdjoint()
+    a.dtype, a.n_features, a.n_eval, a.batch = _lib.DTYPES[dtype], 2, E, B
+    a.t_start, a.t_end, a.t_start_stride, a.t_end_stride, a.t_eval = ends.data_ptr(), ends.data_ptr() + ends.element_size(), 2, 2, dev_at.data_ptr()
+    a.record, ad.iterations, ad.scratch, ad.scratch_bytes = _lib.C.addressof(rec), L, lists.data_ptr(), 4 * lists.numel()
+    assert _lib.load().tode_solve_backward_lists(_lib.C.byref(a), _lib.C.byref(ad), _lib.stream_of(ends)) == 0
+    for b in range(B):
+        hits = []
+        for e in range(E):
+            v = float(sign[b] * at[b, e])
+            reached = [i for i in range(L) if not float(sign[b] * t[i + 1, b]) < v]
+            hits.append(-1 if not reached or (e == 0 and at[b, 0] == t[0, b]) else reached[0])
+        order = sorted(range(E), key=lambda e: hits[e])
+        assert lists[1, b].tolist() == order and lists[0, b].tolist() == [hits[e] for e in order]
+    ad.scratch_bytes -= 1  # (refused on the host)
+    assert _lib.load().tode_solve_backward_lists(_lib.C.byref(a), _lib.C.byref(ad), _lib.stream_of(ends)) == _lib.E_INVALID
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("unordered,points", [(False, 200), (True, 200), (True, 65), (True, 64)])
+def test_lists_are_made_ahead_where_a_row_is_in_no_order(unordered, points, monkeypatch):
+    """A batch with a long row of times in no order has its lists made with a thread to a point: the sweep, which looks a row's points up
+    one after the other, took up to 1.4 times as long.  The last neighbours of the last row are the ones out of order."""
+    lib, made = _lib.load(), []
+    make = lib.tode_solve_backward_lists
+    monkeypatch.setattr(lib, "tode_solve_backward_lists", lambda *args: made.append(1) or make(*args))
+    t_eval = torch.linspace(0, 1, points).repeat(70, 1)
+    if unordered:
+        t_eval[-1, [-2, -1]] = t_eval[-1, [-1, -2]]
+    y, rate = torch.ones(70, 2, device="cuda", requires_grad=True), torch.ones(70, 2, device="cuda", requires_grad=True)
+    solver = to.AutoDiffAdjoint(to.Tsit5(), to.IntegralController(1e-6, 1e-3))
+    for _ in range(2):
+        ys = solver.solve(to.InitialValueProblem(y, t_eval=t_eval.cuda()), to.ODETerm(to.LinearDecay(rate))).ys
+        torch.autograd.grad(ys.sum(), [y, rate])
+    assert len(made) == (2 if unordered and points > 64 else 0)
 
 
 @pytest.mark.gpu
@@ -814,7 +870,7 @@ def test_order_of_a_row_is_checked_to_its_last_point(E, swapped):
     for lists in (False, True):
         leaf, y = k.clone().requires_grad_(), y0.clone().requires_grad_()
         solver = to.AutoDiffAdjoint(to.Tsit5(), to.PIDController(1e-6, 1e-3, 0.2, 0.5, 0.0))
-        solver.backward_points_in_torch = lists
+        solver.backward_points_in_torch, solver.backward_lists_ahead = lists, False
         problem = to.InitialValueProblem(y, torch.zeros(B).cuda(), torch.full((B,), 2.0).cuda(), t_eval.cuda())
         results.append(torch.autograd.grad(solver.solve(problem, to.ODETerm(to.LinearDecay(leaf))).ys, [y, leaf], cotangent))
     for a, b in zip(*results):

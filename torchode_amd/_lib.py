@@ -13,8 +13,12 @@ import torch
 _HERE = os.path.dirname(os.path.abspath(__file__))
 LIB_PATH = os.path.join(_HERE, "libtorchode_amd.so")
 
-ABI_VERSION = 24
+ABI_VERSION = 25
 END_ONLY_MAX_BATCH = 2048 * 64  # TODE_END_ONLY_MAX_BATCH
+# Rows of more evaluation points have lists made ahead of a reverse sweep where one is in no order; shorter ones the sweep looks up by
+# itself, which spares every pass the look at the rows' order (Van der Pol, B = 65 536, two points of every row swapped: 50
+# points 0.65 ms of sweep in float32 and 0.87 in float64; 65 points 0.76 and 1.01, with the lists made ahead 0.60 and 0.75).
+LISTS_AHEAD_POINTS = 64
 MLP_PACKED_SIZE = {"float32": 152 * 256, "bfloat16": 92 * 256}
 MLP_SUMS_SIZE, MLP_REVERSE_PACKED_SIZE = 64 * 256 + 256 + 256 + 64 * 256 + 64, 144 * 256  # TODE_MLP_*_SIZE
 MLP_INPUTS = {"float32": 0, "bfloat16": 1}
@@ -45,6 +49,8 @@ EXPORTS = (
     "tode_solve_builtin_end",
     "tode_solve_builtin_backward",
     "tode_solve_backward_scratch_bytes",
+    "tode_solve_backward_lists",
+    "tode_mark_unordered_rows",
     "tode_solve_workspace_bytes",
     "tode_mlp_pack_weights",
     "tode_mlp_pack_weights_for",
@@ -394,6 +400,10 @@ def load():
         lib.tode_solve_builtin_end.argtypes = [C.POINTER(SolveTicket), C.POINTER(SolveArgs), C.c_void_p, C.c_void_p, C.POINTER(C.c_int32)]
         lib.tode_solve_backward_scratch_bytes.restype = C.c_int64
         lib.tode_solve_backward_scratch_bytes.argtypes = [C.POINTER(SolveArgs)]
+        lib.tode_mark_unordered_rows.restype = C.c_int
+        lib.tode_mark_unordered_rows.argtypes = [C.POINTER(SolveArgs), C.c_void_p]
+        lib.tode_solve_backward_lists.restype = C.c_int
+        lib.tode_solve_backward_lists.argtypes = [C.POINTER(SolveArgs), C.POINTER(SolveAdjoint), C.c_void_p]
         lib.tode_solve_builtin_backward.restype = C.c_int
         lib.tode_solve_builtin_backward.argtypes = [C.POINTER(SolveArgs), C.POINTER(Controller), C.POINTER(SolveAdjoint), C.c_void_p]
         lib.tode_step_begin.restype = C.c_int

@@ -700,6 +700,10 @@ class AutoDiffAdjoint(nn.Module):
             again.iteration_cap = L
             again.record = _lib.C.addressof(rec)
             _lib.check(lib.tode_solve_builtin(_lib.C.byref(again), _lib.C.byref(ctrl), stream), "tode_solve_builtin")
+            if E > _lib.LISTS_AHEAD_POINTS and dtype == ttype:
+                rc = lib.tode_mark_unordered_rows(_lib.C.byref(again), stream)
+                if rc != _lib.E_UNSUPPORTED:  # (more points than one launch takes: not marked)
+                    _lib.check(rc, "tode_mark_unordered_rows")
             record.flags = flags  # (looked at when the backward pass starts: no second wait for the GPU here)
             self._remember_record_entries((B, F, E, dtype, f.builtin_kind), n + 4)  # (the next recording solve of a batch like this one tries it in one kernel)
             record.iterations = L

@@ -128,6 +128,7 @@ class LoopRecord:
         self.arrays = None  # the same record as entry-major arrays, where the whole-solve kernel wrote it
         self.wrote_points = False  # known without a look at the device: some iteration wrote an evaluation point
         self.flags = None  # that kernel's flag words, still on the device
+        self.unordered_rows = False  # some row of evaluation points does not run in the direction of its solve
 
     def snapshot(self, t, dt, y, k0, hist, ints):
         self.states.append((t.clone(), dt.clone(), y.clone(), k0.clone(), hist[0].clone(), hist[1].clone(), ints[0].clone(), ints[3].clone()))
@@ -437,7 +438,8 @@ def reverse_sweep_whole(adjoint, replay: Replay, term, problem, dt0, record, gra
     L, arrays = record.iterations, record.arrays
 
     # Which iteration wrote which evaluation point (adjoints.py:215-234: the first whose new time has passed it): the kernel
-    # tells by the record's times.  The same in torch operations, as lists handed in, for the tests to hold against that.
+    # tells by the record's times, or by lists where the forward pass met a row in no order.  The same in torch operations, as
+    # lists handed in, for the tests to hold against that.
     iterations_sorted = points_by_iteration = None
     if E > 0 and getattr(adjoint, "backward_points_in_torch", False):
         direction = torch.where(t_end > t_start, 1.0, -1.0).to(dtype)
@@ -481,6 +483,11 @@ def reverse_sweep_whole(adjoint, replay: Replay, term, problem, dt0, record, gra
         a.dt0 = dt0.data_ptr()  # (not read: it says that the first step was given)
     ad.scratch, ad.scratch_bytes = scratch.data_ptr(), scratch.numel()
     ad.points_by_iteration, ad.iterations_sorted = _lib.ptr(points_by_iteration), _lib.ptr(iterations_sorted)
+    if E > 0 and record.unordered_rows and iterations_sorted is None and getattr(adjoint, "backward_lists_ahead", True):
+        rc = lib.tode_solve_backward_lists(_lib.C.byref(a), _lib.C.byref(ad), _lib.stream_of(y0))
+        if rc != _lib.E_UNSUPPORTED:  # (more points than one launch takes: the sweep makes its lists by itself)
+            _lib.check(rc, "tode_solve_backward_lists")
+            ad.iterations_sorted, ad.points_by_iteration = scratch.data_ptr(), scratch.data_ptr() + 4 * B * E
     ad.a_y, ad.a_k0 = out_y.data_ptr(), out_k0.data_ptr()
     ad.a_t, ad.a_dt, ad.a_prev, ad.a_pprev = (out_s[i].data_ptr() for i in range(4))
     ad.g_params = g_par.data_ptr()
@@ -912,8 +919,11 @@ class SolveThroughLoop(torch.autograd.Function):
         adjoint, problem, term, params = ctx.adjoint, ctx.problem, ctx.term, list(ctx.params)
         if grad_ys is None:
             grad_ys = torch.zeros((problem.batch_size, max(problem.n_evaluation_points, 1), problem.n_features), dtype=problem.data_dtype, device=problem.device)
-        if ctx.record.flags is not None and ctx.record.flags.tolist()[_lib.FLAG_NEEDS_GENERAL]:
-            raise RuntimeError("the record of the loop state was too short for the solve it was sized from")
+        if ctx.record.flags is not None:
+            flags = ctx.record.flags.tolist()
+            if flags[_lib.FLAG_NEEDS_GENERAL]:
+                raise RuntimeError("the record of the loop state was too short for the solve it was sized from")
+            ctx.record.unordered_rows = bool(flags[_lib.FLAG_NON_MONOTONE])
         # (a second initialized point of some sample was written by an iteration: the usual case, told by one reduction)
         some_iteration_wrote = problem.n_evaluation_points > 1 and (ctx.record.wrote_points or int(ctx.n_initialized.max()) > 1)
         if problem.n_evaluation_points > 0 and not some_iteration_wrote and not ctx.record.any_point_written(problem):

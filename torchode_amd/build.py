@@ -60,6 +60,7 @@ UNITS = [
     ("tode_stepwise.hip", "tode_stepwise.o", []),
     ("tode_backward.hip", "tode_backward_f32.o", ["-DTODE_INSTANTIATE_F32=1"]),
     ("tode_backward.hip", "tode_backward_f64.o", ["-DTODE_INSTANTIATE_F64=1"]),
+    ("tode_backward_lists.hip", "tode_backward_lists.o", []),
     ("tode_ops.hip", "tode_ops.o", []),
     ("tode_grid.hip", "tode_grid.o", []),
     ("tode_mlp.hip", "tode_mlp.o", []),

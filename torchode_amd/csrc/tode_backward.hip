@@ -176,7 +176,8 @@ __device__ __forceinline__ void start_backward(const CtrlParams<T> &cp, const Te
 // a point at t_start, which the loop's set-up writes, and for one the solve never reached), for a row of times in no order:
 // a binary search over the sample's recorded times for each point, and the points sorted by insertion (stable: points of one
 // iteration stay in their order).  One thread per sample; rows whose times run in the direction of the solve, nearly all
-// there are, never come here (the sweep meets their points in order).
+// there are, never come here (the sweep meets their points in order), and long ones in no order have their lists handed in
+// (tode_solve_backward_lists).
 template <typename T>
 __device__ __forceinline__ void list_points(const WholeBackward<T> &w, const long long sample, const T ts, const T dir, const T *t_eval, int32_t *its, int32_t *pts) {
     for (int e = 0; e < w.E; ++e) {
