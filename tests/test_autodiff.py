@@ -858,8 +858,14 @@ def test_lists_are_made_ahead_where_a_row_is_in_no_order(unordered, points, monk
 @pytest.mark.parametrize("E,swapped", [(2, None), (3, 1), (8, None), (9, 7), (10, 8), (12, 8), (12, 9), (12, 10), (17, 15), (18, 16)])
 def test_order_of_a_row_is_checked_to_its_last_point(E, swapped):
     """The whole sweep looks at eight times of a row at once for their order: one pair of neighbours out of order, `swapped` and
-    the next, on either side of eight's edges and at the row's end, against lists made by torch operations: the same bits."""
-    B = 5
+    the next, on either side of eight's edges and at the row's end, against lists made by torch operations: the same bits.
+    No step but the first, which ends at the first point at the latest, is longer than half the way from one point to the next, so
+    swapped points lie in different steps: a row taken for one in order would have the earlier point hide the later one from
+    its own step."""
+    import torchode_amd.autodiff as autodiff
+
+    B, dt_max = 5, 0.05
+    assert E == 2 or 1.9 / (E - 1) > 2 * dt_max
     g = torch.Generator().manual_seed(E)
     k, y0 = (0.1 + 3 * torch.rand(B, 2, generator=g)).cuda(), (torch.rand(B, 2, generator=g) * 2 - 1).cuda()
     t_eval = torch.linspace(0.1, 2, E)[None, :].repeat(B, 1)
@@ -869,10 +875,12 @@ def test_order_of_a_row_is_checked_to_its_last_point(E, swapped):
     results = []
     for lists in (False, True):
         leaf, y = k.clone().requires_grad_(), y0.clone().requires_grad_()
-        solver = to.AutoDiffAdjoint(to.Tsit5(), to.PIDController(1e-6, 1e-3, 0.2, 0.5, 0.0))
+        solver = to.AutoDiffAdjoint(to.Tsit5(), to.PIDController(1e-6, 1e-3, 0.2, 0.5, 0.0, dt_max=dt_max))
         solver.backward_points_in_torch, solver.backward_lists_ahead = lists, False
         problem = to.InitialValueProblem(y, torch.zeros(B).cuda(), torch.full((B,), 2.0).cuda(), t_eval.cuda())
-        results.append(torch.autograd.grad(solver.solve(problem, to.ODETerm(to.LinearDecay(leaf))).ys, [y, leaf], cotangent))
+        sol = solver.solve(problem, to.ODETerm(to.LinearDecay(leaf)))
+        results.append(torch.autograd.grad(sol.ys, [y, leaf], cotangent))
+        assert autodiff.LAST_SWEEP == "whole" and int(sol.stats["n_accepted"].min()) >= 39  # (38 dt_max and a first step of 0.1 at most)
     for a, b in zip(*results):
         assert bool(a.isfinite().all()) and bool((a != 0).any()) and torch.equal(a, b)
 
