@@ -269,3 +269,36 @@ def test_what_a_sweep_needs_of_its_record(batch, points, iterations, sign):
     assert torch.equal(hits.cpu(), hit) and torch.equal(t_start, ends[:, 0]) and torch.equal(t_end, ends[:, 1])
     if iterations:
         assert torch.equal(moved.cpu(), (accepted[1:] > accepted[:-1]).to(torch.int32))
+
+
+def test_hidden_units_against_tanh_in_float64():
+    """The gradient's kernels' tanh, seen through a network whose hidden unit u is tanh of state value u (one weight of one, the
+    rest zeros: the matrix cores pass the value on exactly): magnitudes from 2^-20 to 10, the neighbours of 1, where its two forms
+    meet, saturation and zero.  At most 2.5 units in the last place: 1.8 from the argument's, exponential's and reciprocal's
+    roundings (a quarter of which reaches the result where the exponential form begins, less beyond) or 1.3 from the
+    polynomial's, and half a unit from the last operation.  In the mean 0.35, where correct rounding has 0.25."""
+    B = 4096
+    g = torch.Generator("cuda").manual_seed(3)
+    rand = lambda *shape: torch.rand(shape, generator=g, dtype=torch.float64, device="cuda")
+    y = (2.0 ** (-20 + (20 + math.log2(10.0)) * rand(B, 64))).float()
+    y[: B // 4] = (3 * torch.randn(B // 4, 64, generator=g, dtype=torch.float64, device="cuda")).float()
+    near = (torch.ones(64, device="cuda").view(torch.int32) + torch.arange(-32, 32, device="cuda", dtype=torch.int32)).view(torch.float32)
+    y[0], y[1], y[2] = near, -near, torch.linspace(8, 10, 64, device="cuda")
+    y[3, :6] = torch.tensor([0.0, -0.0, 30.0, -30.0, 1e30, -1e30], device="cuda")
+    y[4::2] = -y[4::2]
+    W1 = torch.zeros(256, 65, device="cuda")
+    W1[torch.arange(256), torch.arange(256) % 64] = 1.0
+    zeros = lambda *shape: torch.zeros(shape, device="cuda")
+    f = to.MLPField(W1, zeros(256), zeros(64, 256), zeros(64))
+    packed = f.builtin_packed(y.device, torch.float32)
+    t, dt, k0, k, inputs, times, hidden, unused = zeros(B), zeros(B), zeros(B, 64), zeros(6, B, 64), zeros(6, B, 64), zeros(6, B), zeros(6, B, 256) + 7, zeros(7, B, 64)
+    p = _lib.MlpReverse(0, 64, 256, 1, B, packed.data_ptr(), packed.data_ptr(), t.data_ptr(), dt.data_ptr(), y.data_ptr(), k0.data_ptr(), k.data_ptr(), inputs.data_ptr(),
+                        times.data_ptr(), hidden.data_ptr(), None, None, *([unused.data_ptr()] * 5))  # fmt: skip
+    _lib.check(_lib.load().tode_mlp_stages(_lib.C.byref(p), _lib.stream_of(y)), "tode_mlp_stages")
+    assert torch.equal(inputs, y.expand(6, B, 64))  # (steps of zero: every stage's input is the state)
+    want = torch.tanh(y.double())
+    _, exponent = torch.frexp(want)
+    unit = torch.where(want == 0, 1.0, torch.ldexp(torch.ones_like(want), exponent - 24))
+    off = (hidden.view(6, B, 4, 64).double() - want[None, :, None, :]).abs() / unit[None, :, None, :]
+    print("units in the last place: most", float(off.max()), "mean", float(off.mean()))
+    assert float(off.max()) <= 2.5 and float(off.mean()) <= 0.35
