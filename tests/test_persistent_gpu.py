@@ -596,6 +596,61 @@ def test_flags_on_the_host_over_more_calls_than_there_are_slots_and_when_the_bat
     assert _fast_call(empty, sync=True)[2] == [0, 2**31 - 1, 0, 0]
 
 
+def test_tickets_end_in_any_order_and_their_slots_come_back():
+    """tode_solve_builtin_begin / _end with every one of the 64 slots of a device held at once, of three batch sizes: one begin more
+    is refused before anything is launched, tickets end in the reverse order with the results and flags of tode_solve_builtin_auto,
+    and after that all slots are free again."""
+    from torchode_amd import _lib
+
+    lib = _lib.load()
+    by = _lib.C.byref
+
+    def call(w):
+        B, F = w.y0.shape
+        E, params = w.t_eval.shape[1], w.f.builtin_params()
+        ys, out = torch.full((B, E, F), float("nan"), dtype=F32, device="cuda"), torch.full((4, B), -7, dtype=torch.int64, device="cuda")
+        spec = dict(w.controller)
+        ctrl = {"pid": to.PIDController, "integral": to.IntegralController}[spec.pop("kind")](**spec).c_struct()
+        a = _lib.SolveArgs()
+        a.dtype, a.method, a.term = _lib.DTYPES[F32], {"dopri5": 0, "tsit5": 1}[w.method], w.f.builtin_kind
+        a.n_features, a.n_eval, a.n_params, a.batch, a.max_steps, a.iteration_cap = F, E, params.shape[1], B, -1, -1
+        a.y0, a.t_start, a.t_end, a.t_eval = w.y0.data_ptr(), w.t_eval[:, 0].data_ptr(), w.t_eval[:, -1].data_ptr(), w.t_eval.data_ptr()
+        a.t_start_stride = a.t_end_stride = E
+        a.params, a.ys = params.data_ptr(), ys.data_ptr()
+        return a, ctrl, ys, out, params
+
+    workloads = [to.workloads.make("vdp", batch=batch, dtype=F32, device="cuda") for batch in (1, 70, 300)]
+    stream = _lib.stream_of(workloads[0].y0)
+    want = []
+    for w in workloads:
+        a, ctrl, ys, out, _ = call(w)
+        workspace, iterations = torch.empty(lib.tode_solve_workspace_bytes(by(a)), dtype=torch.uint8, device="cuda"), _lib.C.c_int64(-1)
+        rc = lib.tode_solve_builtin_auto(by(a), by(ctrl), *(_lib.ptr(out[i]) for i in range(4)), workspace.data_ptr(), workspace.numel(), 1, stream, by(iterations))
+        _lib.check(rc, "tode_solve_builtin_auto")
+        want.append((ys, out, iterations.value))
+    calls = [(n % 3, *call(workloads[n % 3]), _lib.SolveTicket()) for n in range(65)]
+
+    def begin(n):
+        _, a, ctrl, _, out, _, ticket = calls[n]
+        return lib.tode_solve_builtin_begin(by(a), by(ctrl), *(_lib.ptr(out[i]) for i in range(4)), 1, stream, by(ticket))
+
+    def end(n):
+        kind, a, _, ys, out, _, ticket = calls[n]
+        flags = (_lib.C.c_int32 * _lib.FLAG_WORDS)(-1, -1, -1, -1)
+        _lib.check(lib.tode_solve_builtin_end(by(ticket), by(a), _lib.ptr(out[0]), stream, flags), "tode_solve_builtin_end")
+        assert list(flags) == [want[kind][2], 2**31 - 1, 0, 0]
+        assert torch.equal(ys, want[kind][0]) and torch.equal(out, want[kind][1])
+
+    assert [begin(n) for n in range(64)] == [0] * 64
+    assert len({calls[n][-1].slot for n in range(64)}) == 64
+    assert begin(64) == _lib.E_UNSUPPORTED and bool((calls[64][4] == -7).all())
+    for n in reversed(range(64)):
+        end(n)
+    assert [begin(n) for n in (64, *range(63))] == [0] * 64
+    for n in (64, *range(63)):
+        end(n)
+
+
 def test_flags_on_the_host_from_several_threads_and_streams_at_once():
     """Every call takes a flag slot of its own: concurrent solves must not see each other's flags."""
     import threading
