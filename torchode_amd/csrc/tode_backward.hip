@@ -223,6 +223,11 @@ template <typename T> struct Dividends {
 // divisions, the square root and the two powers in the short forms of tode_math.h wherever the wavefront's operands allow
 // them, 0.66 -> 0.53 ms; and the waits for what was loaded ahead only where it is used (they stood behind each point's index,
 // and at the end of the iteration behind the copies of the record's entry): 0.53 -> 0.46, float64, B = 20 000, 0.56 -> 0.49.
+// What is held for all this costs registers: float32 rows of two take up to 182 (two wavefronts per SIMD; three before), rows of four
+// 256 and 7 to 12 accumulation registers (one; two before), float64 rows of eight all 512 and 800 to 900 bytes of scratch.  It pays all the
+// same where a SIMD has wavefronts to choose from.  Backward passes, before and now: Van der Pol float32, B = 262 144, 2.41 -> 1.11 ms,
+// a million 7.9 -> 4.1; decay, float32 rows of four, 262 144, 1.00 -> 0.75, a million 3.00 -> 2.75; float64 rows of eight, 262 144,
+// Dopri5 4.45 -> 4.17 and Tsit5 4.42 -> 3.81, a million 16.3 -> 15.8 and 16.3 -> 14.2.
 template <typename T, int METHOD, int CTRL, typename Term>
 __global__ void __launch_bounds__(64) whole_backward_kernel(const WholeBackward<T> w) {
     using Tab = typename std::conditional<METHOD == 1, Tsit5Tab, Dopri5Tab>::type;

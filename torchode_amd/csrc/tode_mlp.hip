@@ -62,6 +62,11 @@ static __global__ void mlp_pack_kernel(const float *raw, float *packed, int H, i
 // accurate tanh (mlp_tanh_accurate), since it stands where torch's evaluations of the network stood.  Network of 64 and 256 at
 // B = 4096: solve and record in 0.096 ms (0.106 with the math library's tanh and its branches, 2.6 through the per-step kernels
 // around torch's products).
+// Wavefronts per SIMD that the registers are held to.  float32: two, 256 registers.  bfloat16: its weights are half as wide, and with
+// the biases in LDS three workgroups share a compute unit: 168 registers, of which 8 to 23 are spilled (48 to 128 bytes of scratch a
+// lane; at two workgroups it took 196 to 207 and spilled none).  One build for every batch: with the conversions in pairs it is
+// the quicker one as well where no compute unit has more than two workgroups.  Kernel, Dopri5, two workgroups and conversions one by one
+// against this: B = 2000 61.8 -> 58.1 us, 4096 71.9 -> 67.1, 8192 88.9 -> 84.4, 20 011 199 -> 165; Tsit5, 4096: 181 -> 163.
 template <typename Weights> constexpr int mlp_wavefronts = std::is_same<Weights, MlpWeightsBf16>::value ? 3 : 2;  // per SIMD
 
 template <int METHOD, int CTRL, typename Weights, bool FULL, bool RECORD>

@@ -15,9 +15,9 @@
 // What bounds them, network of 64 and 256 at B = 4096 (one workgroup per compute unit, one wavefront per SIMD): six
 // evaluations forward 28 us (three iterations in one launch 63 us, two workgroups to a compute unit), back 29 us, of which the
 // matrix cores are busy 10.6 and 10.2 us -- the rest are the round trips through LDS between two products, the stage sums and
-// 150 KB of weights loaded per workgroup; the outer products of 20 evaluations 69 us (39 us of matrix instructions, 200 MB of
-// rows at 2.9 TB/s).  A solve and its backward pass: 9.75 ms through
-// autograd, 0.80 ms.
+// 150 KB of weights loaded per workgroup; the outer products of 20 evaluations 69 us (34 us of matrix instructions at 2.4 GHz,
+// 200 MB of rows at 2.9 TB/s).  A solve and its backward pass: 9.75 ms through autograd, 0.61 to 0.80 ms by the host's speed (0.42 ms of
+// kernels).
 //
 // All products are on v_mfma_f32_16x16x4_f32.  For the vector-Jacobian product the weights are packed a second time,
 // transposed (tode_mlp_pack_weights_reverse), so that the same two facts hold as in the forward kernel: every lane keeps its
@@ -502,9 +502,9 @@ template <bool QUADS> __device__ __forceinline__ void mlp_outer_rows(const tode_
 
 // dW2[f][u] = sum over rows g[f] h[u],  dW1[u][i] = sum over rows d[u] x[i],  and the biases' and the time column's sums:
 // every workgroup takes a share of the rows and holds all sums of it in registers (wavefront w: units 64w .. 64w + 63, 128
-// accumulators), 32 matrix instructions (0.45 us) per four rows with the operands of the next four such steps on their way:
+// accumulators), 32 matrix instructions (0.43 us at 2.4 GHz) per four rows with the operands of the next four such steps on their way:
 // one wavefront per SIMD has nothing else to cover the memory's latency with.  82 000 rows: 69 us, of which the matrix
-// instructions are 39; 92 with a load per value, half of whose instructions were addresses.  The sums of a share go to the workgroup's
+// instructions are 34; 92 with a load per value, half of whose instructions were addresses.  The sums of a share go to the workgroup's
 // own slot, added to those of earlier calls (`accumulate`).
 template <bool QUADS>
 __global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(1, 1))) mlp_weight_gradient_kernel(const tode_mlp_reverse p, long long rows, long long rows_per_split, int accumulate) {
