@@ -603,7 +603,8 @@ int tode_set_fast_kernel_variant(int variant);
  * A hook for tests: the short forms of division and square root in the small systems' kernels against the compiler's.  Adds the
  * number of results that differ to `mismatches` (one int32 in device memory).  form 0 ... 3: float32 reciprocal, square
  * root, division by the square root of 2 and of 3, over every value of their ranges; 4: float32 quotient, of `samples`
- * pseudo-random pairs; 5 ... 9: the same five in float64, of `samples` pseudo-random operands.
+ * pseudo-random pairs; 5 ... 9: the same five in float64, of `samples` pseudo-random operands; 10, 11: powers in float32 and
+ * float64; 12, 13: sums over a wavefront.
  */
 int tode_check_short_forms(int32_t form, int64_t samples, void *mismatches, void *stream);
 

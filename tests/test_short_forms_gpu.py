@@ -60,3 +60,35 @@ def test_forms_against_the_compilers(form):
     mismatches = torch.zeros(1, dtype=torch.int32, device="cuda")
     _lib.check(_lib.load().tode_check_short_forms(form, 1 << 28, mismatches.data_ptr(), _lib.stream_of(mismatches)), "tode_check_short_forms")
     assert int(mismatches) == 0
+
+
+@pytest.mark.parametrize("form", [10, 11, 12, 13], ids=["power-f32", "power-f64", "sum-f32", "sum-f64"])
+def test_powers_and_sums_against_their_general_forms(form):
+    """2^26 pairs of a base -- any bits, or from around the short forms' range -- and an exponent of either kind; as many
+    values summed over wavefronts."""
+    from torchode_amd import _lib
+
+    mismatches = torch.zeros(1, dtype=torch.int32, device="cuda")
+    _lib.check(_lib.load().tode_check_short_forms(form, 1 << 26, mismatches.data_ptr(), _lib.stream_of(mismatches)), "tode_check_short_forms")
+    assert int(mismatches) == 0
+
+
+@pytest.mark.parametrize("dtype", [torch.float32, torch.float64], ids=["f32", "f64"])
+@pytest.mark.parametrize("n", [16, 64])
+@pytest.mark.parametrize("controller", CONTROLLERS)
+def test_step_factor_of_a_grid(controller, n, dtype):
+    """The grid kernel forms the powers of its step factor on lanes of one wavefront; the per-call operators form them one
+    after the other: the same bits, whichever exponents are zero or outside the short forms' range."""
+    spec = dict(CONTROLLERS[controller])
+    B, F = 5, n * n
+    g = torch.Generator().manual_seed(n)
+    y0 = torch.rand((B, F), generator=g, dtype=torch.float64).to(dtype).cuda()
+    f = to.ReactionDiffusion(torch.tensor([1e-3, 3e-3, 1e-2, 3e-2, 1e-1], dtype=dtype).cuda(), n)
+    t_eval = torch.linspace(0.0, 1.0, 7, dtype=dtype).repeat(B, 1).cuda()
+    make = to.PIDController if spec.pop("kind") == "pid" else to.IntegralController
+    solver = to.AutoDiffAdjoint(to.Tsit5(), make(**spec))
+    fused = solver.solve(to.InitialValueProblem(y0, t_eval=t_eval), to.ODETerm(f))
+    per_call = solver._solve_protocol(to.InitialValueProblem(y0, t_eval=t_eval), to.ODETerm(f), to.ODETerm(f), None, None)
+    assert torch.equal(fused.ys, per_call.ys) and torch.equal(fused.status, per_call.status)
+    for key in ("n_steps", "n_accepted", "n_initialized"):
+        assert torch.equal(fused.stats[key], per_call.stats[key])

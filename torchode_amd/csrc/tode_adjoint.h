@@ -58,10 +58,7 @@ template <typename T> __device__ __forceinline__ void max_backward(T a, T b, T g
 // rows of fewer than 64 features), and one wavefront per sample with its lanes strided over the row (WAVE true); sums
 // over a row are then completed across the wavefront and per-sample results are stored by lane 0.
 template <bool WAVE, typename T> __device__ __forceinline__ T row_sum(T v) {
-    if (WAVE) {
-#pragma unroll
-        for (int off = 32; off > 0; off >>= 1) v += __shfl_xor(v, off);
-    }
+    if constexpr (WAVE) return wave_sum(v);
     return v;
 }
 

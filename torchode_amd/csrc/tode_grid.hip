@@ -14,6 +14,11 @@
 // workgroup carries the same scalar state (t, dt, error ratio, counters), computed
 // redundantly from the same reduced values: there is no divergence inside a sample.
 //
+// A step is a chain of seven barriers with little work between two of them, so what one wavefront does while the others
+// wait counts: the powers of the step factor in their short forms, one per lane of a quad (dt_factor_by_lanes), and the
+// chunk sums by permutations of registers instead of shuffles.  64 x 64, B = 500, three steps and three points: kernel
+// 57 -> 50 us; B = 512 with 100 points 172 -> 164.
+//
 // The dense output is what this kernel is bound by: every evaluation point is one
 // coalesced 4*F-byte row of ys, written with 16-byte stores straight from registers.
 //
@@ -49,37 +54,30 @@ template <typename T> __device__ __forceinline__ void load4(const T *from, T (&v
 }
 template <typename T> __device__ __forceinline__ void store4(T *to, const T (&v)[4]) { *reinterpret_cast<Four<T> *>(to) = Four<T>{v[0], v[1], v[2], v[3]}; }
 
-// Sum over the row of two per-thread partial sums per band, in the fixed order: the chunk of 256 cells that wavefront w
+// Sums over the row of N_SUMS per-thread partial sums per band, in the fixed order: the chunk of 256 cells that wavefront w
 // holds of band r is chunk r * NW + w of the row, and the chunk sums are added in that order.
-template <typename T, int NW, int R> __device__ __forceinline__ void block_sum2(GridShared<T, NW, R> &sh, int &slot, const T (&a)[R], const T (&b)[R], T &A, T &B) {
+template <int N_SUMS, typename T, int NW, int R> __device__ __forceinline__ void block_sums(GridShared<T, NW, R> &sh, int &slot, const T (&parts)[N_SUMS][R], T (&sums)[N_SUMS]) {
     const int wave = threadIdx.x >> 6;
-#pragma unroll
-    for (int r = 0; r < R; ++r) {
-        T u = a[r], v = b[r];
-#pragma unroll
-        for (int off = 32; off > 0; off >>= 1) {
-            u = u + __shfl_xor(u, off);
-            v = v + __shfl_xor(v, off);
-        }
-        if ((threadIdx.x & 63) == 0) {
-            sh.red[slot][r][wave][0] = u;
-            sh.red[slot][r][wave][1] = v;
-        }
-    }
-    lds_barrier();
-    A = 0;
-    B = 0;
 #pragma unroll
     for (int r = 0; r < R; ++r)
 #pragma unroll
-        for (int w = 0; w < NW; ++w) {
-            A = A + sh.red[slot][r][w][0];
-            B = B + sh.red[slot][r][w][1];
+        for (int n = 0; n < N_SUMS; ++n) {
+            const T chunk = wave_sum(parts[n][r]);
+            if ((threadIdx.x & 63) == 0) sh.red[slot][r][wave][n] = chunk;
         }
+    lds_barrier();
+#pragma unroll
+    for (int n = 0; n < N_SUMS; ++n) sums[n] = 0;
+#pragma unroll
+    for (int r = 0; r < R; ++r)
+#pragma unroll
+        for (int w = 0; w < NW; ++w)
+#pragma unroll
+            for (int n = 0; n < N_SUMS; ++n) sums[n] = sums[n] + sh.red[slot][r][w][n];
     slot ^= 1;
 }
 
-// A scalar of the sample that takes hundreds of instructions (a power): worked out by the first wavefront alone and
+// A scalar of the sample that takes a hundred instructions or more (a power): worked out by the first wavefront alone and
 // handed round in LDS, where otherwise all NW wavefronts would work it out, four to a SIMD one after the other.  Same
 // arithmetic on the same operands: same bits.  (Between two uses lies at least one other barrier of the workgroup, so
 // nobody still reads the word when it is written again.)
@@ -166,20 +164,20 @@ __global__ void __launch_bounds__(N *N / 4 / grid_bands(N)) solve_grid_kernel(co
     if (p.dt0) {
         dt = p.dt0[b];
     } else {
-        T inv[R][4], a0[R], a1[R], A0, A1;
+        T inv[R][4], a[2][R], A[2];
 #pragma unroll
         for (int r = 0; r < R; ++r) {
-            a0[r] = 0, a1[r] = 0;
+            a[0][r] = 0, a[1][r] = 0;
 #pragma unroll
             for (int j = 0; j < 4; ++j) {
                 inv[r][j] = inv_scale(cp.atol, cp.rtol, y[r][j]);
                 const T x0 = (y[r][j] * inv[r][j]) / sf, x1 = (k[0][r][j] * inv[r][j]) / sf;
-                a0[r] = fma_(x0, x0, a0[r]);
-                a1[r] = fma_(x1, x1, a1[r]);
+                a[0][r] = fma_(x0, x0, a[0][r]);
+                a[1][r] = fma_(x1, x1, a[1][r]);
             }
         }
-        block_sum2<T, NW, R>(sh, slot, a0, a1, A0, A1);
-        const T d0 = sqrt_(A0), d1 = sqrt_(A1);
+        block_sums<2, T, NW, R>(sh, slot, a, A);
+        const T d0 = sqrt_(A[0]), d1 = sqrt_(A[1]);
         T h0 = (d0 < (T)1e-5 || d1 < (T)1e-5) ? (T)1e-6 : ((T)0.01 * d0) / d1;
         h0 = tmin(h0, abs_(te - ts));
         T y1[R][4], f1[R][4];
@@ -188,19 +186,19 @@ __global__ void __launch_bounds__(N *N / 4 / grid_bands(N)) solve_grid_kernel(co
 #pragma unroll
             for (int j = 0; j < 4; ++j) y1[r][j] = fma_(dir * h0, k[0][r][j], y[r][j]);
         grid_rhs<T, N, NW, R>(sh, buf, D, y1, f1);
-        T a2[R], none[R], A2, unused;
+        T a2[1][R], A2[1];
 #pragma unroll
         for (int r = 0; r < R; ++r) {
-            a2[r] = 0, none[r] = 0;
+            a2[0][r] = 0;
 #pragma unroll
             for (int j = 0; j < 4; ++j) {
                 const T df = f1[r][j] - k[0][r][j];
                 const T x2 = (df * inv[r][j]) / sf;
-                a2[r] = fma_(x2, x2, a2[r]);
+                a2[0][r] = fma_(x2, x2, a2[0][r]);
             }
         }
-        block_sum2<T, NW, R>(sh, slot, a2, none, A2, unused);
-        dt = by_one_wavefront(sh.handed, [&] { return initial_finish<T>(CTRL == 1 ? TODE_CTRL_PID : TODE_CTRL_INTEGRAL, 1.0 / 5.0, dir, h0, d1, sqrt_(A2)); });
+        block_sums<1, T, NW, R>(sh, slot, a2, A2);
+        dt = by_one_wavefront(sh.handed, [&] { return initial_finish<T>(CTRL == 1 ? TODE_CTRL_PID : TODE_CTRL_INTEGRAL, 1.0 / 5.0, dir, h0, d1, sqrt_(A2[0])); });
     }
     dt = tclamp(dt, tlo - t, thi - t);
 
@@ -242,10 +240,10 @@ __global__ void __launch_bounds__(N *N / 4 / grid_bands(N)) solve_grid_kernel(co
         }
 
         // ---- error ratio (runge_kutta.py:267, step_size_controllers.py:389-395); long rows: fused sums ----
-        T part[R], none[R], total, unused;
+        T part[1][R], total[1];
 #pragma unroll
         for (int r = 0; r < R; ++r) {
-            part[r] = 0, none[r] = 0;
+            part[0][r] = 0;
 #pragma unroll
             for (int j = 0; j < 4; ++j) {
                 T err = 0;
@@ -253,13 +251,13 @@ __global__ void __launch_bounds__(N *N / 4 / grid_bands(N)) solve_grid_kernel(co
                 for (int s = 0; s < 7; ++s) err = fma_(dt * (T)Tab::b_err[s], k[s][r][j], err);
                 const T m = tmax(abs_(y[r][j]), abs_(y1[r][j]));
                 const T x = (abs_(err) / fma_(cp.rtol, m, cp.atol)) / sf;
-                part[r] = fma_(x, x, part[r]);
+                part[0][r] = fma_(x, x, part[0][r]);
             }
         }
-        block_sum2<T, NW, R>(sh, slot, part, none, total, unused);
-        const T ratio = tmax(sqrt_(total), (T)1e-38);
+        block_sums<1, T, NW, R>(sh, slot, part, total);
+        const T ratio = tmax(sqrt_(total[0]), (T)1e-38);
         const bool accept = ratio < (T)1;
-        T dt_next = dt * by_one_wavefront(sh.handed, [&] { return dt_factor<T, CTRL>(cp, ratio, prev, pprev); });
+        T dt_next = dt * by_one_wavefront(sh.handed, [&] { return dt_factor_by_lanes<T, CTRL>(cp, ratio, prev, pprev); });
         const int status = limit_dt<T>(cp, ratio, dt_next);
         if (idle) {
             bail = status != 0;

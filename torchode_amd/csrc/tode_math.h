@@ -340,6 +340,20 @@ template <typename T> __device__ __forceinline__ T rpow(T x, double p) {
     return pow_<T>(x, e);
 }
 
+// rpow for code that runs once per step or start, a lane or a wavefront at a time: with the short forms where x is in
+// [2^-50, 2^50) and the exponent at most 1/2 in magnitude, as the powers of a step rule usually are: 140 instructions
+// instead of 350.  Same values (tode_checks.hip).
+template <typename T> __device__ __forceinline__ bool in_power_range(T x) {
+    const unsigned high = sizeof(T) == 4 ? (unsigned)__float_as_uint((float)x) : (unsigned)__double2hiint((double)x);
+    constexpr unsigned bias = sizeof(T) == 4 ? 127 : 1023, one = sizeof(T) == 4 ? 1u << 23 : 1u << 20;
+    return high - (bias - 50) * one < 100 * one;
+}
+template <typename T> __device__ __forceinline__ T rpow_common(T x, double p) {
+    const T e = (T)p;
+    if (in_power_range(x) && abs_(e) <= (T)0.5 && !special_exponent<T>(p)) return expk<true>(dw_mul(logk<true>(x), e));
+    return rpow<T>(x, p);
+}
+
 // ---------------------------------------------------------------------------
 // Butcher tableaux, float64 literals cast to the working type where used
 // (torchode single_step_methods/dopri5.py:11-44, tsit5.py:74-114).
@@ -571,10 +585,10 @@ template <typename T> __device__ __forceinline__ T clamp_ordered(T x, T lo, T hi
 
 // dt factor (step_size_controllers.py:289-294, 598-620).
 template <typename T, int CTRL> __device__ __forceinline__ T dt_factor(const CtrlParams<T> &cp, T ratio, T prev, T prev_prev) {
-    T factor = cp.safety * rpow<T>(ratio, cp.e1);
+    T factor = cp.safety * rpow_common<T>(ratio, cp.e1);
     if (CTRL == 1) {
-        T f2 = cp.skip2 ? (T)1 : rpow<T>(prev, cp.e2);
-        T f3 = cp.skip3 ? (T)1 : rpow<T>(prev_prev, cp.e3);
+        T f2 = cp.skip2 ? (T)1 : rpow_common<T>(prev, cp.e2);
+        T f3 = cp.skip3 ? (T)1 : rpow_common<T>(prev_prev, cp.e3);
         factor = factor * f2;
         factor = factor * f3;
     }

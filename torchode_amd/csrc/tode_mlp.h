@@ -342,11 +342,7 @@ __device__ __forceinline__ void mlp_load_biases(MlpShared &sh, const float *pack
 template <typename Shared> __device__ __forceinline__ void mlp_sum2(Shared &sh, int &slot, const float (&a)[4], const float (&b)[4], float &A, float &B) {
     const int lane = threadIdx.x & 63, w = threadIdx.x >> 6, q = lane >> 4, c = lane & 15;
     float u = (a[0] + a[1]) + (a[2] + a[3]), v = (b[0] + b[1]) + (b[2] + b[3]);
-#pragma unroll
-    for (int off = 16; off < 64; off <<= 1) {
-        u = u + __shfl_xor(u, off);
-        v = v + __shfl_xor(v, off);
-    }
+    u = add_from<32>(add_from<16>(u)), v = add_from<32>(add_from<16>(v));
     if (q == 0) {
         sh.red[slot][w][c][0] = u;
         sh.red[slot][w][c][1] = v;

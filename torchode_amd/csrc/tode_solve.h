@@ -121,6 +121,38 @@ __device__ __forceinline__ int swap_lanes(int v) { return __builtin_amdgcn_mov_d
 __device__ __forceinline__ float swap_lanes(float v) { return __int_as_float(swap_lanes(__float_as_int(v))); }
 __device__ __forceinline__ double swap_lanes(double v) { return __hiloint2double(swap_lanes(__double2hiint(v)), swap_lanes(__double2loint(v))); }
 
+// Sums between the lanes of a wavefront by permutations of registers (a shuffle goes through LDS: a round trip per step).
+// v of every lane plus that of the lane 16 or 32 away: the swap instructions bring both operands to both lanes.
+template <typename T> struct Words {
+    unsigned w[sizeof(T) / 4];
+};
+template <int OFFSET, typename T> __device__ __forceinline__ T add_from(T v) {
+    static_assert(OFFSET == 16 || OFFSET == 32, "the swaps between rows and between halves");
+    const Words<T> own = __builtin_bit_cast(Words<T>, v);
+    Words<T> first, second;
+#pragma unroll
+    for (int i = 0; i < (int)sizeof(T) / 4; ++i) {
+        const auto both = OFFSET == 32 ? __builtin_amdgcn_permlane32_swap(own.w[i], own.w[i], false, false) : __builtin_amdgcn_permlane16_swap(own.w[i], own.w[i], false, false);
+        first.w[i] = both[0], second.w[i] = both[1];
+    }
+    return __builtin_bit_cast(T, first) + __builtin_bit_cast(T, second);
+}
+template <int CONTROL> __device__ __forceinline__ float permuted(float v) { return __int_as_float(__builtin_amdgcn_mov_dpp(__float_as_int(v), CONTROL, 0xf, 0xf, true)); }
+template <int CONTROL> __device__ __forceinline__ double permuted(double v) {
+    return __hiloint2double(__builtin_amdgcn_mov_dpp(__double2hiint(v), CONTROL, 0xf, 0xf, true), __builtin_amdgcn_mov_dpp(__double2loint(v), CONTROL, 0xf, 0xf, true));
+}
+// The sum over all 64 lanes, in every lane, added up as a butterfly over the offsets 32, 16, 8, 4, 2, 1 adds it up: once the
+// sums over an offset are there, lanes at that distance hold the same value, so that a rotation of the sixteen lanes of a
+// row by 8 or by 4 brings what the exchange with the lane at that offset would bring.
+template <typename T> __device__ __forceinline__ T wave_sum(T v) {
+    v = add_from<32>(v);
+    v = add_from<16>(v);
+    v = v + permuted<0x128>(v);  // row rotated by 8
+    v = v + permuted<0x124>(v);  // by 4
+    v = v + permuted<2 | (3 << 2) | (0 << 4) | (1 << 6)>(v);  // in a quad: lanes 2 3 0 1
+    return v + permuted<1 | (0 << 2) | (3 << 4) | (2 << 6)>(v);  // 1 0 3 2
+}
+
 // All F features of a sample from the K a lane holds.
 template <int F, int L, typename T, int K> __device__ __forceinline__ void gather_features(const T (&own)[K], T (&all)[F]) {
     if constexpr (L == 1) {
@@ -377,7 +409,7 @@ __device__ __forceinline__ T initial_step(const CtrlParams<T> &cp, const Term &r
     } else {
         // python_float / tensor is evaluated by torch as reciprocal(tensor) * python_float
         T rm = (T)1 / m;
-        h1 = rpow<T>(rm * (T)0.01, 1.0 / 5.0);
+        h1 = rpow_common<T>(rm * (T)0.01, 1.0 / 5.0);
     }
     return dir * tmin((T)100 * h0, h1);
 }
@@ -395,7 +427,7 @@ template <typename T> __device__ __forceinline__ T initial_finish(int kind, doub
         h1 = tmax((T)1e-6, h0 * (T)1e-3);
     } else {
         const T rm = (T)1 / m;  // python_float / tensor runs as reciprocal(tensor) * python_float
-        h1 = rpow<T>(rm * (T)0.01, inv_order);
+        h1 = rpow_common<T>(rm * (T)0.01, inv_order);
     }
     return dir * tmin((T)100 * h0, h1);
 }
@@ -410,6 +442,22 @@ __device__ __forceinline__ int searchsorted_first_pending(const uint8_t *pending
         if (!pending[mid]) lo = mid + 1; else hi = mid;
     }
     return lo;
+}
+
+// dt_factor of a sample that the whole wavefront holds alike: the lanes of a quad form one of its powers each.
+template <typename T, int CTRL> __device__ __forceinline__ T dt_factor_by_lanes(const CtrlParams<T> &cp, T ratio, T prev, T prev_prev) {
+    if constexpr (CTRL == 1) {
+        const int j = lane_feature<4>();
+        const T x = j == 0 ? ratio : (j == 1 ? prev : prev_prev);
+        const double p = j == 0 ? cp.e1 : (j == 1 ? cp.e2 : cp.e3);
+        const bool one = j == 1 ? cp.skip2 : (j >= 2 ? cp.skip3 : false);
+        const T power = one ? (T)1 : rpow_common<T>(x, p);
+        T factor = cp.safety * from_lane<4, 0>(power);
+        factor = factor * from_lane<4, 1>(power);
+        factor = factor * from_lane<4, 2>(power);
+        return tclamp(factor, cp.fmin, cp.fmax);
+    }
+    return dt_factor<T, CTRL>(cp, ratio, prev, prev_prev);
 }
 
 // x = (t - t0) / (t1 - t0) with a zero interval mapped to 1 (interpolation.py:8-40)
@@ -517,10 +565,11 @@ template <typename T, int NORM, typename Load> __device__ __forceinline__ T wave
                 }
             }
         }
+        if (NORM == TODE_NORM_MAX) {
 #pragma unroll
-        for (int off = 32; off > 0; off >>= 1) {
-            const T o = __shfl_xor(p, off);
-            p = NORM == TODE_NORM_MAX ? tmax(p, o) : p + o;
+            for (int off = 32; off > 0; off >>= 1) p = tmax(p, __shfl_xor(p, off));
+        } else {
+            p = wave_sum(p);
         }
         total = NORM == TODE_NORM_MAX ? tmax(total, p) : total + p;
     }

@@ -514,8 +514,7 @@ template <typename T, typename Load> __device__ __forceinline__ T block_row_rms(
                 part = fma_(x, x, part);
             }
         }
-#pragma unroll
-        for (int off = 32; off > 0; off >>= 1) part = part + __shfl_xor(part, off);
+        part = wave_sum(part);
         if (lane == 0) chunk_sums[c] = part;
     }
     __syncthreads();
