@@ -464,6 +464,25 @@ def load():
         return _lib
 
 
+_host = None
+
+
+def load_host():
+    """The Python extension ``torchode_amd._host``, after the library it calls into; built once if it is absent, no fallback."""
+    global _host
+    if _host is None:
+        load()
+        from . import build
+
+        with _lock:
+            if not os.path.exists(build.HOST_LIB):
+                build.link_host_module()
+        import importlib
+
+        _host = importlib.import_module(__package__ + "._host")
+    return _host
+
+
 def check(rc: int, what: str):
     if rc != 0:
         msg = load().tode_last_error().decode("utf-8", "replace")
@@ -486,7 +505,7 @@ def ptr(t):
 def require_device(*tensors):
     """The kernels run on a HIP device only; anything else is an error, never a fallback."""
     for t in tensors:
-        if t is not None and t.device.type != "cuda":
+        if t is not None and not t.is_cuda:
             raise RuntimeError(
                 "torchode_amd runs on an AMD GPU (HIP device) only; got a tensor on "
                 f"'{t.device}'. There is no CPU implementation to fall back to."

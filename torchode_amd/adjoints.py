@@ -20,7 +20,6 @@ _PROTOCOL_NAMES = (
 )  # fmt: skip
 
 
-_FlagArray = _lib.C.c_int32 * _lib.FLAG_WORDS
 _F_EVAL_VALUES: Dict[int, torch.Tensor] = {}  # count -> 0-dim int64 tensor (never written to)
 
 
@@ -39,31 +38,32 @@ def _f_evals(count: int, batch: int) -> torch.Tensor:
 _PROTOCOL_NAME_SET = frozenset(_PROTOCOL_NAMES)
 
 
-def _library_object(obj, classes) -> bool:
+# (`tracing` in the functions below: a tracing compiler is looking, and only what it can follow may be written)
+def _library_object(obj, classes, tracing: bool = False) -> bool:
     """True if ``obj`` is exactly one of the library's classes with no protocol method replaced on
     the instance; only then may a fused kernel stand in for the calls the loop would make."""
     if type(obj) not in classes:
         return False
-    if torch.compiler.is_compiling():  # (spelled so that a tracing compiler can follow it)
+    if tracing:
         return all(name not in obj.__dict__ for name in _PROTOCOL_NAMES)
     return _PROTOCOL_NAME_SET.isdisjoint(vars(obj))
 
 
-def _sub(module, name):
+def _sub(module, name, tracing: bool = False):
     """``module.name`` for an attribute that usually is a submodule: ``nn.Module`` keeps those in a dict of their own and
     finds them only through ``__getattr__``, several times the cost of this lookup on a path that runs per solve."""
     found = module.__dict__.get(name)
-    if found is None and not torch.compiler.is_compiling():
+    if found is None and not tracing:
         found = module._modules.get(name)
     return getattr(module, name) if found is None else found
 
 
-def _library_plugins(adjoint, term, methods) -> bool:
+def _library_plugins(adjoint, term, methods, tracing: bool = False) -> bool:
     """The part of ``AutoDiffAdjoint._library_setup`` that looks at the plug-in objects only."""
-    m, c = _sub(adjoint, "step_method"), _sub(adjoint, "step_size_controller")
+    m, c = _sub(adjoint, "step_method", tracing), _sub(adjoint, "step_size_controller", tracing)
     return (
-        _library_object(m, methods)
-        and _library_object(c, (IntegralController, PIDController, FixedStepController))
+        _library_object(m, methods, tracing)
+        and _library_object(c, (IntegralController, PIDController, FixedStepController), tracing)
         and c.fusable
         and isinstance(term, ODETerm)  # subclasses that only supply f (the backsolve terms) included
         and type(term).vf is ODETerm.vf
@@ -153,7 +153,7 @@ class AutoDiffAdjoint(nn.Module):
         if (
             term_ is None
             or not isinstance(f, BuiltinTerm)
-            or not self._persistent_ok(problem, term_)
+            or not self._persistent_ok(problem, term_, tracing=True)
             or not problem.y0.is_cuda
             or (torch.is_grad_enabled() and any(x is not None and x.requires_grad for x in [*tensors, *f.buffers(), *f.parameters()]))
             or not self._whole_solve_shape(problem, f)
@@ -237,19 +237,19 @@ class AutoDiffAdjoint(nn.Module):
     def _fused_ok(self, problem: InitialValueProblem, term: ODETerm) -> bool:
         return self._library_setup(problem, term, (Dopri5, Tsit5))
 
-    def _library_setup(self, problem: InitialValueProblem, term: ODETerm, methods) -> bool:
+    def _library_setup(self, problem: InitialValueProblem, term: ODETerm, methods, tracing: bool = False) -> bool:
         """One of ``methods`` and a controller as the library ships them (no overridden protocol method, the RMS
         norm), a plain term, float32 / float64 tensors."""
-        return _library_plugins(self, term, methods) and problem.data_dtype in _lib.DTYPES and problem.time_dtype in _lib.DTYPES
+        return _library_plugins(self, term, methods, tracing) and problem.data_dtype in _lib.DTYPES and problem.time_dtype in _lib.DTYPES
 
-    def _persistent_ok(self, problem: InitialValueProblem, term: ODETerm) -> bool:
-        f = _sub(term, "f")
+    def _persistent_ok(self, problem: InitialValueProblem, term: ODETerm, tracing: bool = False) -> bool:
+        f = _sub(term, "f", tracing)
         return (
             isinstance(f, BuiltinTerm)
-            and self._fused_ok(problem, term)
+            and self._library_setup(problem, term, (Dopri5, Tsit5), tracing)
             # (time and data in different dtypes: the general kernel of the three small systems is built for them)
             and (problem.data_dtype == problem.time_dtype or f.builtin_kind in _lib.GENERAL_TERMS)
-            and type(_sub(self, "step_size_controller")) is not FixedStepController
+            and type(_sub(self, "step_size_controller", tracing)) is not FixedStepController
             and f.builtin_kind in _lib.PERSISTENT_TERMS
             and not term.with_args
         )
@@ -570,10 +570,9 @@ class AutoDiffAdjoint(nn.Module):
         torch.cuda.current_stream(like.device).wait_stream(side)
         return graph
 
-    def _solve_persistent(self, problem: InitialValueProblem, term: ODETerm, dt0, record=None) -> Solution:
-        """``record``: a ``LoopRecord`` to fill with the loop state of every iteration (the solve then runs the general
-        kernel once more, limited to the iterations the first pass took, with a record of that many entries)."""
-        lib = _lib.load()
+    def _solve_persistent(self, problem: InitialValueProblem, term: ODETerm, dt0, record=None) -> Optional[Solution]:
+        """A solve with a built-in term in a whole-solve kernel, or None where none takes it.  ``record``: a ``LoopRecord``
+        to fill with the loop state of every iteration."""
         f: BuiltinTerm = _sub(term, "f")
         if record is not None and f.builtin_kind not in _lib.GENERAL_TERMS:
             # (the record is written for the three small systems and for the network whose reverse sweep has kernels of its own:
@@ -582,132 +581,115 @@ class AutoDiffAdjoint(nn.Module):
 
             if f.builtin_kind != _lib.TERM_MLP or problem.n_evaluation_points == 0 or not self.use_fast_path or not NetworkSweep.takes(self, term, problem.y0, problem.t_start):
                 return None
-        method_id, controller = _sub(self, "step_method").method_id, _sub(self, "step_size_controller")
-        # What depends on the problem's tensors alone is worked out once per problem object and kept on it (checked by
-        # identity, since the attributes of a problem may be reassigned, and by the tensors' version counters, since
-        # the plan may hold a contiguous copy of one of them that an in-place update of the original would not reach).
-        tensors = (problem.y0, problem.t_start, problem.t_end, problem.t_eval)
-        versions = tuple(-1 if x is None else x._version for x in tensors)
-        plan = getattr(problem, "_launch_plan", None)
-        if plan is None or plan[-1] != versions or any(a is not b for a, b in zip(plan[0], tensors)):
-            y0 = problem.y0.contiguous()
-            # t_start / t_end are usually columns of t_eval: hand them over with their stride
-            t_start, t_end = (t if t.stride(0) >= 1 else t.contiguous() for t in (problem.t_start, problem.t_end))
-            t_eval = None if problem.t_eval is None else problem.t_eval.contiguous()
-            ts = problem.t_eval if problem.t_eval is not None else problem.t_end[:, None]
-            plan = (tensors, y0, t_start, t_end, t_eval, ts, y0.device, y0.dtype, y0.shape[0], y0.shape[1], problem.n_evaluation_points,
-                    y0.data_ptr(), t_start.data_ptr(), t_end.data_ptr(), t_start.stride(0), t_end.stride(0),
-                    None if t_eval is None else t_eval.data_ptr(), {}, versions)  # fmt: skip
-            problem._launch_plan = plan
-        _, y0, t_start, t_end, t_eval, ts, dev, dtype, B, F, E, y0_ptr, t_start_ptr, t_end_ptr, t_start_stride, t_end_stride, t_eval_ptr, _, _ = plan
-        params = f.builtin_params()
-        if params.device != dev or params.dtype != dtype:
+        y0 = problem.y0
+        dtype, dev = y0.dtype, y0.device
+        params = shared = None
+        if f.builtin_kind == _lib.TERM_MLP:
+            if dtype != torch.float32 or not 1 <= y0.shape[1] <= 64 or f.W1.shape[1] != y0.shape[1] + 1 or not 1 <= f.W1.shape[0] <= 256:
+                return None  # the matrix-core kernel takes up to 64 features and up to 256 hidden units: the caller takes another path
+            shared = f.builtin_packed(dev, dtype, fresh=record is not None)
+        else:
+            params = f.builtin_params()
+        if record is not None:
+            return self._solve_recording(problem, term, dt0, params, shared, record)
+        scalars = tuple(getattr(f, "builtin_scalars", tuple)())
+        c = _sub(self, "step_size_controller")
+        solved = _lib.load_host().solve(
+            y0, problem.t_start, problem.t_end, problem.t_eval, dt0, params, shared, _sub(self, "step_method").method_id, f.builtin_kind, scalars, self.max_steps,
+            self.use_fast_path, f.builtin_kind in _lib.GENERAL_TERMS, c._kind, c.dt_min, c.dt_max, c._atol_f, c._rtol_f, c.pcoeff, c.icoeff, c.dcoeff, c.safety,
+            c.factor_min, c.factor_max,
+        )  # fmt: skip
+        if solved is None:
+            return None
+        ys, n_steps, n_accepted, n_initialized, status, iterations = solved
+        stats: Dict[str, Any] = {}
+        if term.with_stats:
+            stats["n_f_evals"] = _f_evals((2 if dt0 is None else 1) + 6 * iterations, y0.shape[0])
+        stats["n_steps"], stats["n_accepted"], stats["n_initialized"] = n_steps, n_accepted, n_initialized
+        return Solution(ts=problem.t_eval if problem.t_eval is not None else problem.t_end[:, None], ys=ys, stats=stats, status=status)
+
+    def _solve_recording(self, problem: InitialValueProblem, term: ODETerm, dt0, params, shared, record) -> Optional[Solution]:
+        """The same with the loop state of every iteration kept in ``record``: from one launch where an earlier solve told how
+        many iterations such a batch takes, else by the general kernel once more, limited to the iterations of the first pass."""
+        lib, f = _lib.load(), _sub(term, "f")
+        mlp = f.builtin_kind == _lib.TERM_MLP
+        y0 = problem.y0.contiguous()
+        # t_start / t_end are usually columns of t_eval: hand them over with their stride
+        t_start, t_end = (t if t.stride(0) >= 1 else t.contiguous() for t in (problem.t_start, problem.t_end))
+        t_eval = None if problem.t_eval is None else problem.t_eval.contiguous()
+        ts = problem.t_eval if problem.t_eval is not None else problem.t_end[:, None]
+        dev, dtype, ttype, (B, F), E = y0.device, y0.dtype, t_start.dtype, y0.shape, problem.n_evaluation_points
+        if params is None:
+            params = y0.new_empty((B, 0))
+        elif params.device != dev or params.dtype != dtype:
             params = params.to(device=dev, dtype=dtype)
         if params.numel() == 0 and params.shape[0] != B:  # a term without per-sample parameters
             params = y0.new_empty((B, 0))
         assert params.shape[0] == B, "built-in term parameters do not match the batch size"
-        mlp = f.builtin_kind == _lib.TERM_MLP
-        if mlp and (
-            dtype != torch.float32 or not 1 <= F <= 64 or f.W1.shape[1] != F + 1 or not 1 <= f.W1.shape[0] <= 256
-        ):
-            return None  # the matrix-core kernel takes up to 64 features and up to 256 hidden units: the caller takes another path
-        shared = f.builtin_packed(dev, dtype, fresh=record is not None) if mlp else None
-        ttype = t_start.dtype
         dt0_ = None if dt0 is None else dt0.to(ttype).contiguous()
 
         ys = torch.empty((B, max(E, 1), F), dtype=dtype, device=dev)
-        ctrl = controller.c_struct()
+        ctrl = _sub(self, "step_size_controller").c_struct()
         stream = _lib.stream_of(y0)
-
-        # The argument struct is kept with the plan and copied from there while it describes the same call (same problem
-        # tensors, parameters, first step, method, term and step limit): only the output pointer changes from solve to solve.
-        key = (method_id, f.builtin_kind, self.max_steps, params.data_ptr(), None if dt0_ is None else dt0_.data_ptr(),
-               None if shared is None else shared.data_ptr())  # fmt: skip
-        held = plan[-2]
-        if held.get("key") != key:
-            scal = list(getattr(f, "builtin_scalars", lambda: ())()) + [0.0] * 4
-            a = _lib.SolveArgs(  # positional, in the order of struct tode_solve_args
-                _lib.dtype_code(dtype, ttype), method_id, f.builtin_kind, F, E, params.shape[1], B,
-                -1 if self.max_steps is None else int(self.max_steps), -1, (_lib.C.c_double * 4)(*scal[:4]),
-                y0_ptr, t_start_ptr, t_end_ptr, t_start_stride, t_end_stride, t_eval_ptr, None if dt0_ is None else dt0_.data_ptr(),
-                params.data_ptr() if params.numel() else None,
-                None if shared is None else shared.data_ptr(), 0 if shared is None else shared.numel(),
-            )  # fmt: skip  (what the general kernel needs besides lives in the workspace)
-            held.update(key=key, args=a, scalars=tuple(scal[:4]), keep=(params, dt0_, shared))
-        elif held["scalars"] != tuple((list(getattr(f, "builtin_scalars", lambda: ())()) + [0.0] * 4)[:4]):
-            held.clear()  # (a scalar of the term was reassigned: describe the call anew)
-            return self._solve_persistent(problem, term, dt0, record=record)
-        a = _lib.SolveArgs.from_buffer_copy(held["args"])  # (a copy per call: solves of one problem object may overlap in threads)
+        scal = list(getattr(f, "builtin_scalars", lambda: ())()) + [0.0] * 4
+        a = _lib.SolveArgs(  # positional, in the order of struct tode_solve_args
+            _lib.dtype_code(dtype, ttype), _sub(self, "step_method").method_id, f.builtin_kind, F, E, params.shape[1], B,
+            -1 if self.max_steps is None else int(self.max_steps), -1, (_lib.C.c_double * 4)(*scal[:4]),
+            y0.data_ptr(), t_start.data_ptr(), t_end.data_ptr(), t_start.stride(0), t_end.stride(0), None if t_eval is None else t_eval.data_ptr(),
+            None if dt0_ is None else dt0_.data_ptr(), params.data_ptr() if params.numel() else None,
+            None if shared is None else shared.data_ptr(), 0 if shared is None else shared.numel(),
+        )  # fmt: skip  (what the general kernel needs besides lives in the workspace)
         a.ys = ys.data_ptr()
-        a_ref = _lib.C.byref(a)
+        a_ref, ctrl_ref = _lib.C.byref(a), _lib.C.byref(ctrl)
 
-        # The one-kernel path where the batch is in its shape; the general kernel where it is not or where the first
-        # reported that the batch leaves the common case; the int64 stats as the reference returns them.
+        # int64 stats as the reference returns them
         out = torch.empty((4, B), dtype=torch.int64, device=dev)
         o0, row = out.data_ptr(), 8 * B
-        if record is not None:
-            # Once a recording solve of this solver has told how many iterations such a batch takes: the solve and its
-            # record in one kernel, with a record of a few entries more.  A batch that leaves that kernel's case, or
-            # takes more iterations than the record holds, goes the long way below.
-            solution = self._solve_recording_in_one_kernel(lib, a, ctrl, out, stream, record, dict(
-                B=B, E=E, F=F, dtype=dtype, ttype=ttype, dev=dev, ts=ts, ys=ys, has_dt0=dt0 is not None, with_stats=term.with_stats,
-                ends_at_last_point=E > 1 and B > 0 and (t_end_ptr, t_end_stride) == (t_eval_ptr + (E - 1) * t_eval.element_size(), E)))  # fmt: skip
-            if solution is not None or mlp:
-                return solution
-        ctrl_ref = _lib.C.byref(ctrl)
-        if E == 0:
-            y_idle = torch.empty((B, F), dtype=dtype, device=dev)
-            a.y_idle = y_idle.data_ptr()
-        ticket, flags = _lib.SolveTicket(), _FlagArray()
-        rc = lib.tode_solve_builtin_begin(a_ref, ctrl_ref, o0, o0 + row, o0 + 2 * row, o0 + 3 * row, 1 if self.use_fast_path else 0, stream, _lib.C.byref(ticket))
+        # Once a recording solve of this solver has told how many iterations such a batch takes: the solve and its
+        # record in one kernel, with a record of a few entries more.  A batch that leaves that kernel's case, or
+        # takes more iterations than the record holds, goes the long way below.
+        solution = self._solve_recording_in_one_kernel(lib, a, ctrl, out, stream, record, dict(
+            B=B, E=E, F=F, dtype=dtype, ttype=ttype, dev=dev, ts=ts, ys=ys, has_dt0=dt0 is not None, with_stats=term.with_stats,
+            ends_at_last_point=E > 1 and B > 0 and (t_end.data_ptr(), t_end.stride(0)) == (t_eval.data_ptr() + (E - 1) * t_eval.element_size(), E)))  # fmt: skip
+        if solution is not None or mlp:
+            return solution
+        # The one-kernel path where the batch is in its shape; the general kernel where it is not or where the first
+        # reported that the batch leaves the common case.
+        workspace_bytes, count = lib.tode_solve_workspace_bytes(a_ref), _lib.C.c_int64(0)
+        workspace = torch.empty(workspace_bytes, dtype=torch.uint8, device=dev)
+        rc = lib.tode_solve_builtin_auto(
+            a_ref, ctrl_ref, o0, o0 + row, o0 + 2 * row, o0 + 3 * row, workspace.data_ptr(), workspace_bytes, 1 if self.use_fast_path else 0, stream, _lib.C.byref(count),
+        )  # fmt: skip
         if rc == _lib.E_UNSUPPORTED:
-            return None  # no whole-solve kernel for this case: the caller takes the per-step or the operator path
-        if rc:
-            _lib.check(rc, "tode_solve_builtin_begin")
-        try:  # (while the kernel runs)
-            stats: Dict[str, Any] = {"n_f_evals": None} if term.with_stats else {}
-            stats["n_steps"], stats["n_accepted"], stats["n_initialized"], status = out.unbind(0)
-        finally:
-            rc = lib.tode_solve_builtin_end(_lib.C.byref(ticket), a_ref, o0, stream, flags)  # (the solve's one host synchronisation)
-        if rc:
-            _lib.check(rc, "tode_solve_builtin_end")
-        iterations = flags[_lib.FLAG_MAX_ITERATIONS]
-        if flags[_lib.FLAG_NEEDS_GENERAL]:
-            if f.builtin_kind not in _lib.GENERAL_TERMS:
-                return None
-            workspace_bytes, count = lib.tode_solve_workspace_bytes(a_ref), _lib.C.c_int64(0)
-            workspace = torch.empty(workspace_bytes, dtype=torch.uint8, device=dev)
-            rc = lib.tode_solve_builtin_auto(
-                a_ref, ctrl_ref, o0, o0 + row, o0 + 2 * row, o0 + 3 * row, workspace.data_ptr(), workspace_bytes, 0, stream, _lib.C.byref(count),
-            )  # fmt: skip
-            if rc:
-                _lib.check(rc, "tode_solve_builtin_auto")
-            iterations = count.value
+            return None
+        _lib.check(rc, "tode_solve_builtin_auto")
+        iterations = count.value
+        stats: Dict[str, Any] = {}
         if term.with_stats:
             stats["n_f_evals"] = _f_evals((2 if dt0 is None else 1) + 6 * iterations, B)
-        if record is not None:
-            # The same solve through the general kernel again, stopped where the first pass stopped, writing the
-            # state before every iteration: entry i of every array is what the per-step kernels' loop holds there.
-            L, n = iterations, iterations + 1
-            new = lambda *shape, dt=dtype: torch.empty(shape, dtype=dt, device=dev)
-            fields, rec = self._record_arrays(n, B, F, dtype, ttype, dev)
-            again = _lib.SolveArgs.from_buffer_copy(a)
-            scratch_ys, y_idle = new(B, max(E, 1), F), new(B, F)
-            counters, flags = new(5, B, dt=torch.int32), new(_lib.FLAG_WORDS, dt=torch.int32)
-            pending = new(B, max(E, 1), dt=torch.uint8)
-            again.ys, again.y_idle, again.pending, again.flags = scratch_ys.data_ptr(), y_idle.data_ptr(), pending.data_ptr(), flags.data_ptr()
-            again.n_steps, again.n_accepted, again.n_initialized, again.status_last, again.status_idle = (counters[i].data_ptr() for i in range(5))
-            again.iteration_cap = L
-            again.record = _lib.C.addressof(rec)
-            _lib.check(lib.tode_solve_builtin(_lib.C.byref(again), _lib.C.byref(ctrl), stream), "tode_solve_builtin")
-            if E > _lib.LISTS_AHEAD_POINTS and dtype == ttype:
-                rc = lib.tode_mark_unordered_rows(_lib.C.byref(again), stream)
-                if rc != _lib.E_UNSUPPORTED:  # (more points than one launch takes: not marked)
-                    _lib.check(rc, "tode_mark_unordered_rows")
-            record.flags = flags  # (looked at when the backward pass starts: no second wait for the GPU here)
-            self._remember_record_entries((B, F, E, dtype, f.builtin_kind), n + 4)  # (the next recording solve of a batch like this one tries it in one kernel)
-            record.iterations = L
-            record.arrays = fields  # (entry-major arrays: what tode_solve_builtin_backward reads)
+        stats["n_steps"], stats["n_accepted"], stats["n_initialized"], status = out.unbind(0)
+        # The same solve through the general kernel again, stopped where the first pass stopped, writing the
+        # state before every iteration: entry i of every array is what the per-step kernels' loop holds there.
+        L, n = iterations, iterations + 1
+        new = lambda *shape, dt=dtype: torch.empty(shape, dtype=dt, device=dev)
+        fields, rec = self._record_arrays(n, B, F, dtype, ttype, dev)
+        again = _lib.SolveArgs.from_buffer_copy(a)
+        scratch_ys, y_idle = new(B, max(E, 1), F), new(B, F)
+        counters, flags = new(5, B, dt=torch.int32), new(_lib.FLAG_WORDS, dt=torch.int32)
+        pending = new(B, max(E, 1), dt=torch.uint8)
+        again.ys, again.y_idle, again.pending, again.flags = scratch_ys.data_ptr(), y_idle.data_ptr(), pending.data_ptr(), flags.data_ptr()
+        again.n_steps, again.n_accepted, again.n_initialized, again.status_last, again.status_idle = (counters[i].data_ptr() for i in range(5))
+        again.iteration_cap = L
+        again.record = _lib.C.addressof(rec)
+        _lib.check(lib.tode_solve_builtin(_lib.C.byref(again), _lib.C.byref(ctrl), stream), "tode_solve_builtin")
+        if E > _lib.LISTS_AHEAD_POINTS and dtype == ttype:
+            rc = lib.tode_mark_unordered_rows(_lib.C.byref(again), stream)
+            if rc != _lib.E_UNSUPPORTED:  # (more points than one launch takes: not marked)
+                _lib.check(rc, "tode_mark_unordered_rows")
+        record.flags = flags  # (looked at when the backward pass starts: no second wait for the GPU here)
+        self._remember_record_entries((B, F, E, dtype, f.builtin_kind), n + 4)  # (the next recording solve of a batch like this one tries it in one kernel)
+        record.iterations = L
+        record.arrays = fields  # (entry-major arrays: what tode_solve_builtin_backward reads)
         return Solution(ts=ts, ys=ys, stats=stats, status=status)
 
     def _remember_record_entries(self, shape, entries: int) -> None:

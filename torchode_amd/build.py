@@ -17,6 +17,7 @@ HERE = os.path.dirname(os.path.abspath(__file__))
 CSRC = os.path.join(HERE, "csrc")
 LIB = os.path.join(HERE, "libtorchode_amd.so")
 OPS_LIB = os.path.join(HERE, "libtorchode_amd_ops.so")  # torch.ops.torchode_amd.*: PyTorch operators over the C ABI
+HOST_LIB = os.path.join(HERE, "_host.so")  # torchode_amd._host: what a solve does around its kernel, as a Python extension
 OBJ = os.path.join(HERE, "build")
 
 ARCH = "gfx950"
@@ -122,39 +123,59 @@ def build_library(force: bool = True, verbose: bool = False) -> str:
         return out
 
     with ThreadPoolExecutor(max_workers=min(8, len(UNITS) + 1)) as pool:
-        ops_object = pool.submit(compile_ops_object)  # (host code only, done long before the kernels)
+        host_objects = [pool.submit(compile_ops_object), pool.submit(compile_host_object)]  # (host code only, done long before the kernels)
         checked = pool.submit(check_units_under_register_pressure)
         objs = list(pool.map(compile_unit, UNITS))
-        ops_object = ops_object.result()
+        ops_object, host_object = (x.result() for x in host_objects)
         checked.result()
     _run([hipcc, f"--offload-arch={ARCH}", "-shared", "-fPIC", "-Wno-unused-command-line-argument", "-o", LIB, *objs])
     link_ops_library(ops_object)
+    link_host_module(host_object)
     return LIB
+
+
+def _compile_host_code(source: str) -> str:
+    import sysconfig
+
+    import torch
+    from torch.utils import cpp_extension
+
+    os.makedirs(OBJ, exist_ok=True)
+    out = os.path.join(OBJ, source[: -len(".cpp")] + ".o")
+    includes = [f"-I{p}" for p in cpp_extension.include_paths(device_type="cuda")] + ["-I/opt/rocm/include", "-I" + sysconfig.get_paths()["include"]]
+    abi = int(torch._C._GLIBCXX_USE_CXX11_ABI)
+    _run(["g++", "-O2", "-std=c++17", "-fPIC", "-D__HIP_PLATFORM_AMD__=1", "-DUSE_ROCM=1", f"-D_GLIBCXX_USE_CXX11_ABI={abi}", *includes,
+          "-c", os.path.join(CSRC, source), "-o", out])  # fmt: skip
+    return out
 
 
 def compile_ops_object() -> str:
     """Compiles csrc/tode_torch_ops.cpp (host code only: PyTorch's headers, no kernel) to an object file."""
-    import torch
-    from torch.utils import cpp_extension
+    return _compile_host_code("tode_torch_ops.cpp")
 
-    out = os.path.join(OBJ, "tode_torch_ops.o")
-    includes = [f"-I{p}" for p in cpp_extension.include_paths(device_type="cuda")] + ["-I/opt/rocm/include"]
-    abi = int(torch._C._GLIBCXX_USE_CXX11_ABI)
-    _run(["g++", "-O2", "-std=c++17", "-fPIC", "-D__HIP_PLATFORM_AMD__=1", "-DUSE_ROCM=1", f"-D_GLIBCXX_USE_CXX11_ABI={abi}", *includes,
-          "-c", os.path.join(CSRC, "tode_torch_ops.cpp"), "-o", out])  # fmt: skip
+
+def compile_host_object() -> str:
+    """The same of csrc/tode_host.cpp."""
+    return _compile_host_code("tode_host.cpp")
+
+
+def _link_against_torch(obj: str, out: str, *more: str) -> str:
+    import torch
+
+    torch_lib = os.path.join(os.path.dirname(torch.__file__), "lib")
+    _run(["g++", "-shared", "-fPIC", obj, "-o", out, f"-L{torch_lib}", "-ltorch", "-ltorch_cpu", "-lc10", "-lc10_hip", "-ltorch_hip", *more,
+          f"-L{HERE}", "-l:libtorchode_amd.so", "-Wl,-rpath,$ORIGIN", f"-Wl,-rpath,{torch_lib}"])  # fmt: skip
     return out
 
 
 def link_ops_library(obj=None) -> str:
     """Links the operator library against PyTorch's libraries and against libtorchode_amd.so, which it finds next to itself."""
-    import torch
+    return _link_against_torch(obj or compile_ops_object(), OPS_LIB)
 
-    if obj is None:
-        obj = compile_ops_object()
-    torch_lib = os.path.join(os.path.dirname(torch.__file__), "lib")
-    _run(["g++", "-shared", "-fPIC", obj, "-o", OPS_LIB, f"-L{torch_lib}", "-ltorch", "-ltorch_cpu", "-lc10", "-lc10_hip", "-ltorch_hip",
-          f"-L{HERE}", "-l:libtorchode_amd.so", "-Wl,-rpath,$ORIGIN", f"-Wl,-rpath,{torch_lib}"])  # fmt: skip
-    return OPS_LIB
+
+def link_host_module(obj=None) -> str:
+    """Links the Python extension ``torchode_amd._host`` likewise."""
+    return _link_against_torch(obj or compile_host_object(), HOST_LIB, "-ltorch_python")
 
 
 def emit_assembly(directory: str, units=None) -> list:

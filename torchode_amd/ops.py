@@ -1,7 +1,7 @@
 """``torch.ops.torchode_amd``: the whole-solve entry point of the C ABI as PyTorch operators.
 
-The library's own eager path calls the C ABI through ``ctypes`` (``_lib.py``; fewer microseconds per
-call than the dispatcher).  The operators here are the same entry points for programs that PyTorch
+The library's own eager path calls the C ABI through an extension of its own (``csrc/tode_host.cpp``) or ``ctypes``
+(``_lib.py``): fewer microseconds per call than the dispatcher.  The operators here are the same entry points for programs that PyTorch
 captures: ``torch.compile(solver.solve)`` with a built-in term records the whole solve as one node,
 ``torchode_amd::solve_builtin``, instead of breaking the graph at a foreign function call.  The
 operators are registered by ``libtorchode_amd_ops.so`` (``csrc/tode_torch_ops.cpp``, built by
