@@ -96,6 +96,17 @@ def test_reverse_sweep_against_its_general_forms(sources):
     assert r.returncode == 0 and r.stdout.split() == ["4000", "0"], (r.stdout, r.stderr[-2000:])
 
 
+def test_reverse_sweep_by_one_wavefront(sources):
+    """The same where one wavefront does all of it, as for batches that fill the GPU (rows of up to four values; the test above
+    has them in two)."""
+    build, compiler = sources
+    out = os.path.join(build, "sweep_by_one")
+    subprocess.run([*compiler, "-O1", "-march=native", "-fsanitize=address", "-DTODE_PAIRED_SWEEP_GROUPS=0", os.path.join(HERE, "host_wavefront", "sweep.cpp"), "-o", out], check=True, timeout=600)
+    env = dict(os.environ, ASAN_OPTIONS="verify_asan_link_order=0")
+    r = subprocess.run([out, "0", "1000"], capture_output=True, text=True, timeout=300, env=env)
+    assert r.returncode == 0 and r.stdout.split() == ["2000", "0"], (r.stdout, r.stderr[-2000:])
+
+
 def test_quotients_next_to_a_rounding_boundary(sources):
     """The short form of the float32 quotient, given the correctly rounded reciprocal, on all 46 517 418 pairs of mantissas
     whose quotient lies so close to a boundary that the form's error could take it to the other side."""

@@ -71,6 +71,38 @@ def test_bits_of_the_gradients(case):
             assert torch.equal(got, stored), (attempt, name, float((got - stored).norm() / stored.norm()))
 
 
+@pytest.mark.parametrize("case", ["vdp-f32-tsit5-pid", "vdp-f64-dopri5-integral", "lorenz-f32-dopri5-integral", "lorenz-f64-tsit5-pid", "decay1-f32-tsit5-integral", "decay4-f32-dopri5-integral"])
+def test_one_wavefront_and_two(case):
+    """Samples of a batch of 1025 groups of 64 (one wavefront to a group) and the same in batches of 1 to 512 groups (two): the
+    same gradients, bit for bit, points in order and swapped, some samples over before the others."""
+    import torchode_amd as to
+
+    system, F, method, control, dtype, E = CASES[case]
+    dtype, B = getattr(torch, dtype), 1025 * 64 - 5
+    g = torch.Generator("cuda").manual_seed(11)
+    rand = lambda lo, hi, *shape: (lo + (hi - lo) * torch.rand(shape, generator=g, dtype=torch.float64, device="cuda")).to(dtype)
+    y0, t1 = rand(-1.5, 1.5, B, F), rand(0.5, 1.5, B) * (0.25 if system == "lorenz" else 1)
+    t1[7::64] *= 1e-3
+    par, f = {"vdp": (rand(0.5, 3.0, B), to.VanDerPol), "lorenz": (rand(20.0, 30.0, B), to.Lorenz63), "decay": (rand(0.1, 5.0, B, F), to.LinearDecay)}[system]
+    cotangent = rand(-1.0, 1.0, B, max(E, 1), F)
+    t_eval = t1[:, None] * (torch.arange(E, device="cuda").to(dtype) / 64) if E else None
+    if E:
+        t_eval[64 * 3 + 2] = t_eval[64 * 3 + 2].flip(0)
+    controller = to.PIDController(1e-6, 1e-4, 0.2, 0.5, 0.05) if control == "pid" else to.IntegralController(1e-5, 1e-3)
+
+    def gradients_of(rows):
+        y, p = y0[rows].clone().requires_grad_(), par[rows].clone().requires_grad_()
+        times = dict(t_start=torch.zeros_like(t1[rows]), t_end=t1[rows]) if not E else dict(t_eval=t_eval[rows], t_start=torch.zeros_like(t1[rows]), t_end=t1[rows])
+        sol = to.AutoDiffAdjoint(getattr(to, method)(), controller).solve(to.InitialValueProblem(y, **times), to.ODETerm(f(p)))
+        assert not sol.status.any()
+        return [sol.ys.detach(), sol.stats["n_steps"], *torch.autograd.grad(sol.ys, [y, p], cotangent[rows])]
+
+    whole = gradients_of(slice(0, B))
+    for rows in (slice(0, 1), slice(60, 391), slice(128, 128 + 64 * 64), slice(B - 64 * 512, B)):
+        for found, expected in zip(gradients_of(rows), whole):
+            assert torch.equal(found, expected[rows]), (case, rows)
+
+
 if __name__ == "__main__":
     result = {case: [[float(v).hex() for v in x.double().flatten().tolist()] for x in next(gradients(case))] for case in CASES}
     with open(sys.argv[1] if len(sys.argv) > 1 else GOLDEN, "w") as file:

@@ -12,6 +12,11 @@
 // worked on: its entry of the record, and the evaluation points it may have written.
 #include "tode_adjoint.h"
 
+// Largest number of groups of 64 samples that take two wavefronts each (launch_backward); half as many in float64.
+#ifndef TODE_PAIRED_SWEEP_GROUPS
+#define TODE_PAIRED_SWEEP_GROUPS 1024
+#endif
+
 namespace tode {
 
 template <typename T> struct WholeBackward {
@@ -214,6 +219,173 @@ template <typename T> struct Dividends {
     }
 };
 
+// What the reverse of an iteration needs of the iteration itself: the stages again (runge_kutta.py:255-263), the error ratio
+// and the step factor before its clip.  None of it waits for a cotangent.
+template <typename T, int F> struct Formed {
+    T k[7][F], yi[7][F], y1[F];
+    T err[F], eb[F], per_eb[F], q[F], x[F], r, ratio, F0;
+    bool bounds_outside;  // this lane's error bounds or history are outside the short forms' ranges
+};
+
+template <typename T, int METHOD, int CTRL, typename Term>
+__device__ __forceinline__ void form_iteration(const WholeBackward<T> &w, const Term &rhs, const RecordEntry<T, Term::F> &here, const bool running_new, Formed<T, Term::F> &o) {
+    using Tab = typename std::conditional<METHOD == 1, Tsit5Tab, Dopri5Tab>::type;
+    constexpr int F = Term::F;
+    constexpr bool SHORT = F * sizeof(T) <= 32;
+    const CtrlParams<T> &cp = w.cp;
+    const T sf = (T)__builtin_sqrt((double)F);
+    const T t0 = here.t, dt = here.dt, prev = here.prev, pprev = here.pprev;
+    const T(&y)[F] = here.y;
+#pragma unroll
+    for (int f = 0; f < F; ++f) o.k[0][f] = here.k0[f];
+#pragma unroll
+    for (int s = 1; s < 7; ++s) {
+#pragma unroll
+        for (int f = 0; f < F; ++f) {
+            T sum = 0;
+#pragma unroll
+            for (int j = 0; j < s; ++j) sum = fma_((T)Tab::a[s][j], o.k[j][f], sum);
+            o.yi[s][f] = fma_(dt, sum, y[f]);
+        }
+        rhs(fma_((T)Tab::c[s], dt, t0), o.yi[s], o.k[s]);
+    }
+#pragma unroll
+    for (int f = 0; f < F; ++f) o.y1[f] = o.yi[6][f];
+    using Div = DivSqrtFeatures<T, F>;
+    // error ratio and step factor, in the short forms where every lane's operands are in their ranges (control_common's,
+    // over a wider range of the errors: their squares may vanish in the sum, as they do in the general form).  A sample
+    // that sits through an iteration with a zero step has an error of zero; its controller's results reach nothing.
+    T acc = 0;
+    lanes_t outside = 0, bounds_outside = 0;
+    unsigned smallest = 0xffffffffu;
+    T largest_eb = 0;
+#pragma unroll
+    for (int f = 0; f < F; ++f) {
+        o.err[f] = 0;
+#pragma unroll
+        for (int s = 0; s < 7; ++s) o.err[f] = fma_(dt * (T)Tab::b_err[s], o.k[s][f], o.err[f]);
+        if constexpr (SHORT) {
+            o.eb[f] = fma_(cp.rtol, max_abs(y[f], o.y1[f]), cp.atol);
+            o.per_eb[f] = reciprocal_estimate(o.eb[f]);
+            o.q[f] = quotient_with(abs_(o.err[f]), o.eb[f], o.per_eb[f]);
+            o.x[f] = Div::fast(o.q[f]);
+            smallest = min(smallest, min(high_bits(abs_(o.err[f])) - 1u, high_bits(o.q[f]) - 1u));  // (zero wraps round to the largest)
+            largest_eb = f == 0 ? o.eb[f] : max_ordered(largest_eb, o.eb[f]);
+            acc = fma_(o.x[f], o.x[f], acc);
+        }
+    }
+    if constexpr (SHORT) {
+        constexpr unsigned from = power_of_two_bits<T>(-40), width = power_of_two_bits<T>(16) - from;
+        const bool idle = acc == (T)0 && !running_new;
+        acc = idle ? (T)1 : acc;
+        bounds_outside = lanes_where(!(largest_eb <= (T)0x1p+20));
+        outside = lanes_where(smallest < power_of_two_bits<T>(Dividends<T>::smallest) - 1u) | lanes_where(high_bits(acc) - from >= width) | bounds_outside;
+        o.r = o.ratio = sqrt_plain(acc);
+        o.F0 = cp.safety * expk<true>(dw_mul(logk<true>(o.ratio), (T)cp.e1));
+        if (CTRL == 1 && !cp.skip2) o.F0 = o.F0 * expk<true>(dw_mul(logk<true>(prev), (T)cp.e2));
+        if (CTRL == 1 && !cp.skip3) o.F0 = o.F0 * expk<true>(dw_mul(logk<true>(pprev), (T)cp.e3));
+        constexpr unsigned history = power_of_two_bits<T>(-20), history_width = power_of_two_bits<T>(20) - history;
+        lanes_t history_outside = 0;
+        if (CTRL == 1 && !cp.skip2) history_outside |= lanes_where(high_bits(prev) - history >= history_width);
+        if (CTRL == 1 && !cp.skip3) history_outside |= lanes_where(high_bits(pprev) - history >= history_width);
+        outside |= history_outside, bounds_outside |= history_outside;
+    }
+    if (!SHORT || !w.plain || outside) {
+        acc = 0;
+#pragma unroll
+        for (int f = 0; f < F; ++f) {
+            o.eb[f] = fma_(cp.rtol, tmax(abs_(y[f]), abs_(o.y1[f])), cp.atol);
+            o.q[f] = abs_(o.err[f]) / o.eb[f];
+            o.x[f] = o.q[f] / sf;
+            acc = fma_(o.x[f], o.x[f], acc);
+        }
+        o.r = sqrt_(acc), o.ratio = tmax(o.r, (T)1e-38);
+        o.F0 = cp.safety * rpow<T>(o.ratio, cp.e1);
+        if (CTRL == 1) {
+            o.F0 = o.F0 * (cp.skip2 ? (T)1 : rpow<T>(prev, cp.e2));
+            o.F0 = o.F0 * (cp.skip3 ? (T)1 : rpow<T>(pprev, cp.e3));
+        }
+    }
+    o.bounds_outside = holds(bounds_outside);
+}
+
+// Coefficients of the dense output's derivative, lowest power first.
+template <typename T, int METHOD, int F>
+__device__ __forceinline__ void form_slope(T dt, const T (&y)[F], const T (&y1)[F], const T (&k)[7][F], int f, T (&slope)[4]) {
+    const T ks[7] = {k[0][f], k[1][f], k[2][f], k[3][f], k[4][f], k[5][f], k[6][f]};
+    T q[5][1];
+    quartic_elem<T, METHOD>(dt, y[f], y1[f], ks, true, q);
+    slope[0] = q[1][0], slope[1] = (T)2 * q[2][0], slope[2] = (T)3 * q[3][0], slope[3] = (T)4 * q[4][0];
+}
+
+// What one wavefront forms and another one uses, by way of LDS: 16 bytes of a lane's values at a time, lanes side by side, two
+// iterations' worth.  The stage inputs are left out: the user has their sums in hand when it needs them.
+template <typename T, int F> struct HandOver {
+    static constexpr int PER = 16 / (int)sizeof(T), VALUES = 16 * F + 4, CHUNKS = (VALUES + PER - 1) / PER;
+    struct alignas(16) Chunk {
+        T v[PER];
+    };
+    static constexpr size_t bytes() { return 2 * sizeof(Chunk) * CHUNKS * 64; }
+    Chunk *lane;  // [2][CHUNKS][64], at this lane
+    int phase = 0;
+    __device__ __forceinline__ HandOver(unsigned char *lds) : lane(reinterpret_cast<Chunk *>(lds) + (threadIdx.x & 63)) {}
+    // every value in its place: the slopes last, which only iterations with an evaluation point read
+    template <typename Each> static __device__ __forceinline__ void each(Formed<T, F> &o, Each each) {
+        int at = 0;
+#pragma unroll
+        for (int f = 0; f < F; ++f) {
+#pragma unroll
+            for (int s = 1; s < 7; ++s) each(at++, o.k[s][f]);
+            each(at++, o.y1[f]), each(at++, o.err[f]), each(at++, o.eb[f]), each(at++, o.per_eb[f]), each(at++, o.q[f]), each(at++, o.x[f]);
+        }
+        each(at++, o.r), each(at++, o.ratio), each(at++, o.F0);
+    }
+    static constexpr int SLOPES = 12 * F + 4, FIRST_SLOPE_CHUNK = SLOPES / PER;
+    __device__ __forceinline__ void write(Formed<T, F> &o, const T (&slope)[F][4]) {
+        T v[CHUNKS * PER] = {};
+        each(o, [&](int at, T &value) { v[at] = value; });
+        v[12 * F + 3] = o.bounds_outside ? (T)1 : (T)0;
+#pragma unroll
+        for (int f = 0; f < F; ++f)
+#pragma unroll
+            for (int j = 0; j < 4; ++j) v[SLOPES + 4 * f + j] = slope[f][j];
+        Chunk *const to = lane + phase * CHUNKS * 64;
+#pragma unroll
+        for (int c = 0; c < CHUNKS; ++c) {
+            Chunk chunk;
+#pragma unroll
+            for (int j = 0; j < PER; ++j) chunk.v[j] = v[c * PER + j];
+            to[c * 64] = chunk;
+        }
+        phase ^= 1;
+    }
+    __device__ __forceinline__ void read(Formed<T, F> &o) {
+        T v[(SLOPES + PER - 1) / PER * PER];
+        const Chunk *const from = lane + phase * CHUNKS * 64;
+#pragma unroll
+        for (int c = 0; c * PER < SLOPES; ++c) {
+            const Chunk chunk = from[c * 64];
+#pragma unroll
+            for (int j = 0; j < PER; ++j) v[c * PER + j] = chunk.v[j];
+        }
+        each(o, [&](int at, T &value) { value = v[at]; });
+        o.bounds_outside = v[12 * F + 3] != (T)0;
+        phase ^= 1;
+    }
+    __device__ __forceinline__ void read_slopes(T (&slope)[F][4]) {  // (after read)
+        const Chunk *const from = lane + (phase ^ 1) * CHUNKS * 64;
+#pragma unroll
+        for (int c = FIRST_SLOPE_CHUNK; c < CHUNKS; ++c) {
+            const Chunk chunk = from[c * 64];
+#pragma unroll
+            for (int j = 0; j < PER; ++j) {
+                const int at = c * PER + j - SLOPES;
+                if (at >= 0 && at < 4 * F) slope[at / 4][at % 4] = chunk.v[j];
+            }
+        }
+    }
+};
+
 // What bounds this kernel is one thread's chain: B = 65536 is one wavefront per SIMD, and the slowest sample's 107
 // iterations follow one another.  The evaluation points of an iteration are in registers before the iteration begins: AHEAD
 // of them, from the last one that no iteration has met yet downwards, are loaded as soon as the iteration before has taken
@@ -223,19 +395,22 @@ template <typename T> struct Dividends {
 // divisions, the square root and the two powers in the short forms of tode_math.h wherever the wavefront's operands allow
 // them, 0.66 -> 0.53 ms; and the waits for what was loaded ahead only where it is used (they stood behind each point's index,
 // and at the end of the iteration behind the copies of the record's entry): 0.53 -> 0.46, float64, B = 20 000, 0.56 -> 0.49.
-// What is held for all this costs registers: float32 rows of two take up to 182 (two wavefronts per SIMD; three before), rows of four
+// What does not wait for a cotangent -- the stages, the error ratio and the step factor's powers, the dense output's
+// coefficients, 500 of 1800 instructions -- is formed by a second wavefront one iteration ahead (PAIR, form_iteration, HandOver; one
+// barrier of LDS between them an iteration) where the SIMD has an issue slot to spare: 0.45 -> 0.37 ms at B = 65536.
+// What is held for all this costs registers (one wavefront for everything): float32 rows of two take up to 182 (two wavefronts per SIMD; three before), rows of four
 // 256 and 7 to 12 accumulation registers (one; two before), float64 rows of eight all 512 and 800 to 900 bytes of scratch.  It pays all the
 // same where a SIMD has wavefronts to choose from.  Backward passes, before and now: Van der Pol float32, B = 262 144, 2.41 -> 1.11 ms,
 // a million 7.9 -> 4.1; decay, float32 rows of four, 262 144, 1.00 -> 0.75, a million 3.00 -> 2.75; float64 rows of eight, 262 144,
 // Dopri5 4.45 -> 4.17 and Tsit5 4.42 -> 3.81, a million 16.3 -> 15.8 and 16.3 -> 14.2.
-template <typename T, int METHOD, int CTRL, typename Term>
-__global__ void __launch_bounds__(64) whole_backward_kernel(const WholeBackward<T> w) {
+template <typename T, int METHOD, int CTRL, typename Term, bool PAIR>
+__global__ void __launch_bounds__(PAIR ? 128 : 64) whole_backward_kernel(const WholeBackward<T> w) {
     using Tab = typename std::conditional<METHOD == 1, Tsit5Tab, Dopri5Tab>::type;
     constexpr int F = Term::F, P = Term::P;
     constexpr bool SHORT = F * sizeof(T) <= 32;  // the short forms (rows of eight doubles have no registers left for what they keep)
     constexpr int AHEAD = F <= 4 ? 4 : (SHORT ? 2 : 1);  // points held: a step of these systems passes one to four
     const long long B = w.batch;
-    const long long g = (long long)blockIdx.x * 64 + threadIdx.x;  // this thread's sample
+    const long long g = (long long)blockIdx.x * 64 + (threadIdx.x & 63);  // this thread's sample
     if (g >= B) return;
     Term rhs;
     rhs.load(w.params + g * P, w.scalars);
@@ -245,6 +420,33 @@ __global__ void __launch_bounds__(64) whole_backward_kernel(const WholeBackward<
 
     const CtrlParams<T> &cp = w.cp;
     const int E = w.E;
+    extern __shared__ __align__(16) unsigned char smem_raw[];
+    HandOver<T, F> hand(smem_raw);
+    if constexpr (PAIR) {
+        static_assert(SHORT, "built for the short forms");
+        // (alternating between neighbouring workgroups, so that every SIMD hosts one wavefront of each kind)
+        if ((((threadIdx.x >> 6) + (blockIdx.x >> 1)) & 1) == 0) {
+            const long long L = w.iterations;
+            RecordEntry<T, F> here = load_entry<T, F>(w, L > 0 ? L - 1 : 0, g);
+            bool running_new = w.rec_running[L * B + g] != 0;
+            for (long long i = L - 1; i >= 0; --i) {
+                RecordEntry<T, F> before = load_entry<T, F>(w, i > 0 ? i - 1 : 0, g);
+                if ((E == 0 && i == L - 1) || lanes_where(here.running != 0)) {  // (the iterations that the other wavefront asks for)
+                    Formed<T, F> formed;
+                    form_iteration<T, METHOD, CTRL, Term>(w, rhs, here, running_new, formed);
+                    T slope[F][4];
+#pragma unroll
+                    for (int f = 0; f < F; ++f) form_slope<T, METHOD, F>(here.dt, here.y, formed.y1, formed.k, f, slope[f]);
+                    hand.write(formed, slope);
+                    entry_is_here(before);
+                    lds_barrier();
+                }
+                running_new = here.running != 0;
+                here = before;
+            }
+            return;
+        }
+    }
     const T ts = w.t_start[g * w.ts_stride], te = w.t_end[g * w.te_stride];
     const T tlo = tmin(ts, te), thi = tmax(te, ts);
     const T sf = (T)__builtin_sqrt((double)F);
@@ -332,22 +534,19 @@ __global__ void __launch_bounds__(64) whole_backward_kernel(const WholeBackward<
         const T t0 = here.t, dt = here.dt, prev = here.prev, pprev = here.pprev;
         const bool move = after.n_accepted > here.n_accepted, running_new = after.running != 0;
 
-        // ---- the stages again (runge_kutta.py:255-263) ----
-        T k[7][F], y[F], yi[7][F];
+        T y[F];
 #pragma unroll
-        for (int f = 0; f < F; ++f) y[f] = here.y[f], k[0][f] = here.k0[f];
+        for (int f = 0; f < F; ++f) y[f] = here.y[f];
+        Formed<T, F> o;
+        if constexpr (PAIR) {
+            lds_barrier();
+            hand.read(o);
 #pragma unroll
-        for (int s = 1; s < 7; ++s) {
-#pragma unroll
-            for (int f = 0; f < F; ++f) {
-                T sum = 0;
-#pragma unroll
-                for (int j = 0; j < s; ++j) sum = fma_((T)Tab::a[s][j], k[j][f], sum);
-                yi[s][f] = fma_(dt, sum, y[f]);
-            }
-            rhs(fma_((T)Tab::c[s], dt, t0), yi[s], k[s]);
+            for (int f = 0; f < F; ++f) o.k[0][f] = here.k0[f];
+        } else {
+            form_iteration<T, METHOD, CTRL, Term>(w, rhs, here, running_new, o);
         }
-        const T(&y1)[F] = yi[6];
+        const T(&k)[7][F] = o.k, (&y1)[F] = o.y1;
 
         // ---- everything after the stages, reversed: the operations of finish_backward_sample, in its order ----
         const T t_new = move ? (t0 + dt) : t0;
@@ -355,60 +554,9 @@ __global__ void __launch_bounds__(64) whole_backward_kernel(const WholeBackward<
         T g_t, g_dt, g_prev = 0, g_pprev = 0, g_h, g_lo, g_hi, g_k[7][F], g_y[F], g_y1[F];
         {
             using Div = DivSqrtFeatures<T, F>;
-            // error ratio and step factor, in the short forms where every lane's operands are in their ranges (control_common's,
-            // over a wider range of the errors: their squares may vanish in the sum, as they do in the general form).  A sample
-            // that sits through an iteration with a zero step has an error of zero; its controller's results reach nothing.
-            T acc = 0, err[F], eb[F], per_eb[F], q[F], x[F], r, ratio, F0;
-            lanes_t outside = 0, bounds_outside = 0;
-            unsigned smallest = 0xffffffffu;
-            T largest_eb = 0;
-#pragma unroll
-            for (int f = 0; f < F; ++f) {
-                err[f] = 0;
-#pragma unroll
-                for (int s = 0; s < 7; ++s) err[f] = fma_(dt * (T)Tab::b_err[s], k[s][f], err[f]);
-                if constexpr (SHORT) {
-                    eb[f] = fma_(cp.rtol, max_abs(y[f], y1[f]), cp.atol);
-                    per_eb[f] = reciprocal_estimate(eb[f]);
-                    q[f] = quotient_with(abs_(err[f]), eb[f], per_eb[f]);
-                    x[f] = Div::fast(q[f]);
-                    smallest = min(smallest, min(high_bits(abs_(err[f])) - 1u, high_bits(q[f]) - 1u));  // (zero wraps round to the largest)
-                    largest_eb = f == 0 ? eb[f] : max_ordered(largest_eb, eb[f]);
-                    acc = fma_(x[f], x[f], acc);
-                }
-            }
-            if constexpr (SHORT) {
-                constexpr unsigned from = power_of_two_bits<T>(-40), width = power_of_two_bits<T>(16) - from;
-                const bool idle = acc == (T)0 && !running_new;
-                acc = idle ? (T)1 : acc;
-                bounds_outside = lanes_where(!(largest_eb <= (T)0x1p+20));
-                outside = lanes_where(smallest < power_of_two_bits<T>(Dividends<T>::smallest) - 1u) | lanes_where(high_bits(acc) - from >= width) | bounds_outside;
-                r = ratio = sqrt_plain(acc);
-                F0 = cp.safety * expk<true>(dw_mul(logk<true>(ratio), (T)cp.e1));
-                if (CTRL == 1 && !cp.skip2) F0 = F0 * expk<true>(dw_mul(logk<true>(prev), (T)cp.e2));
-                if (CTRL == 1 && !cp.skip3) F0 = F0 * expk<true>(dw_mul(logk<true>(pprev), (T)cp.e3));
-                constexpr unsigned history = power_of_two_bits<T>(-20), history_width = power_of_two_bits<T>(20) - history;
-                lanes_t history_outside = 0;
-                if (CTRL == 1 && !cp.skip2) history_outside |= lanes_where(high_bits(prev) - history >= history_width);
-                if (CTRL == 1 && !cp.skip3) history_outside |= lanes_where(high_bits(pprev) - history >= history_width);
-                outside |= history_outside, bounds_outside |= history_outside;
-            }
-            if (!SHORT || !w.plain || outside) {
-                acc = 0;
-#pragma unroll
-                for (int f = 0; f < F; ++f) {
-                    eb[f] = fma_(cp.rtol, tmax(abs_(y[f]), abs_(y1[f])), cp.atol);
-                    q[f] = abs_(err[f]) / eb[f];
-                    x[f] = q[f] / sf;
-                    acc = fma_(x[f], x[f], acc);
-                }
-                r = sqrt_(acc), ratio = tmax(r, (T)1e-38);
-                F0 = cp.safety * rpow<T>(ratio, cp.e1);
-                if (CTRL == 1) {
-                    F0 = F0 * (cp.skip2 ? (T)1 : rpow<T>(prev, cp.e2));
-                    F0 = F0 * (cp.skip3 ? (T)1 : rpow<T>(pprev, cp.e3));
-                }
-            }
+            const T(&err)[F] = o.err, (&eb)[F] = o.eb, (&per_eb)[F] = o.per_eb, (&q)[F] = o.q, (&x)[F] = o.x;
+            const T r = o.r, ratio = o.ratio, F0 = o.F0;
+            lanes_t bounds_outside = lanes_where(o.bounds_outside);
             // Quotients of cotangents: the divisors' ranges are known, the dividends are looked at.  divisors_outside: lanes
             // (of those that take part) whose divisor is outside.
             const T per_ratio = reciprocal_estimate(ratio);
@@ -536,11 +684,12 @@ __global__ void __launch_bounds__(64) whole_backward_kernel(const WholeBackward<
         auto build_slopes = [&](int first, int last) {
 #pragma unroll
             for (int f = first; f < last; ++f) {
-                const T ks[7] = {k[0][f], k[1][f], k[2][f], k[3][f], k[4][f], k[5][f], k[6][f]};
-                T q[5][1];
-                quartic_elem<T, METHOD>(dt, y[f], y1[f], ks, true, q);
-                slope[f][0] = q[1][0], slope[f][1] = (T)2 * q[2][0], slope[f][2] = (T)3 * q[3][0], slope[f][3] = (T)4 * q[4][0];
+                form_slope<T, METHOD, F>(dt, y, y1, k, f, slope[f]);
             }
+        };
+        auto slopes_of_all = [&] {
+            if constexpr (PAIR) hand.read_slopes(slope);
+            else build_slopes(0, F);
         };
         auto add_point = [&](const T t, const T(&cotangent)[F], T *g_time) {
             const T from_t0 = t - t0;
@@ -599,7 +748,7 @@ __global__ void __launch_bounds__(64) whole_backward_kernel(const WholeBackward<
                 const bool more = wrote(p, at[p], written_by[p]);
                 takes[p] = lanes_where(more), n += more ? 1 : 0;
             }
-            if (SHORT && takes[0]) build_slopes(0, F);
+            if (SHORT && takes[0]) slopes_of_all();
             if (takes[AHEAD - 1]) {  // (some sample's step passed more points than are held)
                 for (bool more = n == AHEAD; lanes_where(more);) {
                     const int e = max(cursor - n, 0);
@@ -619,7 +768,7 @@ __global__ void __launch_bounds__(64) whole_backward_kernel(const WholeBackward<
             takes[0] = lanes_where(end_point);
 #pragma unroll
             for (int p = 1; p < AHEAD; ++p) takes[p] = 0;
-            if (SHORT && end_point) build_slopes(0, F);
+            if (SHORT && end_point) slopes_of_all();
         }
 #pragma unroll
         for (int p = AHEAD - 1; p >= 0; --p) {
@@ -640,22 +789,23 @@ __global__ void __launch_bounds__(64) whole_backward_kernel(const WholeBackward<
         // ---- the stages reversed ----
 #pragma unroll
         for (int s = 6; s >= 1; --s) {
-            T gk[F], gy[F];
+            T gk[F], gy[F], sums[F], yi[F];
 #pragma unroll
-            for (int f = 0; f < F; ++f) gk[f] = g_k[s][f];
-            rhs.vjp(fma_((T)Tab::c[s], dt, t0), yi[s], gk, gy, gpar);
+            for (int f = 0; f < F; ++f) {
+                gk[f] = g_k[s][f], sums[f] = 0;
+#pragma unroll
+                for (int j = 0; j < s; ++j) sums[f] = fma_((T)Tab::a[s][j], k[j][f], sums[f]);
+                yi[f] = PAIR ? fma_(dt, sums[f], y[f]) : o.yi[s][f];
+            }
+            rhs.vjp(fma_((T)Tab::c[s], dt, t0), yi, gk, gy, gpar);
             T g_step = 0;
 #pragma unroll
             for (int f = 0; f < F; ++f) {
                 const T g_in = s == 6 ? gy[f] + g_y1[f] : gy[f];
                 g_y[f] += g_in;
-                T sum = 0;
 #pragma unroll
-                for (int j = 0; j < s; ++j) {
-                    sum = fma_((T)Tab::a[s][j], k[j][f], sum);
-                    g_k[j][f] += (T)Tab::a[s][j] * dt * g_in;
-                }
-                g_step += g_in * sum;
+                for (int j = 0; j < s; ++j) g_k[j][f] += (T)Tab::a[s][j] * dt * g_in;
+                g_step += g_in * sums[f];
             }
             g_dt += g_step;
         }
@@ -703,7 +853,17 @@ static int launch_backward(const tode_solve_args &a, const tode_controller &c, c
     w.lists = (int32_t *)adj.scratch;
     w.through_start = adj.through_start, w.dt0_given = a.dt0 != nullptr;
     w.ts_stride = a.t_start_stride, w.te_stride = a.t_end_stride;
-    hipLaunchKernelGGL((whole_backward_kernel<T, METHOD, CTRL, Term>), dim3((unsigned)((B + 63) / 64)), dim3(64), 0, stream, w);
+    // Two wavefronts to a group while a SIMD has no second group to issue for: up to one group per SIMD in float32, half of that in
+    // float64, whose hand-over takes twice the LDS (rows of four: 70 KB, two groups to a compute unit).  Kernel in us, one
+    // wavefront and two: Van der Pol float32, Tsit5 + PID, B = 300 367 and 305, 16 384 372 and 310, 65 536 408 and 355 (at 100 000
+    // two would share the SIMD with two more); Lorenz float32 60 000 194 and 163; decay, rows of four, 60 000 217 and 206;
+    // float64: Van der Pol 300 396 and 332, 32 768 426 and 414, 65 536 457 and 464; Lorenz 16 384 216 and 176, 32 768 226 and 187.
+    const long long groups = (B + 63) / 64;
+    constexpr bool paired = Term::F <= 4;
+    if (paired && groups <= TODE_PAIRED_SWEEP_GROUPS * 4 / (long long)sizeof(T))
+        hipLaunchKernelGGL((whole_backward_kernel<T, METHOD, CTRL, Term, paired>), dim3((unsigned)groups), dim3(128), (HandOver<T, Term::F>::bytes()), stream, w);
+    else
+        hipLaunchKernelGGL((whole_backward_kernel<T, METHOD, CTRL, Term, false>), dim3((unsigned)groups), dim3(64), 0, stream, w);
     return check_hip(hipGetLastError(), "tode_solve_builtin_backward launch");
 }
 
