@@ -476,6 +476,29 @@ typedef struct tode_mlp_start {
 } tode_mlp_start;
 int tode_mlp_start_backward(const tode_mlp_reverse *p, const tode_mlp_start *start, const tode_controller *c, void *stream);
 int tode_mlp_weight_gradients(const tode_mlp_reverse *p, void *out, void *stream);
+/*
+ * All of the above for a whole record (tode_solve_record of a solve with the perceptron: times that run in the solve's
+ * direction, no limits of the step size, times that want no gradient): the stages of all iterations, the iterations in reverse in
+ * one kernel, the start of the loop, the outer products and the sums of their shares.  The stage buffers of p hold the rows of
+ * 6 iterations + 2 evaluations, stage by stage over all iterations' samples and the start's two behind them (k: six times
+ * iterations x batch rows); p->g_y receives the cotangent of y0.  The record's pointers are taken from s, not from p.
+ */
+typedef struct tode_mlp_sweep {
+    tode_solve_record record;
+    int64_t iterations;
+    int32_t n_eval;
+    int32_t through_control;          /* gradients through the step sizes */
+    int32_t through_rule;             /* tode_mlp_start */
+    int32_t reserved;
+    const void *t_start, *t_end;      /* sample b at element b * stride */
+    int64_t t_start_stride, t_end_stride;
+    const void *t_eval, *grad_ys;     /* [B,E], [B,E,F] */
+    void *a_y, *a_k0, *a_dt;          /* [B,F], [B,F], [B]: room for the cotangents of the loop's first state */
+    void *t_end_dense;                /* [B] room */
+    void *error_sums, *control;       /* [iterations x B] floats, [iterations x B] times 16 bytes: room */
+    void *weight_gradients;           /* as tode_mlp_weight_gradients leaves them; NULL where p->sums is */
+} tode_mlp_sweep;
+int tode_mlp_sweep_record(const tode_mlp_reverse *p, const tode_mlp_sweep *s, const tode_controller *c, void *stream);
 
 /* ------------------------------------------------------------------------- */
 /* Per-step kernels around a right-hand side that lives outside the library   */

@@ -59,6 +59,7 @@ EXPORTS = (
     "tode_mlp_stages_backward",
     "tode_mlp_sweep_begin",
     "tode_mlp_start_backward",
+    "tode_mlp_sweep_record",
     "tode_mlp_outer_products",
     "tode_mlp_weight_gradients",
     "tode_select_end_point",
@@ -238,6 +239,14 @@ class MlpStart(C.Structure):
     _fields_ = [(name, C.c_void_p) for name in ("t_end", "a_y", "a_k0", "a_dt")] + [("through_rule", C.c_int32), ("n_eval", C.c_int32), ("grad_ys", C.c_void_p), ("t_eval", C.c_void_p)]
 
 
+class MlpSweep(C.Structure):
+    """struct tode_mlp_sweep"""
+
+    _fields_ = [("record", SolveRecord), ("iterations", C.c_int64)] + [(n, C.c_int32) for n in ("n_eval", "through_control", "through_rule", "reserved")] + [
+        ("t_start", C.c_void_p), ("t_end", C.c_void_p), ("t_start_stride", C.c_int64), ("t_end_stride", C.c_int64),
+    ] + [(n, C.c_void_p) for n in ("t_eval", "grad_ys", "a_y", "a_k0", "a_dt", "t_end_dense", "error_sums", "control", "weight_gradients")]  # fmt: skip
+
+
 class StepAdjoint(C.Structure):
     """struct tode_step_adjoint"""
 
@@ -384,6 +393,8 @@ def load():
         lib.tode_mlp_sweep_begin.argtypes = [C.c_int64, C.c_int32, C.c_int64, C.c_void_p, C.c_int64, C.c_void_p, C.c_int64] + [C.c_void_p] * 8
         lib.tode_mlp_start_backward.restype = C.c_int
         lib.tode_mlp_start_backward.argtypes = [C.POINTER(MlpReverse), C.POINTER(MlpStart), C.POINTER(Controller), C.c_void_p]
+        lib.tode_mlp_sweep_record.restype = C.c_int
+        lib.tode_mlp_sweep_record.argtypes = [C.POINTER(MlpReverse), C.POINTER(MlpSweep), C.POINTER(Controller), C.c_void_p]
         lib.tode_mlp_weight_gradients.restype = C.c_int
         lib.tode_mlp_weight_gradients.argtypes = [C.POINTER(MlpReverse), C.c_void_p, C.c_void_p]
         lib.tode_solve_builtin_fast_static.restype = C.c_int

@@ -551,7 +551,71 @@ class NetworkSweep:
             and y0.shape[0] > 0
         )
 
-    def __init__(self, lib, method_id, f, B, F, iterations, g_k, g_y, g_y1, g_t, g_dt, stream, in_arrays):
+    @classmethod
+    def whole(cls, lib, adjoint, replay, f, problem, dt0_given, arrays, iterations, grad_ys, params, ctrl, stream):
+        """The sweep over a whole record in arrays, times that want no gradient, from one call (tode_mlp_sweep_record: the stages of
+        all iterations, the iterations in reverse, the start of the loop, the weights' gradients).  Returns the cotangent of ``y0``
+        and the gradients of ``params``, or None where the rows of all evaluations are more than ROOM or cannot be had."""
+        (B, F), E, H, L = problem.y0.shape, problem.n_evaluation_points, f.W2.shape[1], iterations
+        dev = problem.y0.device
+        weights = (f.W1, f.b1, f.W2, f.b2)
+        wanted = any(x.requires_grad for x in weights)
+        room = 6 * L + 2
+        if 4 * B * (2 * 256 + 3 * F + 1) * room > cls.ROOM:
+            return None
+        splits = max(1, min(256, (room * B) // 64))
+        n_weights = sum(x.numel() for x in weights)
+        # (everything but the hidden units in one allocation, its parts at multiples of 256 bytes)
+        sizes = dict(packed=_lib.MLP_PACKED_SIZE["float32"], packed_reverse=_lib.MLP_REVERSE_PACKED_SIZE, k=6 * L * B * F, stage_inputs=room * B * F, stage_times=room * B,
+                     a_y=B * F, a_k0=B * F, a_dt=B, t_end_dense=B, error_sums=L * B, control=4 * L * B)  # fmt: skip
+        if wanted:
+            sizes.update(hidden_cotangents=room * B * 256, stage_cotangents=room * B * F, sums=splits * _lib.MLP_SUMS_SIZE)
+        offsets, total = {}, 0
+        for name, n in sizes.items():
+            offsets[name] = 4 * total
+            total += (n + 63) // 64 * 64
+        try:
+            hidden = torch.empty((room, B, 256), dtype=torch.float32, device=dev)
+            rest = torch.empty(total, dtype=torch.float32, device=dev)
+        except torch.cuda.OutOfMemoryError:
+            return None
+        base = rest.data_ptr()
+        at = {name: base + offset for name, offset in offsets.items()}
+        with torch.no_grad():
+            raw = f.builtin_shared()
+        _lib.check(lib.tode_mlp_pack_weights_for(raw.data_ptr(), raw.numel(), F, _lib.MLP_INPUTS["float32"], at["packed"], stream), "tode_mlp_pack_weights_for")
+        _lib.check(lib.tode_mlp_pack_weights_reverse(raw.data_ptr(), raw.numel(), F, at["packed_reverse"], stream), "tode_mlp_pack_weights_reverse")
+        g_y = torch.empty((B, F), dtype=torch.float32, device=dev)
+        out = torch.empty(n_weights, dtype=torch.float32, device=dev) if wanted else None
+        t_start, t_end = (x if x.stride(0) >= 1 else x.contiguous() for x in (replay.t_start.detach(), replay.t_end.detach()))
+        t_eval = replay.t_eval.detach().contiguous()
+        if grad_ys.data_ptr() % 16:
+            grad_ys = grad_ys.clone()
+
+        a = _lib.MlpReverse(adjoint.step_method.method_id, F, H, splits, B)
+        for name in ("packed", "packed_reverse", "k", "stage_inputs", "stage_times", "hidden_cotangents", "stage_cotangents", "sums"):
+            setattr(a, name, at.get(name))
+        a.hidden, a.g_y = hidden.data_ptr(), g_y.data_ptr()
+        s = _lib.MlpSweep(_lib.SolveRecord(arrays["t"].shape[0], *(arrays[n].data_ptr() for n in ("t", "dt", "y", "k0", "prev", "pprev", "running", "n_accepted"))), L, E)
+        s.through_control, s.through_rule = int(bool(replay.through_control)), int(dt0_given is None and bool(replay.through_control))
+        s.t_start, s.t_end, s.t_start_stride, s.t_end_stride = t_start.data_ptr(), t_end.data_ptr(), t_start.stride(0), t_end.stride(0)
+        s.t_eval, s.grad_ys = t_eval.data_ptr(), grad_ys.data_ptr()
+        for name in ("a_y", "a_k0", "a_dt", "t_end_dense", "error_sums", "control"):
+            setattr(s, name, at[name])
+        s.weight_gradients = _lib.ptr(out)
+        _lib.check(lib.tode_mlp_sweep_record(_lib.C.byref(a), _lib.C.byref(s), ctrl, stream), "tode_mlp_sweep_record")
+        return g_y, cls.through_weights(weights, out, params) if wanted else [None] * len(params)
+
+    @staticmethod
+    def through_weights(weights, out, params):
+        """The gradients of ``params`` given those of the held tensors, one behind the other: autograd carries them on to the leaves."""
+        if not params:
+            return []
+        grads = [g.view(x.shape) for g, x in zip(out.split([x.numel() for x in weights]), weights)]
+        pairs = [(x, g) for x, g in zip(weights, grads) if x.requires_grad]
+        return list(torch.autograd.grad([x for x, _ in pairs], params, [g for _, g in pairs], allow_unused=True, retain_graph=True))
+
+    def __init__(self, lib, method_id, f, B, F, iterations, g_k, g_y, g_y1, g_t, g_dt, stream, in_arrays, all_rows=True):
         dev, H = g_k.device, f.W2.shape[1]
         new = lambda *shape: torch.empty(shape, dtype=torch.float32, device=dev)
         self.lib, self.stream, self.f, self.started = lib, stream, f, False
@@ -568,7 +632,7 @@ class NetworkSweep:
         # the record alone, and two workgroups to a compute unit then hide each other's waits (B = 4096, three iterations: 90 us
         # in three launches, 63 in one).
         per_evaluation = 4 * B * (2 * 256 + 3 * F + 1)
-        room = max(6, min(6 * iterations + 2, self.ROOM // per_evaluation)) if wanted else 6
+        room = max(6, min(6 * iterations + 2, self.ROOM // per_evaluation)) if wanted and all_rows else 6
         self.held, self.B, self.F = 0, B, F
         self.iterations = iterations if in_arrays and wanted and iterations > 1 and room == 6 * iterations + 2 else 0  # (0: one at a time)
         try:
@@ -669,9 +733,7 @@ class NetworkSweep:
             return [None] * len(params)
         out = torch.empty(sum(x.numel() for x in weights), dtype=torch.float32, device=self.sums.device)
         _lib.check(self.lib.tode_mlp_weight_gradients(self.ref, out.data_ptr(), self.stream), "tode_mlp_weight_gradients")
-        grads = [g.view(x.shape) for g, x in zip(out.split([x.numel() for x in weights]), weights)]
-        pairs = [(x, g) for x, g in zip(weights, grads) if x.requires_grad]
-        return list(torch.autograd.grad([x for x, _ in pairs], params, [g for _, g in pairs], allow_unused=True, retain_graph=True))
+        return self.through_weights(weights, out, params)
 
 
 def reverse_sweep_kernels(adjoint, replay: Replay, term, args, problem, dt0_given, dt0, states, hits, grad_ys, params, params_given, arrays=None, iterations=0):
@@ -698,6 +760,15 @@ def reverse_sweep_kernels(adjoint, replay: Replay, term, args, problem, dt0_give
     fixed = ctrl.kind == _lib.CTRL_FIXED
     fixed_dt = contiguous(dt0, ttype) if fixed else None
     n_iterations = len(states) - 1 if arrays is None else iterations
+    wants = lambda x: x is not None and x.requires_grad
+    one_call = arrays is not None and n_iterations > 0 and not any(wants(x) for x in (replay.t_start, replay.t_end, replay.t_eval, dt0))
+    if one_call:
+        grad_ys = contiguous(grad_ys, dtype)
+        done = NetworkSweep.whole(lib, adjoint, replay, term.f, problem, dt0_given, arrays, n_iterations, grad_ys, params, cref, stream)
+        if done is not None:
+            out = {k: None for k in STATE_NAMES}
+            out.update(y=done[0], through_start=True)
+            return out, done[1]
 
     # which iteration wrote which evaluation point
     hit_iteration = None
@@ -719,7 +790,6 @@ def reverse_sweep_kernels(adjoint, replay: Replay, term, args, problem, dt0_give
     grad_ys = contiguous(grad_ys, dtype)
 
     # gradients of the times, collected by the kernels
-    wants = lambda x: x is not None and x.requires_grad
     g_t_start = zeros(B, dt=ttype) if wants(replay.t_start) else None
     g_t_end = zeros(B, dt=ttype) if wants(replay.t_end) else None
     g_t_eval = zeros(B, E, dt=ttype) if (E > 0 and wants(replay.t_eval)) else None
@@ -759,7 +829,7 @@ def reverse_sweep_kernels(adjoint, replay: Replay, term, args, problem, dt0_give
     f, with_args = term.f, term.with_args
     network = None
     if NetworkSweep.takes(adjoint, term, y0, t_start):  # (always so where `arrays` are given)
-        network = NetworkSweep(lib, method.method_id, f, B, F, n_iterations, g_k, g_y, g_y1, g_t, g_dt, stream, arrays is not None)
+        network = NetworkSweep(lib, method.method_id, f, B, F, n_iterations, g_k, g_y, g_y1, g_t, g_dt, stream, arrays is not None, all_rows=not one_call)
 
     def rhs(tt, yy):
         out = f(tt, yy, args) if with_args else f(tt, yy)

@@ -8,6 +8,8 @@
 //                               iterations in one launch where their rows fit, since they depend on the record alone;
 //   mlp_stages_backward_kernel  the six stages in reverse: the network's vector-Jacobian product and the stage sums' reverse,
 //                               the cotangents of all stage derivatives in registers between them;
+//   mlp_sweep_kernel            the iterations of a whole record in reverse, where the times want no gradient and the rows of all
+//                               evaluations fit: the step rule's and the dense output's reverse between the iterations too;
 //   mlp_weight_gradient_kernel  the two outer products over the rows of all evaluations of several iterations, split over
 //                               the rows;
 //   mlp_weight_gradient_sum_kernel  the splits' sums added in order, once per sweep.
@@ -16,13 +18,14 @@
 // evaluations forward 28 us (three iterations in one launch 63 us, two workgroups to a compute unit), back 29 us, of which the
 // matrix cores are busy 10.6 and 10.2 us -- the rest are the round trips through LDS between two products, the stage sums and
 // 150 KB of weights loaded per workgroup; the outer products of 20 evaluations 69 us (34 us of matrix instructions at 2.4 GHz,
-// 200 MB of rows at 2.9 TB/s).  A solve and its backward pass: 9.75 ms through autograd, 0.61 to 0.80 ms by the host's speed (0.42 ms of
-// kernels).
+// 200 MB of rows at 2.9 TB/s).  A solve and its backward pass: 9.75 ms through autograd, 0.61 to 0.80 ms by the host's speed with the
+// launches per iteration (0.42 ms of kernels), 0.57 in the one kernel and one call of it (0.37 ms).
 //
 // All products are on v_mfma_f32_16x16x4_f32.  For the vector-Jacobian product the weights are packed a second time,
 // transposed (tode_mlp_pack_weights_reverse), so that the same two facts hold as in the forward kernel: every lane keeps its
 // A operands in registers, and the first product's result, lane (q, c) holding the cotangents of hidden units 4q..4q+3 of
 // sample c, is after (1 - h^2) already the second product's B operand.
+#include "tode_adjoint.h"
 #include "tode_mlp.h"
 
 namespace tode {
@@ -75,15 +78,19 @@ __device__ __forceinline__ void mlp_put(float *row, int f0, int FR, const float 
     }
 }
 
-template <int METHOD> __global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2, 2))) mlp_stages_kernel(const tode_mlp_reverse p) {
+// error_sums: where not null, the sum over a row of the squares of its scaled errors, as the solve formed it.
+template <int METHOD>
+__global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2, 2))) mlp_stages_kernel(const tode_mlp_reverse p, float atol, float rtol, float *error_sums) {
     using Tab = typename std::conditional<METHOD == 1, Tsit5Tab, Dopri5Tab>::type;
     __shared__ MlpShared sh;
     const int tid = threadIdx.x, lane = tid & 63, w = tid >> 6, q = lane >> 4, c = lane & 15, FR = p.n_features, f0 = 16 * w + 4 * q;
     const long long B = p.batch, tiles = (B + MLP_TILE - 1) / MLP_TILE;
+    const float sf = (float)__builtin_sqrt((double)FR);
     MlpWeights W;
     mlp_load(W, (const float *)p.packed, tid);
     for (int i = tid; i < MLP_TILE * MLP_XS; i += 256) sh.x[i] = 0.0f;  // also the zero columns from 65 on
     __syncthreads();
+    int slot = 0;
     for (long long tile = blockIdx.x; tile < tiles; tile += gridDim.x) {
         const bool live = tile * MLP_TILE + c < B;
         const long long b = live ? tile * MLP_TILE + c : B - 1;
@@ -109,6 +116,20 @@ template <int METHOD> __global__ void __launch_bounds__(256) __attribute__((amdg
             }
             mlp_rhs<true>(sh, W, tn, yi, k[s], live ? (float *)p.hidden + row * MLP_H : nullptr);
             if (live) mlp_put((float *)p.k + row * FR, f0, FR, k[s]);
+            if (s == 6 && error_sums) {
+                float part[4], none[4] = {0, 0, 0, 0}, acc, unused;
+#pragma unroll
+                for (int r = 0; r < 4; ++r) {
+                    float err = 0;
+#pragma unroll
+                    for (int j = 0; j < 7; ++j) err = fma_(dt * (float)Tab::b_err[j], k[j][r], err);
+                    const float m = tmax(abs_(y[r]), abs_(yi[r]));
+                    const float x = (abs_(err) / fma_(rtol, m, atol)) / sf;
+                    part[r] = f0 + r < FR ? x * x : 0.0f;
+                }
+                mlp_sum2(sh, slot, part, none, acc, unused);
+                if (live && w == 0 && q == 0) error_sums[b] = acc;
+            }
         }
     }
 }
@@ -268,6 +289,257 @@ template <int METHOD> __global__ void __launch_bounds__(256) __attribute__((amdg
                 ((float *)p.g_t)[b] += g_t;
                 ((float *)p.g_dt)[b] += g_dt;
             }
+        }
+    }
+}
+
+// What an iteration of a sample is to the sweep below, ahead of it (one thread per iteration and sample; none of it waits for a
+// cotangent): the error ratio's root mean square from the stages' sum, the step factor before its clip, and the evaluation points
+// the iteration wrote (adjoints.py:215-234: those that its new time has reached and the time before it had not; times run in the
+// direction of the solve).  In a kernel of its own because powers and searches branch lane by lane, and the sweep holds more
+// registers than this compiler keeps whole across such branches (copies_ahead_of_the_exec_restore in build.py).
+struct MlpIteration {
+    float rms, F0;
+    int first, end;
+};
+
+template <int CTRL> __global__ void __launch_bounds__(256) mlp_sweep_control_kernel(const tode_mlp_sweep s, long long B, const CtrlParams<float> cp) {
+    const long long at = (long long)blockIdx.x * 256 + threadIdx.x;
+    if (at >= s.iterations * B) return;
+    const long long n = at / B, b = at - n * B;
+    const tode_solve_record &rec = s.record;
+    MlpIteration *const out = (MlpIteration *)s.control + at;
+    const float te = ((const float *)s.t_end)[b * s.t_end_stride], ts = ((const float *)s.t_start)[b * s.t_start_stride], dir = te > ts ? 1.0f : -1.0f;
+    const float rms = sqrt_(((const float *)s.error_sums)[at]), ratio = tmax(rms, 1e-38f);
+    float F0 = cp.safety * rpow_common<float>(ratio, cp.e1);
+    if (CTRL == 1) {
+        F0 = F0 * (cp.skip2 ? 1.0f : rpow_common<float>(((const float *)rec.prev)[at], cp.e2));
+        F0 = F0 * (cp.skip3 ? 1.0f : rpow_common<float>(((const float *)rec.pprev)[at], cp.e3));
+    }
+    const float *const times = (const float *)s.t_eval + b * s.n_eval;
+    const int lowest = times[0] == ts ? 1 : 0;  // (written by the loop's set-up)
+    auto reached = [&](float t) {  // how many points lie no further than t
+        int lo = 0, hi = s.n_eval;
+        while (lo < hi) {
+            const int mid = (lo + hi) / 2;
+            if (dir * t < dir * times[mid]) hi = mid;
+            else lo = mid + 1;
+        }
+        return max(lo, lowest);
+    };
+    out->rms = rms, out->F0 = F0;
+    out->first = n == 0 ? lowest : reached(((const float *)rec.t)[at]), out->end = reached(((const float *)rec.t)[at + B]);
+    if (n == 0) ((float *)s.t_end_dense)[b] = te;
+}
+
+// The whole loop of a recorded solve in reverse, a tile of 16 samples from its last iteration to its first: what
+// finish_backward_kernel and mlp_stages_backward_kernel do for one iteration, launch by launch, with the cotangents of the state
+// between the iterations in registers and the transposed weights loaded once.  A sample's row lies across sixteen lanes as in the
+// products: lane (q, c) of wavefront w holds features 16w + 4q .. + 3 of sample c, and every lane its sample's scalars.
+//
+// What a feature's cotangents are made of keeps the operations and the order of the two kernels (points in ascending order, five
+// sums a feature, spread once; shorter rows than 64 the former sweeps point by point), so that gradients with the step sizes held
+// constant are theirs bit for bit; sums over a
+// sample's features are the solve kernel's (mlp_sum2).  B = 4096, three iterations: 101 us, where three times the two kernels took 138.
+template <int METHOD, int CTRL>
+__global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(1, 1))) mlp_sweep_kernel(const tode_mlp_reverse p, const tode_mlp_sweep s, const CtrlParams<float> cp) {
+    using Tab = typename std::conditional<METHOD == 1, Tsit5Tab, Dopri5Tab>::type;
+    __shared__ MlpReverseShared sh;
+    const int tid = threadIdx.x, lane = tid & 63, w = tid >> 6, q = lane >> 4, c = lane & 15, FR = p.n_features, f0 = 16 * w + 4 * q, E = s.n_eval;
+    const long long B = p.batch, L = s.iterations, R = L * B, tiles = (B + MLP_TILE - 1) / MLP_TILE;
+    const float sf = (float)__builtin_sqrt((double)FR);
+    const tode_solve_record &rec = s.record;
+    MlpReverseWeights W;
+    mlp_load(W, (const float *)p.packed_reverse, tid);
+    int slot = 0;
+    for (long long tile = blockIdx.x; tile < tiles; tile += gridDim.x) {
+        const bool live = tile * MLP_TILE + c < B;
+        const long long b = live ? tile * MLP_TILE + c : B - 1;
+        const float ts = ((const float *)s.t_start)[b * s.t_start_stride], te = ((const float *)s.t_end)[b * s.t_end_stride];
+        const float tlo = tmin(ts, te), thi = tmax(te, ts);
+        const float *const times = (const float *)s.t_eval + b * E;
+        const float *const grad_ys = (const float *)s.grad_ys + b * E * FR;
+        float a_y[4] = {0, 0, 0, 0}, a_k0[4] = {0, 0, 0, 0}, a_t = 0, a_dt = 0, a_prev = 0, a_pprev = 0;
+        int running_after = rec.running[L * B + b], accepted_after = rec.n_accepted[L * B + b];
+        for (long long n = L - 1; n >= 0; --n) {
+            const long long at = n * B + b;
+            const float t0 = ((const float *)rec.t)[at], dt = ((const float *)rec.dt)[at], prev = ((const float *)rec.prev)[at], pprev = ((const float *)rec.pprev)[at];
+            const int running = rec.running[at], accepted = rec.n_accepted[at];
+            const bool move = accepted_after > accepted, running_new = running_after != 0;
+            float y[4], y1[4], k[7][4];
+            mlp_get((const float *)rec.y + at * FR, f0, FR, y);
+            mlp_get((const float *)rec.k0 + at * FR, f0, FR, k[0]);
+            mlp_get((const float *)p.stage_inputs + (5 * R + at) * FR, f0, FR, y1);
+#pragma unroll
+            for (int j = 1; j < 7; ++j) mlp_get((const float *)p.k + ((j - 1) * R + at) * FR, f0, FR, k[j]);
+
+            const MlpIteration it = ((const MlpIteration *)s.control)[at];
+            const int n_points = it.end - it.first;
+            const float rms = it.rms, F0 = it.F0, ratio = tmax(rms, 1e-38f);
+            const float factor = tclamp(F0, cp.fmin, cp.fmax);
+            const float t_new = move ? (t0 + dt) : t0, lo = tlo - t_new, hi = thi - t_new, dtn = running_new ? dt * factor : dt;
+
+            // ---- clamp of the step to the time range, and the new time ----
+            const float g_self = (dtn >= lo && dtn <= hi) ? a_dt : 0.0f, g_lo = (dtn < lo && lo < hi) ? a_dt : 0.0f, g_hi = (dtn > hi || hi < lo) ? a_dt : 0.0f;
+            const float g_tnew = a_t - (g_lo + g_hi), g_dt_next = running_new ? g_self : 0.0f;
+            float g_t = g_tnew, g_dt = running_new ? 0.0f : g_self;
+            if (move) g_dt += g_tnew;
+
+            // ---- controller history and step proposal ----
+            float g_ratio = 0, g_prev = 0, g_pprev = 0;
+            if (CTRL == 1) {
+                const bool keep = running_new && move;
+                g_ratio = keep ? a_prev : 0.0f;
+                g_prev = keep ? a_pprev : a_prev;
+                g_pprev = keep ? 0.0f : a_pprev;
+            }
+            if (s.through_control) {
+                g_dt += g_dt_next * factor;
+                const float g_factor = g_dt_next * dt, g_F0 = (F0 >= cp.fmin && F0 <= cp.fmax) ? g_factor : 0.0f;
+                g_ratio += g_F0 * F0 * (float)cp.e1 / ratio;
+                if (CTRL == 1) {
+                    if (!cp.skip2) g_prev += g_F0 * F0 * (float)cp.e2 / prev;
+                    if (!cp.skip3) g_pprev += g_F0 * F0 * (float)cp.e3 / pprev;
+                }
+            }
+
+            // ---- error ratio and error estimate; state update ----
+            const float tiny = 1e-38f, g_r = rms > tiny ? g_ratio : (rms == tiny ? g_ratio / 2.0f : 0.0f);
+            float share_t = 0, share_dt = 0;  // (this lane's, summed over the sample's lanes at the end)
+            float gk[7][4], gy[4], gy1[4];
+            const bool through_error = g_r != 0.0f && rms > 0.0f;
+#pragma unroll
+            for (int r = 0; r < 4; ++r) {
+                gy[r] = move ? 0.0f : a_y[r], gy1[r] = move ? a_y[r] : 0.0f;
+#pragma unroll
+                for (int j = 0; j < 7; ++j) gk[j][r] = 0;
+                gk[0][r] = move ? 0.0f : a_k0[r], gk[6][r] = move ? a_k0[r] : 0.0f;
+            }
+            if (lanes_where(through_error)) {  // (what a lane does not have is selected away, as everywhere here)
+#pragma unroll
+                for (int r = 0; r < 4; ++r) {
+                    const bool on = through_error && f0 + r < FR;
+                    float err = 0, bk = 0;
+#pragma unroll
+                    for (int j = 0; j < 7; ++j) err = fma_(dt * (float)Tab::b_err[j], k[j][r], err), bk = fma_((float)Tab::b_err[j], k[j][r], bk);
+                    const float ay = abs_(y[r]), ay1 = abs_(y1[r]);
+                    const float eb = fma_(cp.rtol, tmax(ay, ay1), cp.atol);
+                    const float x = abs_(err) / eb;
+                    const float g_q = g_r * (x / sf) / rms / sf;
+                    const float g_err = on ? g_q / eb * sign_(err) : 0.0f;
+                    const float g_m = on ? -g_q * x / eb * cp.rtol : 0.0f;
+                    float ga, gb;
+                    max_backward<float>(ay, ay1, g_m, ga, gb);
+                    gy[r] += ga * sign_(y[r]);
+                    gy1[r] += gb * sign_(y1[r]);
+#pragma unroll
+                    for (int j = 0; j < 7; ++j) gk[j][r] += g_err * (dt * (float)Tab::b_err[j]);
+                    share_dt += on ? g_err * bk : 0.0f;
+                }
+            }
+
+            // ---- dense output: five sums a feature over the points, then their shares ----
+            float den = (t0 + dt) - t0;
+            const bool flat = !(abs_(den) > 0.0f);
+            if (flat) den = 1.0f;
+            float G[4][5];
+            bool any[4] = {false, false, false, false};
+#pragma unroll
+            for (int r = 0; r < 4; ++r)
+#pragma unroll
+                for (int i = 0; i < 5; ++i) G[r][i] = 0;
+            for (int j = 0; lanes_where(j < n_points); j += 4) {  // (the cotangents of four points are on their way together)
+                float cotangent[4][4];
+#pragma unroll
+                for (int i = 0; i < 4; ++i) mlp_get(grad_ys + (long long)max(min(it.first + j + i, it.end - 1), 0) * FR, f0, FR, cotangent[i]);
+#pragma unroll
+                for (int i = 0; i < 4; ++i) {
+                    const bool taken = j + i < n_points;
+                    const float x = (times[max(min(it.first + j + i, it.end - 1), 0)] - t0) / den;
+#pragma unroll
+                    for (int r = 0; r < 4; ++r) {
+                        float g = cotangent[i][r];
+                        const bool adds = taken && g != 0.0f;  // (zero adds nothing, wherever the point lies: its position may be an infinity)
+                        any[r] = any[r] || adds;
+#pragma unroll
+                        for (int m = 0; m < 5; ++m) G[r][m] = adds ? G[r][m] + g : G[r][m], g = g * x;
+                    }
+                }
+            }
+            float g_points = 0, g_points_x = 0;
+#pragma unroll
+            for (int r = 0; r < 4; ++r) {
+                const float ks[7] = {k[0][r], k[1][r], k[2][r], k[3][r], k[4][r], k[5][r], k[6][r]};
+                float co[5][1], more_dt = 0;
+                quartic_elem<float, METHOD>(dt, y[r], y1[r], ks, true, co);
+                const float *g = G[r];
+                const bool on = any[r];  // (a state that is not finite adds nothing where no cotangent came)
+                g_points += on ? g[0] * co[1][0] + 2.0f * (g[1] * co[2][0]) + 3.0f * (g[2] * co[3][0]) + 4.0f * (g[3] * co[4][0]) : 0.0f;
+                g_points_x += on ? g[1] * co[1][0] + 2.0f * (g[2] * co[2][0]) + 3.0f * (g[3] * co[3][0]) + 4.0f * (g[4] * co[4][0]) : 0.0f;
+                auto add = [&](float &to, float v) { to = on ? to + v : to; };
+                if (METHOD == 1) {
+                    add(gy[r], g[0]);
+                    add(gk[0][r], g[1] * dt);
+                    more_dt += g[1] * ks[0];
+#pragma unroll
+                    for (int j = 0; j < 7; ++j) {
+                        const float u = g[2] * (float)Tsit5Tab::w[0][j] + g[3] * (float)Tsit5Tab::w[1][j] + g[4] * (float)Tsit5Tab::w[2][j];
+                        add(gk[j][r], u * dt);
+                        more_dt += u * ks[j];
+                    }
+                } else {
+                    const float g_f0 = -2.0f * g[4] + 5.0f * g[3] - 4.0f * g[2] + g[1], g_f1 = 2.0f * g[4] - 3.0f * g[3] + g[2];
+                    const float g_mid = 16.0f * g[4] - 32.0f * g[3] + 16.0f * g[2];
+                    add(gy[r], -8.0f * g[4] + 18.0f * g[3] - 11.0f * g[2] + g[0] + g_mid);
+                    add(gy1[r], -8.0f * g[4] + 14.0f * g[3] - 5.0f * g[2]);
+                    add(gk[0][r], g_f0 * dt);
+                    add(gk[6][r], g_f1 * dt);
+                    more_dt += g_f0 * ks[0] + g_f1 * ks[6];
+#pragma unroll
+                    for (int j = 0; j < 7; ++j) {
+                        add(gk[j][r], g_mid * (dt * (float)Dopri5Tab::w[0][j]));
+                        more_dt += g_mid * (float)Dopri5Tab::w[0][j] * ks[j];
+                    }
+                }
+                share_dt += on ? more_dt : 0.0f;
+            }
+            share_t -= g_points / den;
+            share_dt -= flat ? 0.0f : g_points_x / den;
+
+            // ---- the stages reversed (mlp_stages_backward_kernel) ----
+#pragma unroll
+            for (int j = 6; j >= 1; --j) {
+                const long long row = (j - 1) * R + at;
+                if (live && p.stage_cotangents) mlp_put((float *)p.stage_cotangents + row * FR, f0, FR, gk[j]);
+                float gi[4], gt;
+                mlp_vjp(sh, W, gk[j], (const float *)p.hidden + row * MLP_H, live && p.hidden_cotangents ? (float *)p.hidden_cotangents + row * MLP_H : nullptr, gi, gt);
+                share_t += gt;
+                share_dt = fma_((float)Tab::c[j], gt, share_dt);
+#pragma unroll
+                for (int r = 0; r < 4; ++r) {
+                    if (j == 6) gi[r] += gy1[r];
+                    gy[r] += gi[r];
+                    float sum = 0;
+#pragma unroll
+                    for (int i = 0; i < j; ++i) {
+                        sum = fma_((float)Tab::a[j][i], k[i][r], sum);
+                        gk[i][r] += (float)Tab::a[j][i] * dt * gi[r];
+                    }
+                    share_dt = fma_(gi[r], sum, share_dt);
+                }
+            }
+            const float of_t[4] = {share_t, 0, 0, 0}, of_dt[4] = {share_dt, 0, 0, 0};
+            float sum_t, sum_dt;
+            mlp_sum2(sh, slot, of_t, of_dt, sum_t, sum_dt);
+#pragma unroll
+            for (int r = 0; r < 4; ++r) a_y[r] = gy[r], a_k0[r] = gk[0][r];
+            a_t = g_t + sum_t, a_dt = g_dt + sum_dt, a_prev = g_prev, a_pprev = g_pprev;
+            running_after = running, accepted_after = accepted;
+        }
+        if (live) {
+            mlp_put((float *)s.a_y + b * FR, f0, FR, a_y);
+            mlp_put((float *)s.a_k0 + b * FR, f0, FR, a_k0);
+            if (w == 0 && q == 0) ((float *)s.a_dt)[b] = a_dt;
         }
     }
 }
@@ -631,6 +903,13 @@ static unsigned mlp_tiles_grid(const tode_mlp_reverse &p, int per_unit) {
     return (unsigned)(tiles < 256ll * per_unit ? tiles : 256ll * per_unit);
 }
 
+static int launch_stages(const tode_mlp_reverse &p, float atol, float rtol, float *error_sums, hipStream_t stream) {
+    const dim3 grid(mlp_tiles_grid(p, 2));
+    if (p.method == TODE_TSIT5) hipLaunchKernelGGL((mlp_stages_kernel<1>), grid, dim3(256), 0, stream, p, atol, rtol, error_sums);
+    else hipLaunchKernelGGL((mlp_stages_kernel<0>), grid, dim3(256), 0, stream, p, atol, rtol, error_sums);
+    return check_hip(hipGetLastError(), "tode_mlp_stages");
+}
+
 }  // namespace tode
 
 extern "C" {
@@ -651,10 +930,7 @@ int tode_mlp_stages(const tode_mlp_reverse *p, void *stream) {
     using namespace tode;
     const int rc = check_mlp_reverse(p);
     if (rc || p->batch == 0) return rc;
-    const dim3 grid(mlp_tiles_grid(*p, 2));
-    if (p->method == TODE_TSIT5) hipLaunchKernelGGL((mlp_stages_kernel<1>), grid, dim3(256), 0, (hipStream_t)stream, *p);
-    else hipLaunchKernelGGL((mlp_stages_kernel<0>), grid, dim3(256), 0, (hipStream_t)stream, *p);
-    return check_hip(hipGetLastError(), "tode_mlp_stages");
+    return launch_stages(*p, 0, 0, nullptr, (hipStream_t)stream);
 }
 
 int tode_mlp_stages_backward(const tode_mlp_reverse *p, void *stream) {
@@ -714,6 +990,55 @@ int tode_mlp_outer_products(const tode_mlp_reverse *p, int64_t rows, int32_t acc
     if ((p->n_features & 3) == 0) hipLaunchKernelGGL((mlp_weight_gradient_kernel<true>), dim3(p->splits), dim3(256), 0, (hipStream_t)stream, *p, (long long)rows, per_split, accumulate);
     else hipLaunchKernelGGL((mlp_weight_gradient_kernel<false>), dim3(p->splits), dim3(256), 0, (hipStream_t)stream, *p, (long long)rows, per_split, accumulate);
     return check_hip(hipGetLastError(), "tode_mlp_outer_products");
+}
+
+int tode_mlp_sweep_record(const tode_mlp_reverse *p, const tode_mlp_sweep *s, const tode_controller *c, void *stream) {
+    using namespace tode;
+    if (!p || !s || !c) return fail(TODE_E_INVALID, "null argument");
+    tode_mlp_reverse q = *p;
+    q.batch = p->batch * s->iterations, q.stage_rows = 0;
+    q.t = s->record.t, q.dt = s->record.dt, q.y = s->record.y, q.k0 = s->record.k0;
+    q.g_k = q.g_y1 = q.g_t = q.g_dt = p->g_y;  // (not used by the stages; the sweep keeps them in registers)
+    int rc = check_mlp_reverse(&q);
+    if (rc) return rc;
+    if (s->iterations < 1 || s->record.capacity < s->iterations + 1) return fail(TODE_E_INVALID, "%lld iterations, a record of %lld entries", (long long)s->iterations, (long long)s->record.capacity);
+    if (s->n_eval < 1) return fail(TODE_E_INVALID, "n_eval=%d", s->n_eval);
+    if (q.batch > (1ll << 38)) return fail(TODE_E_UNSUPPORTED, "batch too large");
+    if (s->t_start_stride < 1 || s->t_end_stride < 1) return fail(TODE_E_INVALID, "t_start_stride / t_end_stride must be >= 1");
+    if (c->kind != TODE_CTRL_INTEGRAL && c->kind != TODE_CTRL_PID) return fail(TODE_E_INVALID, "unknown controller kind %d", c->kind);
+    if (c->has_dt_min || c->has_dt_max) return fail(TODE_E_UNSUPPORTED, "limits of the step size");
+    if (p->batch == 0) return TODE_OK;
+    const tode_solve_record &r = s->record;
+    if (!r.t || !r.dt || !r.y || !r.k0 || !r.prev || !r.pprev || !r.running || !r.n_accepted || !s->t_start || !s->t_end || !s->t_eval || !s->grad_ys || !s->a_y || !s->a_k0 || !s->a_dt ||
+        !s->t_end_dense || !s->control || !s->error_sums || !p->sums != !s->weight_gradients)
+        return fail(TODE_E_INVALID, "null pointer");
+    if ((p->n_features & 3) == 0 && ((uintptr_t)s->grad_ys & 15)) return fail(TODE_E_INVALID, "grad_ys is not aligned to 16 bytes");  // (as every array whose rows are read so)
+    hipStream_t stream_ = (hipStream_t)stream;
+    const CtrlParams<float> cp = make_ctrl<float>(*c);
+    if ((rc = launch_stages(q, cp.atol, cp.rtol, (float *)s->error_sums, stream_))) return rc;
+    const dim3 blocks((unsigned)((q.batch + 255) / 256));
+    if (c->kind == TODE_CTRL_PID) hipLaunchKernelGGL((mlp_sweep_control_kernel<1>), blocks, dim3(256), 0, stream_, *s, (long long)p->batch, cp);
+    else hipLaunchKernelGGL((mlp_sweep_control_kernel<0>), blocks, dim3(256), 0, stream_, *s, (long long)p->batch, cp);
+    if ((rc = check_hip(hipGetLastError(), "tode_mlp_sweep_record launch"))) return rc;
+
+    q.batch = p->batch;
+    const dim3 grid(mlp_tiles_grid(q, 1));
+    auto launch = [&](auto kernel) { hipLaunchKernelGGL(kernel, grid, dim3(256), 0, stream_, q, *s, cp); };
+    const bool pid = c->kind == TODE_CTRL_PID;
+    if (p->method == TODE_TSIT5) pid ? launch(mlp_sweep_kernel<1, 1>) : launch(mlp_sweep_kernel<1, 0>);
+    else pid ? launch(mlp_sweep_kernel<0, 1>) : launch(mlp_sweep_kernel<0, 0>);
+    if ((rc = check_hip(hipGetLastError(), "tode_mlp_sweep_record launch"))) return rc;
+
+    // the start of the loop: its evaluations' rows lie behind those of the iterations
+    const long long rows = 6 * s->iterations * p->batch, FR = p->n_features;
+    tode_mlp_reverse first = q;
+    first.stage_inputs = (float *)p->stage_inputs + rows * FR, first.stage_times = (float *)p->stage_times + rows, first.hidden = (float *)p->hidden + rows * MLP_H;
+    if (p->sums) first.stage_cotangents = (float *)p->stage_cotangents + rows * FR, first.hidden_cotangents = (float *)p->hidden_cotangents + rows * MLP_H;
+    const tode_mlp_start start = {s->t_end_dense, s->a_y, s->a_k0, s->a_dt, s->through_rule, s->n_eval, s->grad_ys, s->t_eval};
+    if ((rc = tode_mlp_start_backward(&first, &start, c, stream))) return rc;
+    if (!p->sums) return TODE_OK;
+    if ((rc = tode_mlp_outer_products(&q, rows + (s->through_rule ? 2 : 1) * p->batch, 0, stream))) return rc;
+    return tode_mlp_weight_gradients(&q, s->weight_gradients, stream);
 }
 
 int tode_mlp_weight_gradients(const tode_mlp_reverse *p, void *out, void *stream) {
