@@ -449,6 +449,9 @@ typedef struct tode_mlp_reverse {
                                     iterations x samples, and k and the buffers point at the iteration's rows here); 0: batch */
 } tode_mlp_reverse;
 int tode_mlp_pack_weights_reverse(const void *raw, int64_t n_raw, int32_t n_features, void *packed, void *stream);
+/* Both packings of float32 weights in one launch, from the four tensors (contiguous): TODE_MLP_PACKED_SIZE values as
+ * tode_mlp_pack_weights_for leaves them, and TODE_MLP_REVERSE_PACKED_SIZE behind them. */
+int tode_mlp_pack_weights_both(const void *W1, const void *b1, const void *W2, const void *b2, int32_t n_hidden, int32_t n_features, void *packed, void *stream);
 int tode_mlp_stages(const tode_mlp_reverse *p, void *stream);
 int tode_mlp_stages_backward(const tode_mlp_reverse *p, void *stream);
 int tode_mlp_outer_products(const tode_mlp_reverse *p, int64_t rows, int32_t accumulate, void *stream);

@@ -349,3 +349,40 @@ def test_all_iterations_in_one_kernel(monkeypatch, B, F, H, points, control):
             cancelled = bound / 2e-5 * 2.0**-22 * math.sqrt(E) * float(cotangent.double().norm())
             assert bool(a.isfinite().all()) and float((a.double() - b.double()).norm()) <= bound * float(b.double().norm()) + cancelled
     assert len(calls) == 2 and all(c is not None for c in calls)
+
+
+@pytest.mark.parametrize("F, H", [(1, 1), (64, 256), (63, 255), (6, 40)])
+def test_both_packings_in_one_launch(F, H):
+    """The two orders straight from four tensors against the two packings of their concatenation."""
+    g = torch.Generator("cuda").manual_seed(F)
+    weights = [torch.randn(shape, generator=g, device="cuda") for shape in ((H, F + 1), (H,), (F, H), (F,))]
+    weights[0] = torch.cat([weights[0], weights[0]], 1)[:, : F + 1]  # (not contiguous)
+    f, lib = to.MLPField(*weights), _lib.load()
+    forward, reverse = _lib.MLP_PACKED_SIZE["float32"], _lib.MLP_REVERSE_PACKED_SIZE
+    raw, want = f.builtin_shared(), torch.full((forward + reverse,), 7.0, device="cuda")
+    _lib.check(lib.tode_mlp_pack_weights_for(raw.data_ptr(), raw.numel(), F, 0, want.data_ptr(), _lib.stream_of(raw)), "tode_mlp_pack_weights_for")
+    _lib.check(lib.tode_mlp_pack_weights_reverse(raw.data_ptr(), raw.numel(), F, want.data_ptr() + 4 * forward, _lib.stream_of(raw)), "tode_mlp_pack_weights_reverse")
+    assert torch.equal(f.builtin_packed_both(), want)
+
+
+def test_weights_written_between_the_passes(monkeypatch):
+    """The reverse sweep goes by the forward pass's packing of the weights only while the weights are those: written in place or
+    replaced in between, they are packed anew, and both sweeps take the new ones."""
+    from torchode_amd.autodiff import NetworkSweep
+
+    whole, results = NetworkSweep.whole, []
+    for one_kernel in (True, False):
+        monkeypatch.setattr(NetworkSweep, "whole", whole if one_kernel else lambda *a: None)
+        for change in (lambda f: f.W1.mul_(1.01), lambda f: setattr(f, "W2", f.W2 * 0.99), lambda f: None):
+            g = torch.Generator("cuda").manual_seed(9)
+            rand = lambda *shape: 0.2 * (2 * torch.rand(shape, generator=g, device="cuda") - 1)
+            f = to.MLPField(rand(256, 65), rand(256), rand(64, 256), rand(64))
+            y0 = rand(40, 64).requires_grad_()
+            solver = to.AutoDiffAdjoint(to.Dopri5(), to.IntegralController(1e-5, 1e-3), backprop_through_step_size_control=False)
+            sol = solver.solve(to.InitialValueProblem(y0, t_eval=torch.linspace(0, 1, 5, device="cuda").repeat(40, 1)), to.ODETerm(f))
+            with torch.no_grad():
+                change(f)
+            results.append(torch.autograd.grad(sol.ys, y0, torch.ones_like(sol.ys))[0])
+    for a, b in zip(results[:3], results[3:]):
+        assert torch.equal(a, b)
+    assert not torch.equal(results[0], results[2]) and not torch.equal(results[1], results[2])

@@ -55,6 +55,7 @@ EXPORTS = (
     "tode_mlp_pack_weights",
     "tode_mlp_pack_weights_for",
     "tode_mlp_pack_weights_reverse",
+    "tode_mlp_pack_weights_both",
     "tode_mlp_stages",
     "tode_mlp_stages_backward",
     "tode_mlp_sweep_begin",
@@ -393,6 +394,8 @@ def load():
         lib.tode_mlp_sweep_begin.argtypes = [C.c_int64, C.c_int32, C.c_int64, C.c_void_p, C.c_int64, C.c_void_p, C.c_int64] + [C.c_void_p] * 8
         lib.tode_mlp_start_backward.restype = C.c_int
         lib.tode_mlp_start_backward.argtypes = [C.POINTER(MlpReverse), C.POINTER(MlpStart), C.POINTER(Controller), C.c_void_p]
+        lib.tode_mlp_pack_weights_both.restype = C.c_int
+        lib.tode_mlp_pack_weights_both.argtypes = [C.c_void_p] * 4 + [C.c_int32, C.c_int32, C.c_void_p, C.c_void_p]
         lib.tode_mlp_sweep_record.restype = C.c_int
         lib.tode_mlp_sweep_record.argtypes = [C.POINTER(MlpReverse), C.POINTER(MlpSweep), C.POINTER(Controller), C.c_void_p]
         lib.tode_mlp_weight_gradients.restype = C.c_int

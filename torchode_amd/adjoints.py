@@ -591,7 +591,12 @@ class AutoDiffAdjoint(nn.Module):
         if f.builtin_kind == _lib.TERM_MLP:
             if dtype != torch.float32 or not 1 <= y0.shape[1] <= 64 or f.W1.shape[1] != y0.shape[1] + 1 or not 1 <= f.W1.shape[0] <= 256:
                 return None  # the matrix-core kernel takes up to 64 features and up to 256 hidden units: the caller takes another path
-            shared = f.builtin_packed(dev, dtype, fresh=record is not None)
+            if record is None:
+                shared = f.builtin_packed(dev, dtype)
+            else:  # (the weights as this solve takes them are what its reverse sweep goes by: kept with the record)
+                weights = (f.W1, f.b1, f.W2, f.b2)
+                record.packed = (f.builtin_packed_both(), weights, [w._version for w in weights])
+                shared = record.packed[0][: _lib.MLP_PACKED_SIZE["float32"]]
         else:
             params = f.builtin_params()
         if record is not None:

@@ -128,6 +128,7 @@ class LoopRecord:
         self.arrays = None  # the same record as entry-major arrays, where the whole-solve kernel wrote it
         self.wrote_points = False  # known without a look at the device: some iteration wrote an evaluation point
         self.flags = None  # that kernel's flag words, still on the device
+        self.packed = None  # the network's weights as the forward pass packed them, with the tensors and their versions then
         self.unordered_rows = False  # some row of evaluation points does not run in the direction of its solve
 
     def snapshot(self, t, dt, y, k0, hist, ints):
@@ -552,7 +553,7 @@ class NetworkSweep:
         )
 
     @classmethod
-    def whole(cls, lib, adjoint, replay, f, problem, dt0_given, arrays, iterations, grad_ys, params, ctrl, stream):
+    def whole(cls, lib, adjoint, replay, f, problem, dt0_given, arrays, iterations, packed, grad_ys, params, ctrl, stream):
         """The sweep over a whole record in arrays, times that want no gradient, from one call (tode_mlp_sweep_record: the stages of
         all iterations, the iterations in reverse, the start of the loop, the weights' gradients).  Returns the cotangent of ``y0``
         and the gradients of ``params``, or None where the rows of all evaluations are more than ROOM or cannot be had."""
@@ -566,7 +567,7 @@ class NetworkSweep:
         splits = max(1, min(256, (room * B) // 64))
         n_weights = sum(x.numel() for x in weights)
         # (everything but the hidden units in one allocation, its parts at multiples of 256 bytes)
-        sizes = dict(packed=_lib.MLP_PACKED_SIZE["float32"], packed_reverse=_lib.MLP_REVERSE_PACKED_SIZE, k=6 * L * B * F, stage_inputs=room * B * F, stage_times=room * B,
+        sizes = dict(k=6 * L * B * F, stage_inputs=room * B * F, stage_times=room * B,
                      a_y=B * F, a_k0=B * F, a_dt=B, t_end_dense=B, error_sums=L * B, control=4 * L * B)  # fmt: skip
         if wanted:
             sizes.update(hidden_cotangents=room * B * 256, stage_cotangents=room * B * F, sums=splits * _lib.MLP_SUMS_SIZE)
@@ -581,10 +582,13 @@ class NetworkSweep:
             return None
         base = rest.data_ptr()
         at = {name: base + offset for name, offset in offsets.items()}
-        with torch.no_grad():
-            raw = f.builtin_shared()
-        _lib.check(lib.tode_mlp_pack_weights_for(raw.data_ptr(), raw.numel(), F, _lib.MLP_INPUTS["float32"], at["packed"], stream), "tode_mlp_pack_weights_for")
-        _lib.check(lib.tode_mlp_pack_weights_reverse(raw.data_ptr(), raw.numel(), F, at["packed_reverse"], stream), "tode_mlp_pack_weights_reverse")
+        # (the forward pass's packings, unless a weight has been replaced or written since)
+        if packed is not None and all(x is y and x._version == v for x, y, v in zip(weights, packed[1], packed[2])):
+            both = packed[0]
+        else:
+            both = f.builtin_packed_both()
+        at["packed"] = both.data_ptr()
+        at["packed_reverse"] = at["packed"] + 4 * _lib.MLP_PACKED_SIZE["float32"]
         g_y = torch.empty((B, F), dtype=torch.float32, device=dev)
         out = torch.empty(n_weights, dtype=torch.float32, device=dev) if wanted else None
         t_start, t_end = (x if x.stride(0) >= 1 else x.contiguous() for x in (replay.t_start.detach(), replay.t_end.detach()))
@@ -736,7 +740,7 @@ class NetworkSweep:
         return self.through_weights(weights, out, params)
 
 
-def reverse_sweep_kernels(adjoint, replay: Replay, term, args, problem, dt0_given, dt0, states, hits, grad_ys, params, params_given, arrays=None, iterations=0):
+def reverse_sweep_kernels(adjoint, replay: Replay, term, args, problem, dt0_given, dt0, states, hits, grad_ys, params, params_given, arrays=None, iterations=0, packed=None):
     """The iterations in reverse through the library's reverse kernels (tode_step_finish_backward,
     tode_step_stage_backward): per iteration the stage values are recomputed by the forward stage kernel and ``f``
     (six evaluations under grad mode, each a small graph of its own), the finish kernel is reversed in one launch,
@@ -764,7 +768,7 @@ def reverse_sweep_kernels(adjoint, replay: Replay, term, args, problem, dt0_give
     one_call = arrays is not None and n_iterations > 0 and not any(wants(x) for x in (replay.t_start, replay.t_end, replay.t_eval, dt0))
     if one_call:
         grad_ys = contiguous(grad_ys, dtype)
-        done = NetworkSweep.whole(lib, adjoint, replay, term.f, problem, dt0_given, arrays, n_iterations, grad_ys, params, cref, stream)
+        done = NetworkSweep.whole(lib, adjoint, replay, term.f, problem, dt0_given, arrays, n_iterations, packed, grad_ys, params, cref, stream)
         if done is not None:
             out = {k: None for k in STATE_NAMES}
             out.update(y=done[0], through_start=True)
@@ -1048,7 +1052,7 @@ class SolveThroughLoop(torch.autograd.Function):
             hits = simulate_hits(replay, states, E) if arrays is None else None
             if use_kernels:
                 adj, grad_params = reverse_sweep_kernels(
-                    adjoint, replay, term, args, problem, ctx.dt0, dt0, states, hits, grad_ys, params, list(ctx.params), arrays, ctx.record.iterations
+                    adjoint, replay, term, args, problem, ctx.dt0, dt0, states, hits, grad_ys, params, list(ctx.params), arrays, ctx.record.iterations, ctx.record.packed
                 )
             else:
                 adj, grad_params = reverse_sweep_torch(replay, states, hits, grad_ys, params)

@@ -168,15 +168,27 @@ class MLPField(BuiltinTerm):
         """W1 | b1 | W2 | b2, row-major and concatenated."""
         return torch.cat([w.reshape(-1) for w in (self.W1, self.b1, self.W2, self.b2)]).contiguous()
 
-    def builtin_packed(self, device, dtype, fresh: bool = False) -> torch.Tensor:
+    def builtin_packed_both(self) -> torch.Tensor:
+        """float32 weights in the order the whole-solve kernel loads them and, behind it, in that of its reverse sweep: packed
+        for this call, whatever is kept (a training step changes its weights every time)."""
+        from . import _lib
+
+        weights = [w.detach().contiguous() for w in (self.W1, self.b1, self.W2, self.b2)]
+        size = _lib.MLP_PACKED_SIZE["float32"] + _lib.MLP_REVERSE_PACKED_SIZE
+        packed = torch.empty(size, dtype=torch.float32, device=weights[0].device)
+        rc = _lib.load().tode_mlp_pack_weights_both(*(w.data_ptr() for w in weights), self.W2.shape[1], self.W2.shape[0], packed.data_ptr(), _lib.stream_of(packed))
+        _lib.check(rc, "tode_mlp_pack_weights_both")
+        return packed
+
+    def builtin_packed(self, device, dtype) -> torch.Tensor:
         """The weights in the order the whole-solve kernel loads them into registers (a device
         tensor).  Packed once, and again whenever a weight tensor has been replaced or written
-        in place; ``fresh``: for this call, whatever was kept (a training step changes its weights every time)."""
+        in place."""
         from . import _lib
 
         weights = (self.W1, self.b1, self.W2, self.b2)
         key = (tuple((w.data_ptr(), w._version) for w in weights), device, dtype, self.matrix_inputs)
-        if fresh or getattr(self, "_packed_key", None) != key:
+        if getattr(self, "_packed_key", None) != key:
             raw = self.builtin_shared().to(device=device, dtype=dtype)
             packed = torch.empty(_lib.MLP_PACKED_SIZE[self.matrix_inputs], dtype=dtype, device=device)
             rc = _lib.load().tode_mlp_pack_weights_for(

@@ -19,7 +19,8 @@
 // matrix cores are busy 10.6 and 10.2 us -- the rest are the round trips through LDS between two products, the stage sums and
 // 150 KB of weights loaded per workgroup; the outer products of 20 evaluations 69 us (34 us of matrix instructions at 2.4 GHz,
 // 200 MB of rows at 2.9 TB/s).  A solve and its backward pass: 9.75 ms through autograd, 0.61 to 0.80 ms by the host's speed with the
-// launches per iteration (0.42 ms of kernels), 0.57 in the one kernel and one call of it (0.37 ms).
+// launches per iteration (0.42 ms of kernels), 0.46 in the one kernel, one call of it and one launch for
+// the weights (0.37 ms).
 //
 // All products are on v_mfma_f32_16x16x4_f32.  For the vector-Jacobian product the weights are packed a second time,
 // transposed (tode_mlp_pack_weights_reverse), so that the same two facts hold as in the forward kernel: every lane keeps its
@@ -35,9 +36,8 @@ constexpr int MLP_REVERSE_REGS = 64 + 64 + 16;  // packed values per thread: W2 
 constexpr int MLP_SUM_W1T = MLP_F * MLP_H, MLP_SUM_B1 = MLP_SUM_W1T + MLP_H, MLP_SUM_W2 = MLP_SUM_B1 + MLP_H, MLP_SUM_B2 = MLP_SUM_W2 + MLP_F * MLP_H;
 constexpr int MLP_SUMS = MLP_SUM_B2 + MLP_F;
 
-static __global__ void mlp_pack_reverse_kernel(const float *raw, float *packed, int H, int FR) {
-    const int i = blockIdx.x * blockDim.x + threadIdx.x;
-    if (i >= MLP_REVERSE_REGS * 256) return;
+// Where value i of the transposed order comes from in W1 | b1 | W2 | b2, or -1 for zero.
+__device__ __forceinline__ long long mlp_reverse_source(int i, int H, int FR) {
     const int tid = (i / 4) % 256, lane = tid & 63, w = tid >> 6, q = lane >> 4, c = lane & 15;
     int j = 4 * (i / 1024) + i % 4;
     const long long o_w2 = (long long)H * (FR + 1) + H;
@@ -54,7 +54,31 @@ static __global__ void mlp_pack_reverse_kernel(const float *raw, float *packed, 
         const int unit = 64 * w + 16 * (j / 4) + 4 * q + j % 4;
         if (unit < H) src = (long long)unit * (FR + 1) + FR;
     }
+    return src;
+}
+
+static __global__ void mlp_pack_reverse_kernel(const float *raw, float *packed, int H, int FR) {
+    const int i = blockIdx.x * blockDim.x + threadIdx.x;
+    if (i >= MLP_REVERSE_REGS * 256) return;
+    const long long src = mlp_reverse_source(i, H, FR);
     packed[i] = src < 0 ? 0.0f : raw[src];
+}
+
+// Both orders (tode_mlp_pack_weights_for's for float32 and the transposed one behind it) straight from the four tensors, in one
+// launch: a solve whose gradient is wanted packs its weights anew every time, and putting the tensors one behind the other and
+// packing them in two more launches, then all of it again ahead of the reverse sweep, left the GPU waiting for the host five times.
+static __global__ void mlp_pack_both_kernel(const float *W1, const float *b1, const float *W2, const float *b2, float *packed, int H, int FR) {
+    const int i = blockIdx.x * blockDim.x + threadIdx.x;
+    if (i >= (MLP_REGS + MLP_REVERSE_REGS) * 256) return;
+    long long src;
+    if (i < MLP_REGS * 256) {
+        const int tid = (i / 4) % 256, j = 4 * (i / 1024) + i % 4;  // (16-byte chunks: lane-contiguous loads of four values per thread)
+        src = mlp_packed_source(j, tid, H, FR);
+    } else {
+        src = mlp_reverse_source(i - MLP_REGS * 256, H, FR);
+    }
+    const long long o_b1 = (long long)H * (FR + 1), o_w2 = o_b1 + H, o_b2 = o_w2 + (long long)FR * H;
+    packed[i] = src < 0 ? 0.0f : src < o_b1 ? W1[src] : src < o_w2 ? b1[src - o_b1] : src < o_b2 ? W2[src - o_w2] : b2[src - o_b2];
 }
 
 // The lane's four features f0 .. f0 + 3 of a row of FR values: 16 bytes at a time where rows are whole groups of four.
@@ -924,6 +948,17 @@ int tode_mlp_pack_weights_reverse(const void *raw, int64_t n_raw, int32_t n_feat
     if (n_raw < FR || H * (2 * FR + 2) + FR != n_raw || H < 1 || H > MLP_H) return fail(TODE_E_UNSUPPORTED, "%lld weights do not make a network of up to %d hidden units", (long long)n_raw, MLP_H);
     hipLaunchKernelGGL(mlp_pack_reverse_kernel, dim3(MLP_REVERSE_REGS), dim3(256), 0, (hipStream_t)stream, (const float *)raw, (float *)packed, (int)H, (int)FR);
     return check_hip(hipGetLastError(), "tode_mlp_pack_weights_reverse");
+}
+
+int tode_mlp_pack_weights_both(const void *W1, const void *b1, const void *W2, const void *b2, int32_t n_hidden, int32_t n_features, void *packed, void *stream) {
+    using namespace tode;
+    static_assert(TODE_MLP_PACKED_SIZE == MLP_REGS * 256, "sizes");
+    if (!W1 || !b1 || !W2 || !b2 || !packed) return fail(TODE_E_INVALID, "null pointer");
+    if (n_features < 1 || n_features > MLP_F || n_hidden < 1 || n_hidden > MLP_H)
+        return fail(TODE_E_UNSUPPORTED, "the network's kernels take 1 to %d features and 1 to %d hidden units, got %d and %d", MLP_F, MLP_H, n_features, n_hidden);
+    hipLaunchKernelGGL(mlp_pack_both_kernel, dim3(MLP_REGS + MLP_REVERSE_REGS), dim3(256), 0, (hipStream_t)stream, (const float *)W1, (const float *)b1, (const float *)W2, (const float *)b2,
+                       (float *)packed, n_hidden, n_features);
+    return check_hip(hipGetLastError(), "tode_mlp_pack_weights_both");
 }
 
 int tode_mlp_stages(const tode_mlp_reverse *p, void *stream) {
