@@ -128,3 +128,33 @@ def test_threads_and_streams():
     for t in threads:
         t.join()
     assert not wrong
+
+
+@pytest.mark.parametrize("method,controller", [(to.Dopri5, to.IntegralController), (to.Tsit5, to.IntegralController), (to.Heun, to.IntegralController), (to.Euler, to.FixedStepController)])
+@pytest.mark.parametrize("dtype,time_dtype", [(torch.float32, torch.float32), (torch.float64, torch.float32)], ids=["f32", "f64-t32"])
+def test_stages_around_a_users_function(method, controller, dtype, time_dtype):
+    """A user's f gets fresh tensors at every stage, of its problem's types, that stay what they were; what it returns may be of
+    another type, expanded or strided; the loop's result is that of the operator path, evaluation by evaluation."""
+    seen = []
+
+    def f(t, y):
+        assert t.dtype == time_dtype and y.dtype == dtype and t.shape == (9,) and y.shape == (9, 3) and y.is_contiguous()
+        seen.append((t, y, y.clone()))
+        out = -y * (1 + t[:, None].to(dtype))
+        return (out.double(), out[:, :1].expand(9, 3), out.T.contiguous().T)[len(seen) % 3] if method is not to.Euler else out
+
+    g = torch.Generator().manual_seed(2)
+    y0 = torch.rand((9, 1), generator=g, dtype=torch.float64).to(dtype).expand(9, 3).cuda()
+    times = dict(t_eval=torch.linspace(0, 1, 5, dtype=time_dtype, device="cuda").repeat(9, 1))
+    dt0 = torch.full((9,), 0.125, dtype=time_dtype, device="cuda") if controller is to.FixedStepController else None
+    make = lambda: to.AutoDiffAdjoint(method(), controller() if dt0 is not None else controller(atol=1e-4, rtol=1e-3))
+    found = make().solve(to.InitialValueProblem(y0, **times), to.ODETerm(f), dt0=dt0)
+    assert len({id(y) for _, y, _ in seen}) == len(seen) and all(torch.equal(y, copy) for _, y, copy in seen)
+    steps = found.stats["n_f_evals"][0].item()
+    assert steps <= len(seen) <= steps + 12
+    wanted = make()._solve_protocol(to.InitialValueProblem(y0, **times), to.ODETerm(f), to.ODETerm(f), dt0, None)
+    assert torch.equal(found.stats["n_steps"], wanted.stats["n_steps"]) and torch.allclose(found.ys, wanted.ys, rtol=1e-5, atol=1e-6)
+    with pytest.raises(ValueError):
+        _lib.load_host().stage(0, 0, 1, y0, y0, None, None)
+    with pytest.raises(TypeError):
+        _lib.load_host().stage(0, 0)

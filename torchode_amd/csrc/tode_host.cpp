@@ -172,14 +172,44 @@ PyObject *solve_(PyObject *const *arg) {
     return append(result, 5, PyLong_FromLongLong(iterations));
 }
 
-PyObject *solve(PyObject *, PyObject *const *args, Py_ssize_t n) {
-    if (n != N_ARGS) {
-        PyErr_Format(PyExc_TypeError, "solve takes %zd arguments, got %zd", N_ARGS, n);
+// stage(state, controller, i, y, t, k, stream): stage i of an iteration around a user's right-hand side (tode_step_stage): a node time
+// and a stage input made like t and y, the launch that fills them, and (time, input) as the right-hand side's arguments.  k: the
+// derivative of the stage before, contiguous and of y's shape and type, or None.  state, controller, stream: addresses.
+PyObject *stage_(PyObject *const *arg) {
+    tode_step_state *const s = (tode_step_state *)PyLong_AsVoidPtr(arg[0]);
+    const tode_controller *const c = (const tode_controller *)PyLong_AsVoidPtr(arg[1]);
+    const long long i = integer(arg[2]);
+    void *const stream = arg[6] == Py_None ? nullptr : PyLong_AsVoidPtr(arg[6]);
+    if (PyErr_Occurred()) throw PythonError();
+    if (!s || !c || i < 1 || i > 6) {
+        PyErr_SetString(PyExc_ValueError, "stage: null address or stage out of range");
+        throw PythonError();
+    }
+    const Tensor &y = tensor(arg[3], "y"), &t = tensor(arg[4], "t");
+    if (arg[5] != Py_None) s->k[i - 1] = tensor(arg[5], "k").data_ptr();
+    const Tensor input = at::empty(y.sizes(), y.options()), node = at::empty(t.sizes(), t.options());
+    s->ystage[i] = input.data_ptr(), s->tnode = node.data_ptr();
+    int rc;
+    {
+        WithoutGil released;
+        rc = tode_step_stage(s, c, (int32_t)i, stream);
+    }
+    if (rc) library_error("tode_step_stage", rc);
+    PyObject *result = PyTuple_New(2);
+    if (!result) throw PythonError();
+    append(result, 0, THPVariable_Wrap(node));
+    return append(result, 1, THPVariable_Wrap(input));
+}
+
+template <Py_ssize_t N, PyObject *(*F)(PyObject *const *)> PyObject *entry(PyObject *, PyObject *const *args, Py_ssize_t n) {
+
+    if (n != N) {
+        PyErr_Format(PyExc_TypeError, "takes %zd arguments, got %zd", N, n);
         return nullptr;
     }
     HANDLE_TH_ERRORS
     try {
-        return solve_(args);
+        return F(args);
     } catch (const PythonError &) {
         return nullptr;
     }
@@ -187,7 +217,8 @@ PyObject *solve(PyObject *, PyObject *const *args, Py_ssize_t n) {
 }
 
 PyMethodDef methods[] = {
-    {"solve", (PyCFunction)(void (*)())solve, METH_FASTCALL, "One whole solve with a built-in term (see torchode_amd.adjoints)."},
+    {"solve", (PyCFunction)(void (*)())entry<N_ARGS, solve_>, METH_FASTCALL, "One whole solve with a built-in term (see torchode_amd.adjoints)."},
+    {"stage", (PyCFunction)(void (*)())entry<7, stage_>, METH_FASTCALL, "One stage around a user's right-hand side (see torchode_amd.adjoints)."},
     {nullptr, nullptr, 0, nullptr},
 };
 PyModuleDef module = {PyModuleDef_HEAD_INIT, "_host", nullptr, -1, methods, nullptr, nullptr, nullptr, nullptr};
