@@ -91,6 +91,22 @@ def test_library_exports_every_declared_symbol():
     assert lib.tode_last_error() is not None
 
 
+@pytest.mark.parametrize("name", ["HOST_LIB", "OPS_LIB"])
+def test_libraries_between_pytorch_and_the_kernels_have_no_thread_local_storage(name):
+    """Thread-local storage that a thread never reaches slows down every access of that thread to that of other libraries loaded at
+    run time, PyTorch's among them: all its operations, for the rest of the process."""
+    import struct
+
+    from torchode_amd import build
+
+    with open(getattr(build, name), "rb") as file:
+        elf = file.read()
+    assert elf[:6] == b"\x7fELF\x02\x01"
+    (table,), (size, count) = struct.unpack_from("<Q", elf, 32), struct.unpack_from("<HH", elf, 54)
+    kinds = [struct.unpack_from("<I", elf, table + i * size)[0] for i in range(count)]
+    assert 1 in kinds and 7 not in kinds  # PT_LOAD, PT_TLS
+
+
 def test_torch_operators_are_registered_for_the_gpu_only_with_tracing_rules():
     """libtorchode_amd_ops.so registers torch.ops.torchode_amd.solve_builtin / mlp_pack_weights: no CPU implementation
     (a call with CPU tensors fails in the dispatcher), and the shapes, dtypes and devices of the results for a tracer."""

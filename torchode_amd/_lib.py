@@ -474,6 +474,7 @@ def load():
         got = lib.tode_abi_version()
         if got != ABI_VERSION:
             raise RuntimeError(f"libtorchode_amd.so has ABI version {got}, the Python package expects {ABI_VERSION}")
+        lib.tode_last_error()  # (reaches the library's thread-local storage: until then this thread's torch operations are slower, build._compile_host_code)
         _lib = lib
         return _lib
 
