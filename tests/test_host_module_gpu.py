@@ -106,6 +106,19 @@ def test_refusals():
         _lib.load_host().solve(*[None] * 24)
 
 
+@pytest.mark.parametrize("limit,as_int", [(1e4, 10000), (3.9, 3), (True, 1), (torch.tensor(2.0), 2)])
+def test_step_limit_as_any_number(limit, as_int):
+    """``max_steps`` is taken as ``int(max_steps)`` says, with gradients and without."""
+    y0, t_eval = torch.full((5, 2), 0.5, device="cuda"), torch.linspace(0, 3, 4, device="cuda").repeat(5, 1)
+    make = lambda n: to.AutoDiffAdjoint(to.Dopri5(), to.IntegralController(atol=1e-6, rtol=1e-4), max_steps=n)
+    for gradient in (False, True):
+        a, b = (make(n).solve(to.InitialValueProblem(y0.clone().requires_grad_(gradient), t_eval=t_eval), to.ODETerm(to.VanDerPol(torch.ones(5, device="cuda")))) for n in (limit, as_int))
+        assert torch.equal(a.status, b.status) and torch.equal(a.stats["n_steps"], b.stats["n_steps"])
+        assert int(a.stats["n_steps"].max()) <= as_int and bool(a.status.any()) == (as_int < 10)
+        written = torch.arange(4, device="cuda") < a.stats["n_initialized"][:, None]
+        assert torch.equal(a.ys[written], b.ys[written])
+
+
 def test_threads_and_streams():
     """Solves of several host threads, each on a stream of its own: the call releases the interpreter while it waits."""
     solver = to.AutoDiffAdjoint(to.Tsit5(), to.IntegralController(atol=1e-6, rtol=1e-4))

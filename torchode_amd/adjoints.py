@@ -609,9 +609,9 @@ class AutoDiffAdjoint(nn.Module):
         if record is not None:
             return self._solve_recording(problem, term, dt0, params, shared, record)
         scalars = tuple(getattr(f, "builtin_scalars", tuple)())
-        c = _sub(self, "step_size_controller")
+        c, max_steps = _sub(self, "step_size_controller"), None if self.max_steps is None else int(self.max_steps)
         solved = _lib.load_host().solve(
-            y0, problem.t_start, problem.t_end, problem.t_eval, dt0, params, shared, _sub(self, "step_method").method_id, f.builtin_kind, scalars, self.max_steps,
+            y0, problem.t_start, problem.t_end, problem.t_eval, dt0, params, shared, _sub(self, "step_method").method_id, f.builtin_kind, scalars, max_steps,
             self.use_fast_path, f.builtin_kind in _lib.GENERAL_TERMS, c._kind, c.dt_min, c.dt_max, c._atol_f, c._rtol_f, c.pcoeff, c.icoeff, c.dcoeff, c.safety,
             c.factor_min, c.factor_max,
         )  # fmt: skip
