@@ -351,6 +351,40 @@ def test_all_iterations_in_one_kernel(monkeypatch, B, F, H, points, control):
     assert len(calls) == 2 and all(c is not None for c in calls)
 
 
+def test_outer_products_of_a_record_beyond_its_room(monkeypatch):
+    """A record whose rows do not all fit: the outer products are taken of as many iterations' rows at a time as do fit, and the
+    gradients are those of the sweep that holds all rows."""
+    from torchode_amd.autodiff import NetworkSweep
+
+    B, F, H, lib = 40, 64, 256, _lib.load()
+    g = torch.Generator("cuda").manual_seed(12)
+    rand = lambda *shape: torch.rand(shape, generator=g, device="cuda")
+    weights = [(math.sqrt(6.0 / (F + H)) * (2 * rand(*shape) - 1)).requires_grad_() for shape in ((H, F + 1), (H,), (F, H), (F,))]
+    y0 = (2 * rand(B, F) - 1).requires_grad_()
+    t_eval = 2 * torch.linspace(0, 1, 6, device="cuda").repeat(B, 1)
+    cotangent = 2 * rand(B, 6, F) - 1
+    outer, calls, results = lib.tode_mlp_outer_products, [], []
+    monkeypatch.setattr(lib, "tode_mlp_outer_products", lambda p, rows, accumulate, stream: calls.append((rows, accumulate)) or outer(p, rows, accumulate, stream))
+    for held in (None, 15):  # evaluations: two iterations and a remainder that no third fits into
+        if held:
+            monkeypatch.setattr(NetworkSweep, "ROOM", held * 4 * B * (2 * 256 + 3 * F + 1))
+        solver = to.AutoDiffAdjoint(to.Dopri5(), to.IntegralController(1e-6, 1e-5), backprop_through_step_size_control=False)
+        sol = solver.solve(to.InitialValueProblem(y0, t_eval=t_eval), to.ODETerm(to.MLPField(*weights)))
+        results.append(torch.autograd.grad(sol.ys, [y0, *weights], cotangent))
+    L = (int(sol.stats["n_f_evals"][0]) - 2) // 6
+    assert L >= 5
+    expected, rows = [], 0
+    for evaluations in [6] * L + [1]:  # (the start of the loop: its one evaluation where the step rule wants no gradient)
+        if rows + evaluations > 15:
+            expected.append(rows)
+            rows = 0
+        rows += evaluations
+    expected.append(rows)
+    assert calls == [(B * n, int(i > 0)) for i, n in enumerate(expected)]  # (the sweep that holds all rows calls it from native code)
+    for a, b in zip(*results):
+        assert float((a.double() - b.double()).norm()) <= 2e-5 * float(b.double().norm())
+
+
 @pytest.mark.parametrize("F, H", [(1, 1), (64, 256), (63, 255), (6, 40)])
 def test_both_packings_in_one_launch(F, H):
     """The two orders straight from four tensors against the two packings of their concatenation."""

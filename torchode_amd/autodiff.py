@@ -552,18 +552,21 @@ class NetworkSweep:
             and y0.shape[0] > 0
         )
 
+    @staticmethod
+    def evaluation_bytes(B, F) -> int:
+        """Memory that the rows of one evaluation of the network take."""
+        return 4 * B * (2 * 256 + 3 * F + 1)
+
     @classmethod
     def whole(cls, lib, adjoint, replay, f, problem, dt0_given, arrays, iterations, packed, grad_ys, params, ctrl, stream):
         """The sweep over a whole record in arrays, times that want no gradient, from one call (tode_mlp_sweep_record: the stages of
         all iterations, the iterations in reverse, the start of the loop, the weights' gradients).  Returns the cotangent of ``y0``
-        and the gradients of ``params``, or None where the rows of all evaluations are more than ROOM or cannot be had."""
+        and the gradients of ``params``, or None where memory for the rows of all evaluations cannot be had."""
         (B, F), E, H, L = problem.y0.shape, problem.n_evaluation_points, f.W2.shape[1], iterations
         dev = problem.y0.device
         weights = (f.W1, f.b1, f.W2, f.b2)
         wanted = any(x.requires_grad for x in weights)
         room = 6 * L + 2
-        if 4 * B * (2 * 256 + 3 * F + 1) * room > cls.ROOM:
-            return None
         splits = max(1, min(256, (room * B) // 64))
         n_weights = sum(x.numel() for x in weights)
         # (everything but the hidden units in one allocation, its parts at multiples of 256 bytes)
@@ -635,8 +638,7 @@ class NetworkSweep:
         # Where all of them fit and the record is in arrays, one launch forms the stages of every iteration: they depend on
         # the record alone, and two workgroups to a compute unit then hide each other's waits (B = 4096, three iterations: 90 us
         # in three launches, 63 in one).
-        per_evaluation = 4 * B * (2 * 256 + 3 * F + 1)
-        room = max(6, min(6 * iterations + 2, self.ROOM // per_evaluation)) if wanted and all_rows else 6
+        room = max(6, min(6 * iterations + 2, self.ROOM // self.evaluation_bytes(B, F))) if wanted and all_rows else 6
         self.held, self.B, self.F = 0, B, F
         self.iterations = iterations if in_arrays and wanted and iterations > 1 and room == 6 * iterations + 2 else 0  # (0: one at a time)
         try:
@@ -765,7 +767,12 @@ def reverse_sweep_kernels(adjoint, replay: Replay, term, args, problem, dt0_give
     fixed_dt = contiguous(dt0, ttype) if fixed else None
     n_iterations = len(states) - 1 if arrays is None else iterations
     wants = lambda x: x is not None and x.requires_grad
-    one_call = arrays is not None and n_iterations > 0 and not any(wants(x) for x in (replay.t_start, replay.t_end, replay.t_eval, dt0))
+    one_call = (
+        arrays is not None
+        and n_iterations > 0
+        and not any(wants(x) for x in (replay.t_start, replay.t_end, replay.t_eval, dt0))
+        and NetworkSweep.evaluation_bytes(B, F) * (6 * n_iterations + 2) <= NetworkSweep.ROOM
+    )
     if one_call:
         grad_ys = contiguous(grad_ys, dtype)
         done = NetworkSweep.whole(lib, adjoint, replay, term.f, problem, dt0_given, arrays, n_iterations, packed, grad_ys, params, cref, stream)
@@ -833,6 +840,8 @@ def reverse_sweep_kernels(adjoint, replay: Replay, term, args, problem, dt0_give
     f, with_args = term.f, term.with_args
     network = None
     if NetworkSweep.takes(adjoint, term, y0, t_start):  # (always so where `arrays` are given)
+        # (behind a call that found no memory for the rows of all evaluations: those of one iteration; a record too long for that
+        # call: as many as ROOM holds)
         network = NetworkSweep(lib, method.method_id, f, B, F, n_iterations, g_k, g_y, g_y1, g_t, g_dt, stream, arrays is not None, all_rows=not one_call)
 
     def rhs(tt, yy):
