@@ -202,7 +202,7 @@ def emit_assembly(directory: str, units=None) -> list:
 
 # The units whose kernels keep whole per-sample arrays in registers (up to 256 of them, some in accumulation
 # registers): where the compiler has been seen to place copies ahead of the execution mask's restore.
-UNITS_UNDER_REGISTER_PRESSURE = ("tode_backward_f32.o", "tode_backward_f64.o", "tode_mlp_reverse.o")
+UNITS_UNDER_REGISTER_PRESSURE = ("tode_backward_f32.o", "tode_backward_f64.o", "tode_mlp.o", "tode_mlp_reverse.o")
 
 
 def check_units_under_register_pressure() -> None:
