@@ -424,8 +424,13 @@ __global__ void __launch_bounds__(PAIR ? 128 : 64) whole_backward_kernel(const W
     HandOver<T, F> hand(smem_raw);
     if constexpr (PAIR) {
         static_assert(SHORT, "built for the short forms");
-        // (alternating between neighbouring workgroups, so that every SIMD hosts one wavefront of each kind)
-        if ((((threadIdx.x >> 6) + (blockIdx.x >> 1)) & 1) == 0) {
+        // The group's first wavefront forms; for rows of four doubles the second one.  Which of them does matters where groups share
+        // a compute unit -- roles that took turns by the group's number had the users of two groups on one SIMD there -- and to the
+        // registers the compiler chooses.  Taking turns and so, us: Van der Pol float32, 512 groups, 340 and 322, 768 339 and 316, 1024
+        // 360 and 355; float64, 256 387 and 389, 313 468 and 400, 511 484 and 431.  Decay, rows of four doubles, first and second
+        // wavefront: 5 groups 178 and 172, 256 187 and 183, 511 199 and 196.
+        constexpr unsigned FORMS = F * sizeof(T) == 32 ? 1 : 0;
+        if (threadIdx.x >> 6 == FORMS) {
             const long long L = w.iterations;
             RecordEntry<T, F> here = load_entry<T, F>(w, L > 0 ? L - 1 : 0, g);
             bool running_new = w.rec_running[L * B + g] != 0;
