@@ -3,6 +3,7 @@ against the same sweep with torch's evaluations of the network and autograd's ve
 record, at the edges of their tiles: one sample, a full tile of 16 and one more, more tiles than workgroups; one
 feature, rows that are no multiple of four, all 64; one hidden unit, 255, 256."""
 import math
+import types
 
 import pytest
 import torch
@@ -349,6 +350,71 @@ def test_all_iterations_in_one_kernel(monkeypatch, B, F, H, points, control):
             cancelled = bound / 2e-5 * 2.0**-22 * math.sqrt(E) * float(cotangent.double().norm())
             assert bool(a.isfinite().all()) and float((a.double() - b.double()).norm()) <= bound * float(b.double().norm()) + cancelled
     assert len(calls) == 2 and all(c is not None for c in calls)
+
+
+def replay_with(mistake):
+    """The oracle's loop, with one of the ways that a step size takes to later ones left out."""
+    from torchode_amd.autodiff import Replay
+
+    class Planted(Replay):
+        def attempt(self, state):
+            held = {"factor of the last ratio": "prev", "factor of the ratio before": "pprev"}.get(mistake)
+            return super().attempt(state if held is None else dict(state, **{held: state[held].detach()}))
+
+        def advance(self, state, attempt, *rest):
+            ks, y1, ratio, dt_next = attempt
+            if mistake == "ratio kept":
+                attempt = (ks, y1, ratio.detach(), dt_next)
+            if mistake == "ratio handed on":
+                state = dict(state, prev=state["prev"].detach())
+            return super().advance(state, attempt, *rest)
+
+    return Planted
+
+
+MISTAKES = ["factor of the last ratio", "factor of the ratio before", "ratio kept", "ratio handed on"]
+
+
+@pytest.mark.parametrize("F, H, method, first, until", [(64, 256, to.Tsit5, 0.2, 1.5), (7, 40, to.Tsit5, 0.4, 1.5), (64, 256, to.Dopri5, 0.2, 3), (33, 100, to.Dopri5, 0.2, 3)])
+def test_controllers_history_in_one_kernel(monkeypatch, F, H, method, first, until):
+    """A network with strong weights, large tolerances and a controller that looks far back: errors far above rounding, and
+    gradients to which every way through the controller's history adds a hundredth or more.  Against the record's iterations as torch
+    operations in float64 on the CPU, within 1e-3: the same in float32 comes to 5e-5, 2.4e-4, 3e-5 and 3e-5 of them; with one way
+    through the history left out they are 1.9e-2 and more apart, which is looked at too."""
+    from torchode_amd import autodiff
+
+    whole, calls = autodiff.NetworkSweep.whole, []
+    monkeypatch.setattr(autodiff.NetworkSweep, "whole", lambda *a: calls.append(whole(*a)) or calls[-1])
+    B, E, g = 17, 3, torch.Generator().manual_seed(0)
+    rand = lambda *shape: torch.rand(shape, generator=g, dtype=torch.float64)
+    weights = [(4 * math.sqrt(6.0 / (F + H)) * (2 * rand(*shape) - 1)).float() for shape in ((H, F + 1), (H,), (F, H), (F,))]
+    y0 = (2 * rand(B, F) - 1).float()
+    t_eval = (until * (0.8 + 0.4 * rand(B, 1)) * torch.linspace(0, 1, E, dtype=torch.float64)).float()
+    cotangent = (2 * rand(B, E, F) - 1).float()
+    cotangent[:, 0] = 0  # (the point at the start)
+    dt0, controller = torch.full((B,), first), to.PIDController(0.03, 0.03, 0.2, 0.4, -0.3)
+
+    leaves = [x.cuda().requires_grad_() for x in (y0, *weights)]
+    sol = to.AutoDiffAdjoint(method(), controller).solve(to.InitialValueProblem(leaves[0], t_eval=t_eval.cuda()), to.ODETerm(to.MLPField(*leaves[1:])), dt0=dt0.cuda())
+    assert not sol.status.any()
+    record = sol.ys.grad_fn.record
+    found = torch.autograd.grad(sol.ys, leaves, cotangent.cuda())
+    assert len(calls) == 1 and calls[0] is not None
+    states = [{k: v.cpu().double() if v.is_floating_point() else v.cpu() for k, v in state.items()} for state in record.trimmed(record.iterations)]
+
+    def through_the_record(mistake=None):
+        params = [x.double().requires_grad_() for x in weights]
+        problem = to.InitialValueProblem(y0.double(), t_eval=t_eval.double())
+        replay = replay_with(mistake)(method(), controller, to.ODETerm(to.MLPField(*params)), None, problem, True, dt0.double())
+        adj, grads = autodiff.reverse_sweep_torch(replay, states, autodiff.simulate_hits(replay, states, E), cotangent.double(), params)
+        of_y0 = autodiff.SolveThroughLoop.start_backward(types.SimpleNamespace(dt0=dt0), replay, adj, problem.y0, dt0.double(), params, grads)
+        return [of_y0, *grads]
+
+    want = through_the_record()
+    apart = lambda gradients: max(float((a.detach().cpu().double() - b).norm() / b.norm()) for a, b in zip(gradients, want))
+    print("iterations", record.iterations, "apart", apart(found), [apart(through_the_record(m)) for m in MISTAKES])
+    assert apart(found) <= 1e-3
+    assert all(apart(through_the_record(mistake)) >= 1e-2 for mistake in MISTAKES)
 
 
 def test_outer_products_of_a_record_beyond_its_room(monkeypatch):
