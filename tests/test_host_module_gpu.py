@@ -169,5 +169,24 @@ def test_stages_around_a_users_function(method, controller, dtype, time_dtype):
     assert torch.equal(found.stats["n_steps"], wanted.stats["n_steps"]) and torch.allclose(found.ys, wanted.ys, rtol=1e-5, atol=1e-6)
     with pytest.raises(ValueError):
         _lib.load_host().stage(0, 0, 1, y0, y0, None, None)
+    state, control, y = _lib.StepState(), _lib.Controller(), torch.zeros((9, 3), device="cuda")
+    for k in (y.cpu(), y.double(), y[:8], y.T.contiguous().T):
+        with pytest.raises(ValueError, match="of y's shape"):
+            _lib.load_host().stage(_lib.C.addressof(state), _lib.C.addressof(control), 1, y, y[:, 0], k, None)
     with pytest.raises(TypeError):
         _lib.load_host().stage(0, 0)
+
+
+@pytest.mark.parametrize("evaluation", [0, 1, 4, 7])
+def test_a_users_function_off_the_device_is_refused(evaluation):
+    """f's result on the CPU, at the start, at a stage and at the last one of a step, is an error as in torch's own arithmetic."""
+    seen = []
+
+    def f(t, y):
+        seen.append(None)
+        return -y.cpu() if len(seen) > evaluation else -y
+
+    problem = to.InitialValueProblem(torch.ones((5, 2), device="cuda"), t_eval=torch.linspace(0, 1, 3, device="cuda").repeat(5, 1))
+    with torch.no_grad(), pytest.raises(RuntimeError, match="GPU"):
+        to.AutoDiffAdjoint(to.Dopri5(), to.IntegralController(atol=1e-4, rtol=1e-3)).solve(problem, to.ODETerm(f))
+    torch.cuda.synchronize()

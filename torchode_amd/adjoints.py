@@ -452,7 +452,8 @@ class AutoDiffAdjoint(nn.Module):
 
         def rhs(tt, yy):
             out = f(tt, yy, args) if with_args else f(tt, yy)
-            if out.dtype != dtype or not out.is_contiguous() or out.shape != yy.shape:
+            if out.dtype != dtype or not out.is_contiguous() or out.shape != yy.shape or not out.is_cuda:
+                _lib.require_device(out)
                 out = out.to(dtype).expand(yy.shape).contiguous()
             return out
 

@@ -186,7 +186,11 @@ PyObject *stage_(PyObject *const *arg) {
         throw PythonError();
     }
     const Tensor &y = tensor(arg[3], "y"), &t = tensor(arg[4], "t");
-    if (arg[5] != Py_None) s->k[i - 1] = tensor(arg[5], "k").data_ptr();
+    if (arg[5] != Py_None) {
+        const Tensor &k = tensor(arg[5], "k");
+        TORCH_CHECK_VALUE(k.scalar_type() == y.scalar_type() && k.device() == y.device() && k.sizes() == y.sizes() && k.is_contiguous(), "stage: k must be contiguous and of y's shape, type and device");
+        s->k[i - 1] = k.data_ptr();
+    }
     const Tensor input = at::empty(y.sizes(), y.options()), node = at::empty(t.sizes(), t.options());
     s->ystage[i] = input.data_ptr(), s->tnode = node.data_ptr();
     int rc;
@@ -202,7 +206,6 @@ PyObject *stage_(PyObject *const *arg) {
 }
 
 template <Py_ssize_t N, PyObject *(*F)(PyObject *const *)> PyObject *entry(PyObject *, PyObject *const *args, Py_ssize_t n) {
-
     if (n != N) {
         PyErr_Format(PyExc_TypeError, "takes %zd arguments, got %zd", N, n);
         return nullptr;
