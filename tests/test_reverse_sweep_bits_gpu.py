@@ -71,11 +71,11 @@ def test_bits_of_the_gradients(case):
             assert torch.equal(got, stored), (attempt, name, float((got - stored).norm() / stored.norm()))
 
 
-# rows of four doubles hand over the most: 69 632 bytes of LDS
-IN_TWO = dict(CASES, **{"decay4-f64-tsit5-pid": ("decay", 4, "Tsit5", "pid", "float64", 30), "decay4-f64-dopri5-integral": ("decay", 4, "Dopri5", "integral", "float64", 30)})
+# (rows of four doubles hand over the most: 69 632 bytes of LDS)
+IN_TWO = dict(CASES, **{"vdp-f64-tsit5-pid": ("vdp", 2, "Tsit5", "pid", "float64", 33), "decay4-f64-tsit5-pid": ("decay", 4, "Tsit5", "pid", "float64", 30), "decay4-f64-dopri5-integral": ("decay", 4, "Dopri5", "integral", "float64", 30)})
 
 
-@pytest.mark.parametrize("case", ["vdp-f32-tsit5-pid", "vdp-f64-dopri5-integral", "lorenz-f32-dopri5-integral", "lorenz-f64-tsit5-pid", "decay1-f32-tsit5-integral", "decay4-f32-dopri5-integral",
+@pytest.mark.parametrize("case", ["vdp-f32-tsit5-pid", "vdp-f64-dopri5-integral", "vdp-f64-tsit5-pid", "lorenz-f32-dopri5-integral", "lorenz-f64-tsit5-pid", "decay1-f32-tsit5-integral", "decay4-f32-dopri5-integral",
                                   "decay3-f64-tsit5-integral", "decay4-f64-tsit5-pid", "decay4-f64-dopri5-integral"])  # fmt: skip
 def test_one_wavefront_and_two(case):
     """Samples of a batch of 1025 groups of 64 (one wavefront to a group) and the same in batches of 1 to 512 groups (two), of 513

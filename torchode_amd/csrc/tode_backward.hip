@@ -226,15 +226,19 @@ template <typename T, int F> struct Formed {
     T err[F], eb[F], per_eb[F], q[F], x[F], r, ratio, F0;
     bool bounds_outside;  // this lane's error bounds or history are outside the short forms' ranges
 };
+// With the sum of the errors' squares in front of the rest, for the kernels that form the errors later (LATER below).
+template <typename T> struct KeptSum {
+    T acc;
+};
+template <typename T, int F> struct FormedLater : KeptSum<T>, Formed<T, F> {};
+template <typename T, int F> __device__ __forceinline__ T &sum_of_squares(Formed<T, F> &, T &own) { return own; }
+template <typename T, int F> __device__ __forceinline__ T &sum_of_squares(FormedLater<T, F> &o, T &) { return o.acc; }
 
-template <typename T, int METHOD, int CTRL, typename Term>
-__device__ __forceinline__ void form_iteration(const WholeBackward<T> &w, const Term &rhs, const RecordEntry<T, Term::F> &here, const bool running_new, Formed<T, Term::F> &o) {
+template <typename T, int METHOD, typename Term>
+__device__ __forceinline__ void form_stages(const Term &rhs, const RecordEntry<T, Term::F> &here, Formed<T, Term::F> &o) {
     using Tab = typename std::conditional<METHOD == 1, Tsit5Tab, Dopri5Tab>::type;
     constexpr int F = Term::F;
-    constexpr bool SHORT = F * sizeof(T) <= 32;
-    const CtrlParams<T> &cp = w.cp;
-    const T sf = (T)__builtin_sqrt((double)F);
-    const T t0 = here.t, dt = here.dt, prev = here.prev, pprev = here.pprev;
+    const T t0 = here.t, dt = here.dt;
     const T(&y)[F] = here.y;
 #pragma unroll
     for (int f = 0; f < F; ++f) o.k[0][f] = here.k0[f];
@@ -251,11 +255,24 @@ __device__ __forceinline__ void form_iteration(const WholeBackward<T> &w, const 
     }
 #pragma unroll
     for (int f = 0; f < F; ++f) o.y1[f] = o.yi[6][f];
+}
+
+// Returns bounds_outside of all lanes.
+template <typename T, int METHOD, int CTRL, typename Term, typename O>
+__device__ __forceinline__ lanes_t form_errors(const WholeBackward<T> &w, const RecordEntry<T, Term::F> &here, const bool running_new, O &o) {
+    using Tab = typename std::conditional<METHOD == 1, Tsit5Tab, Dopri5Tab>::type;
+    constexpr int F = Term::F;
+    constexpr bool SHORT = F * sizeof(T) <= 32;
+    const CtrlParams<T> &cp = w.cp;
+    const T sf = (T)__builtin_sqrt((double)F);
+    const T dt = here.dt, prev = here.prev, pprev = here.pprev;
+    const T(&y)[F] = here.y;
     using Div = DivSqrtFeatures<T, F>;
     // error ratio and step factor, in the short forms where every lane's operands are in their ranges (control_common's,
     // over a wider range of the errors: their squares may vanish in the sum, as they do in the general form).  A sample
     // that sits through an iteration with a zero step has an error of zero; its controller's results reach nothing.
-    T acc = 0;
+    T own, &acc = sum_of_squares<T, F>(o, own);
+    acc = 0;
     lanes_t outside = 0, bounds_outside = 0;
     unsigned smallest = 0xffffffffu;
     T largest_eb = 0;
@@ -307,6 +324,7 @@ __device__ __forceinline__ void form_iteration(const WholeBackward<T> &w, const 
         }
     }
     o.bounds_outside = holds(bounds_outside);
+    return bounds_outside;
 }
 
 // Coefficients of the dense output's derivative, lowest power first.
@@ -396,7 +414,7 @@ template <typename T, int F> struct HandOver {
 // them, 0.66 -> 0.53 ms; and the waits for what was loaded ahead only where it is used (they stood behind each point's index,
 // and at the end of the iteration behind the copies of the record's entry): 0.53 -> 0.46, float64, B = 20 000, 0.56 -> 0.49.
 // What does not wait for a cotangent -- the stages, the error ratio and the step factor's powers, the dense output's
-// coefficients, 500 of 1800 instructions -- is formed by a second wavefront one iteration ahead (PAIR, form_iteration, HandOver; one
+// coefficients, 500 of 1800 instructions -- is formed by a second wavefront one iteration ahead (PAIR, form_stages, form_errors, HandOver; one
 // barrier of LDS between them an iteration) where the SIMD has an issue slot to spare: 0.45 -> 0.37 ms at B = 65536.
 // What is held for all this costs registers (one wavefront for everything): float32 rows of two take up to 182 (two wavefronts per SIMD; three before), rows of four
 // 256 and 7 to 12 accumulation registers (one; two before), float64 rows of eight all 512 and 800 to 900 bytes of scratch.  It pays all the
@@ -418,6 +436,12 @@ __global__ void __launch_bounds__(PAIR ? 128 : 64) whole_backward_kernel(const W
 #pragma unroll
     for (int j = 0; j < P; ++j) gpar[j] = 0;
 
+    // One wavefront for everything, float64, Tsit5 and PID, systems of several equations with one parameter: the errors are formed
+    // behind the new time instead of right behind the stages.  It is the same arithmetic; what differs is the compiler's allocation,
+    // which elsewhere is the better one with both in one place.  Right behind and later, B = 65 536, us: Van der Pol 482 and 467,
+    // Lorenz 335 and 302; with a rate per value, rows of three and four, 270 and 288, 287 and 297.
+    constexpr bool LATER = !PAIR && sizeof(T) == 8 && METHOD == 1 && CTRL == 1 && F > 1 && P == 1;
+
     const CtrlParams<T> &cp = w.cp;
     const int E = w.E;
     extern __shared__ __align__(16) unsigned char smem_raw[];
@@ -438,7 +462,8 @@ __global__ void __launch_bounds__(PAIR ? 128 : 64) whole_backward_kernel(const W
                 RecordEntry<T, F> before = load_entry<T, F>(w, i > 0 ? i - 1 : 0, g);
                 if ((E == 0 && i == L - 1) || lanes_where(here.running != 0)) {  // (the iterations that the other wavefront asks for)
                     Formed<T, F> formed;
-                    form_iteration<T, METHOD, CTRL, Term>(w, rhs, here, running_new, formed);
+                    form_stages<T, METHOD, Term>(rhs, here, formed);
+                    form_errors<T, METHOD, CTRL, Term>(w, here, running_new, formed);
                     T slope[F][4];
 #pragma unroll
                     for (int f = 0; f < F; ++f) form_slope<T, METHOD, F>(here.dt, here.y, formed.y1, formed.k, f, slope[f]);
@@ -542,14 +567,15 @@ __global__ void __launch_bounds__(PAIR ? 128 : 64) whole_backward_kernel(const W
         T y[F];
 #pragma unroll
         for (int f = 0; f < F; ++f) y[f] = here.y[f];
-        Formed<T, F> o;
+        typename std::conditional<LATER, FormedLater<T, F>, Formed<T, F>>::type o;
         if constexpr (PAIR) {
             lds_barrier();
             hand.read(o);
 #pragma unroll
             for (int f = 0; f < F; ++f) o.k[0][f] = here.k0[f];
         } else {
-            form_iteration<T, METHOD, CTRL, Term>(w, rhs, here, running_new, o);
+            form_stages<T, METHOD, Term>(rhs, here, o);
+            if constexpr (!LATER) form_errors<T, METHOD, CTRL, Term>(w, here, running_new, o);
         }
         const T(&k)[7][F] = o.k, (&y1)[F] = o.y1;
 
@@ -559,9 +585,11 @@ __global__ void __launch_bounds__(PAIR ? 128 : 64) whole_backward_kernel(const W
         T g_t, g_dt, g_prev = 0, g_pprev = 0, g_h, g_lo, g_hi, g_k[7][F], g_y[F], g_y1[F];
         {
             using Div = DivSqrtFeatures<T, F>;
+            lanes_t bounds_outside;
+            if constexpr (LATER) bounds_outside = form_errors<T, METHOD, CTRL, Term>(w, here, running_new, o);
+            else bounds_outside = lanes_where(o.bounds_outside);
             const T(&err)[F] = o.err, (&eb)[F] = o.eb, (&per_eb)[F] = o.per_eb, (&q)[F] = o.q, (&x)[F] = o.x;
             const T r = o.r, ratio = o.ratio, F0 = o.F0;
-            lanes_t bounds_outside = lanes_where(o.bounds_outside);
             // Quotients of cotangents: the divisors' ranges are known, the dividends are looked at.  divisors_outside: lanes
             // (of those that take part) whose divisor is outside.
             const T per_ratio = reciprocal_estimate(ratio);
