@@ -507,8 +507,9 @@ class AutoDiffAdjoint(nn.Module):
                 for i in range(1, n_stages):
                     if watch and stopped_on_device[0]:
                         return  # (the loop has ended on the device: what is left of this iteration would do nothing)
-                    # (buffers, launch and addresses in one native call: 3 us of host time a stage less than as calls of their own,
-                    # where an evaluation of some eight torch operations takes 35: user's Van der Pol, B = 4096, 29.0 -> 27.1 ms)
+                    # (buffers, launch and addresses in one native call: between two evaluations 8.6 -> 5.6 us of host time, where an
+                    # evaluation of some eight torch operations takes 28 to 36 by the process: user's Van der Pol, B = 4096, 537
+                    # stages, 29.2 -> 27.4 ms in processes where it takes 36)
                     tt, yy = stage(state_at, controller_at, i, y, t, slope, stream.value)
                     keep["t", i], keep["y", i], keep["k", i] = tt, yy, rhs(tt, yy)
                     slope = keep["k", i]

@@ -415,7 +415,7 @@ template <typename T, int F> struct HandOver {
 // and at the end of the iteration behind the copies of the record's entry): 0.53 -> 0.46, float64, B = 20 000, 0.56 -> 0.49.
 // What does not wait for a cotangent -- the stages, the error ratio and the step factor's powers, the dense output's
 // coefficients, 500 of 1800 instructions -- is formed by a second wavefront one iteration ahead (PAIR, form_stages, form_errors, HandOver; one
-// barrier of LDS between them an iteration) where the SIMD has an issue slot to spare: 0.45 -> 0.37 ms at B = 65536.
+// barrier of LDS between them an iteration) where the SIMD has an issue slot to spare: 0.45 -> 0.355 ms at B = 65536.
 // What is held for all this costs registers (one wavefront for everything): float32 rows of two take up to 182 (two wavefronts per SIMD; three before), rows of four
 // 256 and 7 to 12 accumulation registers (one; two before), float64 rows of eight all 512 and 800 to 900 bytes of scratch.  It pays all the
 // same where a SIMD has wavefronts to choose from.  Backward passes, before and now: Van der Pol float32, B = 262 144, 2.41 -> 1.11 ms,
@@ -448,9 +448,9 @@ __global__ void __launch_bounds__(PAIR ? 128 : 64) whole_backward_kernel(const W
     HandOver<T, F> hand(smem_raw);
     if constexpr (PAIR) {
         static_assert(SHORT, "built for the short forms");
-        // The group's first wavefront forms; for rows of four doubles the second one.  Which of them does matters where groups share
-        // a compute unit -- roles that took turns by the group's number had the users of two groups on one SIMD there -- and to the
-        // registers the compiler chooses.  Taking turns and so, us: Van der Pol float32, 512 groups, 340 and 322, 768 339 and 316, 1024
+        // The group's first wavefront forms; for rows of four doubles the second one.  Which of them does was measured to matter where
+        // groups share a compute unit, and to the registers the compiler chooses; roles that take turns by the group's number are
+        // slower (which SIMDs two groups' wavefronts share is not known here).  Taking turns and so, us: Van der Pol float32, 512 groups, 340 and 322, 768 339 and 316, 1024
         // 360 and 355; float64, 256 387 and 389, 313 468 and 400, 511 484 and 431.  Decay, rows of four doubles, first and second
         // wavefront: 5 groups 178 and 172, 256 187 and 183, 511 199 and 196.
         constexpr unsigned FORMS = F * sizeof(T) == 32 ? 1 : 0;
@@ -887,10 +887,11 @@ static int launch_backward(const tode_solve_args &a, const tode_controller &c, c
     w.through_start = adj.through_start, w.dt0_given = a.dt0 != nullptr;
     w.ts_stride = a.t_start_stride, w.te_stride = a.t_end_stride;
     // Two wavefronts to a group while a SIMD has no second group to issue for: up to one group per SIMD in float32, half of that in
-    // float64, whose hand-over takes twice the LDS (rows of four: 70 KB, two groups to a compute unit).  Kernel in us, one
-    // wavefront and two: Van der Pol float32, Tsit5 + PID, B = 300 367 and 305, 16 384 372 and 310, 65 536 408 and 355 (at 100 000
-    // two would share the SIMD with two more); Lorenz float32 60 000 194 and 163; decay, rows of four, 60 000 217 and 206;
-    // float64: Van der Pol 300 396 and 332, 32 768 426 and 414, 65 536 457 and 464; Lorenz 16 384 216 and 176, 32 768 226 and 187.
+    // float64, whose hand-over takes twice the LDS (rows of four: 70 KB, two groups to a compute unit).  Kernel in us with Tsit5 and
+    // PID, one wavefront and two: Van der Pol float32, 5 groups 390 and 322, 256 375 and 311, 512 388 and 314, 1024 455 and 356,
+    // beyond the line 1280 450 and 417, 2048 544 and 720; Lorenz float32, 938 206 and 158, beyond it 1563 227 and 298; decay, rows of
+    // four, 938 170 and 147, beyond it 1563 320 and 278.  float64: Van der Pol 256 531 and 391, 511 552 and 418, beyond it 1024 535 and 500;
+    // Lorenz 511 288 and 195, 1024 297 and 363; decay, rows of four, 511 253 and 197, 1024 265 and 380.
     const long long groups = (B + 63) / 64;
     constexpr bool paired = Term::F <= 4;
     if (paired && groups <= TODE_PAIRED_SWEEP_GROUPS * 4 / (long long)sizeof(T))

@@ -1,9 +1,9 @@
 // torchode_amd._host: what AutoDiffAdjoint.solve does around the kernel of a whole solve with a built-in term -- the argument
 // block from the problem's tensors, the outputs from PyTorch's allocator, the launch, the views of the statistics while
 // the kernel runs, and the wait -- as one call of a Python extension.  A small solve's kernel takes 25 to 75 microseconds, and
-// the same steps in Python, one ctypes or tensor call each, took 23 ahead of the launch where they now take 9 (decay, float64, B = 256: 53 -> 42.6 us a
-// solve; Lorenz to its end point, B = 40 009: 79 -> 69; perceptron, B = 4096: 108 -> 92).  No solver logic and no kernel: everything here ends in the C ABI of include/torchode_amd.h, and nothing is
-// kept from one call for the next.
+// the same steps in Python, one ctypes or tensor call each, took 23 ahead of the launch where they now take 9 (decay, float64,
+// B = 256: 52 -> 40 us a solve; Lorenz to its end point, B = 40 009: 80 -> 67; perceptron, B = 4096: 109 -> 91).  No solver logic and
+// no kernel: everything here ends in the C ABI of include/torchode_amd.h, and nothing is kept from one call for the next.
 #include <Python.h>
 
 #include <ATen/ATen.h>

@@ -5,7 +5,9 @@
 //
 //   mlp_stages_kernel           all six stages of an iteration again (a tile of 16 samples per workgroup, laid out as in
 //                               the whole-solve kernel), keeping stage inputs, derivatives and hidden activations; of all
-//                               iterations in one launch where their rows fit, since they depend on the record alone;
+//                               iterations in one launch where their rows fit, since they depend on the record alone, and
+//                               then the sums of the squares of the scaled errors for the sweep of a whole record as well;
+//   mlp_sweep_control_kernel    ahead of that sweep: an iteration's step factor and the points it wrote, a thread each;
 //   mlp_stages_backward_kernel  the six stages in reverse: the network's vector-Jacobian product and the stage sums' reverse,
 //                               the cotangents of all stage derivatives in registers between them;
 //   mlp_sweep_kernel            the iterations of a whole record in reverse, where the times want no gradient and the rows of all
@@ -19,8 +21,10 @@
 // matrix cores are busy 10.6 and 10.2 us -- the rest are the round trips through LDS between two products, the stage sums and
 // 150 KB of weights loaded per workgroup; the outer products of 20 evaluations 69 us (34 us of matrix instructions at 2.4 GHz,
 // 200 MB of rows at 2.9 TB/s).  A solve and its backward pass: 9.75 ms through autograd, 0.61 to 0.80 ms by the host's speed with the
-// launches per iteration (0.42 ms of kernels), 0.46 in the one kernel, one call of it and one launch for
-// the weights (0.37 ms).
+// launches per iteration (0.42 ms of kernels), 0.46 to 0.54 in the one kernel, one call of it and one launch for
+// the weights (0.38 ms).  Against float64 over the same record, 60 solves with rows shorter than 64, the one kernel and
+// the launches per iteration (geometric means): y0 4.5e-7 and 4.6e-7, W1 8.5e-7 and 8.6e-7 with the steps held constant; y0 4.8e-5 and
+// 4.8e-5, W1 1.00e-5 and 1.01e-5 through the step sizes.
 //
 // All products are on v_mfma_f32_16x16x4_f32.  For the vector-Jacobian product the weights are packed a second time,
 // transposed (tode_mlp_pack_weights_reverse), so that the same two facts hold as in the forward kernel: every lane keeps its

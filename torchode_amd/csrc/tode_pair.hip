@@ -14,8 +14,8 @@
 //     interpolant and writes the evaluation points the step passed, while the
 //     stepper is already computing the next step.
 // Records are double-buffered; one s_barrier per loop iteration orders the
-// hand-over.  Stepper and evaluator roles alternate between neighbouring
-// workgroups so that every SIMD hosts one of each.
+// hand-over.  Stepper and evaluator roles alternate between neighbouring pairs of
+// workgroups, meant to give every SIMD one of each.
 //
 // In the smallest batches a sample's features get a lane each (the ...Lanes systems of tode_solve.h), 64 / L samples per
 // wavefront: the same kernel with one feature per lane.
